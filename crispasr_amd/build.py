@@ -4,6 +4,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -66,6 +67,21 @@ def build_host_driver() -> str:
     return HOST_BIN
 
 
+VIEWS_SRC = os.path.join(HERE, "host", "ggml_views.cpp")
+VIEWS_LIB = os.path.join(HERE, "_host.so")
+
+
+def build_host_module() -> str:
+    """The native host path of ggml.py: a CPython extension (plain g++; it is handed the library's entry points at run time)."""
+    cmd = ["g++", "-O2", "-std=c++17", "-Wall", "-Wno-missing-field-initializers", "-fPIC", "-shared", "-I", sysconfig.get_paths()["include"],
+           VIEWS_SRC, "-o", VIEWS_LIB]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("host module build failed:\n" + res.stderr)
+    return VIEWS_LIB
+
+
 if __name__ == "__main__":
     print(build_library(sys.argv[1:]))
+    print(build_host_module())
     print(build_host_driver())

@@ -68,24 +68,18 @@ bool is_contiguous(const mi355x_tensor * t) {
     return true;
 }
 
-struct DeviceCache {
-    int  cus = 0;
-    bool init = false;
-};
-DeviceCache g_dev[64];
-std::mutex  g_mu;
+std::atomic<int> g_cus[64];         // per device: 0 until looked up (racing callers write the same number)
+std::mutex       g_mu;
 
 int device_cus() {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    std::lock_guard<std::mutex> lk(g_mu);
-    if (!g_dev[dev].init) {
-        int cus = 0;
+    int cus = g_cus[dev].load(std::memory_order_relaxed);
+    if (cus == 0) {
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-        g_dev[dev].cus  = cus;
-        g_dev[dev].init = true;
+        g_cus[dev].store(cus, std::memory_order_relaxed);
     }
-    return g_dev[dev].cus;
+    return cus;
 }
 
 // Extents a kernel can index: none negative, each below 2^31, their product below 2^62 (n = that product).
@@ -447,11 +441,13 @@ void fill_args(FattnArgs & a, const mi355x_tensor * q, const mi355x_tensor * k, 
     a.softcap = p->logit_softcap;
     a.scale   = p->logit_softcap != 0.0f ? p->scale / p->logit_softcap : p->scale;
     a.max_bias = p->max_bias;
-    // ALiBi slope bases, as ggml derives them from the head count
-    const uint32_t n2 = 1u << (uint32_t)floorf(log2f((float)a.Hq));
-    a.n_head_log2 = (int)n2;
-    a.m0 = powf(2.0f, -(p->max_bias) / n2);
-    a.m1 = powf(2.0f, -(p->max_bias / 2.0f) / n2);
+    if (p->max_bias > 0.0f) {
+        // ALiBi slope bases, as ggml derives them from the head count
+        const uint32_t n2 = 1u << (uint32_t)floorf(log2f((float)a.Hq));
+        a.n_head_log2 = (int)n2;
+        a.m0 = powf(2.0f, -(p->max_bias) / n2);
+        a.m1 = powf(2.0f, -(p->max_bias / 2.0f) / n2);
+    }
     a.n_splits = 1;
     a.keys_per_split = a.Nkv;
     a.part_acc = a.part_ml = nullptr;
@@ -490,11 +486,11 @@ void make_plan_core(const FattnArgs & a0, int ktype, int vtype, const mi355x_fat
         // 18.0 -> 14.3 us; 24 x 300, 8 heads: 14.2 -> 10.9 us; at 407 x 407, 816 chunks, the tile kernel wins 29 to 31).
         // With f16 K/V the two are within a microsecond of each other and the tile kernel keeps the shape.
         const int64_t chunk_wgs = (int64_t)a.q_chunks * a.Hkv * a.B;
-        bool          chunked   = ktype == MI355X_TYPE_Q8_0 && chunk_wgs <= 2 * (int64_t)device_cus() && a.Nkv <= 1024;
+        bool          chunked   = ktype == MI355X_TYPE_Q8_0 && chunk_wgs <= 2 * (int64_t)a.n_cus && a.Nkv <= 1024;
         // (f16: only the smallest calls - up to one chunk per CU against 64 keys, or 256 keys at 64-wide heads - where the
         //  decode kernel's single round is 1 to 2 us shorter than the tile kernel's 6 to 9: 64 queries x 32 q / 8 kv heads
         //  against 256 keys 8.8 -> 6.9 us)
-        if (ktype == MI355X_TYPE_F16 && a.q_chunks > 1 && chunk_wgs <= device_cus() && (a.Nkv <= 64 || (a.D == 64 && a.Nkv <= 256)))
+        if (ktype == MI355X_TYPE_F16 && a.q_chunks > 1 && chunk_wgs <= a.n_cus && (a.Nkv <= 64 || (a.D == 64 && a.Nkv <= 256)))
             chunked = true;
         // A longer Q8_0 cache under fewer than 128 queries: the tile kernel would dequantise every tile in its loop, once per
         // query head (1.7 us per 64-key tile at 64-wide heads, 2.1 at 128-wide; 5 sequences x 32 q / 8 kv heads x 16 queries
@@ -502,7 +498,7 @@ void make_plan_core(const FattnArgs & a0, int ktype, int vtype, const mi355x_fat
         // after its own key split, the decode kernel's chunks x keys at its measured rate - and the decode kernel has to
         // win by 1.4 (its rate drops with a mask row per query row).
         if (!chunked && ktype == MI355X_TYPE_Q8_0 && a.q_chunks > 1 && a.Nq < 128 && a.Nkv > 1024) {
-            const int     cus     = device_cus();
+            const int     cus     = a.n_cus;
             const int     n_tiles = (a.Nkv + 63) / 64;
             const int64_t wgs     = (int64_t)a.Hq * a.B;
             int ns = 1;
@@ -598,7 +594,7 @@ void make_plan_core(const FattnArgs & a0, int ktype, int vtype, const mi355x_fat
             //  cut in two, are cut towards two workgroups per CU in ranges of at least 16 tiles: 256 queries x 40 heads of
             //  128 against 8192 keys, 160 workgroups, 146 -> 81 us in 3 ranges; the Whisper-base encoder's 24 tiles stay whole.)
             ns = 1;
-            const int cus = device_cus();
+            const int cus = a.n_cus;
             // (the key-split form of 64-wide heads without a mask walks tiles of 128 keys and more)
             const int nt = var.key_split == 2 && a.D == 64 && !a.masked ? (a.Nkv + 127) / 128 : n_tiles;
             if (wgs * 4 <= cus) {
@@ -637,7 +633,7 @@ void make_plan_core(const FattnArgs & a0, int ktype, int vtype, const mi355x_fat
         const int     min_keys = kernel == MI355X_FATTN_VEC ? (a.D > 64 ? (a.Nkv > 448 ? 112 : 56) : 128) : (a.D <= 64 ? 128 : 64);
         int ns = p->n_splits;
         if (ns <= 0) {
-            const int64_t target = kernel == MI355X_FATTN_VEC ? (int64_t)device_cus() * 3 / 2 : (int64_t)device_cus() * 2;
+            const int64_t target = kernel == MI355X_FATTN_VEC ? (int64_t)a.n_cus * 3 / 2 : (int64_t)a.n_cus * 2;
             // whole splits only while they still fit the target: past it a split doubles the grid and adds the merge
             ns = kernel == MI355X_FATTN_VEC ? (int)((target + groups - 1) / (groups > 0 ? groups : 1))
                                             : (int)(target / (groups > 0 ? groups : 1));
@@ -671,22 +667,21 @@ void make_plan_core(const FattnArgs & a0, int ktype, int vtype, const mi355x_fat
                 double t_hbm = ((double)a.Hkv * a.B * a.Nkv *
                                 (double)(a.D / block_size(ktype) * type_size(ktype) + a.D / block_size(vtype) * type_size(vtype)) - 8.0e6) / 5.0e6;
                 if (t_hbm < 0.0) t_hbm = 0.0;       // (the first megabytes are a matter of latency, which the chain prices)
-                double best = 1e30;
-                int    pick = ns;
-                for (int pass = 0; pass < 2; pass++)
-                    for (int n = 1; n <= ns; n++) {
-                        const int kps_n = ((a.Nkv + n - 1) / n + 31) / 32 * 32;
-                        if ((a.Nkv + kps_n - 1) / kps_n != n) continue;             // not a count that whole steps give
-                        double chain = kps_n / 128.0;
-                        if (chain < 1.0) chain = 1.0;
-                        chain *= a.D <= 64 ? 0.7 : 1.3;
-                        const double per_cu = (double)groups * n / device_cus();     // workgroups sharing a CU share its steps
-                        if (per_cu > 1.0) chain *= per_cu;
-                        const double est = (chain > t_hbm ? chain : t_hbm) + (n > 1 ? 1.0 + n * per : 0.0);
-                        if (pass == 0) { if (est < best) best = est; }
-                        else if (est <= best * 1.10) pick = n;
-                    }
-                ns = pick;
+                double best = 1e30, est[257];
+                if (ns > 256) ns = 256;
+                for (int n = 1; n <= ns; n++) {
+                    const int kps_n = ((a.Nkv + n - 1) / n + 31) / 32 * 32;
+                    est[n] = 2e30;
+                    if ((a.Nkv + kps_n - 1) / kps_n != n) continue;             // not a count that whole steps give
+                    double chain = kps_n / 128.0;
+                    if (chain < 1.0) chain = 1.0;
+                    chain *= a.D <= 64 ? 0.7 : 1.3;
+                    const double per_cu = (double)groups * n / a.n_cus;     // workgroups sharing a CU share its steps
+                    if (per_cu > 1.0) chain *= per_cu;
+                    est[n] = (chain > t_hbm ? chain : t_hbm) + (n > 1 ? 1.0 + n * per : 0.0);
+                    if (est[n] < best) best = est[n];
+                }
+                while (ns > 1 && est[ns] > best * 1.10) ns--;
             }
         }
         if (ns > a.Nkv) ns = a.Nkv;
@@ -738,7 +733,7 @@ void make_plan(const FattnArgs & a0, int ktype, int vtype, const mi355x_fattn_pa
                 dec = true;
             } else if (!dec) {
                 const int64_t chunk_wgs = (int64_t)a0.q_chunks * a0.Hkv * a0.B;
-                dec = a0.q_chunks <= 64 && chunk_wgs <= 3 * (int64_t)device_cus() &&
+                dec = a0.q_chunks <= 64 && chunk_wgs <= 3 * (int64_t)a0.n_cus &&
                       (int64_t)a0.q_chunks * a0.Nkv <= (1 << 16) && chunk_wgs * a0.Nkv <= (1 << 19);
             }
             if (dec && plan.kernel != MI355X_FATTN_DECODE_MMA) {

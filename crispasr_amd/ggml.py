@@ -8,6 +8,9 @@ src/crispasr.cpp:2821, 3220, 3280; src/core/attention.h:992; src/core/fastconfor
 ``ggml_cpy`` (src/crispasr.cpp:2810-2811) and ``ggml_set_rows`` (src/core/attention.h:366-376)
 in the reference.  All arithmetic happens in libmi355x_fattn.so; torch only owns the device
 memory and the stream.  There is no CPU fallback: without the built library every op raises.
+
+What runs once per call or view is native (host/ggml_views.cpp, built as _host.so): a decoder step makes a few
+hundred of them around a few microseconds of GPU work each.
 """
 from __future__ import annotations
 
@@ -17,6 +20,11 @@ from typing import Optional, Sequence
 
 import numpy as np
 import torch
+
+try:
+    from . import _host
+except ImportError as e:
+    raise RuntimeError("crispasr_amd/_host.so is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'`") from e
 
 F32, F16, Q4_0, Q4_1, Q5_0, Q5_1, Q8_0 = 0, 1, 2, 3, 6, 7, 8
 QK8_0 = 32
@@ -140,8 +148,20 @@ def lib() -> ctypes.CDLL:
             fn = getattr(L, name)
             if name not in ("mi355x_status_string", "mi355x_last_error"):
                 fn.restype = ctypes.c_int
+        at = lambda name: ctypes.cast(getattr(L, name), ctypes.c_void_p).value
+        _host.bind({name: at(name) for name in
+                    ("mi355x_flash_attn_ext", "mi355x_flash_attn_ext_noalloc", "mi355x_cpy", "mi355x_set_rows", "mi355x_relpos_bias",
+                     "mi355x_flash_attn_relpos", "hipGetDevice", "hipSetDevice")},
+                   _failed, torch._C._cuda_getCurrentRawStream)
         _lib = L
     return _lib
+
+
+def _failed(status: int, message: Optional[str] = None) -> None:
+    """what the native host path calls with a status that is not OK: raises"""
+    if message is None:
+        _check(status)
+    raise InvalidError(status, message)
 
 
 def _check(status: int) -> None:
@@ -202,19 +222,13 @@ class HostBuffer:
             self.ptr = None
 
 
-class Tensor:
-    """A ggml tensor (or view) living in a device buffer (a torch uint8 tensor) or in a HostBuffer."""
+_host.types(HostBuffer, _failed, torch.uint8, torch.int32, torch.int64)
 
-    def __init__(self, buf, type_: int, ne: Sequence[int],
-                 nb: Optional[Sequence[int]] = None, offset: int = 0):
-        self.buf = buf                      # 1-D uint8 device tensor, a HostBuffer, or None (planning only)
-        self.type = int(type_)
-        self.ne = tuple(int(x) for x in ne) + (1,) * (4 - len(ne))
-        self.nb = tuple(int(x) for x in (nb if nb is not None else contiguous_nb(self.type, self.ne)))
-        self.offset = int(offset)
-        self._c = None                      # the C descriptor, built once: a view never changes
-        if buf is not None and not isinstance(buf, HostBuffer):
-            assert buf.dtype == torch.uint8 and buf.dim() == 1 and buf.is_contiguous()
+
+class Tensor(_host.View):
+    """Tensor(buf, type_, ne, nb=None, offset=0): a ggml tensor (or view) living in a device buffer (a 1-D torch uint8 tensor),
+    in a HostBuffer, or nowhere yet (None: planning only).  Attributes buf, type, ne (always 4 extents), nb, offset; a view
+    does not change once a call has used it.  Base class: view(ne, nb, offset=0, type_=None), span(), data_ptr()."""
 
     # -- construction ---------------------------------------------------------------------
     @staticmethod
@@ -241,41 +255,16 @@ class Tensor:
         buf.array[:raw.size] = raw
         return Tensor(buf, type_, ne, nb, offset)
 
-    def view(self, ne, nb, offset: int = 0, type_: Optional[int] = None) -> "Tensor":
-        """ggml_view_{1,2,3,4}d: same buffer, new extents/strides, offset relative to this view"""
-        return Tensor(self.buf, self.type if type_ is None else type_, ne, nb, self.offset + offset)
-
     # -- access -----------------------------------------------------------------------------
-    def span(self) -> int:
-        if any(n == 0 for n in self.ne):
-            return 0
-        last = (self.ne[0] // BLOCK_SIZE[self.type] - 1) * self.nb[0]
-        last += sum((self.ne[i] - 1) * self.nb[i] for i in (1, 2, 3))
-        return last + TYPE_SIZE[self.type]
-
-    def data_ptr(self) -> int:
-        if self.buf is None:
-            # planning before allocation: the predicates never dereference, they only look at the address's low bits
-            # (buffers start on 256 bytes, so the view's offset modulo 256 stands for them)
-            return self.offset % 256
-        if self.offset + self.span() > self.buf.numel():
-            raise InvalidError(ERR_INVALID, "tensor view exceeds its buffer")
-        return self.buf.data_ptr() + self.offset
-
     def c(self) -> CTensor:
-        if self._c is None:
-            t = CTensor()
-            t.data = self.data_ptr()
-            t.type = self.type
-            t.ne = (ctypes.c_int64 * 4)(*self.ne)
-            t.nb = (ctypes.c_size_t * 4)(*self.nb)
-            self._c = (t, ctypes.byref(t))
-        return self._c[0]
+        """the C descriptor, in the view's own memory"""
+        t = CTensor.from_address(self._descriptor())
+        t._view = self
+        return t
 
     def ref(self):
         """pointer to the C descriptor, as the entry points take it"""
-        self.c()
-        return self._c[1]
+        return ctypes.byref(self.c())
 
     def to_host(self) -> np.ndarray:
         """ggml_backend_tensor_get of the whole underlying buffer (uint8)"""
@@ -292,25 +281,6 @@ class Tensor:
         else:
             raw = self.buf[self.offset:self.offset + 4 * n].cpu().numpy()
         return raw.view(np.float32).reshape(self.ne[3], self.ne[2], self.ne[1], self.ne[0]).copy()
-
-
-class _NoSwitch:
-    def __enter__(self):
-        return None
-
-    def __exit__(self, *exc):
-        return False
-
-
-_NO_SWITCH = _NoSwitch()
-
-
-def _on_device(device):
-    """make `device` current for the call; no context switch when it already is"""
-    idx = device.index
-    if idx is None or idx == torch.cuda.current_device():
-        return _NO_SWITCH
-    return torch.cuda.device(device)
 
 
 def _stream_handle(stream) -> int:
@@ -394,13 +364,12 @@ def flash_attn_ext(q: Tensor, k: Tensor, v: Tensor, mask: Optional[Tensor], scal
     immediately reshape_2d to [DV*Hq, Nq])."""
     if out is None:
         out = Tensor.empty(F32, (v.ne[0], q.ne[2], q.ne[1], q.ne[3]), device=q.buf.device)
-    p = _params(scale, max_bias, logit_softcap, prec, kernel, n_splits, workspace, q_quant, tile_variant)
+    if _lib is None:
+        lib()
     # no_alloc: the entry point that takes its scratch from the library's static device array (pass `out`: the result
     # tensor is the caller's to provide there)
-    entry = lib().mi355x_flash_attn_ext_noalloc if no_alloc else lib().mi355x_flash_attn_ext
-    with _on_device(q.buf.device):
-        _check(entry(q.ref(), k.ref(), v.ref(), mask.ref() if mask is not None else None,
-                     out.ref(), ctypes.byref(p), _stream_handle(stream)))
+    _host.flash_attn_ext(q, k, v, mask, out, scale, max_bias, logit_softcap, prec, kernel, n_splits, workspace, stream,
+                         q_quant, tile_variant, no_alloc)
     return out
 
 
@@ -419,11 +388,9 @@ def relpos_bias(q_v: Tensor, r: Tensor, add: Optional[Tensor], scale: float, n_k
         if n_kv is None:
             n_kv = r.ne[1] - q_v.ne[1] + 1
         out = Tensor.empty(F16, (n_kv, q_v.ne[1], q_v.ne[2], q_v.ne[3]), device=q_v.buf.device)
-    with _on_device(q_v.buf.device):
-        _check(lib().mi355x_relpos_bias(q_v.ref(), r.ref(), add.ref() if add is not None else None, out.ref(),
-                                        float(scale), workspace.data_ptr() if workspace is not None else None,
-                                        workspace.numel() * workspace.element_size() if workspace is not None else 0,
-                                        _stream_handle(stream)))
+    if _lib is None:
+        lib()
+    _host.relpos_bias(q_v, r, add, out, scale, workspace, stream)
     return out
 
 
@@ -434,11 +401,9 @@ def flash_attn_relpos(q_u: Tensor, q_v: Tensor, k: Tensor, v: Tensor, r: Tensor,
     softmax(scale * (q_u.k^T + rel_shift(q_v.r^T)) + add) . v, result ne = [DV, H, Nq, B]."""
     if out is None:
         out = Tensor.empty(F32, (v.ne[0], q_u.ne[2], q_u.ne[1], q_u.ne[3]), device=q_u.buf.device)
-    p = _params(scale, 0.0, 0.0, PREC_DEFAULT, kernel, n_splits, workspace)
-    with _on_device(q_u.buf.device):
-        _check(lib().mi355x_flash_attn_relpos(q_u.ref(), q_v.ref(), k.ref(), v.ref(), r.ref(),
-                                              add.ref() if add is not None else None, out.ref(), ctypes.byref(p),
-                                              _stream_handle(stream)))
+    if _lib is None:
+        lib()
+    _host.flash_attn_relpos(q_u, q_v, k, v, r, add, out, scale, kernel, n_splits, workspace, stream)
     return out
 
 
@@ -453,9 +418,9 @@ def flash_attn_relpos_workspace_size(q_u: Tensor, q_v: Tensor, k: Tensor, v: Ten
 
 def cpy(src: Tensor, dst: Tensor, stream=None) -> Tensor:
     """ggml_cpy(ctx, src, dst): convert src's elements into dst's type and layout"""
-    cs, cd = src.c(), dst.c()
-    with torch.cuda.device(dst.buf.device):
-        _check(lib().mi355x_cpy(ctypes.byref(cs), ctypes.byref(cd), _stream_handle(stream)))
+    if _lib is None:
+        lib()
+    _host.cpy(src, dst, stream)
     return dst
 
 
@@ -468,15 +433,9 @@ def set_rows_supports(dst: Tensor, src: Tensor, n_idx: Sequence[int], idx_bits: 
 def set_rows(dst: Tensor, src: Tensor, idx: torch.Tensor, stream=None) -> Tensor:
     """ggml_set_rows(ctx, dst, src, idx): dst[:, idx[i], ...] = src[:, i, ...]; idx int64/int32 device tensor
     of shape [n_rows] (or [I2, I1, n_rows] in numpy order, broadcast over dims 2 and 3)"""
-    assert idx.dtype in (torch.int64, torch.int32) and idx.is_contiguous()
-    shape = (1,) * (3 - idx.dim()) + tuple(idx.shape)
-    ine = (ctypes.c_int64 * 3)(shape[2], shape[1], shape[0])
-    es = idx.element_size()
-    inb = (ctypes.c_size_t * 3)(es, es * shape[2], es * shape[2] * shape[1])
-    cs, cd = src.c(), dst.c()
-    with torch.cuda.device(dst.buf.device):
-        _check(lib().mi355x_set_rows(ctypes.byref(cs), idx.data_ptr(), 64 if idx.dtype == torch.int64 else 32,
-                                     ine, inb, ctypes.byref(cd), _stream_handle(stream)))
+    if _lib is None:
+        lib()
+    _host.set_rows(dst, src, idx, stream)
     return dst
 
 
