@@ -1,12 +1,12 @@
 // GGML_OP_CPY / CONT / DUP / SET_ROWS with the destination in device memory: the KV-cache
 // writes that feed FLASH_ATTN_EXT (src/crispasr.cpp:2810-2811, 3185-3203, 2956-2973;
 // src/core/attention.h:342-378) and the dequantising reads (src/core/attention.h:917-920).
-// HBM-bound byte work: one element (or one element of a block of 32) per lane, coalesced along
-// dimension 0.  Source and destination may have different shapes with equal element
+// HBM-bound byte work, 8 elements per lane wherever rows allow it, coalesced along dimension 0.  Source and destination may have different shapes with equal element
 // counts (the reference copies a [n_state, n_ctx] tensor into a 1-D cache view).
 #include "fattn_common.h"
 
 #include <string.h>
+#include <type_traits>
 
 // The quantisers must round every product and every sum on its own, as the reference's scalar code does: hipcc's default
 // contraction turns x * id + c into one fused multiply-add (so do __fmul_rn / __fadd_rn, which inline as contractible), and
@@ -15,186 +15,282 @@
 
 namespace {
 
-// byte offset of unit i, where a unit is `unit0` elements along dimension 0 and one step of
-// nb[0] covers `per_nb0` elements (32 for a Q8_0 tensor, 1 otherwise)
-__device__ __forceinline__ int64_t offset_of(int64_t i, const int64_t (&ne)[4], const int64_t (&nb)[4],
-                                             int64_t unit0, int64_t per_nb0 = 1) {
-    const int64_t n0 = ne[0] / unit0;
-    const int64_t i0 = i % n0;  i /= n0;
-    const int64_t i1 = i % ne[1]; i /= ne[1];
-    const int64_t i2 = i % ne[2];
-    const int64_t i3 = i / ne[2];
-    return i0 * (unit0 / per_nb0) * nb[0] + i1 * nb[1] + i2 * nb[2] + i3 * nb[3];
+// Which element a thread works on: unit i of `unit0` elements each -> its place along the four dimensions.
+// I = uint32_t (up to 2^31 units): divisions by multiply and shift, four instructions each.  In 64-bit arithmetic the six
+// divisions of a copy are loops of a hundred instructions each and most of a small launch's time (the 5 x 1280 values of a
+// decoder step into their F16 cache: 2.87 us with them, 1.92 without; a token's rows into a Q8_0 cache 2.94 -> 1.96; a
+// dequantising read of 663 x 8 rows of 128 4.8 -> 3.2: the shortest launch takes about 1.3).
+struct Place {
+    int64_t i0, i1, i2, i3;                 // i0 in units
+};
+template <typename I>
+__device__ __forceinline__ Place place_of(I i, const int64_t (&ne)[4], const FastDiv (&div)[3], int64_t unit0) {
+    Place p;
+    if constexpr (sizeof(I) == 4) {
+        const uint32_t r1 = divide(i, div[0]), r2 = divide(r1, div[1]), r3 = divide(r2, div[2]);
+        p.i0 = i - r1 * div[0].d;
+        p.i1 = r1 - r2 * div[1].d;
+        p.i2 = r2 - r3 * div[2].d;
+        p.i3 = r3;
+    } else {
+        const int64_t n0 = ne[0] / unit0;
+        p.i0 = i % n0;    i /= n0;
+        p.i1 = i % ne[1]; i /= ne[1];
+        p.i2 = i % ne[2];
+        p.i3 = i / ne[2];
+    }
+    return p;
 }
+// its byte offset; step0 = bytes from one unit to the next along dimension 0
+__device__ __forceinline__ int64_t offset_at(const Place & p, const int64_t (&nb)[4], int64_t step0) {
+    return p.i0 * step0 + p.i1 * nb[1] + p.i2 * nb[2] + p.i3 * nb[3];
+}
+template <typename I>
+__device__ __forceinline__ void both_places(const CpyArgs & a, I i, int64_t unit0, Place & s, Place & d) {
+    s = place_of<I>(i, a.sne, a.sdiv, unit0);
+    d = s;
+    if (!a.same_shape) d = place_of<I>(i, a.dne, a.ddiv, unit0);
+}
+template <typename I> __device__ __forceinline__ I thread_index() { return (I)blockIdx.x * 256 + threadIdx.x; }
 
-template <typename TS, typename TD>
+template <typename I, typename TS, typename TD>
 __global__ void __launch_bounds__(256) cpy_scalar_kernel(const CpyArgs a) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= a.n) return;
-    const TS x = *(const TS *)(a.src + offset_of(i, a.sne, a.snb, 1));
-    char * dp = a.dst + offset_of(i, a.dne, a.dnb, 1);
+    const I i = thread_index<I>();
+    if (i >= (I)a.n) return;
+    Place sp, tp;
+    both_places<I>(a, i, 1, sp, tp);
+    const TS x = *(const TS *)(a.src + offset_at(sp, a.snb, a.snb[0]));
+    char * dp = a.dst + offset_at(tp, a.dnb, a.dnb[0]);
     *(TD *)dp = (TD)x;                                          // f32 -> f16 is round-to-nearest-even
     if (a.mirror) *(TD *)(dp + a.mirror) = (TD)x;
 }
 
+template <typename T> using Vec8 = T __attribute__((ext_vector_type(8)));
+template <typename T> using Vec4 = T __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+
 // 8 consecutive elements of dimension 0 per lane: 128-bit loads and stores for f16 <-> f32 and same-type copies.
 // Launched only when both sides have ne0 % 8 == 0, unit element stride and 16-byte aligned rows.
-template <typename TS, typename TD>
+template <typename I, typename TS, typename TD>
 __global__ void __launch_bounds__(256) cpy_vec8_kernel(const CpyArgs a) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= a.n) return;
-    const TS * sp = (const TS *)(a.src + offset_of(i, a.sne, a.snb, 8));
-    TD *       dp = (TD *)(a.dst + offset_of(i, a.dne, a.dnb, 8));
-    typedef TS vs8 __attribute__((ext_vector_type(8)));
-    typedef TD vd8 __attribute__((ext_vector_type(8)));
-    const vs8 x = *(const vs8 *)sp;
-    vd8 y;
+    const I i = thread_index<I>();
+    if (i >= (I)a.n) return;
+    Place sp, tp;
+    both_places<I>(a, i, 8, sp, tp);
+    const Vec8<TS> x  = *(const Vec8<TS> *)(a.src + offset_at(sp, a.snb, 8 * sizeof(TS)));
+    Vec8<TD> *     dp = (Vec8<TD> *)(a.dst + offset_at(tp, a.dnb, 8 * sizeof(TD)));
+    Vec8<TD> y;
 #pragma unroll
     for (int e = 0; e < 8; e++) y[e] = (TD)x[e];
-    *(vd8 *)dp = y;
-    if (a.mirror) *(vd8 *)((char *)dp + a.mirror) = y;
+    *dp = y;
+    if (a.mirror) *(Vec8<TD> *)((char *)dp + a.mirror) = y;
 }
 
-// quantise one block of 32 held one element per lane (32 consecutive lanes) and store it
-// (called by every lane of the wave: the reductions run before any divergence).
+// Quantise one block of 32 held by a quad of lanes, 8 consecutive elements each (lane c of the quad: elements 8c .. 8c+7),
+// and store it.  Called by all four lanes: the quad's reductions are two DPP steps, and a lane stores 8 bytes of
+// quants at once.  Against one element per lane, 32 lanes per block and a byte store each: 1 GiB of F32 into Q8_0
+// 1678 -> 275 us (4.9 TB/s, the rate of a plain copy), the 407 x 8 rows of a prompt 5.2 -> 3.3 us.
 //   Q8_0: d = amax/127 (f32), q = rne(x * (1/d)), d stored as fp16
 //   Q4_0 / Q5_0: d = (signed value of largest magnitude, the first one) / -8 (-16), q = min(15 (31), trunc(x/d + 8.5 (16.5)))
 //   Q4_1 / Q5_1: d = (max - min) / 15 (31), m = min, q = min(15 (31), trunc((x - min)/d + 0.5))
 // every product and sum is a single f32 operation, none fused.
 // mirror: 0, or the distance to a second copy of the destination that gets the same bytes
 template <int TYPE>
-__device__ __forceinline__ void quantize_block_store(float x, char * blk, int e, bool ok, int64_t mirror) {
+__device__ __forceinline__ void quantize_block_store(const float (&x)[8], char * blk, int c, bool ok, int64_t mirror) {
     typedef BlockFormat<TYPE> F;
     const int copies = mirror ? 2 : 1;
     if (TYPE == MI355X_TYPE_Q8_0) {
-        const float amax = group_max<32>(fabsf(x));
-        const float d    = amax / 127.0f;
-        const float id   = d != 0.0f ? 1.0f / d : 0.0f;
-        const int   qi   = (int)rintf(x * id);
+        float amax = fabsf(x[0]);
+#pragma unroll
+        for (int e = 1; e < 8; e++) amax = fmaxf(amax, fabsf(x[e]));
+        amax = group_max<4>(amax);
+        const float d  = amax / 127.0f;
+        const float id = d != 0.0f ? 1.0f / d : 0.0f;
+        u32x2_a2 q = {0u, 0u};
+#pragma unroll
+        for (int e = 0; e < 8; e++) q[e >> 2] |= ((uint32_t)(int)rintf(x[e] * id) & 0xFFu) << (8 * (e & 3));
         if (ok) {
-            for (int c = 0; c < copies; c++, blk += mirror) {
-                ((int8_t *)(blk + 2))[e] = (int8_t)qi;
-                if (e == 0) *(_Float16 *)blk = (_Float16)d;
+            for (int k = 0; k < copies; k++, blk += mirror) {
+                *(u32x2_a2 *)(blk + 2 + c * 8) = q;
+                if (c == 0) *(_Float16 *)blk = (_Float16)d;
             }
         }
         return;
     }
-    const int half = (threadIdx.x & 32);                 // which 32 lanes of the wave hold this block
     float d, m = 0.0f;
-    int   qi;
+    uint32_t q[8];
     if (!F::HAS_M) {
-        const float    amax  = group_max<32>(fabsf(x));
-        const uint32_t who   = (uint32_t)(__ballot(fabsf(x) == amax) >> half);
-        const int      first = who ? __ffs(who) - 1 : 0;
-        float ext = __shfl(x, half + first, 64);
-        if (!(amax > 0.0f)) ext = 0.0f;
-        d = ext / (float)(-(F::LEVELS / 2));
+        // the first element of largest magnitude, with its sign: within the lane, then the lowest lane that has it
+        float ext = x[0], amax = fabsf(x[0]);
+#pragma unroll
+        for (int e = 1; e < 8; e++) {
+            if (fabsf(x[e]) > amax || amax != amax) {
+                amax = fabsf(x[e]);
+                ext  = x[e];
+            }
+        }
+        const float top = group_max<4>(amax);
+        float first = 0.0f;
+#pragma unroll
+        for (int k = 3; k >= 0; k--) {
+            const float a = quad_broadcast(amax, k), v = quad_broadcast(ext, k);
+            if (a == top) first = v;
+        }
+        d = (top > 0.0f ? first : 0.0f) / (float)(-(F::LEVELS / 2));
         const float id = d != 0.0f ? 1.0f / d : 0.0f;
-        const float x0 = x * id;
-        qi = (int)(int8_t)(int)(x0 + ((float)(F::LEVELS / 2) + 0.5f));
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float x0 = x[e] * id;
+            const int   qi = (int)(int8_t)(int)(x0 + ((float)(F::LEVELS / 2) + 0.5f));
+            q[e] = (uint32_t)(qi < F::LEVELS - 1 ? qi : F::LEVELS - 1);
+        }
     } else {
-        m = group_min<32>(x);
-        const float mx = group_max<32>(x);
-        d = (mx - m) / (float)(F::LEVELS - 1);
+        float lo = -x[0], hi = x[0];
+#pragma unroll
+        for (int e = 1; e < 8; e++) {
+            lo = fmaxf(lo, -x[e]);
+            hi = fmaxf(hi, x[e]);
+        }
+        m = -group_max<4>(lo);
+        d = (group_max<4>(hi) - m) / (float)(F::LEVELS - 1);
         const float id = d != 0.0f ? 1.0f / d : 0.0f;
-        const float x0 = (x - m) * id;
-        qi = (int)(uint8_t)(int)(x0 + 0.5f);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float x0 = (x[e] - m) * id;
+            const int   qi = (int)(uint8_t)(int)(x0 + 0.5f);
+            q[e] = (uint32_t)(qi < F::LEVELS - 1 ? qi : F::LEVELS - 1);
+        }
     }
-    qi = qi < F::LEVELS - 1 ? qi : F::LEVELS - 1;
-    const int      hi = __shfl(qi, half + (e & 15) + 16, 64);       // the element that shares this lane's byte
-    const uint32_t qh = (uint32_t)(__ballot((qi & 0x10) != 0) >> half);
+    // elements j and j + 16 share a byte: lanes 0 and 1 take the low nibbles from themselves, the high ones from lanes 2 and 3
+    u32x2_a2 lo = {0u, 0u}, by;
+    uint32_t bits = 0;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        lo[e >> 2] |= (q[e] & 15u) << (8 * (e & 3));
+        bits |= ((q[e] >> 4) & 1u) << e;
+    }
+#pragma unroll
+    for (int k = 0; k < 2; k++) by[k] = lo[k] | quad_swap2(lo[k]) << 4;
+    uint32_t qh = bits << (8 * c);                       // the fifth bits of the whole block in every lane
+    qh |= quad_swap1(qh);
+    qh |= quad_swap2(qh);
     if (ok) {
-        for (int c = 0; c < copies; c++, blk += mirror) {
-            if (e < 16) ((uint8_t *)(blk + F::QS))[e] = (uint8_t)((qi & 15) | ((hi & 15) << 4));
-            if (e == 16) *(_Float16 *)blk = (_Float16)d;
-            if (F::HAS_M && e == 17) *(_Float16 *)(blk + 2) = (_Float16)m;
-            if (F::QH && e == 18) *(uint16_t *)(blk + F::QH) = (uint16_t)qh;
-            if (F::QH && e == 19) *(uint16_t *)(blk + F::QH + 2) = (uint16_t)(qh >> 16);
+        for (int k = 0; k < copies; k++, blk += mirror) {
+            if (c < 2) *(u32x2_a2 *)(blk + F::QS + 8 * c) = by;
+            if (c == 2) {
+                *(_Float16 *)blk = (_Float16)d;
+                if (F::HAS_M) *(_Float16 *)(blk + 2) = (_Float16)m;
+            }
+            if (F::QH && c == 3) {
+                *(uint16_t *)(blk + F::QH) = (uint16_t)qh;
+                *(uint16_t *)(blk + F::QH + 2) = (uint16_t)(qh >> 16);
+            }
         }
     }
 }
 
-// F32 -> block type; one block per 32 lanes
-template <int TYPE>
-__global__ void __launch_bounds__(256) cpy_f32_block_kernel(const CpyArgs a) {
-    const int64_t blk = (int64_t)blockIdx.x * 8 + (threadIdx.x >> 5);
-    const int     e   = threadIdx.x & 31;
-    const bool    ok  = blk < a.n;
-    const int64_t bc  = ok ? blk : 0;                       // keep all lanes in the reductions
-    const char *  sp  = a.src + offset_of(bc, a.sne, a.snb, FATTN_QK8_0) + e * a.snb[0];
-    const float   x   = ok ? *(const float *)sp : 0.0f;
-    char * dp = a.dst + offset_of(bc, a.dne, a.dnb, FATTN_QK8_0, FATTN_QK8_0);
-    quantize_block_store<TYPE>(x, dp, e, ok, a.mirror);
+// the 8 elements of a quad's lane: two 16-byte loads where the source's rows allow it
+template <bool VEC>
+__device__ __forceinline__ void load8(const char * p, int64_t nb0, bool ok, float (&x)[8]) {
+    if (VEC) {
+        const Vec4<float> u = ok ? *(const Vec4<float> *)p : Vec4<float>{0.0f, 0.0f, 0.0f, 0.0f};
+        const Vec4<float> v = ok ? *(const Vec4<float> *)(p + 16) : Vec4<float>{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int e = 0; e < 4; e++) { x[e] = u[e]; x[4 + e] = v[e]; }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++) x[e] = ok ? *(const float *)(p + e * nb0) : 0.0f;
+    }
 }
 
-// block type -> F32; 8 elements per lane, four lanes per block
-template <int TYPE>
+// F32 -> block type; one block per 4 lanes
+template <typename I, int TYPE, bool VEC>
+__global__ void __launch_bounds__(256) cpy_f32_block_kernel(const CpyArgs a) {
+    const I    blk = (I)blockIdx.x * 64 + (threadIdx.x >> 2);
+    const int  c   = threadIdx.x & 3;
+    const bool ok  = blk < (I)a.n;
+    Place sp, tp;
+    both_places<I>(a, ok ? blk : 0, FATTN_QK8_0, sp, tp);
+    float x[8];
+    load8<VEC>(a.src + offset_at(sp, a.snb, FATTN_QK8_0 * a.snb[0]) + c * 8 * a.snb[0], a.snb[0], ok, x);
+    quantize_block_store<TYPE>(x, a.dst + offset_at(tp, a.dnb, a.dnb[0]), c, ok, a.mirror);
+}
+
+// block type -> F32; 8 elements per lane, four lanes per block.  VEC: 16-byte stores.
+template <typename I, int TYPE, bool VEC>
 __global__ void __launch_bounds__(256) cpy_block_f32_kernel(const CpyArgs a) {
-    const int64_t t   = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t blk = t >> 2;
-    const int     j0  = (int)(t & 3) * 8;
-    if (blk >= a.n) return;
-    const char * sp = a.src + offset_of(blk, a.sne, a.snb, FATTN_QK8_0, FATTN_QK8_0);
+    const I   blk = (I)blockIdx.x * 64 + (threadIdx.x >> 2);
+    const int j0  = (threadIdx.x & 3) * 8;
+    if (blk >= (I)a.n) return;
+    Place sp, tp;
+    both_places<I>(a, blk, FATTN_QK8_0, sp, tp);
     float y[8];
-    dequant8<TYPE>(sp, j0, y);
-    char * dp = a.dst + offset_of(blk, a.dne, a.dnb, FATTN_QK8_0) + j0 * a.dnb[0];
+    dequant8<TYPE>(a.src + offset_at(sp, a.snb, a.snb[0]), j0, y);
+    char * dp = a.dst + offset_at(tp, a.dnb, FATTN_QK8_0 * a.dnb[0]) + j0 * a.dnb[0];
+    for (int k = 0; k < (a.mirror ? 2 : 1); k++, dp += a.mirror) {
+        if (VEC) {
+            *(Vec4<float> *)dp        = Vec4<float>{y[0], y[1], y[2], y[3]};
+            *(Vec4<float> *)(dp + 16) = Vec4<float>{y[4], y[5], y[6], y[7]};
+        } else {
 #pragma unroll
-    for (int i = 0; i < 8; i++) *(float *)(dp + i * a.dnb[0]) = y[i];
-    if (a.mirror) {
-#pragma unroll
-        for (int i = 0; i < 8; i++) *(float *)(dp + a.mirror + i * a.dnb[0]) = y[i];
+            for (int e = 0; e < 8; e++) *(float *)(dp + e * a.dnb[0]) = y[e];
+        }
     }
 }
 
 // same block type on both sides: move the blocks as halfwords
-template <int TYPE>
+template <typename I, int TYPE>
 __global__ void __launch_bounds__(256) cpy_block_block_kernel(const CpyArgs a) {
     constexpr int HW = BlockFormat<TYPE>::BYTES / 2;
-    const int64_t t   = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t blk = t / HW;
-    const int     w   = (int)(t % HW);
-    if (blk >= a.n) return;
-    const uint16_t * sp = (const uint16_t *)(a.src + offset_of(blk, a.sne, a.snb, FATTN_QK8_0, FATTN_QK8_0));
-    uint16_t *       dp = (uint16_t *)(a.dst + offset_of(blk, a.dne, a.dnb, FATTN_QK8_0, FATTN_QK8_0));
-    dp[w] = sp[w];
-    if (a.mirror) *(uint16_t *)((char *)(dp + w) + a.mirror) = sp[w];
+    const I   t   = thread_index<I>();
+    const I   blk = t / HW;
+    const int w   = (int)(t % HW);
+    if (blk >= (I)a.n) return;
+    Place sp, tp;
+    both_places<I>(a, blk, FATTN_QK8_0, sp, tp);
+    const uint16_t x = ((const uint16_t *)(a.src + offset_at(sp, a.snb, a.snb[0])))[w];
+    char * dp = a.dst + offset_at(tp, a.dnb, a.dnb[0]) + 2 * w;
+    *(uint16_t *)dp = x;
+    if (a.mirror) *(uint16_t *)(dp + a.mirror) = x;
 }
 
 // SET_ROWS: dst[:, idx[i1, i2 % ine1, i3 % ine2], i2, i3] = convert(src[:, i1, i2, i3]), src F32
-template <int DTYPE>
+// UNIT elements of a source row per unit: 32 by a quad of lanes (block types), 8 by a lane (F16 / F32 rows that start on 16
+// bytes), or 1 by a lane.  VEC: the source is read with 16-byte loads.
+template <typename I, int DTYPE, int UNIT, bool VEC>
 __global__ void __launch_bounds__(256) set_rows_kernel(const CpyArgs a) {
-    // one unit = 32 elements of a source row (block types) or 1 element (F16/F32)
     constexpr bool BLOCKS = FATTN_IS_BLOCK_TYPE(DTYPE);
-    constexpr int  UNIT   = BLOCKS ? FATTN_QK8_0 : 1;
-    int64_t u;
-    int     e = 0;
-    if (UNIT == 1) {
-        u = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    } else {
-        u = (int64_t)blockIdx.x * 8 + (threadIdx.x >> 5);
-        e = threadIdx.x & 31;
-    }
-    const bool ok = u < a.n;
-    int64_t    r  = ok ? u : 0;
-    const int64_t n0 = a.sne[0] / UNIT;
-    const int64_t i0 = r % n0;      r /= n0;
-    const int64_t i1 = r % a.sne[1]; r /= a.sne[1];
-    const int64_t i2 = r % a.sne[2];
-    const int64_t i3 = r / a.sne[2];
-    const char * ip = a.idx + i1 * a.inb[0] + (i2 % a.ine[1]) * a.inb[1] + (i3 % a.ine[2]) * a.inb[2];
+    static_assert(BLOCKS ? UNIT == FATTN_QK8_0 : (UNIT == 1 || UNIT == 8), "units");
+    const I    u  = BLOCKS ? (I)blockIdx.x * 64 + (threadIdx.x >> 2) : thread_index<I>();
+    const int  c  = BLOCKS ? threadIdx.x & 3 : 0;
+    const bool ok = u < (I)a.n;
+    const Place p = place_of<I>(ok ? u : 0, a.sne, a.sdiv, UNIT);
+    // (a broadcast of the indices over heads and sequences is the rule: no division then)
+    const int64_t x1 = a.ine[1] == 1 ? 0 : a.ine[1] == a.sne[2] ? p.i2 : p.i2 % a.ine[1];
+    const int64_t x2 = a.ine[2] == 1 ? 0 : a.ine[2] == a.sne[3] ? p.i3 : p.i3 % a.ine[2];
+    const char * ip = a.idx + p.i1 * a.inb[0] + x1 * a.inb[1] + x2 * a.inb[2];
+    const char * sp = a.src + (p.i0 * UNIT + c * 8) * a.snb[0] + p.i1 * a.snb[1] + p.i2 * a.snb[2] + p.i3 * a.snb[3];
+    float x[8];
+    if constexpr (UNIT == 1) x[0] = ok ? *(const float *)sp : 0.0f;
+    else                     load8<VEC>(sp, a.snb[0], ok, x);
     const int64_t drow = a.idx_is_i64 ? *(const int64_t *)ip : (int64_t)*(const int32_t *)ip;
     // A row index outside the destination writes nothing (ggml-cpu asserts 0 <= idx < ne1 instead): a stale or
     // uninitialised index tensor must not become a write outside the cache.  The lanes stay in the block's reduction.
     const bool inside = ok && drow >= 0 && drow < a.dne[1];
-    const char * sp = a.src + (i0 * UNIT + e) * a.snb[0] + i1 * a.snb[1] + i2 * a.snb[2] + i3 * a.snb[3];
-    const float  x  = ok ? *(const float *)sp : 0.0f;
-    char * dp = a.dst + i0 * a.dnb[0] + (inside ? drow : 0) * a.dnb[1] + i2 * a.dnb[2] + i3 * a.dnb[3];
+    char * dp = a.dst + p.i0 * a.dnb[0] * (BLOCKS ? 1 : UNIT) + (inside ? drow : 0) * a.dnb[1] + p.i2 * a.dnb[2] + p.i3 * a.dnb[3];
     if constexpr (BLOCKS) {
-        quantize_block_store<DTYPE>(x, dp, e, inside, a.mirror);
+        quantize_block_store<DTYPE>(x, dp, c, inside, a.mirror);
     } else if (inside) {
-        for (int c = 0; c < (a.mirror ? 2 : 1); c++, dp += a.mirror) {
-            if (DTYPE == MI355X_TYPE_F16) *(_Float16 *)dp = (_Float16)x;
-            else                          *(float *)dp = x;
+        typedef typename std::conditional<DTYPE == MI355X_TYPE_F16, _Float16, float>::type TD;
+        for (int k = 0; k < (a.mirror ? 2 : 1); k++, dp += a.mirror) {
+            if constexpr (UNIT == 1) {
+                *(TD *)dp = (TD)x[0];
+            } else {
+                Vec8<TD> y;
+#pragma unroll
+                for (int e = 0; e < 8; e++) y[e] = (TD)x[e];
+                *(Vec8<TD> *)dp = y;
+            }
         }
     }
 }
@@ -205,38 +301,36 @@ __global__ void __launch_bounds__(256) set_rows_kernel(const CpyArgs a) {
 // and then rounded once.
 // An F32 table [D, n1, n2, n3] with 16-byte aligned rows may ride along (the relative-position table of a FastConformer
 // block, rounded for the same call): the threads behind K's and V's write its contiguous f16 copy.
-template <int TYPE>
-__global__ void __launch_bounds__(256) kv_to_f16_kernel(const FattnArgs a, char * dst, const F32Rider x) {
-    const int     cpr  = a.D / 8;                                  // chunks per row
-    const int64_t half = (int64_t)cpr * a.Nkv * a.Hkv * a.Bk;      // chunks per tensor
-    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+// chunks of 8 elements per row, rows per head and heads per sequence of the copies, and the same of the rider's table
+struct ChunkDivs {
+    FastDiv kv[3], table[3];
+    int64_t kv_ne[4], table_ne[4];
+};
+template <typename I, int TYPE>
+__global__ void __launch_bounds__(256) kv_to_f16_kernel(const FattnArgs a, char * dst, const F32Rider x, const ChunkDivs v) {
+    const I half = (I)((int64_t)(a.D / 8) * a.Nkv * a.Hkv * a.Bk);      // chunks per tensor
+    I i = thread_index<I>();
     if (i >= 2 * half) {
         i -= 2 * half;
-        if (i >= x.n) return;
-        const int c = (int)(i % cpr);
-        int64_t   r = i / cpr;
-        const int64_t i1 = r % x.ne1;  r /= x.ne1;
-        const int64_t i2 = r % x.ne2;
-        const int64_t i3 = r / x.ne2;
-        const char * row = x.src + i1 * x.nb1 + i2 * x.nb2 + i3 * x.nb3;
+        if (i >= (I)x.n) return;
+        const Place p = place_of<I>(i, v.table_ne, v.table, 1);
+        const int   c = (int)p.i0;
+        const char * row = x.src + p.i1 * x.nb1 + p.i2 * x.nb2 + p.i3 * x.nb3;
         const float4 x0 = *(const float4 *)(row + c * 32);
         const float4 x1 = *(const float4 *)(row + c * 32 + 16);
         typedef _Float16 h8 __attribute__((ext_vector_type(8)));
         h8 y;
         y[0] = (_Float16)x0.x; y[1] = (_Float16)x0.y; y[2] = (_Float16)x0.z; y[3] = (_Float16)x0.w;
         y[4] = (_Float16)x1.x; y[5] = (_Float16)x1.y; y[6] = (_Float16)x1.z; y[7] = (_Float16)x1.w;
-        *(h8 *)(x.dst + i * 16) = y;
+        *(h8 *)(x.dst + (int64_t)i * 16) = y;
         return;
     }
     const bool is_v = i >= half;
     if (is_v) i -= half;
-    const int     c = (int)(i % cpr);
-    int64_t       r = i / cpr;
-    const int64_t j = r % a.Nkv;  r /= a.Nkv;
-    const int64_t h = r % a.Hkv;
-    const int64_t b = r / a.Hkv;
-    const char * row = is_v ? a.v + j * a.nbv1 + h * a.nbv2 + b * a.nbv3
-                            : a.k + j * a.nbk1 + h * a.nbk2 + b * a.nbk3;
+    const Place p = place_of<I>(i, v.kv_ne, v.kv, 1);
+    const int   c = (int)p.i0;
+    const char * row = is_v ? a.v + p.i1 * a.nbv1 + p.i2 * a.nbv2 + p.i3 * a.nbv3
+                            : a.k + p.i1 * a.nbk1 + p.i2 * a.nbk2 + p.i3 * a.nbk3;
     typedef _Float16 h8 __attribute__((ext_vector_type(8)));
     h8 y;
     if constexpr (TYPE == MI355X_TYPE_F32) {
@@ -250,7 +344,7 @@ __global__ void __launch_bounds__(256) kv_to_f16_kernel(const FattnArgs a, char 
 #pragma unroll
         for (int e = 0; e < 8; e++) y[e] = (_Float16)f[e];
     }
-    *(h8 *)(dst + ((is_v ? half : 0) + i) * 16) = y;
+    *(h8 *)(dst + (int64_t)((is_v ? half : 0) + i) * 16) = y;
 }
 
 // The same for a K and a V of different storage types (CRISPASR_KV_QUANT_K / _V, src/core/attention.h:132-137; the
@@ -258,24 +352,21 @@ __global__ void __launch_bounds__(256) kv_to_f16_kernel(const FattnArgs a, char 
 // tensor at run time.  Scalar loads: such rows are only as aligned as their type.
 // It is also the launch that pads: the copies' rows are a.D elements long, the first a.Dv of them the source row's
 // (a multiple of 8), zeros behind - how the tile kernel, which has forms for 64- and 128-wide heads, gets the others.
-__global__ void __launch_bounds__(256) kv_to_f16_mixed_kernel(const FattnArgs a, const int ktype, const int vtype, char * dst) {
-    const int     cpr  = a.D / 8;
-    const int64_t half = (int64_t)cpr * a.Nkv * a.Hkv * a.Bk;
-    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+template <typename I>
+__global__ void __launch_bounds__(256) kv_to_f16_mixed_kernel(const FattnArgs a, const int ktype, const int vtype, char * dst, const ChunkDivs v) {
+    const I half = (I)((int64_t)(a.D / 8) * a.Nkv * a.Hkv * a.Bk);
+    I i = thread_index<I>();
     if (i >= 2 * half) return;
     const bool is_v = i >= half;
     if (is_v) i -= half;
-    const int     c = (int)(i % cpr);
+    const Place p = place_of<I>(i, v.kv_ne, v.kv, 1);
+    const int   c = (int)p.i0;
     if (c * 8 >= a.Dv) {
-        *(uint4 *)(dst + ((is_v ? half : 0) + i) * 16) = uint4{0u, 0u, 0u, 0u};
+        *(uint4 *)(dst + (int64_t)((is_v ? half : 0) + i) * 16) = uint4{0u, 0u, 0u, 0u};
         return;
     }
-    int64_t       r = i / cpr;
-    const int64_t j = r % a.Nkv;  r /= a.Nkv;
-    const int64_t h = r % a.Hkv;
-    const int64_t b = r / a.Hkv;
-    const char * row = is_v ? a.v + j * a.nbv1 + h * a.nbv2 + b * a.nbv3
-                            : a.k + j * a.nbk1 + h * a.nbk2 + b * a.nbk3;
+    const char * row = is_v ? a.v + p.i1 * a.nbv1 + p.i2 * a.nbv2 + p.i3 * a.nbv3
+                            : a.k + p.i1 * a.nbk1 + p.i2 * a.nbk2 + p.i3 * a.nbk3;
     float f[8];
     const char * blk = row + (c >> 2) * fattn_block_bytes(is_v ? vtype : ktype);
     switch (is_v ? vtype : ktype) {
@@ -297,7 +388,7 @@ __global__ void __launch_bounds__(256) kv_to_f16_mixed_kernel(const FattnArgs a,
     h8 y;
 #pragma unroll
     for (int e = 0; e < 8; e++) y[e] = (_Float16)f[e];
-    *(h8 *)(dst + ((is_v ? half : 0) + i) * 16) = y;
+    *(h8 *)(dst + (int64_t)((is_v ? half : 0) + i) * 16) = y;
 }
 
 // memset as a kernel: a memset node recorded into a captured graph is what a fill kernel avoids.
@@ -333,14 +424,30 @@ int kv_to_f16_launch(const FattnArgs & a, int ktype, int vtype, void * dst, hipS
     const int64_t n = 2 * (int64_t)(a.D / 8) * a.Nkv * a.Hkv * a.Bk + x.n;
     if (n == 0) return 0;
     if ((n + 255) / 256 > 0x7fffffff) return (int)hipErrorInvalidValue;
-    const unsigned g = (unsigned)((n + 255) / 256);
+    const dim3 g((unsigned)((n + 255) / 256));
+    ChunkDivs v;
+    const int64_t kv_ne[4] = {a.D / 8, a.Nkv, a.Hkv, a.Bk}, table_ne[4] = {a.D / 8, x.ne1, x.ne2, 1};
+    for (int i = 0; i < 4; i++) {
+        v.kv_ne[i]    = kv_ne[i];
+        v.table_ne[i] = table_ne[i];
+        if (i < 3) {
+            v.kv[i]    = fast_div((uint32_t)kv_ne[i]);
+            v.table[i] = fast_div((uint32_t)table_ne[i]);
+        }
+    }
+    const bool small = n + 256 < ((int64_t)1 << 31);             // 32-bit indices do
     if (ktype != vtype || a.Dv != a.D) {
         if (rider) return (int)hipErrorInvalidValue;
-        hipLaunchKernelGGL(kv_to_f16_mixed_kernel, dim3(g), dim3(256), 0, stream, a, ktype, vtype, (char *)dst);
+        if (small) hipLaunchKernelGGL(kv_to_f16_mixed_kernel<uint32_t>, g, dim3(256), 0, stream, a, ktype, vtype, (char *)dst, v);
+        else       hipLaunchKernelGGL(kv_to_f16_mixed_kernel<int64_t>, g, dim3(256), 0, stream, a, ktype, vtype, (char *)dst, v);
         return (int)hipGetLastError();
     }
     switch (ktype) {
-#define KV16(T) case T: hipLaunchKernelGGL((kv_to_f16_kernel<T>), dim3(g), dim3(256), 0, stream, a, (char *)dst, x); break
+#define KV16(T)                                                                                                         \
+    case T:                                                                                                             \
+        if (small) hipLaunchKernelGGL((kv_to_f16_kernel<uint32_t, T>), g, dim3(256), 0, stream, a, (char *)dst, x, v);    \
+        else       hipLaunchKernelGGL((kv_to_f16_kernel<int64_t, T>), g, dim3(256), 0, stream, a, (char *)dst, x, v);     \
+        break
         KV16(MI355X_TYPE_F32);
         KV16(MI355X_TYPE_Q8_0);
         KV16(MI355X_TYPE_Q4_0);
@@ -353,46 +460,79 @@ int kv_to_f16_launch(const FattnArgs & a, int ktype, int vtype, void * dst, hipS
     return (int)hipGetLastError();
 }
 
+// rows of a side whose elements of `es` bytes lie `es` apart and start on multiples of `align` bytes
+static bool rows_aligned(const void * p, const int64_t (&ne)[4], const int64_t (&nb)[4], int64_t es, int64_t align) {
+    if (nb[0] != es || (uintptr_t)p % align) return false;
+    for (int i = 1; i < 4; i++)
+        if (ne[i] > 1 && nb[i] % align) return false;
+    return true;
+}
+
 static bool vec8_ok(const CpyArgs & a, int stype, int dtype) {
     if (FATTN_IS_BLOCK_TYPE(stype) || FATTN_IS_BLOCK_TYPE(dtype)) return false;
     const int64_t ss = stype == MI355X_TYPE_F32 ? 4 : 2, ds = dtype == MI355X_TYPE_F32 ? 4 : 2;
-    if (a.sne[0] % 8 || a.dne[0] % 8 || a.snb[0] != ss || a.dnb[0] != ds) return false;
-    if (((uintptr_t)a.src % (8 * ss)) || ((uintptr_t)a.dst % (8 * ds))) return false;
-    for (int i = 1; i < 4; i++) {
-        if ((a.sne[i] > 1 && a.snb[i] % (8 * ss)) || (a.dne[i] > 1 && a.dnb[i] % (8 * ds))) return false;
+    return a.sne[0] % 8 == 0 && a.dne[0] % 8 == 0 && rows_aligned(a.src, a.sne, a.snb, ss, 8 * ss) &&
+           rows_aligned(a.dst, a.dne, a.dnb, ds, 8 * ds) && (!a.mirror || a.mirror % (8 * ds) == 0);
+}
+
+// the launch's divisors for units of `unit0` elements; whether 32-bit indices do (`threads` = the grid's)
+static bool prepare_index(CpyArgs & a, int64_t unit0, int64_t threads) {
+    a.same_shape = 1;
+    for (int i = 0; i < 4; i++) a.same_shape = a.same_shape && a.sne[i] == a.dne[i];
+    a.sdiv[0] = fast_div((uint32_t)(a.sne[0] / unit0));
+    a.ddiv[0] = fast_div((uint32_t)(a.dne[0] / unit0));
+    for (int i = 1; i < 3; i++) {
+        a.sdiv[i] = fast_div((uint32_t)a.sne[i]);
+        a.ddiv[i] = fast_div((uint32_t)a.dne[i]);
     }
-    return true;
+    return threads + 256 < ((int64_t)1 << 31);
+}
+
+// a kernel of this file over `threads` lanes, with 32-bit indices where they do
+#define CPY_LAUNCH(args, unit0, threads, KERNEL, ...)                                                                    \
+    do {                                                                                                                 \
+        CpyArgs v_ = args;                                                                                               \
+        const int64_t t_ = (threads);                                                                                    \
+        const bool    small_ = prepare_index(v_, unit0, t_);                                                             \
+        const dim3    g_((unsigned)((t_ + 255) / 256));                                                                  \
+        if (small_) hipLaunchKernelGGL((KERNEL<uint32_t, __VA_ARGS__>), g_, dim3(256), 0, stream, v_);                   \
+        else        hipLaunchKernelGGL((KERNEL<int64_t, __VA_ARGS__>), g_, dim3(256), 0, stream, v_);                    \
+    } while (0)
+
+template <typename TS, typename TD>
+static void launch_plain(const CpyArgs & a, bool vec8, hipStream_t stream) {
+    if (vec8) {
+        CpyArgs b = a;
+        b.n = a.n / 8;
+        CPY_LAUNCH(b, 8, b.n, cpy_vec8_kernel, TS, TD);
+    } else {
+        CPY_LAUNCH(a, 1, a.n, cpy_scalar_kernel, TS, TD);
+    }
+}
+
+template <int T>
+static void launch_to_blocks(const CpyArgs & a, hipStream_t stream) {
+    if (rows_aligned(a.src, a.sne, a.snb, 4, 16)) CPY_LAUNCH(a, FATTN_QK8_0, a.n * 4, cpy_f32_block_kernel, T, true);
+    else                                          CPY_LAUNCH(a, FATTN_QK8_0, a.n * 4, cpy_f32_block_kernel, T, false);
+}
+
+template <int T>
+static void launch_from_blocks(const CpyArgs & a, hipStream_t stream) {
+    if (rows_aligned(a.dst, a.dne, a.dnb, 4, 16) && a.mirror % 16 == 0) CPY_LAUNCH(a, FATTN_QK8_0, a.n * 4, cpy_block_f32_kernel, T, true);
+    else                                                                CPY_LAUNCH(a, FATTN_QK8_0, a.n * 4, cpy_block_f32_kernel, T, false);
 }
 
 int cpy_launch(const CpyArgs & a, int stype, int dtype, hipStream_t stream) {
     if (a.n == 0) return 0;
-    if (vec8_ok(a, stype, dtype)) {
-        CpyArgs v = a;
-        v.n = a.n / 8;
-        const unsigned g = (unsigned)((v.n + 255) / 256);
-        if (stype == MI355X_TYPE_F32 && dtype == MI355X_TYPE_F32)      hipLaunchKernelGGL((cpy_vec8_kernel<float, float>), dim3(g), dim3(256), 0, stream, v);
-        else if (stype == MI355X_TYPE_F32 && dtype == MI355X_TYPE_F16) hipLaunchKernelGGL((cpy_vec8_kernel<float, _Float16>), dim3(g), dim3(256), 0, stream, v);
-        else if (stype == MI355X_TYPE_F16 && dtype == MI355X_TYPE_F16) hipLaunchKernelGGL((cpy_vec8_kernel<_Float16, _Float16>), dim3(g), dim3(256), 0, stream, v);
-        else                                                          hipLaunchKernelGGL((cpy_vec8_kernel<_Float16, float>), dim3(g), dim3(256), 0, stream, v);
-        return (int)hipGetLastError();
-    }
-    const unsigned g256 = (unsigned)((a.n + 255) / 256);
-    const unsigned g8   = (unsigned)((a.n + 7) / 8);
-    if (stype == MI355X_TYPE_F32 && dtype == MI355X_TYPE_F32)
-        hipLaunchKernelGGL((cpy_scalar_kernel<float, float>), dim3(g256), dim3(256), 0, stream, a);
-    else if (stype == MI355X_TYPE_F32 && dtype == MI355X_TYPE_F16)
-        hipLaunchKernelGGL((cpy_scalar_kernel<float, _Float16>), dim3(g256), dim3(256), 0, stream, a);
-    else if (stype == MI355X_TYPE_F16 && dtype == MI355X_TYPE_F16)
-        hipLaunchKernelGGL((cpy_scalar_kernel<_Float16, _Float16>), dim3(g256), dim3(256), 0, stream, a);
-    else if (stype == MI355X_TYPE_F16 && dtype == MI355X_TYPE_F32)
-        hipLaunchKernelGGL((cpy_scalar_kernel<_Float16, float>), dim3(g256), dim3(256), 0, stream, a);
+    const bool vec8 = vec8_ok(a, stype, dtype);
+    if (stype == MI355X_TYPE_F32 && dtype == MI355X_TYPE_F32)      launch_plain<float, float>(a, vec8, stream);
+    else if (stype == MI355X_TYPE_F32 && dtype == MI355X_TYPE_F16) launch_plain<float, _Float16>(a, vec8, stream);
+    else if (stype == MI355X_TYPE_F16 && dtype == MI355X_TYPE_F16) launch_plain<_Float16, _Float16>(a, vec8, stream);
+    else if (stype == MI355X_TYPE_F16 && dtype == MI355X_TYPE_F32) launch_plain<_Float16, float>(a, vec8, stream);
 #define BLOCK_CASES(T)                                                                                                    \
-    else if (stype == MI355X_TYPE_F32 && dtype == T)                                                                       \
-        hipLaunchKernelGGL((cpy_f32_block_kernel<T>), dim3(g8), dim3(256), 0, stream, a);                                 \
-    else if (stype == T && dtype == MI355X_TYPE_F32)                                                                       \
-        hipLaunchKernelGGL((cpy_block_f32_kernel<T>), dim3((unsigned)((a.n * 4 + 255) / 256)), dim3(256), 0, stream, a);  \
-    else if (stype == T && dtype == T)                                                                                     \
-        hipLaunchKernelGGL((cpy_block_block_kernel<T>), dim3((unsigned)((a.n * (BlockFormat<T>::BYTES / 2) + 255) / 256)), dim3(256), 0, stream, a);
+    else if (stype == MI355X_TYPE_F32 && dtype == T) launch_to_blocks<T>(a, stream);                                       \
+    else if (stype == T && dtype == MI355X_TYPE_F32) launch_from_blocks<T>(a, stream);                                     \
+    else if (stype == T && dtype == T) CPY_LAUNCH(a, FATTN_QK8_0, a.n * (BlockFormat<T>::BYTES / 2), cpy_block_block_kernel, T);
     BLOCK_CASES(MI355X_TYPE_Q8_0)
     BLOCK_CASES(MI355X_TYPE_Q4_0)
     BLOCK_CASES(MI355X_TYPE_Q4_1)
@@ -404,20 +544,36 @@ int cpy_launch(const CpyArgs & a, int stype, int dtype, hipStream_t stream) {
     return (int)hipGetLastError();
 }
 
+template <int T>
+static void launch_set_rows(const CpyArgs & a, hipStream_t stream) {
+    const bool vec = rows_aligned(a.src, a.sne, a.snb, 4, 16);
+    if constexpr (FATTN_IS_BLOCK_TYPE(T)) {
+        if (vec) CPY_LAUNCH(a, FATTN_QK8_0, a.n * 4, set_rows_kernel, T, FATTN_QK8_0, true);
+        else     CPY_LAUNCH(a, FATTN_QK8_0, a.n * 4, set_rows_kernel, T, FATTN_QK8_0, false);
+    } else {
+        const int64_t ds = T == MI355X_TYPE_F16 ? 2 : 4;
+        if (vec && a.sne[0] % 8 == 0 && rows_aligned(a.dst, a.dne, a.dnb, ds, 8 * ds) && a.mirror % (8 * ds) == 0) {
+            CpyArgs b = a;
+            b.n = a.n / 8;
+            CPY_LAUNCH(b, 8, b.n, set_rows_kernel, T, 8, true);
+        } else {
+            CPY_LAUNCH(a, 1, a.n, set_rows_kernel, T, 1, false);
+        }
+    }
+}
+
 int set_rows_launch(const CpyArgs & a, int dtype, hipStream_t stream) {
     if (a.n == 0) return 0;
     if (a.n > ((int64_t)1 << 38)) return (int)hipErrorInvalidValue;
-    const dim3 gb((unsigned)((a.n + 7) / 8));
-    if (dtype == MI355X_TYPE_Q8_0)      hipLaunchKernelGGL((set_rows_kernel<MI355X_TYPE_Q8_0>), gb, dim3(256), 0, stream, a);
-    else if (dtype == MI355X_TYPE_Q4_0) hipLaunchKernelGGL((set_rows_kernel<MI355X_TYPE_Q4_0>), gb, dim3(256), 0, stream, a);
-    else if (dtype == MI355X_TYPE_Q4_1) hipLaunchKernelGGL((set_rows_kernel<MI355X_TYPE_Q4_1>), gb, dim3(256), 0, stream, a);
-    else if (dtype == MI355X_TYPE_Q5_0) hipLaunchKernelGGL((set_rows_kernel<MI355X_TYPE_Q5_0>), gb, dim3(256), 0, stream, a);
-    else if (dtype == MI355X_TYPE_Q5_1) hipLaunchKernelGGL((set_rows_kernel<MI355X_TYPE_Q5_1>), gb, dim3(256), 0, stream, a);
-    else if (dtype == MI355X_TYPE_F16)
-        hipLaunchKernelGGL((set_rows_kernel<MI355X_TYPE_F16>), dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, stream, a);
-    else if (dtype == MI355X_TYPE_F32)
-        hipLaunchKernelGGL((set_rows_kernel<MI355X_TYPE_F32>), dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, stream, a);
-    else
-        return (int)hipErrorInvalidValue;
+    switch (dtype) {
+        case MI355X_TYPE_Q8_0: launch_set_rows<MI355X_TYPE_Q8_0>(a, stream); break;
+        case MI355X_TYPE_Q4_0: launch_set_rows<MI355X_TYPE_Q4_0>(a, stream); break;
+        case MI355X_TYPE_Q4_1: launch_set_rows<MI355X_TYPE_Q4_1>(a, stream); break;
+        case MI355X_TYPE_Q5_0: launch_set_rows<MI355X_TYPE_Q5_0>(a, stream); break;
+        case MI355X_TYPE_Q5_1: launch_set_rows<MI355X_TYPE_Q5_1>(a, stream); break;
+        case MI355X_TYPE_F16:  launch_set_rows<MI355X_TYPE_F16>(a, stream); break;
+        case MI355X_TYPE_F32:  launch_set_rows<MI355X_TYPE_F32>(a, stream); break;
+        default: return (int)hipErrorInvalidValue;
+    }
     return (int)hipGetLastError();
 }

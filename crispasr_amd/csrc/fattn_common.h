@@ -123,6 +123,18 @@ static __device__ __forceinline__ float group_sum(float x) {
     return x;
 }
 
+// values of the other lanes of a quad (4 lanes): lane ^ 1, lane ^ 2, lane k
+static __device__ __forceinline__ uint32_t quad_swap1(uint32_t x) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xf, 0xf, true); }
+static __device__ __forceinline__ uint32_t quad_swap2(uint32_t x) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xf, 0xf, true); }
+static __device__ __forceinline__ float quad_broadcast(float x, int k) {          // k: a constant after unrolling
+    switch (k) {
+        case 0:  return dpp_mov<0x00>(x);
+        case 1:  return dpp_mov<0x55>(x);
+        case 2:  return dpp_mov<0xAA>(x);
+        default: return dpp_mov<0xFF>(x);
+    }
+}
+
 template <int GROUP>
 static __device__ __forceinline__ float group_max(float x) {
     x = fmaxf(x, dpp_mov<0xB1>(x));
@@ -291,12 +303,28 @@ static __device__ __forceinline__ void dequant8(const char * blk, int j0, float 
     }
 }
 
+// Unsigned division by a number fixed on the host: n / d = (mulhi(n, m) + n) >> s for n < 2^31.
+struct FastDiv {
+    uint32_t d, m, s;
+};
+static inline FastDiv fast_div(uint32_t d) {
+    FastDiv f;
+    f.d = d;
+    f.s = 0;
+    while (((uint64_t)1 << f.s) < d) f.s++;
+    f.m = d ? (uint32_t)((((uint64_t)1 << 32) * (((uint64_t)1 << f.s) - d)) / d + 1) : 0;
+    return f;
+}
+static __device__ __forceinline__ uint32_t divide(uint32_t n, const FastDiv & f) { return (__umulhi(n, f.m) + n) >> f.s; }
+
 // One CPY / SET_ROWS node.
 struct CpyArgs {
     const char * src;
     char *       dst;
     int64_t sne[4], dne[4];
     int64_t snb[4], dnb[4];
+    FastDiv sdiv[3], ddiv[3];  // of the launch's units: units along dimension 0, extents of dimensions 1 and 2 (filled in by the launcher)
+    int32_t same_shape;        // sne == dne (likewise)
     int64_t n;                 // elements (or blocks of 32 when a side is a block type)
     int64_t mirror;            // 0, or the distance in bytes from dst to a second copy that gets the same stores
     // SET_ROWS only
