@@ -366,6 +366,7 @@ struct FattnRelposArgs {
 int fattn_vec_launch(const FattnArgs & a, int ktype, hipStream_t stream);
 int fattn_merge_launch(const FattnArgs & a, hipStream_t stream);
 int fattn_mma_launch(const FattnArgs & a, int ktype, hipStream_t stream);
+int fattn_pipe_launch(const FattnArgs & a, int query_blocks, int key_split, hipStream_t stream);
 // the instantiation of the tile kernel a call takes
 struct FattnMmaVariant {
     int  query_blocks;            // 32-query blocks per wave (1 or 2)

@@ -142,16 +142,10 @@ template <int D> __device__ __forceinline__ int swz_v(int r) { return D == 64 ? 
 
 template <int D> __device__ __forceinline__ int swz_m(int r) { return (r >> 2) & 3; }     // mask half tile: 4 chunks per row
 
-// TK: keys per tile.  64, except in the key-split form of 64-wide heads without a mask - the grids where a wave is alone on
-// its SIMD: tiles of 128 (each wave two 32-key blocks of its half: half the barriers per key, and the second block's
-// operands are on their way while the first is in the softmax), or of 256 when the workgroups number no more than the
-// CUs, since four such tiles are 128 KB of LDS and leave room for one workgroup per CU only.
-// (two query blocks per wave with 128-key tiles: 240 bytes of scratch per lane in the loop, 110 us instead of 60 on the
-//  large-v3 encoder layer)
 // PAD: the head is one of a.Dv elements (a multiple of 8 below D) on K/V copies whose rows are zero-padded to D: a.Dv
 // elements of every q row are read and a.Dv of every dst row written.  An instantiation of its own, so that the others
 // stay the code they were (the guards cost the one-block forms 2% as a run-time branch).
-template <int D, int NQB, int KSP, int TYPE, bool MASK, bool SOFTCAP, bool DIRECT, bool MDMA, int TK = BC, bool PAD = false>
+template <int D, int NQB, int KSP, int TYPE, bool MASK, bool SOFTCAP, bool DIRECT, bool MDMA, bool PAD = false>
 __global__ void __launch_bounds__(MMA_THREADS, 2) fattn_mma_kernel(const FattnArgs a, const int n_qtiles) {
     static_assert(!PAD || (DIRECT && NQB == 1), "zero-padded heads: f16 copies, one query block per wave");
     constexpr bool whole_head = !PAD;
@@ -161,9 +155,7 @@ __global__ void __launch_bounds__(MMA_THREADS, 2) fattn_mma_kernel(const FattnAr
     constexpr int NMH   = NQB * 2;                 // MDMA: loads per wave and half tile (16 rows x 64 bytes each)
     constexpr int MHALF = NQB * 32 * 64;           //       bytes of a wave's half-tile block; a wave owns 2 of them
     constexpr int ROWB  = D * 2;                   // DIRECT: bytes per (unpadded) row
-    constexpr int BCT   = TK;                      // keys per tile
-    static_assert(TK == BC || (KSP == 2 && D == 64 && !MASK && DIRECT), "larger tiles exist for the unmasked key-split form of 64-wide heads");
-    constexpr int TILEB = BCT * ROWB;              //         bytes per K or V tile; LDS = K0 K1 V0 V1
+    constexpr int TILEB = BC * ROWB;              //         bytes per K or V tile; LDS = K0 K1 V0 V1
     constexpr int NLD   = TILEB / 1024 / MMA_WAVES;   //      global->LDS loads per wave, tile and tensor
 
     constexpr int KS   = D / 16;                   // reduction steps of Q.K^T
@@ -175,7 +167,7 @@ __global__ void __launch_bounds__(MMA_THREADS, 2) fattn_mma_kernel(const FattnAr
     constexpr int PV   = Pitch<D>::V;
     constexpr int BMW  = 32 * NQB;                 // queries per wave
     constexpr int BMG  = BMW * MMA_WAVES / KSP;    // queries per workgroup
-    constexpr int NKB  = BCT / 32 / KSP;           // 32-key blocks of a tile that one wave walks
+    constexpr int NKB  = BC / 32 / KSP;           // 32-key blocks of a tile that one wave walks
     // Skipping excluded blocks adds a branch round the block's body.  The instantiations that already fill the register
     // file (two query blocks per wave, 128-wide heads without key split) answer it with spills inside the tile loop, so
     // it is left to the others: the key-split form and one query block of 64-wide heads.
@@ -697,8 +689,8 @@ __global__ void __launch_bounds__(MMA_THREADS, 2) fattn_mma_kernel(const FattnAr
         }
     };
 
-    const int n_tiles = (k_end - k_begin + BCT - 1) / BCT;
-    const int n_full  = (k_end - k_begin) / BCT;
+    const int n_tiles = (k_end - k_begin + BC - 1) / BC;
+    const int n_full  = (k_end - k_begin) / BC;
     if (DIRECT) {
         char * const lb = (char *)lds_raw;               // K0 K1 V0 V1 [mask: per wave 2 half-tile blocks]
         char * const mb = lb + 4 * TILEB;
@@ -720,9 +712,9 @@ __global__ void __launch_bounds__(MMA_THREADS, 2) fattn_mma_kernel(const FattnAr
                 else                                            __builtin_amdgcn_s_setprio(0);
             }
             const int  cur = (t & 1) * TILEB, nxt = TILEB - cur;
-            const int  jn  = t + 1 < n_tiles ? k_begin + (t + 1) * BCT : -1;
+            const int  jn  = t + 1 < n_tiles ? k_begin + (t + 1) * BC : -1;
             const bool mn  = (MDMA || MPRE) && t + 1 < n_full;     // the next tile's mask is requested during this one
-            tile(k_begin + t * BCT, 0, std::false_type{}, lb + cur, lb + 2 * TILEB + cur, lb + nxt, lb + 2 * TILEB + nxt, jn, t + 1 >= n_full, mb, mn);
+            tile(k_begin + t * BC, 0, std::false_type{}, lb + cur, lb + 2 * TILEB + cur, lb + nxt, lb + 2 * TILEB + nxt, jn, t + 1 >= n_full, mb, mn);
             // everything requested during the tile has had at least half a tile to land
             __builtin_amdgcn_s_waitcnt(0x0F70);
             __syncthreads();
@@ -730,8 +722,8 @@ __global__ void __launch_bounds__(MMA_THREADS, 2) fattn_mma_kernel(const FattnAr
         __builtin_amdgcn_s_setprio(0);
         if (n_full < n_tiles) {
             const int cur = (n_full & 1) * TILEB;
-            if (MDMA) stage_mask_tail(k_begin + n_full * BCT, mb);
-            tile(k_begin + n_full * BCT, 0, std::true_type{}, lb + cur, lb + 2 * TILEB + cur, nullptr, nullptr, -1, false, mb, false);
+            if (MDMA) stage_mask_tail(k_begin + n_full * BC, mb);
+            tile(k_begin + n_full * BC, 0, std::true_type{}, lb + cur, lb + 2 * TILEB + cur, nullptr, nullptr, -1, false, mb, false);
         }
     } else {
     load_tile(k_begin);
@@ -900,35 +892,35 @@ __global__ void __launch_bounds__(MMA_THREADS, 2) fattn_mma_kernel(const FattnAr
     }
 }
 
-template <int D, int NQB, int KSP, int TYPE, bool MASK, bool SOFTCAP, bool DIRECT, bool MDMA, int TK, bool PAD>
+template <int D, int NQB, int KSP, int TYPE, bool MASK, bool SOFTCAP, bool DIRECT, bool MDMA, bool PAD>
 int launch_kernel(const FattnArgs & a, hipStream_t stream) {
     const int bmg = 32 * NQB * MMA_WAVES / KSP;
     const int n_qtiles = (a.Nq + bmg - 1) / bmg;
     if ((int64_t)n_qtiles * a.Hq * a.B * a.n_splits > 0x7fffffff) return (int)hipErrorInvalidValue;
     const dim3 grid((unsigned)((int64_t)n_qtiles * a.Hq * a.B * a.n_splits));
-    const size_t lds = DIRECT ? (size_t)4 * TK * D * sizeof(_Float16) + (MDMA ? (size_t)MMA_WAVES * NQB * 4096 : 0)
+    const size_t lds = DIRECT ? (size_t)4 * BC * D * sizeof(_Float16) + (MDMA ? (size_t)MMA_WAVES * NQB * 4096 : 0)
                               : (size_t)2 * BC * (Pitch<D>::K + Pitch<D>::V) * sizeof(_Float16);
     static std::atomic<uint64_t> lds_allowed{0};     // per instantiation
-    const hipError_t ea = fattn_allow_lds((const void *)fattn_mma_kernel<D, NQB, KSP, TYPE, MASK, SOFTCAP, DIRECT, MDMA, TK, PAD>, (int)lds, lds_allowed);
+    const hipError_t ea = fattn_allow_lds((const void *)fattn_mma_kernel<D, NQB, KSP, TYPE, MASK, SOFTCAP, DIRECT, MDMA, PAD>, (int)lds, lds_allowed);
     if (ea != hipSuccess) return (int)ea;
     static const bool debug = getenv("MI355X_FATTN_DEBUG") != nullptr;
     if (debug) {
         int nb = -1;
-        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (const void *)fattn_mma_kernel<D, NQB, KSP, TYPE, MASK, SOFTCAP, DIRECT, MDMA, TK, PAD>, MMA_THREADS, lds);
+        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (const void *)fattn_mma_kernel<D, NQB, KSP, TYPE, MASK, SOFTCAP, DIRECT, MDMA, PAD>, MMA_THREADS, lds);
         fprintf(stderr, "[mi355x] fattn_mma<%d,%d,%d,%d,%d,%d,%d,%d> grid %u lds %zu B, resident workgroups per CU: %d\n",
                 D, NQB, KSP, TYPE, (int)MASK, (int)SOFTCAP, (int)DIRECT, (int)MDMA, grid.x, lds, nb);
     }
-    hipLaunchKernelGGL((fattn_mma_kernel<D, NQB, KSP, TYPE, MASK, SOFTCAP, DIRECT, MDMA, TK, PAD>), grid, dim3(MMA_THREADS), lds, stream, a, n_qtiles);
+    hipLaunchKernelGGL((fattn_mma_kernel<D, NQB, KSP, TYPE, MASK, SOFTCAP, DIRECT, MDMA, PAD>), grid, dim3(MMA_THREADS), lds, stream, a, n_qtiles);
     return (int)hipGetLastError();
 }
 
-template <int D, int NQB, int KSP, int TYPE, bool MASK, bool SOFTCAP, bool DIRECT, bool MDMA, int TK = BC>
+template <int D, int NQB, int KSP, int TYPE, bool MASK, bool SOFTCAP, bool DIRECT, bool MDMA>
 int launch(const FattnArgs & a, hipStream_t stream) {
     if (a.Dv != a.D) {              // a zero-padded head: the forms that exist for it, or none
-        if constexpr (DIRECT && NQB == 1) return launch_kernel<D, NQB, KSP, TYPE, MASK, SOFTCAP, DIRECT, MDMA, TK, true>(a, stream);
+        if constexpr (DIRECT && NQB == 1) return launch_kernel<D, NQB, KSP, TYPE, MASK, SOFTCAP, DIRECT, MDMA, true>(a, stream);
         return (int)hipErrorInvalidValue;
     }
-    return launch_kernel<D, NQB, KSP, TYPE, MASK, SOFTCAP, DIRECT, MDMA, TK, false>(a, stream);
+    return launch_kernel<D, NQB, KSP, TYPE, MASK, SOFTCAP, DIRECT, MDMA, false>(a, stream);
 }
 
 template <int D, int NQB, int KSP, int TYPE, bool DIRECT>
@@ -937,13 +929,9 @@ int launch_mask(const FattnArgs & a, const FattnMmaVariant & v, hipStream_t stre
     if (KSP == 1 && a.softcap != 0.0f)
         return mask ? launch<D, NQB, 1, TYPE, true, true, DIRECT, false>(a, stream) : launch<D, NQB, 1, TYPE, false, true, DIRECT, false>(a, stream);
     if (!mask) {
-        if constexpr (KSP == 2 && D == 64 && DIRECT) {
-            const int64_t wgs = (int64_t)((a.Nq + 63) / 64) * a.Hq * a.B * a.n_splits;
-            if (a.n_cus > 0 && wgs <= a.n_cus) return launch<D, NQB, KSP, TYPE, false, false, DIRECT, false, 4 * BC>(a, stream);
-            return launch<D, NQB, KSP, TYPE, false, false, DIRECT, false, 2 * BC>(a, stream);
-        } else {
-            return launch<D, NQB, KSP, TYPE, false, false, DIRECT, false>(a, stream);
-        }
+        // (the others are the pipelined kernel's, see fattn_mma_launch)
+        if constexpr (DIRECT && !(D == 128 && KSP == 2)) return (int)hipErrorInvalidValue;
+        else return launch<D, NQB, KSP, TYPE, false, false, DIRECT, false>(a, stream);
     }
     if (KSP == 1 && DIRECT && v.mask_dma) return launch<D, NQB, 1, TYPE, true, false, DIRECT, DIRECT>(a, stream);
     return launch<D, NQB, KSP, TYPE, true, false, DIRECT, false>(a, stream);
@@ -1031,6 +1019,11 @@ bool fattn_mma_supported(const FattnArgs & a, int ktype) {
 int fattn_mma_launch(const FattnArgs & a, int ktype, hipStream_t stream) {
     FattnMmaVariant v;
     fattn_mma_variant(a, ktype, v);
+    // Plain attention over f16 rows is the pipelined kernel's, but for the key-split form of 128-wide heads: there a wave has
+    // few blocks, and the longer prologue costs what the loop gains (300 tokens x 30 heads 10.8 against 11.9 us a launch, 500
+    // x 20 and 800 x 8 within 2%).
+    if (ktype == MI355X_TYPE_F16 && v.direct && !a.masked && a.softcap == 0.0f && !(a.D == 128 && v.key_split == 2))
+        return fattn_pipe_launch(a, v.query_blocks, v.key_split, stream);
     switch (ktype) {
         case MI355X_TYPE_F16:  return launch_type<MI355X_TYPE_F16>(a, v, stream);
         case MI355X_TYPE_F32:  return launch_type<MI355X_TYPE_F32>(a, v, stream);

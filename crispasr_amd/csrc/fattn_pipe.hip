@@ -1,0 +1,551 @@
+// Software-pipelined f16-MFMA tile kernel for prefill / encoder attention on gfx950 (CDNA4, wave64).
+//
+// The products are those of fattn_mma.hip: v_mfma_f32_32x32x16_f16 in transposed form (S^T = K.Q^T, O^T = V^T.P^T), a
+// lane owns one query column, probabilities never leave registers.  What differs is the order.  A wave's work is a chain
+// of units - 32 queries x 32 keys - and while the exponentials of unit u run on the vector ALU, the matrix cores work on
+// the scores of unit u + 1 and on V^T.P^T of unit u - 1: nothing in a region of the loop waits for anything else in it.
+// Matrix and vector instructions of ONE wave do overlap on this chip (16 independent 32x32x16 MFMAs with 2 exponentials
+// and a conversion behind each: 299 cycles per 8, 271 for the MFMAs alone, 171 for the exponentials), so a wave alone on
+// its SIMD keeps the matrix cores busy too.
+//
+// What the loop had to be rid of to get there, each measured on the 20 x 64-wide encoder layer: taken branches in the
+// common path (about 40 cycles each for a wave alone: the steady-state loop is straight-line code and the rare path lies
+// behind it), copies of the C operand (16 registers per unit; see `first_mfma`), waits on loads just issued.
+//
+// K and V blocks of 32 keys go global -> LDS (global_load_lds_dwordx4, chunks XOR-swizzled) into a ring of 4 slots each, one
+// barrier per block; what a block's start requests is needed two or three blocks later (8 slots are no faster: a CU's path
+// from L2 into LDS gives 53 B/clk from two blocks ahead on).
+//
+// Against the tile-wise kernel it replaced for these forms, per launch: 20 x 64 x 1500^2 in batches of 4 60.2 -> 56.8 us
+// (1.08 PFLOP/s, the card's power limit: the clock falls to 1.8 GHz), 8 x 64 x 1500 against 1536 keys 14.4 -> 12.8, 8 x 128 x
+// 1500^2 x 4 55.2 -> 52.6, 10 x 128 x 1500^2 31.2 -> 23.6, 64 x 128 x 300^2 14.9 -> 12.5, 30 x 64 x 300^2 8.8 -> 7.7.
+// What is left above the MFMAs of a wave alone on its SIMD is instruction issue (about 5 cycles an instruction); where two
+// share a SIMD, the exponentials and the power limit.
+#include "fattn_row.h"
+
+#include <type_traits>
+
+namespace {
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef float    float16v __attribute__((ext_vector_type(16)));
+typedef float    float4v __attribute__((ext_vector_type(4)));
+typedef short    short4v __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+
+constexpr int   PIPE_WAVES   = 4;
+constexpr int   PIPE_THREADS = PIPE_WAVES * 64;
+constexpr int   RING         = 4;                  // slots per tensor (a power of two)
+constexpr float LOG2E        = 1.4426950408889634f;
+
+template <int D> __device__ __forceinline__ int pipe_swz_k(int r) { return D == 64 ? (r >> 1) & 7 : r & 15; }
+// (for a 32-lane half of a transposing read, rows 0 .. 3, to fall into distinct banks: 64-wide rows lie two to a bank line)
+template <int D> __device__ __forceinline__ int pipe_swz_v(int r) { return D == 64 ? ((r >> 1) & 1) << 2 : (r & 3) << 2; }
+
+// the larger of lane l's and lane (l ^ 32)'s value, without the LDS crossbar (whose traffic would blur the waits of the loop)
+__device__ __forceinline__ float max_of_halves(float x) {
+    uint32_t a = __float_as_uint(x), b = a;
+    asm volatile("" : "+v"(b));                    // (the swap of a value with itself is folded wrongly)
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// The first MFMA of a chain, whose destination is not its C operand.  As asm because the compiler ties the two in code
+// where the C operand is redefined on a rare path, and then copies 16 registers in the common one.
+__device__ __forceinline__ void first_mfma(float16v & d, half8 a, half8 b, const float16v & c) {
+    asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(d) : "v"(a), "v"(b), "v"(c));
+}
+
+// LDS by number: a kernel without static LDS finds its dynamic LDS at 0
+typedef __attribute__((address_space(3))) const half8 lds_half8;
+typedef __attribute__((address_space(3))) short4v     lds_short4;
+
+// instructions stay on their side of it
+#define PIPE_FENCE() __builtin_amdgcn_sched_barrier(0)
+
+constexpr int pipe_lds_bytes(int D, int NQB, int KSP) {
+    const int ring  = 2 * RING * KSP * 32 * D * 2;
+    const int stage = PIPE_WAVES * 32 * D * 4;                                  // result rows / the pairs' partial results
+    return ring > stage ? ring : stage;
+}
+
+// NQB: 32-query blocks per wave.  KSP = 2: waves w and w + 2 share their queries and take alternate 32-key blocks.
+// PAD: heads of a.Dv elements (a multiple of 8 below D) on copies of K and V whose rows are zero-padded to D.
+template <int D, int NQB, int KSP, bool PAD>
+__global__ void __launch_bounds__(PIPE_THREADS, 2) fattn_pipe_kernel(const FattnArgs a, const int n_qtiles) {
+    static_assert(NQB == 1 || (NQB == 2 && D == 64 && KSP == 1 && !PAD), "forms");
+    constexpr int KS   = D / 16;                                  // reduction steps of Q.K^T
+    constexpr int DB   = D / 32;                                  // 32-wide blocks of the output's d
+    constexpr int CH   = D / 8;                                   // 16-byte chunks per row
+    constexpr int ROWB = D * 2;
+    constexpr int BLKB = 32 * ROWB;                               // bytes of a block
+    constexpr int STEPB = KSP * BLKB;                             // ... of a step: one block for every wave of a pair
+    constexpr int SKEYS = KSP * 32;
+    constexpr int NLD  = STEPB / 1024 / PIPE_WAVES;               // loads per wave, step and tensor
+    constexpr int R    = RING;
+    // steps ahead of the current one that its start requests, and loads that may still be under way then
+    constexpr int DK   = R, DV = NQB == 2 ? R - 1 : R - 2;
+    constexpr int OPEN = (NQB == 2 ? R - 2 : R - 3) * 2 * NLD;
+    constexpr int BMW  = 32 * NQB;
+    constexpr int BMG  = BMW * PIPE_WAVES / KSP;
+    constexpr int NM   = KS + 2 * DB;                             // MFMAs of a region
+    constexpr int EPS  = 16 / NM;                                 // exponentials per MFMA
+    // The reference m enters the scores as the C operand of their first MFMA, 16 registers of one value, and the exponentials
+    // need no subtraction.  128-wide heads have vector instructions to spare and no registers: they subtract.
+    constexpr bool SPLAT = D == 64;
+    constexpr uint32_t VRING = R * STEPB, RMASK = R * STEPB - 1;
+
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+
+    const int tid  = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63;
+    const int l32  = lane & 31;
+    const int hh   = lane >> 5;
+    const int qgroup = KSP == 2 ? wave & 1 : wave;
+    const int kgroup = KSP == 2 ? wave >> 1 : 0;
+
+    // Workgroups go to the 8 XCDs round-robin; renumbered so that the query tiles of one (head, batch), which share K/V, sit
+    // on one XCD and meet in its L2.
+    int bid = blockIdx.x;
+    {
+        const int nb = gridDim.x;
+        const int per = nb / 8;
+        if (bid < per * 8) bid = (bid % 8) * per + bid / 8;
+    }
+    const int split = bid % a.n_splits;
+    bid /= a.n_splits;
+    const int k_begin = split * a.keys_per_split;
+    const int k_end   = min(a.Nkv, k_begin + a.keys_per_split);
+    const int qt = bid % n_qtiles;
+    const int h  = (bid / n_qtiles) % a.Hq;
+    const int b  = bid / (n_qtiles * a.Hq);
+    const int hk = h / a.gqa;
+    const int bk = b / a.bq;
+    const int q0 = qt * BMG + qgroup * BMW;
+
+    // ---- Q rows: requested first, converted behind the first requests of K and V, so that all of them are one round trip ---
+    float4v qraw[NQB][KS][2];
+#pragma unroll
+    for (int qb = 0; qb < NQB; qb++) {
+        const int qi = min(q0 + qb * 32 + l32, a.Nq - 1);
+        const float * qrow = (const float *)(a.q + (int64_t)qi * a.nbq1 + (int64_t)h * a.nbq2 + (int64_t)b * a.nbq3);
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            // (padded: a lane with nothing behind Dv reads the row's first 8 elements and scales them by zero)
+            const float * q8 = qrow + (!PAD || ks * 16 + hh * 8 < a.Dv ? ks * 16 + hh * 8 : 0);
+            qraw[qb][ks][0] = *(const float4v *)q8;
+            qraw[qb][ks][1] = *(const float4v *)(q8 + 4);
+        }
+    }
+
+    const int n_keys  = k_end - k_begin;
+    const int n_steps = (n_keys + SKEYS - 1) / SKEYS;
+    const uint64_t kbase = (uint64_t)(a.k + (int64_t)hk * a.nbk2 + (int64_t)bk * a.nbk3 + (int64_t)k_begin * a.nbk1);
+    const uint64_t vbase = (uint64_t)(a.v + (int64_t)hk * a.nbv2 + (int64_t)bk * a.nbv3 + (int64_t)k_begin * a.nbv1);
+
+    // ---- global -> LDS: slot L = (wave * NLD + j) * 64 + lane of a step holds chunk (L % CH) ^ swizzle of row L / CH ------
+    int      row[NLD];
+    uint32_t kch[NLD], vch[NLD];
+#pragma unroll
+    for (int j = 0; j < NLD; j++) {
+        const int L = (wave * NLD + j) * 64 + lane, c = L % CH;
+        row[j] = L / CH;
+        kch[j] = (uint32_t)((c ^ pipe_swz_k<D>(row[j] & 31)) * 16);
+        vch[j] = (uint32_t)((c ^ pipe_swz_v<D>(row[j] & 31)) * 16);
+    }
+    const uint32_t lds0 = wave * (NLD * 1024);
+    // (as asm: the compiler's own bookkeeping of such loads makes every LDS read that may alias them wait.  The addresses
+    //  are uniform; readfirstlane says so to the register allocator and costs nothing where it knows.)
+    auto dma = [&](uint64_t base, uint32_t off, uint32_t to) __attribute__((always_inline)) {
+        const uint64_t p = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(base >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)base);
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane((int)to)), "v"(off), "s"(p) : "memory");
+    };
+    // Requests go step by step; behind the last step they go on with its rows, and rows past its end repeat the last one
+    // (their scores are excluded, or nobody looks), so that the waits can count.
+    struct Stream {
+        uint64_t at;          // first row of the next step to be requested
+        int      left;        // its last row, counted from there
+    };
+    Stream kst = {kbase, n_keys - 1}, vst = {vbase, n_keys - 1};
+    const uint32_t nb1k = (uint32_t)a.nbk1, nb1v = (uint32_t)a.nbv1;          // (below 2^24)
+    auto request = [&](Stream & st, uint32_t nb1, const uint32_t (&ch)[NLD], uint32_t slot) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < NLD; j++) dma(st.at, __umul24((uint32_t)min(row[j], st.left), nb1) + ch[j], lds0 + slot + j * 1024);
+        const bool more = st.left >= SKEYS;
+        st.at   += more ? (uint64_t)SKEYS * nb1 : 0;
+        st.left -= more ? SKEYS : 0;
+    };
+
+    // Operand reads inside this wave's block of a slot: the address of reduction step 0 (of d block 0); step ks (block db) is
+    // that with 2 ks (4 db) XORed into the chunk index, which the swizzle passes through.
+    const uint32_t kaddr = (uint32_t)((l32 * CH + (hh ^ pipe_swz_k<D>(l32))) * 16 + kgroup * BLKB);
+    uint32_t vaddr;
+    {
+        const int i16 = lane & 15;
+        const int kr0 = hh * 4 + (i16 >> 2);
+        const int c = ((lane >> 4) & 1) * 2 + ((i16 & 3) >> 1);
+        vaddr = (uint32_t)((kr0 * CH + (c ^ pipe_swz_v<D>(kr0))) * 16 + 8 * (i16 & 1) + VRING + kgroup * BLKB);
+    }
+#pragma unroll
+    for (int j = 0; j < DK; j++) {
+        request(kst, nb1k, kch, j * STEPB);
+        if (j >= DK - DV) request(vst, nb1v, vch, VRING + (j - (DK - DV)) * STEPB);
+    }
+
+    half8 qreg[NQB][KS];                       // f16 B operands in log2 units
+#pragma unroll
+    for (int qb = 0; qb < NQB; qb++)
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            asm volatile("" : "+v"(qraw[qb][ks][0]), "+v"(qraw[qb][ks][1]));          // (not before here)
+            const float qs = !PAD || ks * 16 + hh * 8 < a.Dv ? a.scale * LOG2E : 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; e++) qreg[qb][ks][e] = (_Float16)(qraw[qb][ks][e >> 2][e & 3] * qs);
+        }
+
+    float16v oacc[NQB][DB], negm[SPLAT ? NQB : 1], s[2];
+    half8    p[2][2];
+    float    m[NQB];
+    float4v  lacc[NQB];                       // row sums: four times the same number
+#pragma unroll
+    for (int qb = 0; qb < NQB; qb++) {
+        lacc[qb] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) oacc[qb][db][r] = 0.0f;
+    }
+    half8 zero8;
+#pragma unroll
+    for (int e = 0; e < 8; e++) zero8[e] = (_Float16)0.0f;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int k = 0; k < 2; k++) p[i][k] = zero8;
+    // Row sums by the matrix cores: row i of this constant operand of v_mfma_f32_16x16x32_f16 has ones where
+    // (i / 4) % 2 == (k / 8) % 2, so that every lane finds in its accumulators the sum of the probabilities that it and
+    // the lane 32 away supply for their query - the rounded ones that V is multiplied by.
+    half8 ones;
+#pragma unroll
+    for (int e = 0; e < 8; e++) ones[e] = (_Float16)(((lane >> 2) & 1) == ((lane >> 4) & 1) ? 1.0f : 0.0f);
+
+    // Operand registers.  Two query blocks per wave: K of one block, V of one block, each used twice.  One query block: two
+    // sets of 4 MFMA operands, Y and X, that take turns - 128-wide heads: the first and second half of K, then of V.
+    constexpr bool TURNS = NQB == 1 && D == 128;
+    half8 ka[TURNS ? 4 : KS], va[TURNS ? 4 : 2 * DB];             // TURNS: Y = ka, X = va
+#pragma unroll
+    for (int i = 0; i < (TURNS ? 4 : 2 * DB); i++) va[i] = zero8;
+    auto read_k = [&](half8 (&to)[4], uint32_t slot, int ks0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) to[i] = *(lds_half8 *)((slot + kaddr) ^ (uint32_t)((ks0 + i) * 32));
+    };
+    auto read_v1 = [&](uint32_t slot, int k2, int db) __attribute__((always_inline)) {
+        lds_short4 * p0 = (lds_short4 *)(((slot + vaddr) ^ (uint32_t)(db * 64)) + k2 * 16 * ROWB);
+        const half4 lo = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(p0));
+        const half4 hi = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(p0 + ROWB));
+        return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    auto read_v = [&](half8 (&to)[4], uint32_t slot, int i0) __attribute__((always_inline)) {      // operands i0 .. i0 + 3 of (k2, db)
+#pragma unroll
+        for (int i = 0; i < 4; i++) to[i] = read_v1(slot, (i0 + i) / DB, (i0 + i) % DB);
+    };
+
+    if (NQB == 1) {
+        // the first unit multiplies the V of a step before the first one by zeros: it must be finite
+#pragma unroll
+        for (int i = 0; i < STEPB / 16 / PIPE_THREADS; i++) *(float4 *)(lds + VRING + (R - 1) * STEPB + (i * PIPE_THREADS + tid) * 16) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    // the first two blocks of K have landed
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((DK - 2 + DV) * NLD) : "memory");
+    __builtin_amdgcn_s_barrier();
+    auto exclude_past_end = [&](float16v & x, int step) __attribute__((always_inline)) {
+        int lim = n_keys - step * SKEYS - kgroup * 32 - hh * 4;
+        asm volatile("" : "+v"(lim));            // (nothing of this is worth a register in the loop)
+#pragma unroll
+        for (int r = 0; r < 16; r++) x[r] = (r >> 2) * 8 + (r & 3) < lim ? x[r] : -INFINITY;
+    };
+    // the first reference of every row: its largest score in the first block
+    {
+        half8 k1[4];
+        read_k(ka, 0, 0);
+        if (KS == 8) read_k(k1, 0, KS - 4);
+#pragma unroll
+        for (int qb = NQB - 1; qb >= 0; qb--) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) s[0][r] = 0.0f;
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) s[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ks < 4 ? ka[ks & 3] : k1[ks & 3], qreg[qb][ks], s[0], 0, 0, 0);
+            if (n_keys < SKEYS) exclude_past_end(s[0], 0);
+            float mx = s[0][0];
+#pragma unroll
+            for (int r = 1; r < 16; r++) mx = fmaxf(mx, s[0][r]);
+            mx = max_of_halves(mx);
+            m[qb] = mx > -INFINITY ? mx : 0.0f;
+            if (SPLAT) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) negm[SPLAT ? qb : 0][r] = -m[qb];
+            }
+        }
+        if (SPLAT) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) s[0][r] -= m[0];
+        }
+        if (NQB == 1) read_k(ka, STEPB, 0);      // (of a single step: what the slot holds, multiplied and not used)
+    }
+
+    int      step = 0;
+    uint32_t cur  = 0;                                            // slot of the current step
+
+    // One unit: the softmax of s[U] (query block QB), with the scores of the next unit into s[1 - U] and V^T.P^T of the one
+    // before on the matrix cores.
+    auto region = [&](auto u_tag, auto start_tag) __attribute__((always_inline)) {
+        constexpr int  U     = decltype(u_tag)::value;
+        constexpr bool START = decltype(start_tag)::value;        // the first unit of a step
+        constexpr int  QB    = NQB == 2 ? U : 0, NX = NQB == 2 ? 1 - U : 0;
+        if (START) {
+            // what was requested OPEN loads ago and earlier has landed, in every wave's share
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(OPEN) : "memory");
+            __builtin_amdgcn_s_barrier();
+            request(kst, nb1k, kch, (cur + DK * STEPB) & RMASK);
+            request(vst, nb1v, vch, VRING + ((cur + DV * STEPB) & RMASK));
+        }
+        if (__builtin_expect((step + 1) * SKEYS > n_keys, 0)) exclude_past_end(s[U], step);
+        // (one query block) operands of this region's second half
+        if (TURNS)          read_k(va, (cur + STEPB) & RMASK, KS - 4);
+        else if (NQB == 1)  read_v(va, (cur - STEPB) & RMASK, 0);
+        PIPE_FENCE();
+        float e[16];
+        float lprev;                                              // (a copy by force: else all four old sums stay in registers)
+        asm volatile("v_mov_b32 %0, %1" : "=v"(lprev) : "v"(lacc[QB][0]));
+        auto pack = [&](int i) __attribute__((always_inline)) {          // probabilities 2i, 2i + 1
+            p[U][i >> 2][(2 * i) & 7]     = (_Float16)e[2 * i];
+            p[U][i >> 2][(2 * i + 1) & 7] = (_Float16)e[2 * i + 1];
+        };
+        auto add_sums = [&](int k) __attribute__((always_inline)) { lacc[QB] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, p[U][k], lacc[QB], 0, 0, 0); };
+        int done = 0, packed = 0;
+#pragma unroll
+        for (int j = 0; j < NM; j++) {
+            // operands that take the place of those that the MFMA before has read for the last time
+            if (TURNS && j == 4)                         read_v(ka, (cur - STEPB) & RMASK, 0);
+            if (TURNS && j == 8)                         read_v(va, (cur - STEPB) & RMASK, 4);
+            if (TURNS && j == 12)                        read_k(ka, (cur + 2 * STEPB) & RMASK, 0);
+            if (!TURNS && NQB == 1 && j == KS)           read_k(ka, (cur + 2 * STEPB) & RMASK, 0);
+            if (NQB == 2 && U == 0 && j == KS)           read_k(ka, (cur + STEPB) & RMASK, 0);
+            PIPE_FENCE();
+            if (j == 0) {
+                if (SPLAT) {
+                    first_mfma(s[1 - U], ka[0], qreg[NX][0], negm[SPLAT ? NX : 0]);
+                } else {
+                    float16v none;
+#pragma unroll
+                    for (int r = 0; r < 16; r++) none[r] = 0.0f;
+                    s[1 - U] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[0], qreg[NX][0], none, 0, 0, 0);
+                }
+            }
+            else if (j < KS)  s[1 - U] = __builtin_amdgcn_mfma_f32_32x32x16_f16(TURNS && j >= 4 ? va[j & 3] : ka[j & 3], qreg[NX][j], s[1 - U], 0, 0, 0);
+            else {
+                const int i = j - KS, k2 = i / DB, db = i % DB;
+                oacc[NX][db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(TURNS ? (k2 ? va[db & 3] : ka[db & 3]) : va[i % (2 * DB)], p[1 - U][k2], oacc[NX][db], 0, 0, 0);
+            }
+#pragma unroll
+            for (int k = 0; k < EPS; k++) { e[done] = __builtin_amdgcn_exp2f(SPLAT ? s[U][done] : s[U][done] - m[QB]); done++; }
+            while (packed * 2 + 2 <= done - EPS) { pack(packed); packed++; }
+            if (j == NM - 2) add_sums(0);
+            PIPE_FENCE();
+        }
+        if (NQB == 2 && U == 0) read_v(va, cur, 0);
+#pragma unroll
+        for (; packed < 8; packed++) pack(packed);
+        add_sums(1);
+        if (NQB == 1 || U == 1) cur = (cur + STEPB) & RMASK;
+        PIPE_FENCE();
+        // A probability that left f16's range (inf, or NaN from an infinite score) shows in the row's sum: the reference has
+        // fallen 16 binary orders behind.  Wave-uniform and rare.
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(lacc[QB][0] <= 1e30f)) != 0, 0)) {
+            float mx = s[U][0];
+#pragma unroll
+            for (int r = 1; r < 16; r++) mx = fmaxf(mx, s[U][r]);
+            const float delta = fmaxf(max_of_halves(mx) - (SPLAT ? 0.0f : m[QB]), 0.0f);
+            const float f = __builtin_amdgcn_exp2f(-delta);
+            const float base = SPLAT ? delta : m[QB] + delta;      // what the scores at hand still have to come down by
+            m[QB] += delta;
+#pragma unroll
+            for (int r = 0; r < 4; r++) lacc[QB][r] = lprev * f;
+#pragma unroll
+            for (int db = 0; db < DB; db++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) oacc[QB][db][r] *= f;
+            if (SPLAT) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) negm[SPLAT ? QB : 0][r] -= delta;
+                if (NQB == 1) {          // the next unit's scores stand on the old reference
+#pragma unroll
+                    for (int r = 0; r < 16; r++) s[1 - U][r] -= delta;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                e[2 * i]     = __builtin_amdgcn_exp2f(s[U][2 * i] - base);
+                e[2 * i + 1] = __builtin_amdgcn_exp2f(s[U][2 * i + 1] - base);
+                pack(i);
+                PIPE_FENCE();
+            }
+            add_sums(0);
+            add_sums(1);
+        }
+    };
+    typedef std::integral_constant<int, 0> I0;
+    typedef std::integral_constant<int, 1> I1;
+    // V^T.P^T of the last unit
+    auto last_pv = [&](auto u_tag) __attribute__((always_inline)) {
+        constexpr int U = decltype(u_tag)::value, QB = NQB == 2 ? U : 0;
+#pragma unroll
+        for (int k2 = 0; k2 < 2; k2++)
+#pragma unroll
+            for (int db = 0; db < DB; db++) {
+                const half8 v = NQB == 2 ? va[(k2 * DB + db) % (2 * DB)] : read_v1((cur - STEPB) & RMASK, k2, db);
+                oacc[QB][db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, p[U][k2], oacc[QB][db], 0, 0, 0);
+            }
+    };
+    // (One query block: an odd number of steps is made even by one whose keys all lie past the end.  Leaving the loop in the
+    //  middle would cost the accumulators' 64 registers a copy in every turn.)
+#pragma unroll 1
+    while (step < n_steps) {
+        region(I0{}, std::true_type{});
+        if (NQB == 1) step++;
+        region(I1{}, std::integral_constant<bool, NQB == 1>{});
+        step++;
+    }
+    last_pv(I1{});
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // (what was requested behind the last step)
+
+    __syncthreads();                                   // every wave is done with the ring
+    // ---- the pairs' second waves hand their state to the first ones through LDS -------------------------------------------
+    if (KSP == 2) {
+        constexpr int XREGS = DB * 16 + 2;                 // accumulators, reference, sum: one dword per lane each
+        static_assert(2 * XREGS * 256 <= pipe_lds_bytes(D, NQB, KSP), "hand-over");
+        float * xs = (float *)lds + qgroup * (XREGS * 64) + lane;
+        if (kgroup == 1) {
+#pragma unroll
+            for (int db = 0; db < DB; db++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) xs[(db * 16 + r) * 64] = oacc[0][db][r];
+            xs[(DB * 16) * 64]     = m[0];
+            xs[(DB * 16 + 1) * 64] = lacc[0][0];
+        }
+        __syncthreads();
+        if (kgroup == 1) return;
+        // (a wave without a key of its own has a sum of zero and stands on reference 0)
+        const float mo = xs[(DB * 16) * 64], lo = xs[(DB * 16 + 1) * 64];
+        const float mn = lo == 0.0f ? m[0] : lacc[0][0] == 0.0f ? mo : fmaxf(m[0], mo);
+        const float fa = lacc[0][0] == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(m[0] - mn);
+        const float fo = lo == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(mo - mn);
+        lacc[0][0] = lacc[0][0] * fa + lo * fo;
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) oacc[0][db][r] = oacc[0][db][r] * fa + xs[(db * 16 + r) * 64] * fo;
+        m[0] = mn;
+    }
+
+    // ---- normalise and write dst[D, Hq, Nq, B], or hand the unnormalised partial to the merge kernel -----------------------
+    const int dv = PAD ? a.Dv : D;                      // dst rows are dv floats; partial rows are D apart
+    if constexpr (KSP == 1) {
+        // whole rows through LDS (32 x D floats per wave, chunks XOR-swizzled by row), 16 or 32 adjacent lanes on one row
+        constexpr int CPR = D / 4;                         // 16-byte chunks per output row
+        constexpr int RPI = 64 / CPR;                      // rows per store instruction
+        float * const stg = (float *)lds + qgroup * (32 * D);
+        const int64_t row_stride = a.n_splits > 1 ? (int64_t)a.Hq * a.n_splits * D : (int64_t)a.Hq * dv;    // floats between queries
+#pragma unroll
+        for (int qb = 0; qb < NQB; qb++) {
+            const float ltot = lacc[qb][0];
+            const float inv  = a.n_splits > 1 ? 1.0f : (ltot > 0.0f ? 1.0f / ltot : 0.0f);
+            const int   qi   = q0 + qb * 32 + l32;
+#pragma unroll
+            for (int db = 0; db < DB; db++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    float4 o;
+                    o.x = oacc[qb][db][g * 4 + 0] * inv;
+                    o.y = oacc[qb][db][g * 4 + 1] * inv;
+                    o.z = oacc[qb][db][g * 4 + 2] * inv;
+                    o.w = oacc[qb][db][g * 4 + 3] * inv;
+                    const int c = db * 8 + g * 2 + hh;
+                    *(float4 *)(stg + l32 * D + ((c ^ (l32 & (CPR - 1))) * 4)) = o;
+                }
+            __builtin_amdgcn_wave_barrier();               // (LDS serves a wave's requests in order)
+            const int     q_first = q0 + qb * 32;
+            const int64_t row0    = ((int64_t)b * a.Nq + q_first) * a.Hq + h;
+            float * const out0    = a.n_splits > 1 ? a.part_acc + (row0 * a.n_splits + split) * D : a.dst + row0 * dv;
+#pragma unroll
+            for (int k = 0; k < 32 / RPI; k++) {
+                const int row = k * RPI + lane / CPR, c = lane % CPR;
+                const float4 o = *(const float4 *)(stg + row * D + ((c ^ (row & (CPR - 1))) * 4));
+                typedef float f32x4 __attribute__((ext_vector_type(4)));
+                if (q_first + row < a.Nq && (!PAD || a.n_splits > 1 || c * 4 < a.Dv))
+                    __builtin_nontemporal_store(f32x4{o.x, o.y, o.z, o.w}, (f32x4 *)(out0 + row * row_stride + c * 4));
+            }
+            __builtin_amdgcn_wave_barrier();               // the next query block reuses the staging rows
+            if (a.n_splits > 1 && hh == 0 && qi < a.Nq) {
+                // (reference, sum) in natural-log units; a range with no visible key contributes nothing
+                float * pm = a.part_ml + ((((int64_t)b * a.Nq + qi) * a.Hq + h) * a.n_splits + split) * 2;
+                pm[0] = ltot == 0.0f ? -INFINITY : m[qb] * 0.6931471805599453f;
+                pm[1] = ltot;
+            }
+        }
+    } else {
+        // (short launches: straight from the accumulators, the detour would cost them a round trip)
+        const float ltot = lacc[0][0];
+        const float inv  = a.n_splits > 1 ? 1.0f : (ltot > 0.0f ? 1.0f / ltot : 0.0f);
+        const int   qi   = q0 + l32;
+        if (qi < a.Nq) {
+            const int64_t row = ((int64_t)b * a.Nq + qi) * a.Hq + h;
+            float * out = a.n_splits > 1 ? a.part_acc + (row * a.n_splits + split) * D : a.dst + row * dv;
+#pragma unroll
+            for (int db = 0; db < DB; db++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    float4 o;
+                    o.x = oacc[0][db][g * 4 + 0] * inv;
+                    o.y = oacc[0][db][g * 4 + 1] * inv;
+                    o.z = oacc[0][db][g * 4 + 2] * inv;
+                    o.w = oacc[0][db][g * 4 + 3] * inv;
+                    if (!PAD || a.n_splits > 1 || db * 32 + g * 8 + hh * 4 < a.Dv) *(float4 *)(out + db * 32 + g * 8 + hh * 4) = o;
+                }
+            if (a.n_splits > 1 && hh == 0) {
+                float * pm = a.part_ml + (row * a.n_splits + split) * 2;
+                pm[0] = ltot == 0.0f ? -INFINITY : m[0] * 0.6931471805599453f;
+                pm[1] = ltot;
+            }
+        }
+    }
+}
+
+template <int D, int NQB, int KSP, bool PAD>
+int launch(const FattnArgs & a, hipStream_t stream) {
+    constexpr int bmg = 32 * NQB * PIPE_WAVES / KSP, lds = pipe_lds_bytes(D, NQB, KSP);
+    const int     n_qtiles = (a.Nq + bmg - 1) / bmg;
+    const int64_t wgs = (int64_t)n_qtiles * a.Hq * a.B * a.n_splits;
+    if (wgs > 0x7fffffff) return (int)hipErrorInvalidValue;
+    static std::atomic<uint64_t> lds_allowed{0};
+    const hipError_t e = fattn_allow_lds((const void *)fattn_pipe_kernel<D, NQB, KSP, PAD>, lds, lds_allowed);
+    if (e != hipSuccess) return (int)e;
+    hipLaunchKernelGGL((fattn_pipe_kernel<D, NQB, KSP, PAD>), dim3((unsigned)wgs), dim3(PIPE_THREADS), (size_t)lds, stream, a, n_qtiles);
+    return (int)hipGetLastError();
+}
+
+}  // namespace
+
+int fattn_pipe_launch(const FattnArgs & a, int query_blocks, int key_split, hipStream_t stream) {
+    const bool pad = a.Dv != a.D;
+    if (a.D == 64) {
+        if (query_blocks == 2) return pad ? (int)hipErrorInvalidValue : launch<64, 2, 1, false>(a, stream);
+        if (key_split == 2) return pad ? launch<64, 1, 2, true>(a, stream) : launch<64, 1, 2, false>(a, stream);
+        return pad ? launch<64, 1, 1, true>(a, stream) : launch<64, 1, 1, false>(a, stream);
+    }
+    if (key_split == 2) return (int)hipErrorInvalidValue;         // (not a form of this kernel: see fattn_mma_launch)
+    return pad ? launch<128, 1, 1, true>(a, stream) : launch<128, 1, 1, false>(a, stream);
+}
