@@ -11,6 +11,20 @@
 #define FATTN_Q8_0_BYTES 34
 #define FATTN_IS_BLOCK_TYPE(t) ((t) == MI355X_TYPE_Q8_0 || (t) == MI355X_TYPE_Q4_0 || (t) == MI355X_TYPE_Q4_1 || (t) == MI355X_TYPE_Q5_0 || (t) == MI355X_TYPE_Q5_1)
 
+// Unsigned division by a number fixed on the host: n / d = (mulhi(n, m) + n) >> s for n < 2^31.
+struct FastDiv {
+    uint32_t d, m, s;
+};
+static inline FastDiv fast_div(uint32_t d) {
+    FastDiv f;
+    f.d = d;
+    f.s = 0;
+    if (d > 1) f.s = 32 - (uint32_t)__builtin_clz(d - 1);       // the smallest s with 2^s >= d
+    f.m = d ? (uint32_t)((((uint64_t)1 << 32) * (((uint64_t)1 << f.s) - d)) / d + 1) : 0;
+    return f;
+}
+static __device__ __forceinline__ uint32_t divide(uint32_t n, const FastDiv & f) { return (__umulhi(n, f.m) + n) >> f.s; }
+
 // Everything a kernel needs about one FLASH_ATTN_EXT node, by value.
 struct FattnArgs {
     const char * q;      // F32  [D, Nq, Hq, B]
@@ -57,6 +71,8 @@ struct FattnArgs {
     // workgroups that share output rows (zero between launches): every workgroup adds one when its partials are out, and
     // the one that finds the set complete merges the rows itself and leaves the counter at zero again.
     unsigned * counters;
+    // decode kernel: filled in by its launcher
+    FastDiv by_splits, by_chunks, by_hkv, by_gqa, by_bq, by_hm, by_bm;
 };
 
 // Workgroups that use more than 64 KiB of dynamic LDS need hipFuncAttributeMaxDynamicSharedMemorySize raised, and that
@@ -151,6 +167,10 @@ static __device__ __forceinline__ float group_max(float x) {
 // dies are not, for ordinary accesses): what workgroups of one launch hand to each other goes through these.
 static __device__ __forceinline__ void device_store(float * p, float v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// (p: a multiple of 8 bytes)
+static __device__ __forceinline__ void device_store2(float * p, float v0, float v1) {
+    __hip_atomic_store((uint64_t *)p, __builtin_bit_cast(uint64_t, make_float2(v0, v1)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 static __device__ __forceinline__ float2 device_load2(const float2 * p) {
     const uint64_t u = __hip_atomic_load((const uint64_t *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -302,20 +322,6 @@ static __device__ __forceinline__ void dequant8(const char * blk, int j0, float 
         }
     }
 }
-
-// Unsigned division by a number fixed on the host: n / d = (mulhi(n, m) + n) >> s for n < 2^31.
-struct FastDiv {
-    uint32_t d, m, s;
-};
-static inline FastDiv fast_div(uint32_t d) {
-    FastDiv f;
-    f.d = d;
-    f.s = 0;
-    while (((uint64_t)1 << f.s) < d) f.s++;
-    f.m = d ? (uint32_t)((((uint64_t)1 << 32) * (((uint64_t)1 << f.s) - d)) / d + 1) : 0;
-    return f;
-}
-static __device__ __forceinline__ uint32_t divide(uint32_t n, const FastDiv & f) { return (__umulhi(n, f.m) + n) >> f.s; }
 
 // One CPY / SET_ROWS node.
 struct CpyArgs {

@@ -27,6 +27,10 @@
 // register stage instead of two.  Q4_0 / Q4_1 / Q5_0 / Q5_1 rows are streamed the same way into raw K and V stages and
 // dequantised out of LDS (V into the f16 stage).  Streams and f16 rows are loaded non-temporal: they are read once.
 // Loads of the next step are in flight while the current one is consumed.  Waves are merged through LDS, splits by fattn_merge_kernel.
+//
+// Masked calls walk only the steps that one of their rows sees, and a step's mask values are requested with its K and V:
+// one step for 64 sequences of 500 to 4096 Q8_0 entries (32 query, 8 KV heads of 128) 117.6 -> 84.9 us with the pass's two
+// row writes, 3.8 TB/s over the entries seen; the bound is the bytes in flight of the longest sequences' splits.
 #include "fattn_row.h"
 
 #include <stdlib.h>
@@ -53,6 +57,7 @@ constexpr float SUM_LIMIT   = 4096.0f;             // 8 probabilities per lane a
 typedef uint32_t u32x2    __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4    __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
 
 // ---- Q8_0 in registers ------------------------------------------------------------------
 
@@ -262,7 +267,7 @@ constexpr int decode_lds_bytes() {
     constexpr int wave   = V8 ? RAWSZ + STEP * v8_pitch<D>() + D / 32 * STEP * 2
                               : STEP * (D + 32) * 2 + (RAW ? 2 * RAWSZ : 0);
     constexpr int stage  = DEC_WAVES * wave;
-    constexpr int red    = DEC_WAVES * 16 * (D + 1 + 2) * 4;
+    constexpr int red    = DEC_WAVES * 16 * (D + 4 + 2) * 4;
     return stage > red ? stage : red;
 }
 
@@ -330,8 +335,9 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
     char * v_rawst     = k_rawst + RAWSZ;                               // (!V8)
     char * v8_stage    = wave_mem + RAWSZ;                              // (V8) [32 keys][VP8]
     char * vsc_stage   = v8_stage + STEP * VP8;                         // (V8) f16 [KS][32 keys]
-    float (*red_o)[16][D + 1]      = (float (*)[16][D + 1])smem;
-    float (*red_ml)[16][2]         = (float (*)[16][2])(smem + DEC_WAVES * 16 * (D + 1) * 4);
+    // (rows D + 4 floats apart: the 16 columns of a 128-bit store start 4 banks apart)
+    float (*red_o)[16][D + 4]      = (float (*)[16][D + 4])smem;
+    float (*red_ml)[16][2]         = (float (*)[16][2])(smem + DEC_WAVES * 16 * (D + 4) * 4);
 
     const int tid  = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);     // uniform: loop control and row bases stay scalar
@@ -345,34 +351,30 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
     // the spare workgroups leave here, before any barrier, and belong to no set of the merge).
     int     split, chunk, hk, b;
     int64_t set;                                   // index of (chunk, KV head, batch): the merge's counter
-    if (a.q_chunks == 1) {
-        split = blockIdx.x % a.n_splits;
-        chunk = 0;
-        hk    = (blockIdx.x / a.n_splits) % a.Hkv;
-        b     = blockIdx.x / (a.n_splits * a.Hkv);
-        set   = blockIdx.x / a.n_splits;
-    } else {
-        // (32-bit arithmetic: the grid has fewer than 2^31 workgroups, and 64-bit divisions are loops of a hundred
-        //  instructions each - 1 us before the first request leaves)
+    // (divisions by multiply and shift: a call that is one or two steps long spends 0.3 us on five ordinary ones)
+    uint32_t pair = blockIdx.x;
+    chunk = 0;
+    if (a.q_chunks != 1) {
         const uint32_t w  = blockIdx.x >> 3;
-        const uint32_t p  = (w / (uint32_t)a.q_chunks) * 8u + (blockIdx.x & 7u);
-        const uint32_t sh = (uint32_t)a.n_splits * (uint32_t)a.Hkv;           // (<= pairs <= the grid)
-        if (p >= sh * (uint32_t)a.B) return;
-        chunk = (int)(w % (uint32_t)a.q_chunks);
-        split = (int)(p % (uint32_t)a.n_splits);
-        hk    = (int)((p / (uint32_t)a.n_splits) % (uint32_t)a.Hkv);
-        b     = (int)(p / sh);
-        set   = ((int64_t)b * a.Hkv + hk) * a.q_chunks + chunk;
+        const uint32_t wc = divide(w, a.by_chunks);
+        pair  = wc * 8u + (blockIdx.x & 7u);
+        chunk = (int)(w - wc * (uint32_t)a.q_chunks);
+        if (pair >= (uint32_t)a.n_splits * (uint32_t)a.Hkv * (uint32_t)a.B) return;      // (<= the grid)
     }
-    const int bk    = b / a.bq;
+    const uint32_t head = divide(pair, a.by_splits);
+    b     = (int)divide(head, a.by_hkv);
+    split = (int)(pair - head * (uint32_t)a.n_splits);
+    hk    = (int)head - b * a.Hkv;
+    set   = (int64_t)head * a.q_chunks + chunk;
+    const int bk    = (int)divide((uint32_t)b, a.by_bq);
 
     // row r = iq1 * gqa + gg of this KV head  <->  query iq1 of q head hk*gqa + gg; column j is row chunk*16 + j
     const int  R      = a.Nq * a.gqa;
     const int  row0   = chunk * 16;
     const bool col_ok = row0 + j < R;
     const int  jc     = col_ok ? row0 + j : row0;
-    const int  iq1    = jc / a.gqa;
-    const int  h      = hk * a.gqa + jc % a.gqa;
+    const int  iq1    = (int)divide((uint32_t)jc, a.by_gqa);
+    const int  h      = hk * a.gqa + jc - iq1 * a.gqa;
 
     const int k_begin = split * a.keys_per_split;
     const int k_end   = min(a.Nkv, k_begin + a.keys_per_split);
@@ -381,7 +383,8 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
     const char * kbase = a.k + (int64_t)hk * a.nbk2 + (int64_t)bk * a.nbk3;
     const char * vbase = a.v + (int64_t)hk * a.nbv2 + (int64_t)bk * a.nbv3;
     const uint16_t * mrow = MASK
-        ? (const uint16_t *)(a.mask + (int64_t)iq1 * a.nbm1 + (int64_t)(h % a.Hm) * a.nbm2 + (int64_t)(b % a.Bm) * a.nbm3)
+        ? (const uint16_t *)(a.mask + (int64_t)iq1 * a.nbm1 + (int64_t)(h - (int)divide((uint32_t)h, a.by_hm) * a.Hm) * a.nbm2 +
+                             (int64_t)(b - (int)divide((uint32_t)b, a.by_bm) * a.Bm) * a.nbm3)
         : nullptr;
     const float mslope = MASK ? fattn_slope(a, h) * LOG2E : 0.0f;
 
@@ -391,6 +394,41 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
     float m = 0.0f, l = 0.0f;
     bool  have = false;
 
+    const int n_steps = k_end > k_begin ? (k_end - k_begin + STEP - 1) / STEP : 0;
+
+    // (MASK) Which of the wave's steps any of the chunk's rows sees: bit t of `todo` stands for step wave + 4 t.  A step
+    // without a visible key is neither loaded nor computed - all its probabilities would be exact zeros.  The mask is looked
+    // at in up to LOOKS places of 512 keys (a lane takes 8, four lanes a step): one row over 4096 keys, or up to 8 rows over
+    // 512.  Other splits count every step as visible, and so does a slope that has underflowed to zero (0 * -inf is NaN, as
+    // it is on the CPU).  Reads stay inside [k_begin, k_end) by moving the last ones back: at worst a step is taken for
+    // visible because the one before it is.
+    constexpr int LOOKS = 8;
+    const uint32_t EXCLUDED2 = 0xFC00FC00u;                 // two masked-out keys
+    uint64_t   todo     = 0;
+    const int  windows  = (n_steps + 15) >> 4;
+    const int  mrow_0   = MASK && a.Hm == 1 ? (int)divide((uint32_t)row0, a.by_gqa) : row0;
+    const int  mrow_1   = MASK && a.Hm == 1 ? (int)divide((uint32_t)min(row0 + 15, R - 1), a.by_gqa) : min(row0 + 15, R - 1);
+    const int  looks    = mrow_1 == mrow_0 ? windows : mrow_1 - mrow_0 + 1;
+    const bool skipping = MASK && k_end - k_begin >= 8 && looks <= LOOKS && (windows == 1 || mrow_1 == mrow_0) &&
+                          __builtin_amdgcn_ballot_w64(!(mslope > 0.0f)) == 0;
+    auto look_at = [&](int i) __attribute__((always_inline)) {
+        const int r   = mrow_1 == mrow_0 ? mrow_0 : min(mrow_0 + i, mrow_1);
+        const int riq = a.Hm == 1 ? r : (int)divide((uint32_t)r, a.by_gqa);
+        const int rh  = a.Hm == 1 ? 0 : hk * a.gqa + r - riq * a.gqa;
+        const int hm  = a.Hm == 1 ? 0 : rh - (int)divide((uint32_t)rh, a.by_hm) * a.Hm;
+        const int key = min(k_begin + (mrow_1 == mrow_0 ? i * 512 : 0) + lane * 8, k_end - 8);
+        return *(const u32x4_a2 *)(a.mask + (int64_t)riq * a.nbm1 + (int64_t)hm * a.nbm2 +
+                                   (int64_t)(b - (int)divide((uint32_t)b, a.by_bm) * a.Bm) * a.nbm3 + (int64_t)key * 2);
+    };
+    // takes the wave's next visible step (n_steps or more: none left) after step `it`
+    auto next_step = [&](int it) __attribute__((always_inline)) {
+        if (!skipping) return it + DEC_WAVES;
+        if (todo == 0) return n_steps;
+        const int t = (int)__builtin_ctzll(todo);
+        todo &= todo - 1;
+        return wave + t * DEC_WAVES;
+    };
+
     // loads of one step: K in operand layout (key = kb*16 + j, chunk = ks*4 + g4), V in row order
     Chunk kraw[2][RAW ? 1 : 2][RAW ? 1 : KS];
     Chunk vraw[2][RAW ? 1 : NV];
@@ -399,11 +437,26 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
     unit_t kun[2][RAW ? NU : 1], vun[2][RAW ? NU : 1];
     // (V8) LDS offsets from wave_mem of the pieces of this lane's V units, two to a register
     uint32_t vdst[V8 ? NU : 1][V8 ? PCS / 2 : 1];
+    // mask values of the lane's eight keys of the step, in the order of its scores
+    u32x2_a2 mraw[2][MASK ? 2 : 1];
     // a partial last step: its loads are clamped to the last valid row or unit (branch-free, in bounds) and the
     // keys they stand for are excluded in the step
     auto issue = [&](int it, auto stage) __attribute__((always_inline)) {
         constexpr int s = decltype(stage)::value;
         const int j0 = k_begin + it * STEP;
+        if constexpr (MASK) {
+#pragma unroll
+            for (int kb = 0; kb < 2; kb++) {
+                const int key = j0 + (V8 ? g4 * 8 + kb * 4 : kb * 16 + g4 * 4);
+                if (j0 + STEP <= k_end) {
+                    mraw[ONE ? 0 : s][kb] = *(const u32x2_a2 *)(mrow + key);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 2; r++)
+                        mraw[ONE ? 0 : s][kb][r] = (uint32_t)mrow[min(key + 2 * r, k_end - 1)] | (uint32_t)mrow[min(key + 2 * r + 1, k_end - 1)] << 16;
+                }
+            }
+        }
         if (RAW) {
             // one coalesced stream per tensor
             const int last = min(STEP, k_end - j0) * (RS / UNIT) - 1;
@@ -436,16 +489,20 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
         }
     };
 
-    const int n_steps = k_end > k_begin ? (k_end - k_begin + STEP - 1) / STEP : 0;
     typedef std::integral_constant<int, 0> S0;
 
-    // one step of 32 keys out of register stage s; the following step is requested into the other stage
-    auto step = [&](const int it, auto stage) __attribute__((always_inline)) {
+    // one step of 32 keys out of register stage s; the wave's following step `nxt` is requested into the other stage
+    auto step = [&](const int it, const int nxt, auto stage) __attribute__((always_inline)) {
         constexpr int s = decltype(stage)::value;
         const int  j0   = k_begin + it * STEP;
         const bool tail = j0 + STEP > k_end;                  // wave-uniform
         // the following step's loads: into the other register stage, or (V8) into this one as soon as it is in LDS
-        if (!ONE && it + DEC_WAVES < n_steps) issue(it + DEC_WAVES, std::integral_constant<int, 1 - s>{});
+        if (!ONE && nxt < n_steps) issue(nxt, std::integral_constant<int, 1 - s>{});
+        u32x2_a2 mcur[2];                                     // (V8's next request overwrites the stage)
+        if (MASK) {
+            mcur[0] = mraw[ONE ? 0 : s][0];
+            mcur[1] = mraw[ONE ? 0 : s][MASK ? 1 : 0];
+        }
 
         if (RAW) {
 #pragma unroll
@@ -476,7 +533,7 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
                     }
                 }
             }
-            if (ONE && it + DEC_WAVES < n_steps) issue(it + DEC_WAVES, stage);
+            if (ONE && nxt < n_steps) issue(nxt, stage);
             if (!V8 && tail) {
                 // rows past k_end hold bytes of no row: a zero scale keeps what is made of them finite
 #pragma unroll
@@ -533,7 +590,7 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
             for (int r = 0; r < 4; r++) {
                 const int key = V8 ? j0 + g4 * 8 + kb * 4 + r : j0 + kb * 16 + g4 * 4 + r;
                 float x = sc[kb][r];
-                if (MASK) x = fmaf(mslope, h2f_bits(mrow[min(key, k_end - 1)]), x);
+                if (MASK) x = fmaf(mslope, h2f_bits((uint16_t)(mcur[kb][r >> 1] >> (16 * (r & 1)))), x);
                 if (tail && key >= k_end) x = -INFINITY;
                 sv[kb * 4 + r] = x - m;
             }
@@ -607,7 +664,44 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
         }
         __builtin_amdgcn_wave_barrier();
     };
+    // The look at the mask goes out ahead of the first K/V request, and that ahead of its answer: the request is for the
+    // wave's first step, seen or not, and repeated for the first seen one.
+    u32x4_a2 look[LOOKS];
+    if (skipping) {
+#pragma unroll
+        for (int i = 0; i < LOOKS; i++) look[i] = u32x4_a2{EXCLUDED2, EXCLUDED2, EXCLUDED2, EXCLUDED2};
+        look[0] = look_at(0);
+        if (looks > 1) {
+#pragma unroll
+            for (int i = 1; i < LOOKS; i++) look[i] = look_at(i);
+        }
+    }
     if (wave < n_steps) issue(wave, S0{});
+    int it = wave;
+    if (skipping) {
+        auto any = [&](const u32x4_a2 & w) __attribute__((always_inline)) {
+            return ((w[0] ^ EXCLUDED2) | (w[1] ^ EXCLUDED2) | (w[2] ^ EXCLUDED2) | (w[3] ^ EXCLUDED2)) != 0;
+        };
+        // lane t takes over step wave + 4 t: lanes 4 (step % 16) .. + 3 of window t / 4
+        const int mine = wave + lane * DEC_WAVES;
+        uint64_t  win  = 0;
+        if (mrow_1 == mrow_0) {
+#pragma unroll
+            for (int i = 0; i < LOOKS; i++) {
+                const uint64_t v = __builtin_amdgcn_ballot_w64(any(look[i]));
+                win = mine >> 4 == i ? v : win;
+            }
+        } else {
+            bool seen = false;
+#pragma unroll
+            for (int i = 0; i < LOOKS; i++) seen = seen || any(look[i]);
+            const uint64_t v = __builtin_amdgcn_ballot_w64(seen);
+            win = mine < 16 ? v : 0;
+        }
+        todo = __builtin_amdgcn_ballot_w64(mine < n_steps && ((uint32_t)(win >> ((mine & 15) * 4)) & 15u) != 0);
+        it = next_step(wave);
+        if (it != wave && it < n_steps) issue(it, S0{});
+    }
 
     // (V8) where the pieces of this lane's V units go: read behind the first K/V request, needed when that has arrived
     if (V8) {
@@ -641,9 +735,14 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
             qreg[ks] = v;
         }
     }
-    for (int it = wave; it < n_steps; it += 2 * DEC_WAVES) {
-        step(it, S0{});
-        if (it + DEC_WAVES < n_steps) step(it + DEC_WAVES, std::integral_constant<int, ONE ? 0 : 1>{});
+    while (it < n_steps) {
+        const int n1 = next_step(it);
+        step(it, n1, S0{});
+        it = n1;
+        if (n1 < n_steps) {
+            it = next_step(n1);
+            step(n1, it, std::integral_constant<int, ONE ? 0 : 1>{});
+        }
     }
 
     // ---- column totals, then the four waves through LDS ----------------------------------------------
@@ -652,16 +751,14 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
     if (!have) m = -INFINITY;
     __syncthreads();                           // every wave is done with its stage
 #pragma unroll
-    for (int db = 0; db < DBK; db++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) red_o[wave][j][db * 16 + g4 * 4 + r] = oacc[db][r];
+    for (int db = 0; db < DBK; db++) *(float4v *)&red_o[wave][j][db * 16 + g4 * 4] = oacc[db];
     if (g4 == 0) {
         red_ml[wave][j][0] = m;
         red_ml[wave][j][1] = l;
     }
     __syncthreads();
 
-    // thread t: column t / 16, a strided set of d
+    // thread t: column t / 16, D / 64 groups of four d
     const int col = tid >> 4;
     bool bad = false;                           // this column's result is not finite
     if (row0 + col < R) {
@@ -677,21 +774,36 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
             L += red_ml[w][col][1] * f[w];
         }
         bad = not_finite(L);
-        const int     ciq1 = (row0 + col) / a.gqa;
-        const int     ch   = hk * a.gqa + (row0 + col) % a.gqa;
+        const int     ciq1 = (int)divide((uint32_t)(row0 + col), a.by_gqa);
+        const int     ch   = hk * a.gqa + row0 + col - ciq1 * a.gqa;
         const int64_t row  = ((int64_t)b * a.Nq + ciq1) * a.Hq + ch;
         const int dv = PAD ? a.Dv : D;              // dst rows are dv floats; partial rows stay D apart
-        for (int d = tid & 15; d < dv; d += 16) {
-            float acc = 0.0f;
 #pragma unroll
-            for (int w = 0; w < DEC_WAVES; w++) acc += red_o[w][col][d] * f[w];
-            bad = bad || not_finite(acc);
+        for (int k = 0; k < D / 64; k++) {
+            const int d = ((tid & 15) + k * 16) * 4;
+            if (PAD && d >= dv) continue;
+            float4v acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int w = 0; w < DEC_WAVES; w++) {
+                const float4v o = *(const float4v *)&red_o[w][col][d];
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[e] += o[e] * f[w];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++) bad = bad || not_finite(acc[e]);
             if (a.n_splits == 1) {
-                a.dst[row * dv + d] = L > 0.0f ? acc / L : 0.0f;
-            } else if (a.counters) {
-                device_store(a.part_acc + (row * a.n_splits + split) * D + d, acc);
+                float4v o;
+#pragma unroll
+                for (int e = 0; e < 4; e++) o[e] = L > 0.0f ? acc[e] / L : 0.0f;
+                *(float4v *)(a.dst + row * dv + d) = o;
             } else {
-                a.part_acc[(row * a.n_splits + split) * D + d] = acc;
+                float * pa = a.part_acc + (row * a.n_splits + split) * D + d;
+                if (a.counters) {
+                    device_store2(pa, acc[0], acc[1]);
+                    device_store2(pa + 2, acc[2], acc[3]);
+                } else {
+                    *(float4v *)pa = acc;
+                }
             }
         }
         if (a.n_splits > 1 && (tid & 15) == 0) {
@@ -699,8 +811,7 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
             float * pm = a.part_ml + (row * a.n_splits + split) * 2;
             const float mn = M == -INFINITY ? -INFINITY : M * 0.6931471805599453f;
             if (a.counters) {
-                device_store(pm, mn);
-                device_store(pm + 1, L);
+                device_store2(pm, mn, L);
             } else {
                 pm[0] = mn;
                 pm[1] = L;
@@ -732,13 +843,21 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
         constexpr int LPR = D / 4;                  // lanes per row: 8 or 4 rows per pass
         for (int c = tid / LPR; c < 16 && row0 + c < R; c += DEC_THREADS / LPR) {
             const int r = row0 + c;
-            fattn_merge_row<true>(a, ((int64_t)b * a.Nq + r / a.gqa) * a.Hq + hk * a.gqa + r % a.gqa, tid % LPR);
+            const int riq = (int)divide((uint32_t)r, a.by_gqa);
+            fattn_merge_row<true>(a, ((int64_t)b * a.Nq + riq) * a.Hq + hk * a.gqa + r - riq * a.gqa, tid % LPR);
         }
     }
 }
 
 template <int D, int TYPE, bool MASK, bool RAW, bool V8 = false, bool PAD = false>
-int launch_one(const FattnArgs & a, hipStream_t stream) {
+int launch_one(FattnArgs a, hipStream_t stream) {
+    a.by_splits = fast_div((uint32_t)a.n_splits);
+    a.by_chunks = fast_div((uint32_t)a.q_chunks);
+    a.by_hkv    = fast_div((uint32_t)a.Hkv);
+    a.by_gqa    = fast_div((uint32_t)a.gqa);
+    a.by_bq     = fast_div((uint32_t)a.bq);
+    a.by_hm     = fast_div((uint32_t)a.Hm);
+    a.by_bm     = fast_div((uint32_t)a.Bm);
     const int64_t pairs = (int64_t)a.n_splits * a.Hkv * a.B;
     const int64_t wgs   = a.q_chunks == 1 ? pairs : (pairs + 7) / 8 * 8 * a.q_chunks;      // as the kernel numbers them
     if (wgs > 0x7fffffff || a.q_chunks != (a.Nq * a.gqa + 15) / 16) return (int)hipErrorInvalidValue;
