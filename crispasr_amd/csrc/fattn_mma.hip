@@ -60,6 +60,8 @@ constexpr int   MMA_THREADS = MMA_WAVES * 64;
 constexpr int   BC          = 64;                 // keys per tile
 constexpr float LOG2E       = 1.4426950408889634f;
 
+constexpr int   TRIM_TILES  = 8;                  // see `trim`: a shorter loop has less to lose than the look costs (about 1 us)
+
 template <int D> struct Pitch {
     static constexpr int K = D + 8;               // halves: (2D + 16) bytes = 16 mod 128
     static constexpr int V = D + 32;              // halves: (2D + 64) bytes = 64 mod 128
@@ -172,6 +174,8 @@ __global__ void __launch_bounds__(MMA_THREADS, 2) fattn_mma_kernel(const FattnAr
     // file (two query blocks per wave, 128-wide heads without key split) answer it with spills inside the tile loop, so
     // it is left to the others: the key-split form and one query block of 64-wide heads.
     constexpr bool SKIP = MASK && (KSP == 2 || (D == 64 && NQB == 1));
+    // The others do not walk the tiles at the end of the key range that none of the workgroup's queries sees: see `trim`.
+    constexpr bool TRIM = MASK && DIRECT && !SKIP;
 
     extern __shared__ __attribute__((aligned(16))) _Float16 lds_raw[];
     _Float16 (*k_lds)[BC * PK] = (_Float16 (*)[BC * PK])lds_raw;
@@ -186,20 +190,31 @@ __global__ void __launch_bounds__(MMA_THREADS, 2) fattn_mma_kernel(const FattnAr
     // Workgroups are handed to the 8 XCDs round-robin; renumber them so that the query tiles
     // of one (head, batch) - which share K/V - sit on one XCD and hit its L2.
     int bid = blockIdx.x;
-    {
-        const int nb = gridDim.x;
-        const int per = nb / 8;
-        if (bid < per * 8) bid = (bid % 8) * per + bid / 8;
-    }
+    const int nb = gridDim.x, per = nb / 8;
+    if (bid < per * 8) bid = (bid % 8) * per + bid / 8;
     // key range of this workgroup: everything, or one of n_splits ranges of whole tiles (few query tiles on many
     // CUs; the partial results then go through fattn_merge_kernel)
     const int split = bid % a.n_splits;
     bid /= a.n_splits;
     const int k_begin = split * a.keys_per_split;
     const int k_end   = min(a.Nkv, k_begin + a.keys_per_split);
-    const int qt = bid % n_qtiles;
-    const int h  = (bid / n_qtiles) % a.Hq;
-    const int b  = bid / (n_qtiles * a.Hq);
+    int qt = bid % n_qtiles, pair = bid / n_qtiles;
+    if (MASK && a.n_splits == 1 && per * 8 == nb && per % n_qtiles == 0) {
+        // Workgroups of a masked call differ in length (causal rows, padded sequences).  An XCD's are ordered from the last
+        // query tile to the first, and every second group of n_cus / 8 - the ones that join the group before on its CUs -
+        // backwards, so that a CU's two add up to about the same (2048 causal tokens, 32 heads of 128, with what `trim`
+        // saves: 76 us a layer against 79 without the turn and 89 in the plain order; 16 heads of 64, which skip block by
+        // block instead: 56 -> 51).
+        const int cus = a.n_cus >= 8 ? a.n_cus / 8 : 32, heads = per / n_qtiles;
+        int i = blockIdx.x / 8;
+        const int seg = i / cus * cus;
+        if ((i / cus) & 1) i = seg + min(cus, per - seg) - 1 - (i - seg);
+        qt   = n_qtiles - 1 - i / heads;
+        pair = (int)(blockIdx.x % 8) * heads + i % heads;
+    }
+    // (masked: the batch runs faster than the head, or the longest sequence of a padded batch would be one XCD's alone)
+    const int h = MASK ? pair / a.B : pair % a.Hq;
+    const int b = MASK ? pair % a.B : pair / a.Hq;
     const int hk = h / a.gqa;
     const int bk = b / a.bq;
 
@@ -689,15 +704,65 @@ __global__ void __launch_bounds__(MMA_THREADS, 2) fattn_mma_kernel(const FattnAr
         }
     };
 
-    const int n_tiles = (k_end - k_begin + BC - 1) / BC;
-    const int n_full  = (k_end - k_begin) / BC;
+    int n_tiles = (k_end - k_begin + BC - 1) / BC;
+    int n_full  = (k_end - k_begin) / BC;
+
+    // TRIM: a wave looks at the last 64 keys of its last 8 queries while the first tile is on its way (that is all an
+    // unpadded sequence costs: one row of 512 keys for each query of 8 cost a launch over per-head masks 4 of 73 us); if
+    // none of them is seen, at the rows of all its queries, 4 tiles at a time from the end on, until it meets a visible key.
+    // What is read there is what the tiles themselves would have read.  Requests stay inside the rows by moving the last
+    // ones back: at worst a tile is kept because the one before it is seen.  A slope that has underflowed to zero trims
+    // nothing (0 * -inf is NaN, as it is on the CPU).
+    // 2048 causal tokens behind 2048 rows, 32 query and 8 KV heads of 128: 171 -> 146 us a layer with its row writes, without
+    // the 2048 rows 106 -> 76; 8 sequences of 400 to 750 frames under per-head masks 51.3 -> 48.8 (the masks' own bytes are
+    // read either way).  In the forms that skip block by block the look costs more than it saves (300 tokens, key split: 17.3
+    // -> 20 us).
+    typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+    const bool trim = TRIM && n_tiles >= TRIM_TILES && mslope > 0.0f;
+    auto mask_keys = [&](int row, int key) __attribute__((always_inline)) {
+        return *(const u32x4_a2 *)(a.mask + (int64_t)(h % a.Hm) * a.nbm2 + (int64_t)(b % a.Bm) * a.nbm3 +
+                                   (int64_t)min(q0 + row, a.Nq - 1) * a.nbm1 + (int64_t)min(key, k_end - 8) * 2);
+    };
+    auto any_seen = [&](const u32x4_a2 & w) __attribute__((always_inline)) {                   // (0xFC00: a masked-out key)
+        return (w[0] ^ 0xFC00FC00u) | (w[1] ^ 0xFC00FC00u) | (w[2] ^ 0xFC00FC00u) | (w[3] ^ 0xFC00FC00u);
+    };
+    auto last_seen = [&]() __attribute__((always_inline)) {        // tiles up to the last one that the wave's queries see
+        for (int hi = n_tiles; hi > 0;) {
+            const int lo  = max(hi - 4, 0);
+            const int key = k_begin + lo * BC + (lane & 31) * 8;   // 32 lanes a row, 8 keys a lane
+            u32x4_a2  w[16];
+            uint32_t  any = 0;
+#pragma unroll
+            for (int r = 0; r < BMW / 2; r += 16) {
+#pragma unroll
+                for (int i = 0; i < 16; i++) w[i] = mask_keys((r + i) * 2 + (lane >> 5), key);
+#pragma unroll
+                for (int i = 0; i < 16; i++) any |= any_seen(w[i]);
+            }
+            const uint64_t v2 = __builtin_amdgcn_ballot_w64(any != 0);
+            const uint32_t v  = (uint32_t)v2 | (uint32_t)(v2 >> 32);
+            if (v) return min(hi, lo + (31 - __builtin_clz(v)) / 8 + 1);
+            hi = lo;
+        }
+        return 1;
+    };
+
     if (DIRECT) {
         char * const lb = (char *)lds_raw;               // K0 K1 V0 V1 [mask: per wave 2 half-tile blocks]
         char * const mb = lb + 4 * TILEB;
         load_direct(k_begin, lb, lb + 2 * TILEB, n_full == 0);
         if (MDMA && n_full > 0) load_mask_half(k_begin, 0, mb, 0.0f);
         if (MPRE && n_full > 0) load_mask_ahead(k_begin);
+        u32x4_a2 end_keys = {0u, 0u, 0u, 0u};
+        if (trim) end_keys = mask_keys(BMW - 8 + (lane >> 3), k_begin + (n_tiles - 1) * BC + (lane & 7) * 8);
         load_q();
+        if (trim) {
+            int * const wn = (int *)(lb + TILEB);    // (K1 is not requested before the second barrier)
+            wn[wave] = __builtin_amdgcn_ballot_w64(any_seen(end_keys) != 0) ? n_tiles : last_seen();
+            __syncthreads();
+            const int nt = max(max(wn[0], wn[1]), max(wn[2], wn[3]));
+            if (nt < n_tiles) n_tiles = n_full = nt; // (no partial tile is left then)
+        }
         __builtin_amdgcn_s_waitcnt(0x0F70);          // vmcnt(0): this wave's share of the tile is in LDS
         __syncthreads();
         // Two workgroups share a CU, and the SIMD's arbiter prefers the older wave: left alone, the first
