@@ -22,11 +22,17 @@
 //   mask = f16(scale * BD + add), s = S + mask in log2 units, online softmax against a reference that is raised
 //          only when a row's maximum outgrows it by a factor 256, P -> f16
 //   O^T += V^T . P^T                            8 MFMAs, A = V tile through ds_read_b64_tr_b16, B = P from registers
-// The four waves need the same table rows one step apart, so the table is staged once per workgroup in a ring of five
-// 32-row blocks.  K tiles and table blocks move global -> LDS without passing registers (global_load_lds_dwordx4, the
-// 16-byte chunks of a row XOR-swizzled so that the operand reads are conflict-free), requested behind the first barrier
-// of a step and waited for before the second; V is fetched one step ahead into registers and written behind the second.  K, V and the table are f16 with 16-byte aligned rows (the caller rounds F32 ones first, as
-// the reference's own graph does for the mask product's operands).
+// The waves need the same table rows one step apart, so the table is staged once per workgroup in a ring of 32-row blocks,
+// one more than there are waves.  K and V tiles and table blocks move global -> LDS without passing registers
+// (global_load_lds_dwordx4, the 16-byte chunks of a row XOR-swizzled so that the operand reads are conflict-free).  A step
+// requests the next one's into the halves and the slot that the step before it has left, and one barrier at its end waits
+// for them: K and V have two halves each.  K, V and the table are f16 with 16-byte aligned rows (the caller rounds F32 ones
+// first, as the reference's own graph does for the mask product's operands).
+//
+// What bounds it: the chain of a step - operand reads, product, un-skew, exponentials, product - with 1 to 2 waves on a SIMD
+// (8 x 8 heads of 128 x 750: matrix cores busy 17%, vector ALU 25%, waves waiting 41% of their cycles; neither the
+// additive mask's loads nor the blocks' are what they wait for).  Against one half, two barriers a step and operand reads two
+// at a time: 8 heads x 128, calls of 1000 tokens x 4 78.4 -> 72.6 us, 750 x 8 90.9 -> 87.7; 8 x 64, 750 x 8 62.7 -> 57.
 #include "fattn_row.h"
 
 #include <stdlib.h>
@@ -52,8 +58,8 @@ constexpr float FR_SUM_LIMIT = 4096.0f;               // a tile's 16 probabiliti
 template <int D> constexpr int fr_kp() { return 2 * D; }          // bytes per K / table row in LDS (chunks swizzled, no padding)
 template <int D> __device__ __forceinline__ int fr_swz(int r) { return D == 64 ? (r >> 1) & 7 : r & 15; }
 template <int D> __device__ __forceinline__ int fr_swz_v(int r) { return D == 64 ? r & 7 : (r & 3) << 2; }
-// K tile, V tile, NW + 1 table blocks (NW in use, one being written), one un-skew square per wave
-template <int D, int NW> constexpr int fr_lds_bytes() { return (2 + NW + 1) * 32 * fr_kp<D>() + NW * 32 * FR_SQP * 4; }
+// two K tiles, two V tiles, NW + 1 table blocks (NW in use, one being written), one un-skew square per wave
+template <int D, int NW> constexpr int fr_lds_bytes() { return (4 + NW + 1) * 32 * fr_kp<D>() + NW * 32 * FR_SQP * 4; }
 
 template <int D, int NW, bool ADD, bool ADD_F16>
 __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) fattn_relpos_kernel(const FattnRelposArgs a) {
@@ -63,10 +69,10 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     constexpr int CH  = D / 8;                      // 16-byte chunks per row
     constexpr int KP  = fr_kp<D>();
 
-    extern __shared__ __attribute__((aligned(16))) char fr_lds[];
-    char * const kt   = fr_lds;
-    char * const vt   = kt + 32 * KP;
-    char * const ring = vt + 32 * KP;
+    extern __shared__ __attribute__((aligned(256))) char fr_lds[];
+    char * const kt   = fr_lds;                     // tile t: half t % 2
+    char * const vt   = kt + 2 * 32 * KP;
+    char * const ring = vt + 2 * 32 * KP;
     const int tid  = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
@@ -105,26 +111,46 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     // tile, the ends of the table) repeat the nearest valid row: they belong to excluded keys or to no key at all.
     constexpr int TI  = 32 * CH * 16 / 1024;                  // 64-lane instructions per tile
     constexpr int NDM = (TI + NW - 1) / NW;                   // ... per wave: instruction j of wave w is number j * NW + w
-    typedef __attribute__((address_space(3))) void * lds_vptr;
-    typedef const __attribute__((address_space(1))) void * glb_vptr;
+    // Instruction number ins moves rows ins * RPI .. + RPI - 1: the lane's row and chunk in it are the same for every ins but
+    // for one or two bits of the K layout's swizzle, so that an instruction's addresses cost two operations.
+    constexpr int RPI = 64 / CH;
+    const int      lr = lane / CH, lc = lane % CH;
+    const uint32_t ck = (uint32_t)((lc ^ fr_swz<D>(lr)) * 16), cv = (uint32_t)((lc ^ fr_swz_v<D>(lr)) * 16);
+    static_assert(RPI == 4 || RPI == 8, "the swizzles of rows r and r + RPI * ins differ by 4 * (ins % (16 / RPI)) (K) or not at all (V)");
+    // (as asm: the compiler's own bookkeeping of such loads makes every LDS read that may alias them wait)
+    auto dma = [&](uint64_t at, uint32_t off, uint32_t to) __attribute__((always_inline)) {
+        const uint64_t p = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at);
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane((int)to)), "v"(off), "s"(p) : "memory");
+    };
+    // Rows row0 .. row0 + 31 of a tensor, in one of two layouts.  (NW = 3: the last wave repeats an instruction of the one before.)
     auto dma_rows = [&](char * dst, const char * base, int64_t nb1, int row0, int last_row, auto is_v) __attribute__((always_inline)) {
-        const bool inside = row0 >= 0 && row0 + 31 <= last_row;      // uniform
-        const char * p = base + (int64_t)(inside ? row0 : 0) * nb1;
+        constexpr bool V      = decltype(is_v)::value;
+        const uint32_t to     = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)dst;
+        const uint32_t nb     = (uint32_t)nb1;                        // (row offsets inside a tile are 32-bit)
+        uint32_t       lrow   = (uint32_t)lr;
+        asm volatile("" : "+v"(lrow));                                // (its products are not worth registers in the loop)
+        if (__builtin_expect(row0 >= 0 && row0 + 31 <= last_row, 1)) {
+            const uint64_t at = (uint64_t)(base + (int64_t)row0 * nb1);
 #pragma unroll
-        for (int j = 0; j < NDM; j++) {
-            const int ins = j * NW + wave;                            // uniform
-            if (TI % NW != 0 && ins >= TI) break;
-            const int L = ins * 64 + lane, r = L / CH;
-            const int c = (L % CH) ^ (decltype(is_v)::value ? fr_swz_v<D>(r) : fr_swz<D>(r));
-            const int rr = inside ? r : min(max(row0 + r, 0), last_row);
-            __builtin_amdgcn_global_load_lds((glb_vptr)(p + ((uint32_t)rr * (uint32_t)nb1 + (uint32_t)c * 16u)),
-                                             (lds_vptr)(dst + ins * 1024), 16, 0, 0);
+            for (int j = 0; j < NDM; j++) {
+                const uint32_t ins = min((uint32_t)(j * NW + wave), (uint32_t)TI - 1);         // uniform
+                dma(at + ins * RPI * nb, lrow * nb + (V ? cv : ck ^ ((ins & (16 / RPI - 1)) * 64)), to + ins * 1024);
+            }
+        } else {
+            const int      first = min(max(row0, 0), last_row);
+            const uint64_t at    = (uint64_t)(base + (int64_t)first * nb1);
+#pragma unroll 1
+            for (int j = 0; j < NDM; j++) {
+                const uint32_t ins = min((uint32_t)(j * NW + wave), (uint32_t)TI - 1);
+                const uint32_t rr  = (uint32_t)(min(max(row0 + (int)ins * RPI + lr, 0), last_row) - first);
+                dma(at, rr * nb + (V ? cv : ck ^ ((ins & (16 / RPI - 1)) * 64)), to + ins * 1024);
+            }
         }
     };
     typedef std::integral_constant<bool, false> KLayout;
     typedef std::integral_constant<bool, true>  VLayout;
-    auto dma_k = [&](int t) __attribute__((always_inline)) { dma_rows(kt, kbase, a.nbk1, 32 * t, a.Nkv - 1, KLayout{}); };
-    auto dma_v = [&](int t) __attribute__((always_inline)) { dma_rows(vt, vbase, a.nbv1, 32 * t, a.Nkv - 1, VLayout{}); };
+    auto dma_k = [&](int t) __attribute__((always_inline)) { dma_rows(kt + (t & 1) * 32 * KP, kbase, a.nbk1, 32 * t, a.Nkv - 1, KLayout{}); };
+    auto dma_v = [&](int t) __attribute__((always_inline)) { dma_rows(vt + (t & 1) * 32 * KP, vbase, a.nbv1, 32 * t, a.Nkv - 1, VLayout{}); };
     auto slot_of = [&](int beta) { return ring + ((beta + NW - 1) % FR_SLOTS) * 32 * KP; };   // beta >= 1 - NW
     auto dma_r = [&](int beta) __attribute__((always_inline)) { dma_rows(slot_of(beta), rbase, a.nbr1, p_base0 + 32 * beta, NR - 1, KLayout{}); };
 
@@ -150,9 +176,8 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
         }
     }
     constexpr int AES = ADD_F16 ? 2 : 4;
-    const char * addrow = nullptr;                  // the query's row of the additive mask; addp walks it, 32 keys a step
+    const char * addrow = nullptr;                  // the query's row of the additive mask
     if (ADD) addrow = a.add + (int64_t)iq * a.nba1 + (int64_t)(h % a.Ha) * a.nba2 + (int64_t)(b % a.Ba) * a.nba3;
-    const char * addp = addrow + 4 * hh * AES;
     // Keys beyond the length of a padded sequence carry -inf in the additive mask for every query: tiles that are masked
     // out entirely at the END of the key range add nothing and are not walked at all.  Each wave looks at its queries'
     // last tile while the first blocks are on their way (that is all an unpadded sequence costs) and, if that one is
@@ -205,44 +230,51 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
         // (the four floats behind each row of a square are padding that nothing else writes)
         if (lane == 0) ((int *)(ring + FR_SLOTS * 32 * KP))[32 + wave] = live;
     }
-    __builtin_amdgcn_s_waitcnt(0x0F70);               // vmcnt(0): this wave's share of the blocks is in LDS
-    __syncthreads();
+    // every wave's share of what it requested is in LDS, and every wave is done with what it read there
+    auto meet = [&]() __attribute__((always_inline)) {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    meet();
     if (ADD) {
         NTL = 0;
 #pragma unroll
         for (int w = 0; w < NW; w++) NTL = max(NTL, ((const int *)(ring + FR_SLOTS * 32 * KP))[32 + w]);
     }
 
-    // operand reads of a K or table block: lane (il, hh) takes d = 16 ks + 8 hh .. +7 of row il
-    uint32_t opaddr[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) opaddr[ks] = (uint32_t)((il * CH + ((ks * 2 + hh) ^ fr_swz<D>(il))) * 16);
+    // operand reads of a K or table block: lane (il, hh) takes d = 16 ks + 8 hh .. +7 of row il.  (Tiles and blocks lie at
+    // multiples of their size, so the address of operand ks is that of operand 0 with the bits of ks turned over.)
+    const uint32_t op0 = (uint32_t)((il * CH + (hh ^ fr_swz<D>(il))) * 16);
     // transposing reads of the V tile: lane j16 of a group of 16 addresses key 4 hh + j16 / 4 (+ 8, + 16 ks) and four
     // values of d from 32 db + 16 (group % 2) + 4 (j16 % 4) on; the swizzle depends on key % 8 only
-    uint32_t vaddr[DBO];
+    uint32_t va0;
     {
         const int j16 = lane & 15, G16 = lane >> 4, kr0 = 4 * (G16 >> 1) + (j16 >> 2);
-#pragma unroll
-        for (int db = 0; db < DBO; db++) {
-            const int c = 4 * db + 2 * (G16 & 1) + ((j16 & 3) >> 1);
-            vaddr[db] = (uint32_t)((kr0 * CH + (c ^ fr_swz_v<D>(kr0))) * 16 + 8 * (j16 & 1));
-        }
+        const int c = 2 * (G16 & 1) + ((j16 & 3) >> 1);
+        va0 = (uint32_t)((kr0 * CH + (c ^ fr_swz_v<D>(kr0))) * 16 + 8 * (j16 & 1));
     }
+    typedef __attribute__((address_space(3))) const half8 lds_half8;
+    typedef __attribute__((address_space(3))) short4v lds_short4;
+    auto lds_at = [&](const char * p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char *)p; };
 
-    auto block_times_q = [&](const char * blk, const half8 (&q)[KS]) __attribute__((always_inline)) {
+    auto read_block = [&](half8 (&to)[KS], const char * blk) __attribute__((always_inline)) {
+        const uint32_t at = lds_at(blk) + op0;
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) to[ks] = *(lds_half8 *)(uintptr_t)(at ^ (ks * 32));
+    };
+    auto times_q = [&](const half8 (&block)[KS], const half8 (&q)[KS]) __attribute__((always_inline)) {
         float16v acc;
+        asm("v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=&v"(acc) : "v"(block[0]), "v"(q[0]));       // (no 16 registers to clear)
 #pragma unroll
-        for (int r = 0; r < 16; r++) acc[r] = 0.0f;
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            const half8 av = *(const half8 *)(blk + opaddr[ks]);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, q[ks], acc, 0, 0, 0);
-        }
+        for (int ks = 1; ks < KS; ks++) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(block[ks], q[ks], acc, 0, 0, 0);
         return acc;
     };
 
     // the wave's block 0 (= block -wave in wave 0's numbering): its lower-right triangle is the first tile's
-    float16v bd_prev = block_times_q(slot_of(-wave), qv);
+    half8 ops[KS];
+    read_block(ops, slot_of(-wave));
+    float16v bd_prev = times_q(ops, qv);
 
     float16v oacc[DBO];
 #pragma unroll
@@ -257,49 +289,57 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     const int x_lane = il + 4 * hh + 1;
     const int sq_new = il * FR_SQP + x_lane, sq_prev = sq_new - 32;
 
+    // the additive mask's values of a tile: requested when the tile before is done with its own, waited for with that
+    // tile's blocks
+    typedef typename std::conditional<ADD_F16, half4_a2, float4_a4>::type araw_t;
+    araw_t araw[ADD ? 4 : 1];
+    auto load_add = [&](int t) __attribute__((always_inline)) {
+        if (__builtin_expect(32 * t + 32 <= a.Nkv, 1)) {
+#pragma unroll
+            for (int g = 0; g < 4; g++) araw[ADD ? g : 0] = *(const araw_t *)(addrow + ((int64_t)32 * t + 8 * g + 4 * hh) * AES);
+        } else {
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    const int key = min(32 * t + 8 * g + 4 * hh + c, a.Nkv - 1);
+                    if constexpr (ADD_F16) araw[ADD ? g : 0][c] = *(const _Float16 *)(addrow + (int64_t)key * 2);
+                    else                   araw[ADD ? g : 0][c] = *(const float *)(addrow + (int64_t)key * 4);
+                }
+        }
+    };
+    // (the compiler's wait for them belongs here, behind that of `meet`: further down it would wait for the blocks on their way)
+    auto have_add = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int g = 0; g < 4; g++) asm volatile("" : "+v"(araw[ADD ? g : 0]));
+    };
+    if (ADD) load_add(0);
+    meet();                                            // block 1 - NW has been read: its slot takes the next one
+    if (ADD) have_add();
+
 #pragma unroll 1
     for (int t = 0; t < NTL; t++) {
         const bool tail = 32 * t + 32 > a.Nkv;             // uniform
-        // the additive mask of this tile: requested first, used after the products.  The values stay as loaded until
-        // then (a conversion inside the branch below would have to wait for its load right there, four round trips a step)
-        typedef typename std::conditional<ADD_F16, half4_a2, float4_a4>::type araw_t;
-        araw_t araw[4];
-        if (ADD) {
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const int key0 = 32 * t + 8 * g + 4 * hh;
-                if (!tail) {
-                    araw[g] = *(const araw_t *)(addp + 8 * g * AES);
-                } else {
-#pragma unroll
-                    for (int c = 0; c < 4; c++) {
-                        const int key = min(key0 + c, a.Nkv - 1);
-                        if constexpr (ADD_F16) araw[g][c] = *(const _Float16 *)(addrow + (int64_t)key * 2);
-                        else                   araw[g][c] = *(const float *)(addrow + (int64_t)key * 4);
-                    }
-                }
-            }
-        }
-        if (ADD) addp += 32 * AES;
-        // ---- the position product against this step's table block; select per slot, un-skew through the square ------
-        {
-            const float16v bd_new = block_times_q(slot_of(t + 1 - wave), qv);
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int  k_r  = 8 * (r >> 2) + (r & 3);
-                const bool prev = x_lane + k_r >= 32;
-                sq[(prev ? sq_prev : sq_new) + k_r] = prev ? bd_prev[r] : bd_new[r];
-            }
-            bd_prev = bd_new;
-        }
-        // ---- the content product against this step's K tile -------------------------------------------------------------
-        const float16v s = block_times_q(kt, qu);
-        __builtin_amdgcn_s_waitcnt(0x0F70);               // vmcnt(0): this wave's share of the V tile is in LDS
-        __syncthreads();                                  // every wave has read the K tile and its table block; the V tile is complete
+        read_block(ops, slot_of(t + 1 - wave));
+        // the next step's blocks: into the halves and the slot that the step before this one has left
         if (t + 1 < NTL) {
             dma_k(t + 1);
             dma_r(t + 2);
+            dma_v(t + 1);
         }
+        // ---- the position product against this step's table block, the content product against its K tile -------------
+        half8 kops[KS];
+        read_block(kops, kt + (t & 1) * 32 * KP);
+        const float16v bd_new = times_q(ops, qv);
+        const float16v s = times_q(kops, qu);
+        // (beside the second product) select per slot, un-skew through the square
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int  k_r  = 8 * (r >> 2) + (r & 3);
+            const bool prev = x_lane + k_r >= 32;
+            sq[(prev ? sq_prev : sq_new) + k_r] = prev ? bd_prev[r] : bd_new[r];
+        }
+        bd_prev = bd_new;
 
         // ---- mask = f16(scale * BD + add); scores in log2 units ------------------------------------------------------
         float s2[16];
@@ -319,7 +359,8 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
                 for (int e = 0; e < 2; e++) s2[4 * g + c + e] = fmaf((float)mh[e], FR_LOG2E, s[4 * g + c + e]);
             }
         }
-        if (tail) {                                        // keys past the end of the last tile
+        if (ADD && t + 1 < NTL) load_add(t + 1);
+        if (__builtin_expect(tail, 0)) {                   // keys past the end of the last tile
 #pragma unroll
             for (int r = 0; r < 16; r++)
                 if (32 * t + 8 * (r >> 2) + 4 * hh + (r & 3) >= a.Nkv) s2[r] = -INFINITY;
@@ -366,21 +407,21 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 
         // ---- O^T += V^T . P^T -------------------------------------------------------------------------------------------
         {
+            const uint32_t v_at = lds_at(vt + (t & 1) * 32 * KP) + va0;
 #pragma unroll
             for (int db = 0; db < DBO; db++) {
 #pragma unroll
                 for (int ks = 0; ks < 2; ks++) {
-                    const char * p0 = vt + vaddr[db] + 16 * ks * KP;
-                    const half4 lo = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)p0));
-                    const half4 hi = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)(p0 + 8 * KP)));
+                    const uint32_t p0 = (v_at ^ (db * 64)) + 16 * ks * KP;
+                    const half4 lo = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)(uintptr_t)p0));
+                    const half4 hi = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)(uintptr_t)(p0 + 8 * KP)));
                     const half8 va = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
                     oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, p[ks], oacc[db], 0, 0, 0);
                 }
             }
         }
-        __builtin_amdgcn_s_waitcnt(0x0F70);               // vmcnt(0): this wave's share of the next K tile and table block is in LDS
-        __syncthreads();                                  // every wave has read the V tile; the next K tile and table block are complete
-        if (t + 1 < NTL) dma_v(t + 1);
+        meet();
+        if (ADD) have_add();
     }
 
     // ---- normalise and store: lane (il, hh) holds d = 32 db + 8 g + 4 hh + c of its query -------------------------------
@@ -454,11 +495,19 @@ bool fattn_relpos_supported(const FattnRelposArgs & a) {
 
 int fattn_relpos_launch(const FattnRelposArgs & a, hipStream_t stream) {
     if (!fattn_relpos_supported(a)) return (int)hipErrorInvalidValue;
-    // Workgroups of 2, 3 or 4 waves (32 queries each).  Every workgroup stages all K, V and table tiles of its head and pays
-    // a step's barriers and waits whatever its width, so the widest one that the queries fill is taken (measured at
-    // 8 heads x 128, T = 750, batch 8: 4 waves, 384 workgroups: 74 us; 3 waves, 512 workgroups: 80 us; 2 waves, 768: 81 us).
+    // Workgroups of 2, 3 or 4 waves (32 queries each): the widest one that the queries fill.  128-wide heads have LDS for one
+    // workgroup of 4 waves on a CU or for two of 3, and take what fills the chip in fewer rounds.  A 32-key step was measured
+    // to take about 1.8 us with 4 waves on the CU, 1.7 with 3 and 3.0 with two times 3 (8 heads: 750 tokens x 8 87.7 us a
+    // call with 3 waves against 112 with 4, 1000 x 4 88.9 against 72.6; 4 heads, 1000 x 4 56.8 against 59.1).
     int best = (a.Nq + 31) / 32;
     best = best < 2 ? 2 : best > 4 ? 4 : best;
+    if (a.D == 128 && best == 4) {
+        const int64_t heads = (int64_t)a.H * a.B, cus = a.n_cus > 0 ? a.n_cus : 256;
+        const int64_t wg3 = (a.Nq + 95) / 96 * heads, wg4 = (a.Nq + 127) / 128 * heads;
+        const int64_t rest = wg3 % (2 * cus);
+        const int64_t t3 = wg3 / (2 * cus) * 30 + (rest == 0 ? 0 : rest <= cus ? 17 : 30), t4 = (wg4 + cus - 1) / cus * 18;
+        if (t3 < t4) best = 3;
+    }
     static const char * force = getenv("MI355X_RELPOS_WAVES");            // experiments only
     if (force && atoi(force) >= 2 && atoi(force) <= 4) best = atoi(force);
     switch (best) {
