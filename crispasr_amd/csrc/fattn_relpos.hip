@@ -32,7 +32,7 @@
 // What bounds it: the chain of a step - operand reads, product, un-skew, exponentials, product - with 1 to 2 waves on a SIMD
 // (8 x 8 heads of 128 x 750: matrix cores busy 17%, vector ALU 25%, waves waiting 41% of their cycles; neither the
 // additive mask's loads nor the blocks' are what they wait for).  Against one half, two barriers a step and operand reads two
-// at a time: 8 heads x 128, calls of 1000 tokens x 4 78.4 -> 72.6 us, 750 x 8 90.9 -> 87.7; 8 x 64, 750 x 8 62.7 -> 57.
+// at a time: 8 heads x 128, calls of 1000 tokens x 4 78.4 -> 73.0 us, 750 x 8 90.9 -> 86.0; 8 x 64, 750 x 8 62.7 -> 56.9.
 #include "fattn_row.h"
 
 #include <stdlib.h>
@@ -123,13 +123,14 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane((int)to)), "v"(off), "s"(p) : "memory");
     };
     // Rows row0 .. row0 + 31 of a tensor, in one of two layouts.  (NW = 3: the last wave repeats an instruction of the one before.)
-    auto dma_rows = [&](char * dst, const char * base, int64_t nb1, int row0, int last_row, auto is_v) __attribute__((always_inline)) {
+    auto dma_rows = [&](char * dst, const char * base, int64_t nb1, int row0, int last_row, auto is_v, auto is_first) __attribute__((always_inline)) {
         constexpr bool V      = decltype(is_v)::value;
+        constexpr bool FIRST  = decltype(is_first)::value;            // before the loop: one form for all, instructions are cold
         const uint32_t to     = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)dst;
         const uint32_t nb     = (uint32_t)nb1;                        // (row offsets inside a tile are 32-bit)
         uint32_t       lrow   = (uint32_t)lr;
         asm volatile("" : "+v"(lrow));                                // (its products are not worth registers in the loop)
-        if (__builtin_expect(row0 >= 0 && row0 + 31 <= last_row, 1)) {
+        if (!FIRST && __builtin_expect(row0 >= 0 && row0 + 31 <= last_row, 1)) {
             const uint64_t at = (uint64_t)(base + (int64_t)row0 * nb1);
 #pragma unroll
             for (int j = 0; j < NDM; j++) {
@@ -139,7 +140,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
         } else {
             const int      first = min(max(row0, 0), last_row);
             const uint64_t at    = (uint64_t)(base + (int64_t)first * nb1);
-#pragma unroll 1
+#pragma unroll (FIRST ? NDM : 1)
             for (int j = 0; j < NDM; j++) {
                 const uint32_t ins = min((uint32_t)(j * NW + wave), (uint32_t)TI - 1);
                 const uint32_t rr  = (uint32_t)(min(max(row0 + (int)ins * RPI + lr, 0), last_row) - first);
@@ -149,16 +150,16 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     };
     typedef std::integral_constant<bool, false> KLayout;
     typedef std::integral_constant<bool, true>  VLayout;
-    auto dma_k = [&](int t) __attribute__((always_inline)) { dma_rows(kt + (t & 1) * 32 * KP, kbase, a.nbk1, 32 * t, a.Nkv - 1, KLayout{}); };
-    auto dma_v = [&](int t) __attribute__((always_inline)) { dma_rows(vt + (t & 1) * 32 * KP, vbase, a.nbv1, 32 * t, a.Nkv - 1, VLayout{}); };
+    auto dma_k = [&](int t, auto first) __attribute__((always_inline)) { dma_rows(kt + (t & 1) * 32 * KP, kbase, a.nbk1, 32 * t, a.Nkv - 1, KLayout{}, first); };
+    auto dma_v = [&](int t, auto first) __attribute__((always_inline)) { dma_rows(vt + (t & 1) * 32 * KP, vbase, a.nbv1, 32 * t, a.Nkv - 1, VLayout{}, first); };
     auto slot_of = [&](int beta) { return ring + ((beta + NW - 1) % FR_SLOTS) * 32 * KP; };   // beta >= 1 - NW
-    auto dma_r = [&](int beta) __attribute__((always_inline)) { dma_rows(slot_of(beta), rbase, a.nbr1, p_base0 + 32 * beta, NR - 1, KLayout{}); };
+    auto dma_r = [&](int beta, auto first) __attribute__((always_inline)) { dma_rows(slot_of(beta), rbase, a.nbr1, p_base0 + 32 * beta, NR - 1, KLayout{}, first); };
 
     // ---- prologue: table blocks 1 - NW .. 1, the first K and V tiles, Q_u and Q_v as B operands ---------------------
 #pragma unroll 1
-    for (int beta = 1 - NW; beta <= 1; beta++) dma_r(beta);
-    dma_k(0);
-    dma_v(0);
+    for (int beta = 1 - NW; beta <= 1; beta++) dma_r(beta, std::true_type{});
+    dma_k(0, std::true_type{});
+    dma_v(0, std::true_type{});
     half8 qu[KS], qv[KS];
     {
         const float * pu = (const float *)(a.qu + (int64_t)iq * a.nbu1 + (int64_t)h * a.nbu2 + (int64_t)b * a.nbu3);
@@ -265,9 +266,10 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     };
     auto times_q = [&](const half8 (&block)[KS], const half8 (&q)[KS]) __attribute__((always_inline)) {
         float16v acc;
-        asm("v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=&v"(acc) : "v"(block[0]), "v"(q[0]));       // (no 16 registers to clear)
 #pragma unroll
-        for (int ks = 1; ks < KS; ks++) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(block[ks], q[ks], acc, 0, 0, 0);
+        for (int r = 0; r < 16; r++) acc[r] = 0.0f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(block[ks], q[ks], acc, 0, 0, 0);
         return acc;
     };
 
@@ -323,9 +325,9 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
         read_block(ops, slot_of(t + 1 - wave));
         // the next step's blocks: into the halves and the slot that the step before this one has left
         if (t + 1 < NTL) {
-            dma_k(t + 1);
-            dma_r(t + 2);
-            dma_v(t + 1);
+            dma_k(t + 1, std::false_type{});
+            dma_r(t + 2, std::false_type{});
+            dma_v(t + 1, std::false_type{});
         }
         // ---- the position product against this step's table block, the content product against its K tile -------------
         half8 kops[KS];
@@ -499,8 +501,11 @@ int fattn_relpos_launch(const FattnRelposArgs & a, hipStream_t stream) {
     // workgroup of 4 waves on a CU or for two of 3, and take what fills the chip in fewer rounds.  A 32-key step was measured
     // to take about 1.8 us with 4 waves on the CU, 1.7 with 3 and 3.0 with two times 3 (8 heads: 750 tokens x 8 87.7 us a
     // call with 3 waves against 112 with 4, 1000 x 4 88.9 against 72.6; 4 heads, 1000 x 4 56.8 against 59.1).
+    // 64-wide heads are never slower with 3 waves than with 4 (120 tokens x 4 heads 12.6 against 13.9 us, 180 x 4 13.6 against
+    // 15.0, 750 x 64 56.7 against 57.6).
+    const int most = a.D == 64 ? 3 : 4;
     int best = (a.Nq + 31) / 32;
-    best = best < 2 ? 2 : best > 4 ? 4 : best;
+    best = best < 2 ? 2 : best > most ? most : best;
     if (a.D == 128 && best == 4) {
         const int64_t heads = (int64_t)a.H * a.B, cus = a.n_cus > 0 ? a.n_cus : 256;
         const int64_t wg3 = (a.Nq + 95) / 96 * heads, wg4 = (a.Nq + 127) / 128 * heads;
@@ -509,10 +514,10 @@ int fattn_relpos_launch(const FattnRelposArgs & a, hipStream_t stream) {
         if (t3 < t4) best = 3;
     }
     static const char * force = getenv("MI355X_RELPOS_WAVES");            // experiments only
-    if (force && atoi(force) >= 2 && atoi(force) <= 4) best = atoi(force);
+    if (force && atoi(force) >= 2 && atoi(force) <= most) best = atoi(force);
     switch (best) {
         case 2:  return a.D == 64 ? launch_d<64, 2>(a, stream) : launch_d<128, 2>(a, stream);
         case 3:  return a.D == 64 ? launch_d<64, 3>(a, stream) : launch_d<128, 3>(a, stream);
-        default: return a.D == 64 ? launch_d<64, 4>(a, stream) : launch_d<128, 4>(a, stream);
+        default: return launch_d<128, 4>(a, stream);
     }
 }
