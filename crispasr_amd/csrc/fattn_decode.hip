@@ -28,9 +28,9 @@
 // dequantised out of LDS (V into the f16 stage).  Streams and f16 rows are loaded non-temporal: they are read once.
 // Loads of the next step are in flight while the current one is consumed.  Waves are merged through LDS, splits by fattn_merge_kernel.
 //
-// Masked calls walk only the steps that one of their rows sees, and a step's mask values are requested with its K and V:
-// one step for 64 sequences of 500 to 4096 Q8_0 entries (32 query, 8 KV heads of 128) 117.6 -> 84.9 us with the pass's two
-// row writes, 3.8 TB/s over the entries seen; the bound is the bytes in flight of the longest sequences' splits.
+// Masked calls walk the steps between the first and the last that one of their rows sees, and a step's mask values are
+// requested with its K and V: one step for 64 sequences of 500 to 4096 Q8_0 entries (32 query, 8 KV heads of 128) 115 -> 81 us,
+// 3.8 TB/s over the entries seen; the bound is the bytes in flight of the longest sequences' splits.
 #include "fattn_row.h"
 
 #include <stdlib.h>
@@ -382,10 +382,10 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
     half8 qreg[KS];
     const char * kbase = a.k + (int64_t)hk * a.nbk2 + (int64_t)bk * a.nbk3;
     const char * vbase = a.v + (int64_t)hk * a.nbv2 + (int64_t)bk * a.nbv3;
-    const uint16_t * mrow = MASK
-        ? (const uint16_t *)(a.mask + (int64_t)iq1 * a.nbm1 + (int64_t)(h - (int)divide((uint32_t)h, a.by_hm) * a.Hm) * a.nbm2 +
-                             (int64_t)(b - (int)divide((uint32_t)b, a.by_bm) * a.Bm) * a.nbm3)
-        : nullptr;
+    const char * mhead = MASK ? a.mask + (int64_t)(h - (int)divide((uint32_t)h, a.by_hm) * a.Hm) * a.nbm2 +
+                                (int64_t)(b - (int)divide((uint32_t)b, a.by_bm) * a.Bm) * a.nbm3
+                              : nullptr;
+    const uint16_t * mrow = (const uint16_t *)(mhead + (int64_t)iq1 * a.nbm1);
     const float mslope = MASK ? fattn_slope(a, h) * LOG2E : 0.0f;
 
     float4v oacc[DBK];
@@ -396,37 +396,28 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
 
     const int n_steps = k_end > k_begin ? (k_end - k_begin + STEP - 1) / STEP : 0;
 
-    // (MASK) Which of the wave's steps any of the chunk's rows sees: bit t of `todo` stands for step wave + 4 t.  A step
-    // without a visible key is neither loaded nor computed - all its probabilities would be exact zeros.  The mask is looked
-    // at in up to LOOKS places of 512 keys (a lane takes 8, four lanes a step): one row over 4096 keys, or up to 8 rows over
-    // 512.  Other splits count every step as visible, and so does a slope that has underflowed to zero (0 * -inf is NaN, as
-    // it is on the CPU).  Reads stay inside [k_begin, k_end) by moving the last ones back: at worst a step is taken for
-    // visible because the one before it is.
-    constexpr int LOOKS = 8;
+    // (MASK) Which of the wave's steps any of the chunk's rows sees: a step without a visible key adds exact zeros, so the wave
+    // walks those between its first and its last visible one.  Two requests of 8 keys a lane, four lanes a step, see one row
+    // over 32 steps of the wave (a split of 4096 keys) or 8 rows of a mask without heads over 4 (512 keys).  Other splits count
+    // every step as visible, and so does a slope that has underflowed to zero (0 * -inf is NaN, as it is on the CPU).  Reads stay
+    // inside [k_begin, k_end) by moving the last ones back: at worst a step is taken for visible because the one before it is.
+    // A look costs 0.3 us and is worth it from two steps a wave on, where it can save one: 5 beams against 140 entries, 20 heads
+    // of 64, 4.8 us without it, 5.2 with it, 6.1 where every wave looked at all of its split; a 2048-entry cache of which 100
+    // are written, 16 query, 8 KV heads of 128, 10.3, 9.2 and 9.9 us.  Splits of one step a wave never look.
     const uint32_t EXCLUDED2 = 0xFC00FC00u;                 // two masked-out keys
-    uint64_t   todo     = 0;
-    const int  windows  = (n_steps + 15) >> 4;
-    const int  mrow_0   = MASK && a.Hm == 1 ? (int)divide((uint32_t)row0, a.by_gqa) : row0;
-    const int  mrow_1   = MASK && a.Hm == 1 ? (int)divide((uint32_t)min(row0 + 15, R - 1), a.by_gqa) : min(row0 + 15, R - 1);
-    const int  looks    = mrow_1 == mrow_0 ? windows : mrow_1 - mrow_0 + 1;
-    const bool skipping = MASK && k_end - k_begin >= 8 && looks <= LOOKS && (windows == 1 || mrow_1 == mrow_0) &&
-                          __builtin_amdgcn_ballot_w64(!(mslope > 0.0f)) == 0;
-    auto look_at = [&](int i) __attribute__((always_inline)) {
-        const int r   = mrow_1 == mrow_0 ? mrow_0 : min(mrow_0 + i, mrow_1);
-        const int riq = a.Hm == 1 ? r : (int)divide((uint32_t)r, a.by_gqa);
-        const int rh  = a.Hm == 1 ? 0 : hk * a.gqa + r - riq * a.gqa;
-        const int hm  = a.Hm == 1 ? 0 : rh - (int)divide((uint32_t)rh, a.by_hm) * a.Hm;
-        const int key = min(k_begin + (mrow_1 == mrow_0 ? i * 512 : 0) + lane * 8, k_end - 8);
-        return *(const u32x4_a2 *)(a.mask + (int64_t)riq * a.nbm1 + (int64_t)hm * a.nbm2 +
-                                   (int64_t)(b - (int)divide((uint32_t)b, a.by_bm) * a.Bm) * a.nbm3 + (int64_t)key * 2);
+    int        walk = wave, walk_end = n_steps;             // the steps that the wave walks
+    const int  iq_0    = MASK ? (int)divide((uint32_t)row0, a.by_gqa) : 0;
+    const int  iq_1    = MASK ? (int)divide((uint32_t)min(row0 + 15, R - 1), a.by_gqa) : 0;
+    const bool one_row = iq_1 == iq_0;
+    const bool looking = MASK && n_steps > DEC_WAVES && (one_row ? n_steps <= 128 : n_steps <= 16 && iq_1 - iq_0 < 8) && (a.Hm == 1 || R == 1) &&
+                         __builtin_amdgcn_ballot_w64(!(mslope > 0.0f)) == 0;
+    auto look_key = [&](int i) __attribute__((always_inline)) {         // the first of the lane's 8 keys of request i
+        const int t = one_row ? i * 16 + (lane >> 2) : (lane >> 2) & 3;
+        return k_begin + (wave + t * DEC_WAVES) * STEP + (lane & 3) * 8;
     };
-    // takes the wave's next visible step (n_steps or more: none left) after step `it`
-    auto next_step = [&](int it) __attribute__((always_inline)) {
-        if (!skipping) return it + DEC_WAVES;
-        if (todo == 0) return n_steps;
-        const int t = (int)__builtin_ctzll(todo);
-        todo &= todo - 1;
-        return wave + t * DEC_WAVES;
+    auto look_at = [&](int i) __attribute__((always_inline)) {
+        const int row = one_row ? iq_0 : min(iq_0 + i * 4 + (lane >> 4), iq_1);
+        return *(const u32x4_a2 *)(mhead + (int64_t)row * a.nbm1 + (int64_t)min(look_key(i), k_end - 8) * 2);
     };
 
     // loads of one step: K in operand layout (key = kb*16 + j, chunk = ks*4 + g4), V in row order
@@ -444,17 +435,30 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
     auto issue = [&](int it, auto stage) __attribute__((always_inline)) {
         constexpr int s = decltype(stage)::value;
         const int j0 = k_begin + it * STEP;
-        if constexpr (MASK) {
+        // (One branch for the eight values where a step's registers are many; the int8 V form, with one register stage, is up to
+        //  3% faster on large batches with one branch for each four.)
+        if constexpr (MASK && V8) {
 #pragma unroll
             for (int kb = 0; kb < 2; kb++) {
-                const int key = j0 + (V8 ? g4 * 8 + kb * 4 : kb * 16 + g4 * 4);
+                const int key = j0 + g4 * 8 + kb * 4;
                 if (j0 + STEP <= k_end) {
-                    mraw[ONE ? 0 : s][kb] = *(const u32x2_a2 *)(mrow + key);
+                    mraw[0][kb] = *(const u32x2_a2 *)(mrow + key);
                 } else {
 #pragma unroll
                     for (int r = 0; r < 2; r++)
-                        mraw[ONE ? 0 : s][kb][r] = (uint32_t)mrow[min(key + 2 * r, k_end - 1)] | (uint32_t)mrow[min(key + 2 * r + 1, k_end - 1)] << 16;
+                        mraw[0][kb][r] = (uint32_t)mrow[min(key + 2 * r, k_end - 1)] | (uint32_t)mrow[min(key + 2 * r + 1, k_end - 1)] << 16;
                 }
+            }
+        } else if constexpr (MASK) {
+            if (__builtin_expect(j0 + STEP <= k_end, 1)) {
+#pragma unroll
+                for (int kb = 0; kb < 2; kb++) mraw[s][kb] = *(const u32x2_a2 *)(mrow + j0 + kb * 16 + g4 * 4);
+            } else {
+                uint32_t w[8];
+#pragma unroll
+                for (int e = 0; e < 8; e++) w[e] = mrow[min(j0 + (e >> 2) * 16 + g4 * 4 + (e & 3), k_end - 1)];
+#pragma unroll
+                for (int e = 0; e < 8; e += 2) mraw[s][e >> 2][(e >> 1) & 1] = w[e] | w[e + 1] << 16;
             }
         }
         if (RAW) {
@@ -497,7 +501,7 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
         const int  j0   = k_begin + it * STEP;
         const bool tail = j0 + STEP > k_end;                  // wave-uniform
         // the following step's loads: into the other register stage, or (V8) into this one as soon as it is in LDS
-        if (!ONE && nxt < n_steps) issue(nxt, std::integral_constant<int, 1 - s>{});
+        if (!ONE && nxt < walk_end) issue(nxt, std::integral_constant<int, 1 - s>{});
         u32x2_a2 mcur[2];                                     // (V8's next request overwrites the stage)
         if (MASK) {
             mcur[0] = mraw[ONE ? 0 : s][0];
@@ -533,7 +537,7 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
                     }
                 }
             }
-            if (ONE && nxt < n_steps) issue(nxt, stage);
+            if (ONE && nxt < walk_end) issue(nxt, stage);
             if (!V8 && tail) {
                 // rows past k_end hold bytes of no row: a zero scale keeps what is made of them finite
 #pragma unroll
@@ -664,43 +668,63 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
         }
         __builtin_amdgcn_wave_barrier();
     };
-    // The look at the mask goes out ahead of the first K/V request, and that ahead of its answer: the request is for the
-    // wave's first step, seen or not, and repeated for the first seen one.
-    u32x4_a2 look[LOOKS];
-    if (skipping) {
+    // ---- Q: requested here and converted to f16 B operands, in log2 units, once the loads that follow are on their way ------
+    float qraw[KS][8];
+    auto request_q = [&]() __attribute__((always_inline)) {
+        const float * qrow = (const float *)(a.q + (int64_t)iq1 * a.nbq1 + (int64_t)h * a.nbq2 + (int64_t)b * a.nbq3);
 #pragma unroll
-        for (int i = 0; i < LOOKS; i++) look[i] = u32x4_a2{EXCLUDED2, EXCLUDED2, EXCLUDED2, EXCLUDED2};
-        look[0] = look_at(0);
-        if (looks > 1) {
+        for (int ks = 0; ks < KS; ks++) {
+            // (PAD: every lane reads 8 elements that exist, its own or the row's first 8 where it has none, and the lanes
+            //  without scale them by zero: under a guard each, the 8 * KS loads waited for one another - 2 us per call.  A q row
+            //  with inf or NaN in it gives NaN either way.)
+            const float * q8 = qrow + (!PAD || ks * 32 + g4 * 8 < a.Dv ? ks * 32 + g4 * 8 : 0);
 #pragma unroll
-            for (int i = 1; i < LOOKS; i++) look[i] = look_at(i);
+            for (int e = 0; e < 8; e++) qraw[ks][e] = q8[e];
         }
-    }
-    if (wave < n_steps) issue(wave, S0{});
-    int it = wave;
-    if (skipping) {
-        auto any = [&](const u32x4_a2 & w) __attribute__((always_inline)) {
-            return ((w[0] ^ EXCLUDED2) | (w[1] ^ EXCLUDED2) | (w[2] ^ EXCLUDED2) | (w[3] ^ EXCLUDED2)) != 0;
-        };
-        // lane t takes over step wave + 4 t: lanes 4 (step % 16) .. + 3 of window t / 4
-        const int mine = wave + lane * DEC_WAVES;
-        uint64_t  win  = 0;
-        if (mrow_1 == mrow_0) {
+    };
+    auto convert_q = [&]() __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < LOOKS; i++) {
-                const uint64_t v = __builtin_amdgcn_ballot_w64(any(look[i]));
-                win = mine >> 4 == i ? v : win;
+        for (int ks = 0; ks < KS; ks++) {
+            const float qs = !PAD || ks * 32 + g4 * 8 < a.Dv ? a.scale * LOG2E : 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; e++) qreg[ks][e] = (_Float16)(qraw[ks][e] * qs);
+        }
+    };
+
+    // The look at the mask and Q go out ahead of the first K/V request, that ahead of their answers, so that all of them are
+    // one round trip; the request is for the wave's first step, seen or not.
+    if constexpr (MASK) {
+        u32x4_a2 look[2] = {{EXCLUDED2, EXCLUDED2, EXCLUDED2, EXCLUDED2}, {EXCLUDED2, EXCLUDED2, EXCLUDED2, EXCLUDED2}};
+        if (looking) {
+            look[0] = look_at(0);
+            if (one_row ? n_steps > 64 : iq_1 - iq_0 >= 4) look[1] = look_at(1);
+        }
+        request_q();
+        // (a loop of one turn, or of two where the wave's first step is not seen: the request exists once)
+        for (bool asked = false;; asked = true) {
+            if (walk < walk_end) issue(walk, S0{});
+            if (!looking || asked) break;
+            uint64_t seen[2];                               // bits 4 t .. 4 t + 3: keys of the wave's step t (one row)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                seen[i] = __builtin_amdgcn_ballot_w64(look_key(i) < k_end && ((look[i][0] ^ EXCLUDED2) | (look[i][1] ^ EXCLUDED2) |
+                                                                              (look[i][2] ^ EXCLUDED2) | (look[i][3] ^ EXCLUDED2)) != 0);
+            if (!one_row) {                                 // 16 bits a row
+                uint64_t v = seen[0] | seen[1];
+                v |= v >> 32;
+                v |= v >> 16;
+                seen[0] = v & 0xFFFFu;
+                seen[1] = 0;
             }
-        } else {
-            bool seen = false;
-#pragma unroll
-            for (int i = 0; i < LOOKS; i++) seen = seen || any(look[i]);
-            const uint64_t v = __builtin_amdgcn_ballot_w64(seen);
-            win = mine < 16 ? v : 0;
+            const int first = seen[0] ? (int)__builtin_ctzll(seen[0]) >> 2 : 16 + ((int)__builtin_ctzll(seen[1] | 1ull << 63) >> 2);
+            const int last  = seen[1] ? 31 - ((int)__builtin_clzll(seen[1]) >> 2) : seen[0] ? 15 - ((int)__builtin_clzll(seen[0]) >> 2) : -1;
+            walk_end = last < 0 ? 0 : min(n_steps, wave + last * DEC_WAVES + 1);
+            if (first == 0 || last < 0) break;
+            walk = wave + first * DEC_WAVES;
         }
-        todo = __builtin_amdgcn_ballot_w64(mine < n_steps && ((uint32_t)(win >> ((mine & 15) * 4)) & 15u) != 0);
-        it = next_step(wave);
-        if (it != wave && it < n_steps) issue(it, S0{});
+        convert_q();
+    } else {
+        if (wave < n_steps) issue(wave, S0{});
     }
 
     // (V8) where the pieces of this lane's V units go: read behind the first K/V request, needed when that has arrived
@@ -712,46 +736,14 @@ __global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const Fatt
 #pragma unroll
             for (int k = 0; k < PCS / 2; k++) vdst[i][k] = places[(i * 64 + lane) * (PCS / 2) + k];
     }
-    // ---- Q -> f16 B operands in log2 units (after the first K/V request: the two cold misses overlap) ----
-    {
-        const float * qrow = (const float *)(a.q + (int64_t)iq1 * a.nbq1 + (int64_t)h * a.nbq2 + (int64_t)b * a.nbq3);
-        const float   qs   = a.scale * LOG2E;
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            half8 v;
-            if constexpr (PAD) {
-                // every lane reads 8 elements that exist (its own, or the row's first 8 where it has none) and the lanes
-                // without scale them by zero: under a guard each, the 8 * KS loads waited for one another - 2 us per call.
-                // (A q row with inf or NaN in it gives NaN either way.)
-                const bool    own = ks * 32 + g4 * 8 < a.Dv;
-                const float * q8  = qrow + (own ? ks * 32 + g4 * 8 : 0);
-                const float   qsl = own ? qs : 0.0f;
-#pragma unroll
-                for (int e = 0; e < 8; e++) v[e] = (_Float16)(q8[e] * qsl);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; e++) v[e] = (_Float16)(qrow[ks * 32 + g4 * 8 + e] * qs);
-            }
-            qreg[ks] = v;
-        }
+    if constexpr (!MASK) {                         // (after the first K/V request: the two cold misses overlap)
+        request_q();
+        convert_q();
     }
-    if constexpr (!MASK) {
-        // (steps a fixed distance apart: with the next one in a variable the 64-wide f16 form takes 146 registers for 127, three
-        //  workgroups a CU for four.  At the sizes measured that is no time: 32 sequences x 32 query, 8 KV heads of 64 against
-        //  2048 keys 25.5 us either way, 64 x 20 heads against 1500 74.0)
-        for (; it < n_steps; it += 2 * DEC_WAVES) {
-            step(it, it + DEC_WAVES, S0{});
-            if (it + DEC_WAVES < n_steps) step(it + DEC_WAVES, it + 2 * DEC_WAVES, std::integral_constant<int, ONE ? 0 : 1>{});
-        }
-    }
-    while (MASK && it < n_steps) {
-        const int n1 = next_step(it);
-        step(it, n1, S0{});
-        it = n1;
-        if (n1 < n_steps) {
-            it = next_step(n1);
-            step(n1, it, std::integral_constant<int, ONE ? 0 : 1>{});
-        }
+    typedef std::integral_constant<int, ONE ? 0 : 1> S1;
+    for (int it = walk; it < walk_end; it += 2 * DEC_WAVES) {
+        step(it, it + DEC_WAVES, S0{});
+        if (it + DEC_WAVES < walk_end) step(it + DEC_WAVES, it + 2 * DEC_WAVES, S1{});
     }
 
     // ---- column totals, then the four waves through LDS ----------------------------------------------

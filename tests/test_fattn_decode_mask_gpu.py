@@ -69,3 +69,22 @@ def test_hidden_nan_rows(D, ktype):
     print("case", D, ktype, flush=True)
     assert_parity(run_gpu(case, kernel=ggml.KERNEL_DECODE_MMA), ref)
     assert_parity(run_gpu(case, kernel=ggml.KERNEL_DECODE_MMA, n_splits=1), ref)
+
+
+# the look at the mask: from five steps a split on, up to 128 for one row (two requests from 65 on) and 16 for 2 .. 8 rows
+LIMITS = [(1, 128), (1, 129), (1, 2048), (1, 2049), (1, 4096), (1, 4097), (2, 161), (4, 512), (5, 512), (8, 507), (9, 512), (8, 513)]
+
+
+@pytest.mark.parametrize("D,ktype", [(64, ora.F16), (128, ora.Q8_0), (64, ora.Q5_1)])
+@pytest.mark.parametrize("Nq,Nkv", LIMITS)
+def test_looks_at_their_limits(D, ktype, Nq, Nkv):
+    """one visible key, or none, for each row: the first and the last of a wave's steps, of a request and of the split"""
+    keys = sorted({0, 31, 32, 127, 128, 159, 160, 511, 512, 2047, 2048, 2175, Nkv - 33, Nkv - 8, Nkv - 1})
+    keys = [k for k in keys if 0 <= k < Nkv]
+    visible = np.zeros((len(keys), 1, Nq, Nkv), bool)                    # a sequence for each key, rows from the last one up
+    for b, k in enumerate(keys):
+        for i in range(Nq):
+            visible[b, 0, Nq - 1 - i, max(k - 37 * i, 0)] = i == 0 or (b + i) % 3 != 0
+    print("case", D, ktype, Nq, Nkv, flush=True)
+    case = masked_case(visible, 4300 + Nkv + Nq, D, 2, 2, ktype)
+    assert_parity(run_gpu(case, kernel=ggml.KERNEL_DECODE_MMA, n_splits=1), run_oracle(case))

@@ -49,3 +49,9 @@ def test_decode_without_a_mask(resources):
     for pad in (0, 1):
         assert forms[(64, F16, 0, 0, 0, pad)]["VGPRs"] <= 128
     assert all(r["ScratchSize"] == 0 for r in forms.values())
+
+
+def test_decode_under_a_mask(resources):
+    """the int8 V form of 64-wide heads: the look at the mask takes no workgroup from a CU"""
+    forms = _forms(resources, "fattn_decode_kernel")
+    assert forms[(64, Q8_0, 1, 1, 1, 0)]["VGPRs"] <= 128
