@@ -258,6 +258,16 @@ __device__ __forceinline__ half8 chunk_to_half8(const Chunk & r) {
 // row pitch in bytes of the int8 V stage: the 16 rows one half of a transpose read touches start 4 banks apart
 template <int D> constexpr int v8_pitch() { return D == 128 ? 136 : 80; }
 
+// Waves a SIMD is to hold, at least and at most, where the compiler's own guess is a bad one.  Streamed 64-wide rows come to
+// a register or two above or below 128, with which four workgroups share a CU, for three (Q4_0, 64 sequences x 16 heads
+// against 160 masked entries: 10.7 us with 129 registers, 8.5 with 128; Q5_0 takes 143 under a mask and would spill).  The LDS
+// of streamed 128-wide rows of narrow types holds two workgroups: a schedule that keeps registers free for a third is slower
+// for nothing (Q4_0, 64 sequences of 500 to 4096 entries, 167 registers 73.4 us, 177 registers 67.1).
+template <int D, int TYPE, bool RAW> constexpr int decode_waves_min() {
+    return D == 64 && RAW && (TYPE == MI355X_TYPE_Q4_0 || TYPE == MI355X_TYPE_Q4_1 || TYPE == MI355X_TYPE_Q5_1) ? 4 : 2;
+}
+template <int D, bool RAW, bool V8> constexpr int decode_waves_max() { return D == 128 && RAW && !V8 ? 2 : 8; }
+
 // LDS bytes per workgroup: the per-wave f16 V stages, plus per-wave raw K and V stages when RAW; with V8 the V side is
 // one int8 stage and the scales of its 32 x D/32 blocks instead
 template <int D, int TYPE, bool RAW, bool V8>
@@ -303,7 +313,8 @@ template <int D> __device__ const V8Places<D> v8_places_table = v8_places<D>();
 // PAD: f16 rows of a.Dv elements (a multiple of 8 below D) read in place: the chunks of a row behind Dv are zeros in the
 // registers, q is read and dst written up to Dv.  An instantiation of its own: the others stay the code they were.
 template <int D, int TYPE, bool MASK, bool RAW, bool V8, bool PAD = false>
-__global__ void __launch_bounds__(DEC_THREADS, 2) fattn_decode_kernel(const FattnArgs a) {
+__global__ void __launch_bounds__(DEC_THREADS) __attribute__((amdgpu_waves_per_eu((decode_waves_min<D, TYPE, RAW>()), (decode_waves_max<D, RAW, V8>()))))
+fattn_decode_kernel(const FattnArgs a) {
     static_assert(!PAD || (TYPE == MI355X_TYPE_F16 && !RAW && !V8), "other head sizes: f16 rows, read per lane");
     static_assert(!V8 || RAW, "the int8 V stage belongs to the streamed Q8_0 path");
     constexpr int KS  = D / 32;                    // reduction steps of Q.K^T (one Q8_0 block each)

@@ -9,7 +9,7 @@ import pytest
 from crispasr_amd import build
 
 # 512 registers a lane and SIMD, given out in eighths: 128 leave room for four waves, 168 for three, 256 for two
-F16, Q8_0 = 1, 8
+F16, Q4_0, Q4_1, Q5_1, Q8_0 = 1, 2, 3, 7, 8
 
 
 def _resources(source):
@@ -52,6 +52,8 @@ def test_decode_without_a_mask(resources):
 
 
 def test_decode_under_a_mask(resources):
-    """the int8 V form of 64-wide heads: the look at the mask takes no workgroup from a CU"""
+    """64-wide streamed caches: the look at the mask takes no workgroup from a CU"""
     forms = _forms(resources, "fattn_decode_kernel")
     assert forms[(64, Q8_0, 1, 1, 1, 0)]["VGPRs"] <= 128
+    for ktype in (Q4_0, Q4_1, Q5_1):
+        assert forms[(64, ktype, 1, 1, 0, 0)]["VGPRs"] <= 128
