@@ -10,7 +10,8 @@
 //
 // What the loop had to be rid of to get there, each measured on the 20 x 64-wide encoder layer: taken branches in the
 // common path (about 40 cycles each for a wave alone: the steady-state loop is straight-line code and the rare path lies
-// behind it), copies of the C operand (16 registers per unit; see `first_mfma`), waits on loads just issued.
+// behind it), waits on loads just issued.  Matrix instructions and what reads their results are the compiler's, none of them
+// inline assembly: it puts the wait states between the two, and leaves them out around instructions it does not know.
 //
 // K and V blocks of 32 keys go global -> LDS (global_load_lds_dwordx4, chunks XOR-swizzled) into a ring of 4 slots each, one
 // barrier per block; what a block's start requests is needed two or three blocks later (8 slots are no faster: a CU's path
@@ -50,12 +51,6 @@ __device__ __forceinline__ float max_of_halves(float x) {
     asm volatile("" : "+v"(b));                    // (the swap of a value with itself is folded wrongly)
     const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
     return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-
-// The first MFMA of a chain, whose destination is not its C operand.  As asm because the compiler ties the two in code
-// where the C operand is redefined on a rare path, and then copies 16 registers in the common one.
-__device__ __forceinline__ void first_mfma(float16v & d, half8 a, half8 b, const float16v & c) {
-    asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(d) : "v"(a), "v"(b), "v"(c));
 }
 
 // LDS by number: a kernel without static LDS finds its dynamic LDS at 0
@@ -240,10 +235,10 @@ __global__ void __launch_bounds__(PIPE_THREADS, 2) fattn_pipe_kernel(const Fattn
     for (int i = 0; i < (TURNS ? 4 : 2 * DB); i++) va[i] = zero8;
     auto read_k = [&](half8 (&to)[4], uint32_t slot, int ks0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) to[i] = *(lds_half8 *)((slot + kaddr) ^ (uint32_t)((ks0 + i) * 32));
+        for (int i = 0; i < 4; i++) to[i] = *(lds_half8 *)(uintptr_t)((slot + kaddr) ^ (uint32_t)((ks0 + i) * 32));
     };
     auto read_v1 = [&](uint32_t slot, int k2, int db) __attribute__((always_inline)) {
-        lds_short4 * p0 = (lds_short4 *)(((slot + vaddr) ^ (uint32_t)(db * 64)) + k2 * 16 * ROWB);
+        lds_short4 * p0 = (lds_short4 *)(uintptr_t)(((slot + vaddr) ^ (uint32_t)(db * 64)) + k2 * 16 * ROWB);
         const half4 lo = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(p0));
         const half4 hi = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(p0 + ROWB));
         return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -318,8 +313,8 @@ __global__ void __launch_bounds__(PIPE_THREADS, 2) fattn_pipe_kernel(const Fattn
         else if (NQB == 1)  read_v(va, (cur - STEPB) & RMASK, 0);
         PIPE_FENCE();
         float e[16];
-        float lprev;                                              // (a copy by force: else all four old sums stay in registers)
-        asm volatile("v_mov_b32 %0, %1" : "=v"(lprev) : "v"(lacc[QB][0]));
+        float lprev = lacc[QB][0];                                // (a copy by force: else all four old sums stay in registers)
+        asm volatile("" : "+v"(lprev));
         auto pack = [&](int i) __attribute__((always_inline)) {          // probabilities 2i, 2i + 1
             p[U][i >> 2][(2 * i) & 7]     = (_Float16)e[2 * i];
             p[U][i >> 2][(2 * i + 1) & 7] = (_Float16)e[2 * i + 1];
@@ -337,7 +332,7 @@ __global__ void __launch_bounds__(PIPE_THREADS, 2) fattn_pipe_kernel(const Fattn
             PIPE_FENCE();
             if (j == 0) {
                 if (SPLAT) {
-                    first_mfma(s[1 - U], ka[0], qreg[NX][0], negm[SPLAT ? NX : 0]);
+                    s[1 - U] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[0], qreg[NX][0], negm[SPLAT ? NX : 0], 0, 0, 0);
                 } else {
                     float16v none;
 #pragma unroll

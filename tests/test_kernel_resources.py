@@ -30,6 +30,15 @@ def _resources(source):
     return out
 
 
+def test_matrix_instructions_are_the_compilers():
+    """none in inline assembly, nor moves of their results: the wait states between the two are the compiler's to place"""
+    for f in sorted(os.listdir(build.CSRC)):
+        if f.endswith((".hip", ".h")):
+            code = open(os.path.join(build.CSRC, f)).read()
+            for m in re.finditer(r'\basm\b[^;]*;', re.sub(r"//.*", "", code)):
+                assert not re.search(r"v_mfma|v_smfmac|v_mov_b32|v_accvgpr", m[0]), (f, m[0])
+
+
 @pytest.fixture(scope="module")
 def resources():
     if not os.path.exists(build._hipcc()):
