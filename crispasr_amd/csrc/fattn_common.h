@@ -151,6 +151,23 @@ static __device__ __forceinline__ float quad_broadcast(float x, int k) {        
     }
 }
 
+// lane l's and lane (l ^ 32)'s values, the lower lane's first, without the LDS crossbar (whose traffic would blur the waits of
+// a loop, and whose addresses cost registers)
+static __device__ __forceinline__ float2 both_halves(float x) {
+    uint32_t a = __float_as_uint(x), b = a;
+    asm volatile("" : "+v"(b));                    // (the swap of a value with itself is folded wrongly)
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    return make_float2(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+static __device__ __forceinline__ float max_of_halves(float x) {
+    const float2 v = both_halves(x);
+    return fmaxf(v.x, v.y);
+}
+static __device__ __forceinline__ float sum_of_halves(float x) {
+    const float2 v = both_halves(x);
+    return v.x + v.y;
+}
+
 template <int GROUP>
 static __device__ __forceinline__ float group_max(float x) {
     x = fmaxf(x, dpp_mov<0xB1>(x));

@@ -45,14 +45,6 @@ template <int D> __device__ __forceinline__ int pipe_swz_k(int r) { return D == 
 // (for a 32-lane half of a transposing read, rows 0 .. 3, to fall into distinct banks: 64-wide rows lie two to a bank line)
 template <int D> __device__ __forceinline__ int pipe_swz_v(int r) { return D == 64 ? ((r >> 1) & 1) << 2 : (r & 3) << 2; }
 
-// the larger of lane l's and lane (l ^ 32)'s value, without the LDS crossbar (whose traffic would blur the waits of the loop)
-__device__ __forceinline__ float max_of_halves(float x) {
-    uint32_t a = __float_as_uint(x), b = a;
-    asm volatile("" : "+v"(b));                    // (the swap of a value with itself is folded wrongly)
-    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-
 // LDS by number: a kernel without static LDS finds its dynamic LDS at 0
 typedef __attribute__((address_space(3))) const half8 lds_half8;
 typedef __attribute__((address_space(3))) short4v     lds_short4;

@@ -178,7 +178,14 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     }
     constexpr int AES = ADD_F16 ? 2 : 4;
     const char * addrow = nullptr;                  // the query's row of the additive mask
-    if (ADD) addrow = a.add + (int64_t)iq * a.nba1 + (int64_t)(h % a.Ha) * a.nba2 + (int64_t)(b % a.Ba) * a.nba3;
+    // (The head's and the sequence's offsets in scalar registers: the divisions leave theirs in vector ones, and the 128-wide
+    //  forms held them through the loop in scratch, for the rows that are done again.  What is left of it, one register in the
+    //  form of 3 waves and three in that of 2, belongs to the epilogue; a build without it is 1% slower at 750 tokens.)
+    const char * add_head = nullptr;
+    if (ADD) {
+        add_head = a.add + (int64_t)__builtin_amdgcn_readfirstlane(h % a.Ha) * a.nba2 + (int64_t)__builtin_amdgcn_readfirstlane(b % a.Ba) * a.nba3;
+        addrow   = add_head + (int64_t)iq * a.nba1;
+    }
     // Keys beyond the length of a padded sequence carry -inf in the additive mask for every query: tiles that are masked
     // out entirely at the END of the key range add nothing and are not walked at all.  Each wave looks at its queries'
     // last tile while the first blocks are on their way (that is all an unpadded sequence costs) and, if that one is
@@ -396,7 +403,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
             float tmax = s2[0];
 #pragma unroll
             for (int r = 1; r < 16; r++) tmax = fmaxf(tmax, s2[r]);
-            tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));      // both halves of a query must agree
+            tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));// both halves of a query must agree
             const float mn = tmax > m ? tmax : m;
             const float f  = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mn);     // m = -inf: nothing accumulated yet, f = 0
             l *= f;
@@ -427,7 +434,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     }
 
     // ---- normalise and store: lane (il, hh) holds d = 32 db + 8 g + 4 hh + c of its query -------------------------------
-    l += __shfl_xor(l, 32, 64);
+    l = sum_of_halves(l);
     // Excluded keys (add = -inf) were multiplied by probabilities of exactly zero, not skipped: the same for finite K/V, NaN
     // otherwise.  Queries whose result is not finite are computed again below, excluded keys unread, as the CPU op does it.
     uint64_t badbits = 0;
@@ -459,7 +466,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
             while (bits != 0) {
                 const int qi = i0w + __builtin_ctz(bits);
                 bits &= bits - 1;
-                if (qi < a.Nq) attn_row_redo_relpos<D>(a, qi, h, b);
+                if (qi < a.Nq) attn_row_redo_relpos<D>(a, qi, h, b, add_head);
             }
         }
     }

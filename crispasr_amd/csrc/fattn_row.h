@@ -258,8 +258,9 @@ struct RowMaskRelpos {
     }
 };
 
+// add_head: the (head, sequence)'s additive mask, or nullptr
 template <int D>
-static __device__ __forceinline__ void attn_row_redo_relpos(const FattnRelposArgs & a, int iq, int h, int b) {
+static __device__ __forceinline__ void attn_row_redo_relpos(const FattnRelposArgs & a, int iq, int h, int b, const char * add_head) {
     constexpr int LPR = D / 8;
     const int lane = threadIdx.x & 63;
     const int d0   = (lane % LPR) * 8;
@@ -276,7 +277,7 @@ static __device__ __forceinline__ void attn_row_redo_relpos(const FattnRelposArg
     }
     mask.rrow0   = a.r + (int64_t)(h % a.Hr) * a.nbr2 + (int64_t)(b % a.Br) * a.nbr3 + (int64_t)(a.Nq - 1 - iq) * a.nbr1;
     mask.nbr1    = a.nbr1;
-    mask.addrow  = a.add ? a.add + (int64_t)iq * a.nba1 + (int64_t)(h % a.Ha) * a.nba2 + (int64_t)(b % a.Ba) * a.nba3 : nullptr;
+    mask.addrow  = add_head ? add_head + (int64_t)iq * a.nba1 : nullptr;
     mask.add_f16 = a.add_f16 != 0;
     mask.scale   = a.scale;
     mask.d0      = d0;

@@ -43,7 +43,7 @@ def test_matrix_instructions_are_the_compilers():
 def resources():
     if not os.path.exists(build._hipcc()):
         pytest.skip("no hipcc")
-    sources = ["fattn_decode.hip"]
+    sources = ["fattn_decode.hip", "fattn_relpos.hip"]
     with ThreadPoolExecutor(len(sources)) as ex:
         return {k: v for r in ex.map(_resources, sources) for k, v in r.items()}
 
@@ -66,3 +66,11 @@ def test_decode_under_a_mask(resources):
     assert forms[(64, Q8_0, 1, 1, 1, 0)]["VGPRs"] <= 128
     for ktype in (Q4_0, Q4_1, Q5_1):
         assert forms[(64, ktype, 1, 1, 0, 0)]["VGPRs"] <= 128
+
+
+def test_relpos_scratch(resources):
+    """none inside the step loop; the forms that fill the register file hold up to three registers of the epilogue there"""
+    forms = _forms(resources, "fattn_relpos_kernel")
+    assert {k[0] for k in forms} == {64, 128}
+    for args, r in forms.items():
+        assert r["ScratchSize"] <= (16 if args[0] == 128 else 0), (args, r)
