@@ -186,6 +186,28 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
         add_head = a.add + (int64_t)__builtin_amdgcn_readfirstlane(h % a.Ha) * a.nba2 + (int64_t)__builtin_amdgcn_readfirstlane(b % a.Ba) * a.nba3;
         addrow   = add_head + (int64_t)iq * a.nba1;
     }
+    // the additive mask's values of a tile: requested when the tile before is done with its own, waited for with that
+    // tile's blocks
+    typedef typename std::conditional<ADD_F16, half4_a2, float4_a4>::type araw_t;
+    araw_t araw[ADD ? 4 : 1];
+    auto load_add = [&](int t) __attribute__((always_inline)) {
+        if (__builtin_expect(32 * t + 32 <= a.Nkv, 1)) {
+#pragma unroll
+            for (int g = 0; g < 4; g++) araw[ADD ? g : 0] = *(const araw_t *)(addrow + ((int64_t)32 * t + 8 * g + 4 * hh) * AES);
+        } else {
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    const int key = min(32 * t + 8 * g + 4 * hh + c, a.Nkv - 1);
+                    if constexpr (ADD_F16) araw[ADD ? g : 0][c] = *(const _Float16 *)(addrow + (int64_t)key * 2);
+                    else                   araw[ADD ? g : 0][c] = *(const float *)(addrow + (int64_t)key * 4);
+                }
+        }
+    };
+    // (the first tile's with the first blocks: behind the barrier they were a round trip of their own, 0.2 us of a call of two
+    //  tiles - 50 tokens x 4 heads of 64 7.6 -> 7.4 us)
+    if (ADD) load_add(0);
     // Keys beyond the length of a padded sequence carry -inf in the additive mask for every query: tiles that are masked
     // out entirely at the END of the key range add nothing and are not walked at all.  Each wave looks at its queries'
     // last tile while the first blocks are on their way (that is all an unpadded sequence costs) and, if that one is
@@ -298,31 +320,11 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     const int x_lane = il + 4 * hh + 1;
     const int sq_new = il * FR_SQP + x_lane, sq_prev = sq_new - 32;
 
-    // the additive mask's values of a tile: requested when the tile before is done with its own, waited for with that
-    // tile's blocks
-    typedef typename std::conditional<ADD_F16, half4_a2, float4_a4>::type araw_t;
-    araw_t araw[ADD ? 4 : 1];
-    auto load_add = [&](int t) __attribute__((always_inline)) {
-        if (__builtin_expect(32 * t + 32 <= a.Nkv, 1)) {
-#pragma unroll
-            for (int g = 0; g < 4; g++) araw[ADD ? g : 0] = *(const araw_t *)(addrow + ((int64_t)32 * t + 8 * g + 4 * hh) * AES);
-        } else {
-#pragma unroll
-            for (int g = 0; g < 4; g++)
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    const int key = min(32 * t + 8 * g + 4 * hh + c, a.Nkv - 1);
-                    if constexpr (ADD_F16) araw[ADD ? g : 0][c] = *(const _Float16 *)(addrow + (int64_t)key * 2);
-                    else                   araw[ADD ? g : 0][c] = *(const float *)(addrow + (int64_t)key * 4);
-                }
-        }
-    };
     // (the compiler's wait for them belongs here, behind that of `meet`: further down it would wait for the blocks on their way)
     auto have_add = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int g = 0; g < 4; g++) asm volatile("" : "+v"(araw[ADD ? g : 0]));
     };
-    if (ADD) load_add(0);
     meet();                                            // block 1 - NW has been read: its slot takes the next one
     if (ADD) have_add();
 
