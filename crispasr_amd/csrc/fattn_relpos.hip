@@ -506,27 +506,38 @@ bool fattn_relpos_supported(const FattnRelposArgs & a) {
 
 int fattn_relpos_launch(const FattnRelposArgs & a, hipStream_t stream) {
     if (!fattn_relpos_supported(a)) return (int)hipErrorInvalidValue;
-    // Workgroups of 2, 3 or 4 waves (32 queries each): the widest one that the queries fill.  128-wide heads have LDS for one
-    // workgroup of 4 waves on a CU or for two of 3, and take what fills the chip in fewer rounds.  A 32-key step was measured
-    // to take about 1.8 us with 4 waves on the CU, 1.7 with 3 and 3.0 with two times 3 (8 heads: 750 tokens x 8 87.7 us a
-    // call with 3 waves against 112 with 4, 1000 x 4 88.9 against 72.6; 4 heads, 1000 x 4 56.8 against 59.1).
-    // 64-wide heads are never slower with 3 waves than with 4 (120 tokens x 4 heads 12.6 against 13.9 us, 180 x 4 13.6 against
-    // 15.0, 750 x 64 56.7 against 57.6).
-    const int most = a.D == 64 ? 3 : 4;
-    int best = (a.Nq + 31) / 32;
-    best = best < 2 ? 2 : best > most ? most : best;
+    // Workgroups of 2, 3 or 4 waves (32 queries each): no wider than the queries fill, and of those what prices lowest.
+    const int64_t heads = (int64_t)a.H * a.B, cus = a.n_cus > 0 ? a.n_cus : 256;
+    const int     most  = (a.Nq + 31) / 32 < 4 ? (a.Nq + 31) / 32 : 4;
+    auto groups = [&](int waves) { return (a.Nq + 32 * waves - 1) / (32 * waves) * heads; };
+    int best = most < 2 ? 2 : most;
     if (a.D == 128 && best == 4) {
-        const int64_t heads = (int64_t)a.H * a.B, cus = a.n_cus > 0 ? a.n_cus : 256;
-        const int64_t wg3 = (a.Nq + 95) / 96 * heads, wg4 = (a.Nq + 127) / 128 * heads;
-        const int64_t rest = wg3 % (2 * cus);
+        // 128-wide heads have LDS for one workgroup of 4 waves on a CU or for two of 3, and take what fills the chip in fewer
+        // rounds.  A 32-key step was measured to take about 1.8 us with 4 waves on the CU, 1.7 with 3 and 3.0 with two times 3 (8
+        // heads: 750 tokens x 8 60 us a call with 3 waves against 92 with 4, 1000 x 4 73 against 60; where both are one round, 120
+        // x 8 16.1 against 17.7).
+        const int64_t wg3 = groups(3), wg4 = groups(4), rest = wg3 % (2 * cus);
         const int64_t t3 = wg3 / (2 * cus) * 30 + (rest == 0 ? 0 : rest <= cus ? 17 : 30), t4 = (wg4 + cus - 1) / cus * 18;
         if (t3 < t4) best = 3;
+    } else if (a.D == 64) {
+        // 64-wide heads fit by their registers: 8 waves on a CU, as four workgroups of 2, two of 3 or two of 4.  A round takes
+        // what the CU with the most waves takes (1000 tokens, us: 33 with 2 waves, 35 with 3, 39 with 4, 47 with 6, 52 with 8).
+        // Over 154 calls of 50 to 1500 tokens x 4 to 512 heads this is 0.3% off the best of the three, 7% at worst; 3 waves
+        // for all calls, as it was, is 12.5% off (1000 tokens x 64 heads 61.5 us with 2, 96.5 with 3, 61.3 with 4; 120 x 32
+        // 10.9, 12.4, 12.4; 750 x 32 38.3, 35.6, 39.1).
+        static const int round_of[5][5] = {{}, {}, {0, 33, 40, 47, 52}, {0, 35, 48}, {0, 39, 51}};      // [waves][workgroups on the CU]
+        int64_t least = INT64_MAX;
+        for (int w = best; w >= 2; w--) {
+            const int64_t fit = w == 2 ? 4 : 2, rest = groups(w) % (fit * cus);
+            const int64_t t = groups(w) / (fit * cus) * round_of[w][fit] + round_of[w][(rest + cus - 1) / cus];
+            if (t < least) { least = t; best = w; }
+        }
     }
     static const char * force = getenv("MI355X_RELPOS_WAVES");            // experiments only
-    if (force && atoi(force) >= 2 && atoi(force) <= most) best = atoi(force);
+    if (force && atoi(force) >= 2 && atoi(force) <= 4) best = atoi(force);
     switch (best) {
         case 2:  return a.D == 64 ? launch_d<64, 2>(a, stream) : launch_d<128, 2>(a, stream);
         case 3:  return a.D == 64 ? launch_d<64, 3>(a, stream) : launch_d<128, 3>(a, stream);
-        default: return launch_d<128, 4>(a, stream);
+        default: return a.D == 64 ? launch_d<64, 4>(a, stream) : launch_d<128, 4>(a, stream);
     }
 }

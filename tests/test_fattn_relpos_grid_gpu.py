@@ -36,3 +36,10 @@ def test_edges_of_tiles_and_widths(D, add, add_type, Nq, Nkv):
 @pytest.mark.parametrize("T,H,B", [(150, 8, 16), (390, 8, 8), (200, 8, 24), (260, 4, 50)])
 def test_grids(D, T, H, B):
     check(6100 + T, D, T, T, H, B, "padlong")
+
+
+# 64-wide heads: calls that run with 2, 3 and 4 waves a workgroup, one and several workgroups on a CU
+@pytest.mark.parametrize("add,add_type", [(None, ora.F32), ("padlong", ora.F32), ("padlong", ora.F16)])
+@pytest.mark.parametrize("T,H,B", [(100, 4, 4), (129, 8, 16), (200, 8, 24), (70, 8, 20), (97, 8, 22), (128, 8, 20), (121, 8, 40)])
+def test_widths_by_grid(T, H, B, add, add_type):
+    check(6200 + T, 64, T, T, H, B, add, add_type)
