@@ -43,7 +43,7 @@ def test_matrix_instructions_are_the_compilers():
 def resources():
     if not os.path.exists(build._hipcc()):
         pytest.skip("no hipcc")
-    sources = ["fattn_decode.hip", "fattn_relpos.hip"]
+    sources = ["fattn_mma.hip", "fattn_decode.hip", "fattn_relpos.hip"]
     with ThreadPoolExecutor(len(sources)) as ex:
         return {k: v for r in ex.map(_resources, sources) for k, v in r.items()}
 
@@ -66,6 +66,13 @@ def test_decode_under_a_mask(resources):
     assert forms[(64, Q8_0, 1, 1, 1, 0)]["VGPRs"] <= 128
     for ktype in (Q4_0, Q4_1, Q5_1):
         assert forms[(64, ktype, 1, 1, 0, 0)]["VGPRs"] <= 128
+
+
+def test_tile_kernel_under_a_mask(resources):
+    """f16 rows moved straight to LDS: no form keeps anything in scratch"""
+    forms = {k: r for k, r in _forms(resources, "fattn_mma_kernel").items() if k[6]}
+    assert {(k[0], k[1]) for k in forms} == {(64, 1), (64, 2), (128, 1)}
+    assert [k for k, r in forms.items() if r["ScratchSize"]] == []
 
 
 def test_relpos_scratch(resources):
