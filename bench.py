@@ -123,19 +123,19 @@ def bench_encoder(args, ca, ora, torch):
     # HBM bytes per launch of the same kernel from the committed rocprofv3 FETCH_SIZE / WRITE_SIZE runs
     traffic = None
     try:
-        for ln in open(os.path.join(ROOT, "profiles", "fattn_mma_whisper_large_v3_encoder.txt")):
+        for ln in open(os.path.join(ROOT, "profiles", "fattn_pipe_whisper_encoders.txt")):
             if ln.startswith("traffic_bytes_per_launch"):
                 traffic = float(ln.split()[1])
     except OSError:
         pass
     pd = ca.ggml.flash_attn_plan_details(layers[0]["q"], layers[0]["k"], layers[0]["v"], None, scale)
-    kname = (f"fattn_mma_kernel<D={D}, query_blocks={pd['query_blocks']}, key_split={pd['key_split']}, F16, "
+    kname = (f"fattn_pipe_kernel<D={D}, query_blocks={pd['query_blocks']}, key_split={pd['key_split']}, F16, "
              f"direct={pd['direct']}>" if pd["kernel"] == ca.ggml.KERNEL_MMA else f"kernel {pd['kernel']}")
     res = {
         "value": value, "ms_per_step": ms_per_step,
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": PEAK_F16_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_F16_TFLOPS, "traffic": traffic,
-                     "traffic_source": "profiles/fattn_mma_whisper_large_v3_encoder.txt: rocprofv3 FETCH_SIZE + WRITE_SIZE of this "
+                     "traffic_source": "profiles/fattn_pipe_whisper_encoders.txt: rocprofv3 FETCH_SIZE + WRITE_SIZE of this "
                                        "command in runs of their own, scaled by a plain copy; a constant of that profile, not "
                                        "measured by this run",
                      "kernel": kname, "queries_per_workgroup": pd["queries_per_workgroup"], "n_splits": pd["n_splits"],
