@@ -595,7 +595,10 @@ void make_plan_core(const FattnArgs & a0, int ktype, int vtype, const mi355x_fat
             //  128 against 8192 keys, 160 workgroups, 146 -> 81 us in 3 ranges; the Whisper-base encoder's 24 tiles stay whole.)
             ns = 1;
             const int cus = a.n_cus;
-            // (the key-split form of 64-wide heads without a mask walks tiles of 128 keys and more)
+            // (64-wide heads without a mask, key split: the pipelined kernel takes a key in half the time, and a range must be
+            //  twice as long to be worth its merge.  180 calls of 32 .. 400 queries x 1 .. 20 heads x 512 .. 8192 keys, eight forced
+            //  counts each: AUTO is 4.8% off the best count, 1.24 at worst (1024 keys, 2 ranges where 8 are best); counted
+            //  in tiles of 64 6.2% and 1.38 (512 keys, where any range loses).)
             const int nt = var.key_split == 2 && a.D == 64 && !a.masked ? (a.Nkv + 127) / 128 : n_tiles;
             if (wgs * 4 <= cus) {
                 int want = (int)(cus / wgs);

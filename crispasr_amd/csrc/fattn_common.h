@@ -11,7 +11,8 @@
 #define FATTN_Q8_0_BYTES 34
 #define FATTN_IS_BLOCK_TYPE(t) ((t) == MI355X_TYPE_Q8_0 || (t) == MI355X_TYPE_Q4_0 || (t) == MI355X_TYPE_Q4_1 || (t) == MI355X_TYPE_Q5_0 || (t) == MI355X_TYPE_Q5_1)
 
-// Unsigned division by a number fixed on the host: n / d = (mulhi(n, m) + n) >> s for n < 2^31.
+// Unsigned division by a number fixed on the host, as multiply and shift (Granlund and Montgomery, "Division by invariant
+// integers using multiplication", 1994): n / d = (mulhi(n, m) + n) >> s for n < 2^31.
 struct FastDiv {
     uint32_t d, m, s;
 };

@@ -18,10 +18,12 @@
 // from L2 into LDS gives 53 B/clk from two blocks ahead on).
 //
 // Against the tile-wise kernel it replaced for these forms, per launch: 20 x 64 x 1500^2 in batches of 4 60.2 -> 56.8 us
-// (1.08 PFLOP/s, the card's power limit: the clock falls to 1.8 GHz), 8 x 64 x 1500 against 1536 keys 14.4 -> 12.8, 8 x 128 x
-// 1500^2 x 4 55.2 -> 52.6, 10 x 128 x 1500^2 31.2 -> 23.6, 64 x 128 x 300^2 14.9 -> 12.5, 30 x 64 x 300^2 8.8 -> 7.7.
-// What is left above the MFMAs of a wave alone on its SIMD is instruction issue (about 5 cycles an instruction); where two
-// share a SIMD, the exponentials and the power limit.
+// (0.81 PFLOP/s), 8 x 64 x 1500 against 1536 keys 14.4 -> 12.8, 8 x 128 x 1500^2 x 4 55.2 -> 52.6, 10 x 128 x 1500^2 31.2 ->
+// 23.6, 64 x 128 x 300^2 14.9 -> 12.5, 30 x 64 x 300^2 8.8 -> 7.7.
+// What is left above the MFMAs of a wave alone on its SIMD is instruction issue (about 5 cycles an instruction).  Where two
+// share a SIMD nothing is full: by the counters of the first of these launches the matrix cores are busy for 49% of it (at
+// 1.85 GHz) and the vector ALU for 38%, and a wave stands ready for another instruction to end for 39% of its cycles and
+// waits at a counter or barrier for 21%.
 #include "fattn_row.h"
 
 #include <type_traits>

@@ -405,7 +405,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
             float tmax = s2[0];
 #pragma unroll
             for (int r = 1; r < 16; r++) tmax = fmaxf(tmax, s2[r]);
-            tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));// both halves of a query must agree
+            tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));      // both halves of a query must agree
             const float mn = tmax > m ? tmax : m;
             const float f  = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mn);     // m = -inf: nothing accumulated yet, f = 0
             l *= f;
