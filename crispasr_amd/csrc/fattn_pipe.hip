@@ -146,12 +146,6 @@ __global__ void __launch_bounds__(PIPE_THREADS, 2) fattn_pipe_kernel(const Fattn
         vch[j] = (uint32_t)((c ^ pipe_swz_v<D>(row[j] & 31)) * 16);
     }
     const uint32_t lds0 = wave * (NLD * 1024);
-    // (as asm: the compiler's own bookkeeping of such loads makes every LDS read that may alias them wait.  The addresses
-    //  are uniform; readfirstlane says so to the register allocator and costs nothing where it knows.)
-    auto dma = [&](uint64_t base, uint32_t off, uint32_t to) __attribute__((always_inline)) {
-        const uint64_t p = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(base >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)base);
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane((int)to)), "v"(off), "s"(p) : "memory");
-    };
     // Requests go step by step; behind the last step they go on with its rows, and rows past its end repeat the last one
     // (their scores are excluded, or nobody looks), so that the waits can count.
     struct Stream {
@@ -162,7 +156,7 @@ __global__ void __launch_bounds__(PIPE_THREADS, 2) fattn_pipe_kernel(const Fattn
     const uint32_t nb1k = (uint32_t)a.nbk1, nb1v = (uint32_t)a.nbv1;          // (below 2^24)
     auto request = [&](Stream & st, uint32_t nb1, const uint32_t (&ch)[NLD], uint32_t slot) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < NLD; j++) dma(st.at, __umul24((uint32_t)min(row[j], st.left), nb1) + ch[j], lds0 + slot + j * 1024);
+        for (int j = 0; j < NLD; j++) load_to_lds16<false>(st.at, __umul24((uint32_t)min(row[j], st.left), nb1) + ch[j], lds0 + slot + j * 1024);
         const bool more = st.left >= SKEYS;
         st.at   += more ? (uint64_t)SKEYS * nb1 : 0;
         st.left -= more ? SKEYS : 0;

@@ -117,11 +117,6 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     const int      lr = lane / CH, lc = lane % CH;
     const uint32_t ck = (uint32_t)((lc ^ fr_swz<D>(lr)) * 16), cv = (uint32_t)((lc ^ fr_swz_v<D>(lr)) * 16);
     static_assert(RPI == 4 || RPI == 8, "the swizzles of rows r and r + RPI * ins differ by 4 * (ins % (16 / RPI)) (K) or not at all (V)");
-    // (as asm: the compiler's own bookkeeping of such loads makes every LDS read that may alias them wait)
-    auto dma = [&](uint64_t at, uint32_t off, uint32_t to) __attribute__((always_inline)) {
-        const uint64_t p = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at);
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane((int)to)), "v"(off), "s"(p) : "memory");
-    };
     // Rows row0 .. row0 + 31 of a tensor, in one of two layouts.  (NW = 3: the last wave repeats an instruction of the one before.)
     auto dma_rows = [&](char * dst, const char * base, int64_t nb1, int row0, int last_row, auto is_v, auto is_first) __attribute__((always_inline)) {
         constexpr bool V      = decltype(is_v)::value;
@@ -135,7 +130,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
             for (int j = 0; j < NDM; j++) {
                 const uint32_t ins = min((uint32_t)(j * NW + wave), (uint32_t)TI - 1);         // uniform
-                dma(at + ins * RPI * nb, lrow * nb + (V ? cv : ck ^ ((ins & (16 / RPI - 1)) * 64)), to + ins * 1024);
+                load_to_lds16<true>(at + ins * RPI * nb, lrow * nb + (V ? cv : ck ^ ((ins & (16 / RPI - 1)) * 64)), to + ins * 1024);
             }
         } else {
             const int      first = min(max(row0, 0), last_row);
@@ -144,7 +139,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
             for (int j = 0; j < NDM; j++) {
                 const uint32_t ins = min((uint32_t)(j * NW + wave), (uint32_t)TI - 1);
                 const uint32_t rr  = (uint32_t)(min(max(row0 + (int)ins * RPI + lr, 0), last_row) - first);
-                dma(at, rr * nb + (V ? cv : ck ^ ((ins & (16 / RPI - 1)) * 64)), to + ins * 1024);
+                load_to_lds16<true>(at, rr * nb + (V ? cv : ck ^ ((ins & (16 / RPI - 1)) * 64)), to + ins * 1024);
             }
         }
     };

@@ -1,4 +1,5 @@
-"""Registers and scratch of kernels whose speed rests on them, as the compiler reports them for the library's own flags."""
+"""Registers and scratch of kernels whose speed rests on them, and the wait states around inline assembly, in what the compiler
+makes of the sources with the library's own flags."""
 import os
 import re
 import subprocess
@@ -12,10 +13,10 @@ from crispasr_amd import build
 F16, Q4_0, Q4_1, Q5_1, Q8_0 = 1, 2, 3, 7, 8
 
 
-def _resources(source):
-    """{(kernel, template arguments): {"VGPRs": .., "ScratchSize": ..}} of a source's kernels"""
-    res = subprocess.run([build._hipcc(), *build.HIPCC_FLAGS, "--offload-device-only", "-Rpass-analysis=kernel-resource-usage", "-c",
-                          os.path.join(build.CSRC, source), "-o", os.devnull], capture_output=True, text=True, timeout=600)
+def _resources(source, listing):
+    """{(kernel, template arguments): {"VGPRs": .., "ScratchSize": ..}} of a source's kernels; their assembly goes to `listing`"""
+    res = subprocess.run([build._hipcc(), *build.HIPCC_FLAGS, "--offload-device-only", "-Rpass-analysis=kernel-resource-usage", "-S",
+                          os.path.join(build.CSRC, source), "-o", str(listing)], capture_output=True, text=True, timeout=600)
     assert res.returncode == 0, res.stderr[-2000:]
     out, name = {}, None
     for line in res.stderr.splitlines():
@@ -39,13 +40,62 @@ def test_matrix_instructions_are_the_compilers():
                 assert not re.search(r"v_mfma|v_smfmac|v_mov_b32|v_accvgpr", m[0]), (f, m[0])
 
 
+SOURCES = ["fattn_mma.hip", "fattn_decode.hip", "fattn_relpos.hip", "fattn_pipe.hip"]
+
+
 @pytest.fixture(scope="module")
-def resources():
+def compiled(tmp_path_factory):
+    """(resources of all kernels, {source: its assembly's path})"""
     if not os.path.exists(build._hipcc()):
         pytest.skip("no hipcc")
-    sources = ["fattn_mma.hip", "fattn_decode.hip", "fattn_relpos.hip"]
-    with ThreadPoolExecutor(len(sources)) as ex:
-        return {k: v for r in ex.map(_resources, sources) for k, v in r.items()}
+    listings = {s: tmp_path_factory.mktemp("asm") / (s + ".s") for s in SOURCES}
+    with ThreadPoolExecutor(len(SOURCES)) as ex:
+        return {k: v for r in ex.map(_resources, SOURCES, listings.values()) for k, v in r.items()}, listings
+
+
+@pytest.fixture(scope="module")
+def resources(compiled):
+    return compiled[0]
+
+
+def _sgprs(operand):
+    """the scalar registers that an operand names"""
+    m = re.fullmatch(r"s(\d+)|s\[(\d+):(\d+)\]", operand)
+    return set() if not m else {int(m[1])} if m[1] else set(range(int(m[2]), int(m[3]) + 1))
+
+
+def early_loads(lines):
+    """memory instructions that read a scalar register fewer than five wait states after a vector instruction wrote it"""
+    found, writes, clock = [], {}, 0
+    for line in lines:
+        line = line.split(";")[0].strip()
+        if not line or line[0] in ".#" or line.endswith(":"):
+            continue
+        op, *rest = line.split(None, 1)
+        operands = [x.split()[0] for x in rest[0].split(",") if x.strip()] if rest else []
+        if op.startswith(("global_", "buffer_")):
+            read = set().union(*(_sgprs(x) for x in operands))
+            found += [line for r in read if clock - writes.get(r, -9) < 5]
+        clock += 1 + int(operands[0], 0) if op == "s_nop" else 1
+        if op.startswith(("v_readlane", "v_readfirstlane", "v_cmp")):
+            writes.update({r: clock for r in _sgprs(operands[0])})
+    return found
+
+
+def test_early_loads_are_found():
+    read = ["v_readlane_b32 s49, v255, 26", "s_mov_b32 m0, s87", "s_nop 0", "global_load_lds_dwordx4 v72, s[48:49]"]
+    assert early_loads(read) == [read[3]]
+    assert early_loads([read[0], "s_nop 3", read[3]]) == [read[3]]
+    assert early_loads([read[0], "s_nop 4", read[3]]) == []
+    assert early_loads(["v_readlane_b32 s50, v255, 26", read[3]]) == []
+
+
+@pytest.mark.parametrize("source", SOURCES)
+def test_no_load_reads_a_scalar_too_early(compiled, source):
+    """the compiler places these wait states itself, but not between its code and inline assembly"""
+    lines = open(compiled[1][source]).read().splitlines()
+    assert any("global_load" in x for x in lines)
+    assert early_loads(lines) == []
 
 
 def _forms(resources, kernel):
