@@ -3,7 +3,7 @@
 // src/core/attention.h:342-378) and the dequantising reads (src/core/attention.h:917-920).
 // HBM-bound byte work, 8 elements per lane wherever rows allow it, coalesced along dimension 0.  Source and destination may have different shapes with equal element
 // counts (the reference copies a [n_state, n_ctx] tensor into a 1-D cache view).
-#include "fattn_common.h"
+#include "copy_forms.h"
 
 #include <string.h>
 #include <type_traits>
@@ -14,6 +14,8 @@
 #pragma clang fp contract(off)
 
 namespace {
+
+typedef float float4v __attribute__((ext_vector_type(4)));
 
 // Which element a thread works on: unit i of `unit0` elements each -> its place along the four dimensions.
 // I = uint32_t (up to 2^31 units): divisions by multiply and shift, four instructions each.  In 64-bit arithmetic the six
@@ -45,45 +47,83 @@ __device__ __forceinline__ Place place_of(I i, const int64_t (&ne)[4], const Fas
 __device__ __forceinline__ int64_t offset_at(const Place & p, const int64_t (&nb)[4], int64_t step0) {
     return p.i0 * step0 + p.i1 * nb[1] + p.i2 * nb[2] + p.i3 * nb[3];
 }
-template <typename I>
-__device__ __forceinline__ void both_places(const CpyArgs & a, I i, int64_t unit0, Place & s, Place & d) {
-    s = place_of<I>(i, a.sne, a.sdiv, unit0);
-    d = s;
-    if (!a.same_shape) d = place_of<I>(i, a.dne, a.ddiv, unit0);
-}
 template <typename I> __device__ __forceinline__ I thread_index() { return (I)blockIdx.x * 256 + threadIdx.x; }
+// Lanes of the grid, by which the kernels that give a lane four elements of 64-bit indices walk on: a grid has fewer than 2^32.
+template <typename I> __device__ __forceinline__ I grid_lanes() { return (I)gridDim.x * 256; }
+constexpr int64_t MAX_WALKED = (int64_t)1 << 31;
 
-template <typename I, typename TS, typename TD>
-__global__ void __launch_bounds__(256) cpy_scalar_kernel(const CpyArgs a) {
+// the wide form of a copy or SET_ROWS: everything the narrow one does not hold
+template <typename I> struct WideCopy : CpyArgs {
+    typedef I       index;
+    typedef int64_t offset;
+};
+template <typename I>
+__device__ __forceinline__ void offsets(const WideCopy<I> & a, I i, int unit0, int64_t sstep, int64_t dstep, int64_t & so, int64_t & to) {
+    const Place s = place_of<I>(i, a.sne, a.sdiv, unit0);
+    Place d = s;
+    if (!a.same_shape) d = place_of<I>(i, a.dne, a.ddiv, unit0);
+    so = offset_at(s, a.snb, sstep);
+    to = offset_at(d, a.dnb, dstep);
+}
+
+// bytes from one source element to the next (a destination's are always adjacent)
+template <typename T> __device__ __forceinline__ int64_t element_pitch(const NarrowCopy &) { return sizeof(T); }
+template <typename T, typename I> __device__ __forceinline__ int64_t element_pitch(const WideCopy<I> & a) { return a.snb[0]; }
+
+// Sixteen bytes a lane, whole lines a wave.  Written through, they leave the dies' L2 caches while the launch still runs instead of
+// at its end; marked non-temporal (STREAM) they do not stay in the memory-side cache either.  us a launch, plain / written through /
+// both: F32 -> F16 rows of 128, 663 x 8 2.40 / 2.29 / 2.29, 2048 x 64 24.1 / 23.2 / 22.6; Q8_0 -> F32, 663 x 8 2.32 / 2.15 / 2.15, 2048 x 8
+// 3.84 / 3.88 / 2.78, 2048 x 64 17.9 / 17.7 / 11.4.  So dequantised reads, which outgrow the caches, are both; what the next
+// launch reads is written through only (six encoder layers whose K and V are copied to F16 first: 119 us plain, 118 written
+// through, 124 both).  Pieces of lines written through cost up to twice the plain stores: other kernels keep plain ones.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+template <bool STREAM, typename T> __device__ __forceinline__ void store16(const NarrowCopy & a, uint32_t to, T x) {
+    // (a buffer store, because only its builtin takes the cache bits: 2 = non-temporal, 16 = write through)
+    const auto r = __builtin_amdgcn_make_buffer_rsrc(a.dst, 0, -1, 0x00020000);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), r, (int)to, 0, STREAM ? 18 : 16);
+}
+template <bool STREAM, typename I, typename T> __device__ __forceinline__ void store16(const WideCopy<I> & a, int64_t to, T x) {
+    if (STREAM) __builtin_nontemporal_store(x, (T *)(a.dst + to));
+    else        *(T *)(a.dst + to) = x;
+}
+
+template <typename A, typename TS, typename TD>
+__global__ void __launch_bounds__(256) cpy_scalar_kernel(const A a) {
+    typedef typename A::index I;
     const I i = thread_index<I>();
     if (i >= (I)a.n) return;
-    Place sp, tp;
-    both_places<I>(a, i, 1, sp, tp);
-    const TS x = *(const TS *)(a.src + offset_at(sp, a.snb, a.snb[0]));
-    char * dp = a.dst + offset_at(tp, a.dnb, a.dnb[0]);
+    typename A::offset so, to;
+    offsets(a, i, 1, element_pitch<TS>(a), sizeof(TD), so, to);
+    const TS x = *(const TS *)(a.src + so);
+    char * dp = a.dst + to;
     *(TD *)dp = (TD)x;                                          // f32 -> f16 is round-to-nearest-even
     if (a.mirror) *(TD *)(dp + a.mirror) = (TD)x;
 }
 
-template <typename T> using Vec8 = T __attribute__((ext_vector_type(8)));
-template <typename T> using Vec4 = T __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
 
-// 8 consecutive elements of dimension 0 per lane: 128-bit loads and stores for f16 <-> f32 and same-type copies.
-// Launched only when both sides have ne0 % 8 == 0, unit element stride and 16-byte aligned rows.
-template <typename I, typename TS, typename TD>
-__global__ void __launch_bounds__(256) cpy_vec8_kernel(const CpyArgs a) {
-    const I i = thread_index<I>();
-    if (i >= (I)a.n) return;
-    Place sp, tp;
-    both_places<I>(a, i, 8, sp, tp);
-    const Vec8<TS> x  = *(const Vec8<TS> *)(a.src + offset_at(sp, a.snb, 8 * sizeof(TS)));
-    Vec8<TD> *     dp = (Vec8<TD> *)(a.dst + offset_at(tp, a.dnb, 8 * sizeof(TD)));
-    Vec8<TD> y;
+// What a lane's 16-byte store of TD holds, 8 or 4 consecutive elements of dimension 0, for f16 <-> f32 and same-type copies.
+// Launched only when dimension 0 is whole such units on both sides, the elements are adjacent and rows start on the 16 bytes
+// (8 where four f16 are read) that a lane moves at once.
+template <typename TD> constexpr int vec_elements() { return 16 / (int)sizeof(TD); }
+template <typename A, typename TS, typename TD>
+__global__ void __launch_bounds__(256) cpy_vec_kernel(const A a) {
+    typedef typename A::index I;
+    constexpr int E = vec_elements<TD>();
+    constexpr int SAL = E * (int)sizeof(TS) < 16 ? E * (int)sizeof(TS) : 16;
+    typedef TS Src __attribute__((ext_vector_type(E), aligned(SAL)));
+    typedef TD Dst __attribute__((ext_vector_type(E)));
+    for (I i = thread_index<I>(); i < (I)a.n; i += grid_lanes<I>()) {
+        typename A::offset so, to;
+        offsets(a, i, E, E * sizeof(TS), E * sizeof(TD), so, to);
+        const Src x = *(const Src *)(a.src + so);
+        Dst y;
 #pragma unroll
-    for (int e = 0; e < 8; e++) y[e] = (TD)x[e];
-    *dp = y;
-    if (a.mirror) *(Vec8<TD> *)((char *)dp + a.mirror) = y;
+        for (int e = 0; e < E; e++) y[e] = (TD)x[e];
+        store16<false>(a, to, y);
+        if (a.mirror) *(Dst *)(a.dst + to + a.mirror) = y;
+        if (sizeof(I) == 4) return;
+    }
 }
 
 // Quantise one block of 32 held by a quad of lanes, 8 consecutive elements each (lane c of the quad: elements 8c .. 8c+7),
@@ -191,105 +231,146 @@ __device__ __forceinline__ void quantize_block_store(const float (&x)[8], char *
 
 // the 8 elements of a quad's lane: two 16-byte loads where the source's rows allow it
 template <bool VEC>
-__device__ __forceinline__ void load8(const char * p, int64_t nb0, bool ok, float (&x)[8]) {
+__device__ __forceinline__ void load8(const char * p, int64_t nb0, float (&x)[8]) {
     if (VEC) {
-        const Vec4<float> u = ok ? *(const Vec4<float> *)p : Vec4<float>{0.0f, 0.0f, 0.0f, 0.0f};
-        const Vec4<float> v = ok ? *(const Vec4<float> *)(p + 16) : Vec4<float>{0.0f, 0.0f, 0.0f, 0.0f};
+        const float4v u = *(const float4v *)p, v = *(const float4v *)(p + 16);
 #pragma unroll
         for (int e = 0; e < 4; e++) { x[e] = u[e]; x[4 + e] = v[e]; }
     } else {
 #pragma unroll
-        for (int e = 0; e < 8; e++) x[e] = ok ? *(const float *)(p + e * nb0) : 0.0f;
+        for (int e = 0; e < 8; e++) x[e] = *(const float *)(p + e * nb0);
     }
 }
 
 // F32 -> block type; one block per 4 lanes
-template <typename I, int TYPE, bool VEC>
-__global__ void __launch_bounds__(256) cpy_f32_block_kernel(const CpyArgs a) {
+template <typename A, int TYPE, bool VEC>
+__global__ void __launch_bounds__(256) cpy_f32_block_kernel(const A a) {
+    typedef typename A::index I;
     const I    blk = (I)blockIdx.x * 64 + (threadIdx.x >> 2);
     const int  c   = threadIdx.x & 3;
     const bool ok  = blk < (I)a.n;
-    Place sp, tp;
-    both_places<I>(a, ok ? blk : 0, FATTN_QK8_0, sp, tp);
+    const int64_t es = VEC ? 4 : element_pitch<float>(a);              // bytes from one F32 element to the next
+    typename A::offset so, to;
+    offsets(a, ok ? blk : 0, FATTN_QK8_0, FATTN_QK8_0 * es, BlockFormat<TYPE>::BYTES, so, to);
     float x[8];
-    load8<VEC>(a.src + offset_at(sp, a.snb, FATTN_QK8_0 * a.snb[0]) + c * 8 * a.snb[0], a.snb[0], ok, x);
-    quantize_block_store<TYPE>(x, a.dst + offset_at(tp, a.dnb, a.dnb[0]), c, ok, a.mirror);
+    load8<VEC>(a.src + so + c * 8 * es, es, x);
+    quantize_block_store<TYPE>(x, a.dst + to, c, ok, a.mirror);
 }
 
-// block type -> F32; 8 elements per lane, four lanes per block.  VEC: 16-byte stores.
-template <typename I, int TYPE, bool VEC>
-__global__ void __launch_bounds__(256) cpy_block_f32_kernel(const CpyArgs a) {
-    const I   blk = (I)blockIdx.x * 64 + (threadIdx.x >> 2);
-    const int j0  = (threadIdx.x & 3) * 8;
-    if (blk >= (I)a.n) return;
-    Place sp, tp;
-    both_places<I>(a, blk, FATTN_QK8_0, sp, tp);
-    float y[8];
-    dequant8<TYPE>(a.src + offset_at(sp, a.snb, a.snb[0]), j0, y);
-    char * dp = a.dst + offset_at(tp, a.dnb, FATTN_QK8_0 * a.dnb[0]) + j0 * a.dnb[0];
-    for (int k = 0; k < (a.mirror ? 2 : 1); k++, dp += a.mirror) {
+// block type -> F32; 4 elements per lane, eight lanes per block, so that with 16-byte stores (VEC) a wave writes 1 KB that lies
+// together: with 8 elements, two stores and half as many lanes 663 x 8 rows of 128 took 2.51 us instead of 2.15, 2048 x 64 20.6 instead of 11.4.
+template <typename A, int TYPE, bool VEC>
+__global__ void __launch_bounds__(256) cpy_block_f32_kernel(const A a) {
+    typedef typename A::index I;
+    const int j0  = (threadIdx.x & 7) * 4;
+    for (I blk = (I)blockIdx.x * 32 + (threadIdx.x >> 3); blk < (I)a.n; blk += grid_lanes<I>() / 8) {
+        typename A::offset so, to;
+        offsets(a, blk, FATTN_QK8_0, BlockFormat<TYPE>::BYTES, FATTN_QK8_0 * 4, so, to);
+        float y[4];
+        dequant<TYPE>(a.src + so, j0, y);
         if (VEC) {
-            *(Vec4<float> *)dp        = Vec4<float>{y[0], y[1], y[2], y[3]};
-            *(Vec4<float> *)(dp + 16) = Vec4<float>{y[4], y[5], y[6], y[7]};
+            const float4v v = {y[0], y[1], y[2], y[3]};
+            store16<true>(a, to + j0 * 4, v);
+            if (a.mirror) *(float4v *)(a.dst + to + j0 * 4 + a.mirror) = v;
         } else {
+            char * dp = a.dst + to + j0 * 4;
+            for (int k = 0; k < (a.mirror ? 2 : 1); k++, dp += a.mirror)
 #pragma unroll
-            for (int e = 0; e < 8; e++) *(float *)(dp + e * a.dnb[0]) = y[e];
+                for (int e = 0; e < 4; e++) ((float *)dp)[e] = y[e];
         }
+        if (sizeof(I) == 4) return;
     }
 }
 
 // same block type on both sides: move the blocks as halfwords
-template <typename I, int TYPE>
-__global__ void __launch_bounds__(256) cpy_block_block_kernel(const CpyArgs a) {
+template <typename A, int TYPE>
+__global__ void __launch_bounds__(256) cpy_block_block_kernel(const A a) {
+    typedef typename A::index I;
     constexpr int HW = BlockFormat<TYPE>::BYTES / 2;
     const I   t   = thread_index<I>();
     const I   blk = t / HW;
     const int w   = (int)(t % HW);
     if (blk >= (I)a.n) return;
-    Place sp, tp;
-    both_places<I>(a, blk, FATTN_QK8_0, sp, tp);
-    const uint16_t x = ((const uint16_t *)(a.src + offset_at(sp, a.snb, a.snb[0])))[w];
-    char * dp = a.dst + offset_at(tp, a.dnb, a.dnb[0]) + 2 * w;
+    typename A::offset so, to;
+    offsets(a, blk, FATTN_QK8_0, BlockFormat<TYPE>::BYTES, BlockFormat<TYPE>::BYTES, so, to);
+    const uint16_t x = ((const uint16_t *)(a.src + so))[w];
+    char * dp = a.dst + to + 2 * w;
     *(uint16_t *)dp = x;
     if (a.mirror) *(uint16_t *)(dp + a.mirror) = x;
 }
 
+// bytes of a unit of a destination row
+template <int DTYPE, int UNIT> constexpr int row_unit_bytes() {
+    if constexpr (FATTN_IS_BLOCK_TYPE(DTYPE)) return BlockFormat<DTYPE>::BYTES;
+    else return UNIT * (DTYPE == MI355X_TYPE_F16 ? 2 : 4);
+}
+
+struct RowPlace {
+    int64_t      so, to;                   // of the source unit; of the destination's unit in row 0
+    const char * ip;                       // the row's index
+    int64_t      row_pitch, rows, mirror;
+    bool         i64;
+};
+__device__ __forceinline__ RowPlace row_place(const NarrowRows & a, uint32_t i, int, int64_t sstep, int64_t dstep) {
+    uint32_t so, to, xo;
+    offsets(a, i, (uint32_t)sstep, (uint32_t)dstep, so, to, xo);
+    return {so, to, a.idx + xo, a.dnb[0], a.rows, 0, (a.x2_is_i64 & 1) != 0};
+}
+template <typename I>
+__device__ __forceinline__ RowPlace row_place(const WideCopy<I> & a, I i, int unit0, int64_t sstep, int64_t dstep) {
+    const Place q = place_of<I>(i, a.sne, a.sdiv, unit0);
+    // (a broadcast of the indices over heads and sequences is the rule: no division then)
+    const int64_t x1 = a.ine[1] == 1 ? 0 : a.ine[1] == a.sne[2] ? q.i2 : q.i2 % a.ine[1];
+    const int64_t x2 = a.ine[2] == 1 ? 0 : a.ine[2] == a.sne[3] ? q.i3 : q.i3 % a.ine[2];
+    RowPlace p;
+    p.so = offset_at(q, a.snb, sstep);
+    p.to = q.i0 * dstep + q.i2 * a.dnb[2] + q.i3 * a.dnb[3];
+    p.ip = a.idx + q.i1 * a.inb[0] + x1 * a.inb[1] + x2 * a.inb[2];
+    p.row_pitch = a.dnb[1];
+    p.rows = a.dne[1];
+    p.mirror = a.mirror;
+    p.i64 = a.idx_is_i64;
+    return p;
+}
+template <typename T> __device__ __forceinline__ int64_t element_pitch(const NarrowRows &) { return sizeof(T); }
+
 // SET_ROWS: dst[:, idx[i1, i2 % ine1, i3 % ine2], i2, i3] = convert(src[:, i1, i2, i3]), src F32
 // UNIT elements of a source row per unit: 32 by a quad of lanes (block types), 8 by a lane (F16 / F32 rows that start on 16
 // bytes), or 1 by a lane.  VEC: the source is read with 16-byte loads.
-template <typename I, int DTYPE, int UNIT, bool VEC>
-__global__ void __launch_bounds__(256) set_rows_kernel(const CpyArgs a) {
+template <typename A, int DTYPE, int UNIT, bool VEC>
+__global__ void __launch_bounds__(256) set_rows_kernel(const A a) {
+    typedef typename A::index I;
     constexpr bool BLOCKS = FATTN_IS_BLOCK_TYPE(DTYPE);
     static_assert(BLOCKS ? UNIT == FATTN_QK8_0 : (UNIT == 1 || UNIT == 8), "units");
     const I    u  = BLOCKS ? (I)blockIdx.x * 64 + (threadIdx.x >> 2) : thread_index<I>();
     const int  c  = BLOCKS ? threadIdx.x & 3 : 0;
     const bool ok = u < (I)a.n;
-    const Place p = place_of<I>(ok ? u : 0, a.sne, a.sdiv, UNIT);
-    // (a broadcast of the indices over heads and sequences is the rule: no division then)
-    const int64_t x1 = a.ine[1] == 1 ? 0 : a.ine[1] == a.sne[2] ? p.i2 : p.i2 % a.ine[1];
-    const int64_t x2 = a.ine[2] == 1 ? 0 : a.ine[2] == a.sne[3] ? p.i3 : p.i3 % a.ine[2];
-    const char * ip = a.idx + p.i1 * a.inb[0] + x1 * a.inb[1] + x2 * a.inb[2];
-    const char * sp = a.src + (p.i0 * UNIT + c * 8) * a.snb[0] + p.i1 * a.snb[1] + p.i2 * a.snb[2] + p.i3 * a.snb[3];
+    const int64_t es = VEC ? 4 : element_pitch<float>(a);
+    const RowPlace p = row_place(a, ok ? u : 0, UNIT, UNIT * es, row_unit_bytes<DTYPE, UNIT>());
+    const char * sp = a.src + p.so + c * 8 * es;
     float x[8];
-    if constexpr (UNIT == 1) x[0] = ok ? *(const float *)sp : 0.0f;
-    else                     load8<VEC>(sp, a.snb[0], ok, x);
-    const int64_t drow = a.idx_is_i64 ? *(const int64_t *)ip : (int64_t)*(const int32_t *)ip;
+    // (lanes behind the last unit read the first one: nothing here stands under a guard, so that all loads are one round trip)
+    if constexpr (UNIT == 1) x[0] = *(const float *)sp;
+    else                     load8<VEC>(sp, es, x);
+    const int32_t lo = *(const int32_t *)p.ip, hi = *(const int32_t *)(p.ip + (p.i64 ? 4 : 0));
+    const int64_t drow = (int64_t)((uint64_t)(uint32_t)(p.i64 ? hi : lo >> 31) << 32 | (uint32_t)lo);
     // A row index outside the destination writes nothing (ggml-cpu asserts 0 <= idx < ne1 instead): a stale or
     // uninitialised index tensor must not become a write outside the cache.  The lanes stay in the block's reduction.
-    const bool inside = ok && drow >= 0 && drow < a.dne[1];
-    char * dp = a.dst + p.i0 * a.dnb[0] * (BLOCKS ? 1 : UNIT) + (inside ? drow : 0) * a.dnb[1] + p.i2 * a.dnb[2] + p.i3 * a.dnb[3];
+    const bool inside = ok && drow >= 0 && drow < p.rows;
+    char * dp = a.dst + p.to + (inside ? drow : 0) * p.row_pitch;
     if constexpr (BLOCKS) {
-        quantize_block_store<DTYPE>(x, dp, c, inside, a.mirror);
+        quantize_block_store<DTYPE>(x, dp, c, inside, p.mirror);
     } else if (inside) {
         typedef typename std::conditional<DTYPE == MI355X_TYPE_F16, _Float16, float>::type TD;
-        for (int k = 0; k < (a.mirror ? 2 : 1); k++, dp += a.mirror) {
+        for (int k = 0; k < (p.mirror ? 2 : 1); k++, dp += p.mirror) {
             if constexpr (UNIT == 1) {
                 *(TD *)dp = (TD)x[0];
             } else {
-                Vec8<TD> y;
+                typedef TD V8 __attribute__((ext_vector_type(8)));
+                V8 y;
 #pragma unroll
                 for (int e = 0; e < 8; e++) y[e] = (TD)x[e];
-                *(Vec8<TD> *)dp = y;
+                *(V8 *)dp = y;
             }
         }
     }
@@ -340,7 +421,7 @@ __global__ void __launch_bounds__(256) kv_to_f16_kernel(const FattnArgs a, char 
         y[4] = (_Float16)x1.x; y[5] = (_Float16)x1.y; y[6] = (_Float16)x1.z; y[7] = (_Float16)x1.w;
     } else {
         float f[8];
-        dequant8<TYPE>(row + (c >> 2) * fattn_block_bytes(TYPE), (c & 3) * 8, f);
+        dequant<TYPE>(row + (c >> 2) * fattn_block_bytes(TYPE), (c & 3) * 8, f);
 #pragma unroll
         for (int e = 0; e < 8; e++) y[e] = (_Float16)f[e];
     }
@@ -378,11 +459,11 @@ __global__ void __launch_bounds__(256) kv_to_f16_mixed_kernel(const FattnArgs a,
 #pragma unroll
             for (int e = 0; e < 8; e++) f[e] = h2f_bits(((const uint16_t *)row)[c * 8 + e]);
             break;
-        case MI355X_TYPE_Q8_0: dequant8<MI355X_TYPE_Q8_0>(blk, (c & 3) * 8, f); break;
-        case MI355X_TYPE_Q4_0: dequant8<MI355X_TYPE_Q4_0>(blk, (c & 3) * 8, f); break;
-        case MI355X_TYPE_Q4_1: dequant8<MI355X_TYPE_Q4_1>(blk, (c & 3) * 8, f); break;
-        case MI355X_TYPE_Q5_0: dequant8<MI355X_TYPE_Q5_0>(blk, (c & 3) * 8, f); break;
-        default:               dequant8<MI355X_TYPE_Q5_1>(blk, (c & 3) * 8, f); break;
+        case MI355X_TYPE_Q8_0: dequant<MI355X_TYPE_Q8_0>(blk, (c & 3) * 8, f); break;
+        case MI355X_TYPE_Q4_0: dequant<MI355X_TYPE_Q4_0>(blk, (c & 3) * 8, f); break;
+        case MI355X_TYPE_Q4_1: dequant<MI355X_TYPE_Q4_1>(blk, (c & 3) * 8, f); break;
+        case MI355X_TYPE_Q5_0: dequant<MI355X_TYPE_Q5_0>(blk, (c & 3) * 8, f); break;
+        default:               dequant<MI355X_TYPE_Q5_1>(blk, (c & 3) * 8, f); break;
     }
     typedef _Float16 h8 __attribute__((ext_vector_type(8)));
     h8 y;
@@ -468,14 +549,15 @@ static bool rows_aligned(const void * p, const int64_t (&ne)[4], const int64_t (
     return true;
 }
 
-static bool vec8_ok(const CpyArgs & a, int stype, int dtype) {
-    if (FATTN_IS_BLOCK_TYPE(stype) || FATTN_IS_BLOCK_TYPE(dtype)) return false;
-    const int64_t ss = stype == MI355X_TYPE_F32 ? 4 : 2, ds = dtype == MI355X_TYPE_F32 ? 4 : 2;
-    return a.sne[0] % 8 == 0 && a.dne[0] % 8 == 0 && rows_aligned(a.src, a.sne, a.snb, ss, 8 * ss) &&
-           rows_aligned(a.dst, a.dne, a.dnb, ds, 8 * ds) && (!a.mirror || a.mirror % (8 * ds) == 0);
+// f16 <-> f32 and same-type copies: whether cpy_vec_kernel takes them
+template <typename TS, typename TD>
+static bool vec_ok(const CpyArgs & a) {
+    constexpr int E = vec_elements<TD>(), sal = E * (int)sizeof(TS) < 16 ? E * (int)sizeof(TS) : 16;
+    return a.sne[0] % E == 0 && a.dne[0] % E == 0 && rows_aligned(a.src, a.sne, a.snb, sizeof(TS), sal) &&
+           rows_aligned(a.dst, a.dne, a.dnb, sizeof(TD), 16) && a.mirror % 16 == 0;
 }
 
-// the launch's divisors for units of `unit0` elements; whether 32-bit indices do (`threads` = the grid's)
+// the wide form's divisors for units of `unit0` elements; whether 32-bit indices do (`threads` = the grid's)
 static bool prepare_index(CpyArgs & a, int64_t unit0, int64_t threads) {
     a.same_shape = 1;
     for (int i = 0; i < 4; i++) a.same_shape = a.same_shape && a.sne[i] == a.dne[i];
@@ -488,51 +570,82 @@ static bool prepare_index(CpyArgs & a, int64_t unit0, int64_t threads) {
     return threads + 256 < ((int64_t)1 << 31);
 }
 
-// a kernel of this file over `threads` lanes, with 32-bit indices where they do
-#define CPY_LAUNCH(args, unit0, threads, KERNEL, ...)                                                                    \
-    do {                                                                                                                 \
-        CpyArgs v_ = args;                                                                                               \
-        const int64_t t_ = (threads);                                                                                    \
-        const bool    small_ = prepare_index(v_, unit0, t_);                                                             \
-        const dim3    g_((unsigned)((t_ + 255) / 256));                                                                  \
-        if (small_) hipLaunchKernelGGL((KERNEL<uint32_t, __VA_ARGS__>), g_, dim3(256), 0, stream, v_);                   \
-        else        hipLaunchKernelGGL((KERNEL<int64_t, __VA_ARGS__>), g_, dim3(256), 0, stream, v_);                    \
+// a kernel of this file over `threads` lanes for units of `unit0` elements, a.n of them: in the narrow form where `narrow` filled
+// it in, else in the wide one, with 32-bit indices where they do.  walked: its 64-bit form goes on from the grid's end.
+#define FORM_LAUNCH(a, unit0, threads, walked, narrow, v, KERNEL, ...)                                                         \
+    do {                                                                                                                  \
+        const dim3 g_((unsigned)(((threads) + 255) / 256));                                                               \
+        if (narrow) {                                                                                                     \
+            hipLaunchKernelGGL((KERNEL<decltype(v), __VA_ARGS__>), g_, dim3(256), 0, stream, v);                          \
+            break;                                                                                                        \
+        }                                                                                                                 \
+        WideCopy<uint32_t> w_;                                                                                            \
+        (CpyArgs &)w_ = a;                                                                                                \
+        if (prepare_index(w_, unit0, threads)) {                                                                          \
+            hipLaunchKernelGGL((KERNEL<WideCopy<uint32_t>, __VA_ARGS__>), g_, dim3(256), 0, stream, w_);                  \
+        } else {                                                                                                          \
+            WideCopy<int64_t> l_;                                                                                         \
+            (CpyArgs &)l_ = w_;                                                                                           \
+            const dim3 lg_((unsigned)((((walked) && (threads) > MAX_WALKED ? MAX_WALKED : (threads)) + 255) / 256));      \
+            hipLaunchKernelGGL((KERNEL<WideCopy<int64_t>, __VA_ARGS__>), lg_, dim3(256), 0, stream, l_);                  \
+        }                                                                                                                 \
+    } while (0)
+// (es: bytes of a source element, whole blocks counted as one)
+#define CPY_LAUNCH(a, unit0, es, sstep, dstep, threads, walked, KERNEL, ...)                                                   \
+    do {                                                                                                                  \
+        NarrowCopy v_;                                                                                                    \
+        const bool n_ = (a).snb[0] == (int64_t)(es) && narrow_copy(a, unit0, sstep, dstep, threads, v_);                  \
+        FORM_LAUNCH(a, unit0, threads, walked, n_, v_, KERNEL, __VA_ARGS__);                                                      \
+    } while (0)
+#define ROWS_LAUNCH(a, unit0, threads, ...)                                                                               \
+    do {                                                                                                                  \
+        NarrowRows v_;                                                                                                    \
+        const bool n_ = narrow_rows(a, unit0, threads, v_);                                                               \
+        FORM_LAUNCH(a, unit0, threads, false, n_, v_, set_rows_kernel, __VA_ARGS__);                                             \
     } while (0)
 
 template <typename TS, typename TD>
-static void launch_plain(const CpyArgs & a, bool vec8, hipStream_t stream) {
-    if (vec8) {
+static void launch_plain(const CpyArgs & a, hipStream_t stream) {
+    if (vec_ok<TS, TD>(a)) {
+        constexpr int E = vec_elements<TD>();
         CpyArgs b = a;
-        b.n = a.n / 8;
-        CPY_LAUNCH(b, 8, b.n, cpy_vec8_kernel, TS, TD);
+        b.n = a.n / E;
+        CPY_LAUNCH(b, E, sizeof(TS), E * sizeof(TS), E * sizeof(TD), b.n, true, cpy_vec_kernel, TS, TD);
     } else {
-        CPY_LAUNCH(a, 1, a.n, cpy_scalar_kernel, TS, TD);
+        CPY_LAUNCH(a, 1, sizeof(TS), sizeof(TS), sizeof(TD), a.n, false, cpy_scalar_kernel, TS, TD);
     }
 }
 
 template <int T>
 static void launch_to_blocks(const CpyArgs & a, hipStream_t stream) {
-    if (rows_aligned(a.src, a.sne, a.snb, 4, 16)) CPY_LAUNCH(a, FATTN_QK8_0, a.n * 4, cpy_f32_block_kernel, T, true);
-    else                                          CPY_LAUNCH(a, FATTN_QK8_0, a.n * 4, cpy_f32_block_kernel, T, false);
+    constexpr int U = FATTN_QK8_0, BB = BlockFormat<T>::BYTES;
+    if (rows_aligned(a.src, a.sne, a.snb, 4, 16)) CPY_LAUNCH(a, U, 4, U * 4, BB, a.n * 4, false, cpy_f32_block_kernel, T, true);
+    else                                          CPY_LAUNCH(a, U, 4, U * 4, BB, a.n * 4, false, cpy_f32_block_kernel, T, false);
 }
 
 template <int T>
 static void launch_from_blocks(const CpyArgs & a, hipStream_t stream) {
-    if (rows_aligned(a.dst, a.dne, a.dnb, 4, 16) && a.mirror % 16 == 0) CPY_LAUNCH(a, FATTN_QK8_0, a.n * 4, cpy_block_f32_kernel, T, true);
-    else                                                                CPY_LAUNCH(a, FATTN_QK8_0, a.n * 4, cpy_block_f32_kernel, T, false);
+    constexpr int U = FATTN_QK8_0, BB = BlockFormat<T>::BYTES;
+    if (rows_aligned(a.dst, a.dne, a.dnb, 4, 16) && a.mirror % 16 == 0) CPY_LAUNCH(a, U, BB, BB, U * 4, a.n * 8, true, cpy_block_f32_kernel, T, true);
+    else                                                                CPY_LAUNCH(a, U, BB, BB, U * 4, a.n * 8, true, cpy_block_f32_kernel, T, false);
+}
+
+template <int T>
+static void launch_blocks(const CpyArgs & a, hipStream_t stream) {
+    constexpr int U = FATTN_QK8_0, BB = BlockFormat<T>::BYTES;
+    CPY_LAUNCH(a, U, BB, BB, BB, a.n * (BB / 2), false, cpy_block_block_kernel, T);
 }
 
 int cpy_launch(const CpyArgs & a, int stype, int dtype, hipStream_t stream) {
     if (a.n == 0) return 0;
-    const bool vec8 = vec8_ok(a, stype, dtype);
-    if (stype == MI355X_TYPE_F32 && dtype == MI355X_TYPE_F32)      launch_plain<float, float>(a, vec8, stream);
-    else if (stype == MI355X_TYPE_F32 && dtype == MI355X_TYPE_F16) launch_plain<float, _Float16>(a, vec8, stream);
-    else if (stype == MI355X_TYPE_F16 && dtype == MI355X_TYPE_F16) launch_plain<_Float16, _Float16>(a, vec8, stream);
-    else if (stype == MI355X_TYPE_F16 && dtype == MI355X_TYPE_F32) launch_plain<_Float16, float>(a, vec8, stream);
+    if (stype == MI355X_TYPE_F32 && dtype == MI355X_TYPE_F32)      launch_plain<float, float>(a, stream);
+    else if (stype == MI355X_TYPE_F32 && dtype == MI355X_TYPE_F16) launch_plain<float, _Float16>(a, stream);
+    else if (stype == MI355X_TYPE_F16 && dtype == MI355X_TYPE_F16) launch_plain<_Float16, _Float16>(a, stream);
+    else if (stype == MI355X_TYPE_F16 && dtype == MI355X_TYPE_F32) launch_plain<_Float16, float>(a, stream);
 #define BLOCK_CASES(T)                                                                                                    \
     else if (stype == MI355X_TYPE_F32 && dtype == T) launch_to_blocks<T>(a, stream);                                       \
     else if (stype == T && dtype == MI355X_TYPE_F32) launch_from_blocks<T>(a, stream);                                     \
-    else if (stype == T && dtype == T) CPY_LAUNCH(a, FATTN_QK8_0, a.n * (BlockFormat<T>::BYTES / 2), cpy_block_block_kernel, T);
+    else if (stype == T && dtype == T) launch_blocks<T>(a, stream);
     BLOCK_CASES(MI355X_TYPE_Q8_0)
     BLOCK_CASES(MI355X_TYPE_Q4_0)
     BLOCK_CASES(MI355X_TYPE_Q4_1)
@@ -548,16 +661,16 @@ template <int T>
 static void launch_set_rows(const CpyArgs & a, hipStream_t stream) {
     const bool vec = rows_aligned(a.src, a.sne, a.snb, 4, 16);
     if constexpr (FATTN_IS_BLOCK_TYPE(T)) {
-        if (vec) CPY_LAUNCH(a, FATTN_QK8_0, a.n * 4, set_rows_kernel, T, FATTN_QK8_0, true);
-        else     CPY_LAUNCH(a, FATTN_QK8_0, a.n * 4, set_rows_kernel, T, FATTN_QK8_0, false);
+        if (vec) ROWS_LAUNCH(a, FATTN_QK8_0, a.n * 4, T, FATTN_QK8_0, true);
+        else     ROWS_LAUNCH(a, FATTN_QK8_0, a.n * 4, T, FATTN_QK8_0, false);
     } else {
         const int64_t ds = T == MI355X_TYPE_F16 ? 2 : 4;
         if (vec && a.sne[0] % 8 == 0 && rows_aligned(a.dst, a.dne, a.dnb, ds, 8 * ds) && a.mirror % (8 * ds) == 0) {
             CpyArgs b = a;
             b.n = a.n / 8;
-            CPY_LAUNCH(b, 8, b.n, set_rows_kernel, T, 8, true);
+            ROWS_LAUNCH(b, 8, b.n, T, 8, true);
         } else {
-            CPY_LAUNCH(a, 1, a.n, set_rows_kernel, T, 1, false);
+            ROWS_LAUNCH(a, 1, a.n, T, 1, false);
         }
     }
 }

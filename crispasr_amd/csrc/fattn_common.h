@@ -24,7 +24,7 @@ static inline FastDiv fast_div(uint32_t d) {
     f.m = d ? (uint32_t)((((uint64_t)1 << 32) * (((uint64_t)1 << f.s) - d)) / d + 1) : 0;
     return f;
 }
-static __device__ __forceinline__ uint32_t divide(uint32_t n, const FastDiv & f) { return (__umulhi(n, f.m) + n) >> f.s; }
+static __host__ __device__ __forceinline__ uint32_t divide(uint32_t n, const FastDiv & f) { return ((uint32_t)(((uint64_t)n * f.m) >> 32) + n) >> f.s; }
 
 // Everything a kernel needs about one FLASH_ATTN_EXT node, by value.
 struct FattnArgs {
@@ -323,16 +323,16 @@ static inline __host__ __device__ int fattn_block_bytes(int type) {
     }
 }
 
-// elements j0 .. j0+7 (j0 = 0, 8, 16 or 24) of one block as f32: q*d is exact, q*d + m is one product and one sum,
-// each rounded to f32 (not fused).  Blocks are only 2-byte aligned: halfword reads.
-template <int TYPE>
-static __device__ __forceinline__ void dequant8(const char * blk, int j0, float (&out)[8]) {
+// elements j0 .. j0+N-1 (N = 4 or 8, j0 a multiple of it) of one block as f32: q*d is exact, q*d + m is one product and one
+// sum, each rounded to f32 (not fused).  Blocks are only 2-byte aligned: halfword reads.
+template <int TYPE, int N>
+static __device__ __forceinline__ void dequant(const char * blk, int j0, float (&out)[N]) {
     typedef BlockFormat<TYPE> F;
     const float d = h2f_bits(*(const uint16_t *)blk);
     if (TYPE == MI355X_TYPE_Q8_0) {
         const uint16_t * qs = (const uint16_t *)(blk + 2 + j0);
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < N / 2; i++) {
             const uint16_t w = qs[i];
             out[2 * i]     = (float)(int8_t)(w & 0xff) * d;
             out[2 * i + 1] = (float)(int8_t)(w >> 8) * d;
@@ -340,7 +340,7 @@ static __device__ __forceinline__ void dequant8(const char * blk, int j0, float 
         return;
     }
     const float m = F::HAS_M ? h2f_bits(*(const uint16_t *)(blk + 2)) : 0.0f;
-    const uint16_t * qs = (const uint16_t *)(blk + F::QS + (j0 & 8));       // elements j and j + 16 share a byte
+    const uint16_t * qs = (const uint16_t *)(blk + F::QS + (j0 & 15));      // elements j and j + 16 share a byte
     const int sh = (j0 & 16) ? 4 : 0;
     uint32_t hb = 0;
     if (F::QH) {
@@ -348,7 +348,7 @@ static __device__ __forceinline__ void dequant8(const char * blk, int j0, float 
         hb = (((uint32_t)qh[0] | (uint32_t)qh[1] << 16) >> j0) & 0xffu;
     }
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < N / 2; i++) {
         const uint32_t w  = qs[i];
         const int      q0 = (int)(((w >> sh) & 15u) | (((hb >> (2 * i)) & 1u) << 4));
         const int      q1 = (int)(((w >> (8 + sh)) & 15u) | (((hb >> (2 * i + 1)) & 1u) << 4));

@@ -43,7 +43,7 @@ static __device__ __forceinline__ void row_load8(const char * row, int d0, bool 
             for (int i = 0; i < 8; i++) out[i] = i < nvalid ? f[i] : 0.0f;
         }
     } else {  // block-32 types: blocks are only 2-byte aligned
-        dequant8<TYPE>(row + (size_t)(d0 / FATTN_QK8_0) * fattn_block_bytes(TYPE), d0 % FATTN_QK8_0, out);
+        dequant<TYPE>(row + (size_t)(d0 / FATTN_QK8_0) * fattn_block_bytes(TYPE), d0 % FATTN_QK8_0, out);
     }
 }
 
