@@ -18,7 +18,7 @@ static __device__ __align__(256) unsigned char scratch[MI355X_NOALLOC_SCRATCH_BY
 // loaded, and left at zero by every launch.  Set 0 serves calls that run on the library's own scratch block, set 1 the
 // allocation-free entry point: each of the two is one-call-at-a-time per GPU by its contract, and a call of one may
 // overlap a call of the other.  A call on a caller's workspace may overlap anything and merges in a launch of its own.
-constexpr int MERGE_COUNTERS = 16384;
+constexpr int MERGE_COUNTERS = FATTN_COUNTERS;
 static __device__ __align__(256) unsigned merge_counters[2 * MERGE_COUNTERS];
 
 namespace {
@@ -697,7 +697,9 @@ void make_plan_core(const FattnArgs & a0, int ktype, int vtype, const mi355x_fat
         plan.n_splits = ns;
         plan.keys_per_split = a.Nkv > 0 ? kps : 0;
         if (ns > 1) plan.workspace += (size_t)rows * ns * (a.D + 2) * sizeof(float);
-        if (ns > 1 && groups <= MERGE_COUNTERS) plan.merge_sets = groups;      // (vector kernel: one set per row)
+        // (vector kernel: one set per row.  Decode kernel: a wave merges up to four rows of a set, whose partials it reads within
+        //  4 GiB of the first one's - with 128-wide heads, 16384 heads in 128 ranges are too many)
+        if (ns > 1 && groups <= MERGE_COUNTERS && (int64_t)a.Hq * ns * a.D * 16 < 0xFFF00000LL) plan.merge_sets = groups;
     }
 }
 

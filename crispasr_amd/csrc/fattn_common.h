@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <atomic>
+#include <type_traits>
 
 #include "../../include/mi355x_fattn.h"
 
@@ -211,39 +212,65 @@ static __device__ __forceinline__ void device_store(float * p, float v) {
 static __device__ __forceinline__ void device_store2(float * p, float v0, float v1) {
     __hip_atomic_store((uint64_t *)p, __builtin_bit_cast(uint64_t, make_float2(v0, v1)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-static __device__ __forceinline__ float2 device_load2(const float2 * p) {
-    const uint64_t u = __hip_atomic_load((const uint64_t *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return __builtin_bit_cast(float2, u);
-}
-static __device__ __forceinline__ float4 device_load4(const float4 * p) {
-    const float2 lo = device_load2((const float2 *)p), hi = device_load2((const float2 *)p + 1);
-    return make_float4(lo.x, lo.y, hi.x, hi.y);
-}
 
-// out[row] = sum_s acc_s * exp(m_s - M) / sum_s l_s * exp(m_s - M), for the four values d4*4 .. d4*4+3 of the row.
-// The (m, l) pairs and the accumulators of FATTN_MERGE_BATCH splits are requested together, and the next batch is
-// requested before the current one is folded in: a row costs about one memory round trip however many splits it has
-// (folded in split order, one batch after the other, whatever is in flight).  DEVICE: the partials come from other
-// workgroups of this launch.
-constexpr int FATTN_MERGE_BATCH = 8;
+// `bytes` bytes from `base` on as a buffer, base and length the same for every lane: loads behind its end give zeros and do not
+// reach memory.  (Descriptor word 3: raw dwords.)
+static __device__ __forceinline__ __amdgpu_buffer_rsrc_t fattn_buffer(const void * base, uint32_t bytes) {
+    const uint64_t b = (uint64_t)base;
+    const uint64_t u = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
+    return __builtin_amdgcn_make_buffer_rsrc((void *)u, 0, __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000);
+}
+constexpr uint32_t FATTN_NO_ADDRESS = 0xFFFFFFF0u;          // an offset behind every buffer's end
+
+// out[row] = sum_s acc_s * exp(m_s - M) / sum_s l_s * exp(m_s - M), for the four values d4*4 .. d4*4+3 of the row, folded in in
+// split order.  DEVICE: the partials come from other workgroups of this launch (and the rows of a wave rise with its lanes, all
+// their partials within 4 GiB).
+// The (m, l) pairs and the accumulators of 4, 8 or 16 splits are requested together, so that a row costs one memory round trip
+// up to 16 splits.  What counts beside that round trip is the number of requests: they take 16 bytes (two pairs, or four values)
+// and ask memory for nothing behind the last split.  Against batches of 8 in 8-byte requests, the next batch behind a branch
+// (for which the compiler waited as if for both), with the counters below, us a call inside a graph: 5 rows x 20 heads of 64,
+// 8 splits 7.83 -> 7.0; 8 heads of 128, 7 splits of Q8_0 7.8 -> 7.45, 13 splits of f16 9.9 -> 9.1, 16 of Q4_0 9.9 -> 8.8.
 template <bool DEVICE>
 static __device__ __forceinline__ void fattn_merge_row(const FattnArgs & a, int64_t row, int d4) {
-    constexpr int NB = FATTN_MERGE_BATCH;
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    const int n   = a.n_splits;
     const int lpr = a.D / 4;
-    const float2 * pm = (const float2 *)(a.part_ml + (size_t)row * a.n_splits * 2);
-    const float4 * pa = (const float4 *)(a.part_acc + (size_t)row * a.n_splits * a.D) + d4;
+    const float2 * pm = (const float2 *)(a.part_ml + (size_t)row * n * 2);
+    const float4 * pa = (const float4 *)(a.part_acc + (size_t)row * n * a.D) + d4;
     float4 out = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     float  M = -INFINITY, L = 0.0f;
-    auto request = [&](int s0, float2 (&ml)[NB], float4 (&v)[NB]) __attribute__((always_inline)) {
+    auto fold = [&](auto batch, int s0) __attribute__((always_inline)) {
+        constexpr int NB = decltype(batch)::value;
+        float2 ml[NB];
+        float4 v[NB];
+        if constexpr (DEVICE) {
+            const int64_t  first = (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(row >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)row);
+            const uint64_t after = (uint64_t)((int64_t)a.Nq * a.Hq * a.B - first) * n;          // splits of the rows from there on
+            const auto     bm = fattn_buffer(a.part_ml + (size_t)first * n * 2, (uint32_t)min(after * 8, (uint64_t)0xFFFFFFE0u));
+            const auto     ba = fattn_buffer(a.part_acc + (size_t)first * n * a.D, (uint32_t)min(after * a.D * 4, (uint64_t)0xFFFFFFE0u));
+            const uint32_t at = (uint32_t)(row - first) * (uint32_t)n;
 #pragma unroll
-        for (int i = 0; i < NB; i++) {
-            const int s = min(s0 + i, a.n_splits - 1);          // (past the end: a second look at the last one, not used)
-            ml[i] = DEVICE ? device_load2(pm + s) : pm[s];
-            v[i]  = DEVICE ? device_load4(pa + (size_t)s * lpr) : pa[(size_t)s * lpr];
-            if (s0 + i >= a.n_splits) ml[i] = make_float2(-INFINITY, 0.0f);
+            for (int i = 0; i < NB; i += 2) {
+                const u4 x = __builtin_amdgcn_raw_buffer_load_b128(bm, (int)(s0 + i < n ? (at + s0 + i) * 8 : FATTN_NO_ADDRESS), 0, 16);      // sc1
+                ml[i]     = make_float2(__uint_as_float(x[0]), __uint_as_float(x[1]));
+                ml[i + 1] = make_float2(__uint_as_float(x[2]), __uint_as_float(x[3]));
+            }
+#pragma unroll
+            for (int i = 0; i < NB; i++) {
+                const u4 x = __builtin_amdgcn_raw_buffer_load_b128(ba, (int)(s0 + i < n ? ((at + s0 + i) * lpr + d4) * 16 : FATTN_NO_ADDRESS), 0, 16);
+                v[i] = make_float4(__uint_as_float(x[0]), __uint_as_float(x[1]), __uint_as_float(x[2]), __uint_as_float(x[3]));
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < NB; i++) {
+                const int s = min(s0 + i, n - 1);           // (past the end: a second look at the last one, not used)
+                ml[i] = pm[s];
+                v[i]  = pa[(size_t)s * lpr];
+            }
         }
-    };
-    auto fold = [&](const float2 (&ml)[NB], const float4 (&v)[NB]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NB; i++)
+            if (s0 + i >= n) ml[i].x = -INFINITY;
         float Mb = M;
 #pragma unroll
         for (int i = 0; i < NB; i++) Mb = fmaxf(Mb, ml[i].x);
@@ -263,17 +290,10 @@ static __device__ __forceinline__ void fattn_merge_row(const FattnArgs & a, int6
             out.w += seen ? v[i].w * w : 0.0f;
         }
     };
-    float2 ml0[NB], ml1[NB];
-    float4 v0[NB], v1[NB];
-    request(0, ml0, v0);
-    for (int s0 = 0; s0 < a.n_splits; s0 += 2 * NB) {
-        const bool more1 = s0 + NB < a.n_splits, more2 = s0 + 2 * NB < a.n_splits;
-        if (more1) request(s0 + NB, ml1, v1);
-        fold(ml0, v0);
-        if (!more1) break;
-        if (more2) request(s0 + 2 * NB, ml0, v0);
-        fold(ml1, v1);
-    }
+    if (n <= 4)      fold(std::integral_constant<int, 4>{}, 0);
+    else if (n <= 8) fold(std::integral_constant<int, 8>{}, 0);
+    else
+        for (int s0 = 0; s0 < n; s0 += 16) fold(std::integral_constant<int, 16>{}, s0);
     const float inv = L > 0.0f ? 1.0f / L : 0.0f;
     out.x *= inv; out.y *= inv; out.z *= inv; out.w *= inv;
     // (dst rows are Dv floats - the head size - also where the partial rows are those of a head zero-padded to D)
@@ -285,17 +305,20 @@ static __device__ __forceinline__ void fattn_merge_row(const FattnArgs & a, int6
 // used ordinary stores says so with `wrote_plain`, and pays for a write-back of its die's whole L2): every thread waits
 // for its stores to be acknowledged before the workgroup counts itself done, and the merging workgroup reads by
 // device_load.  All threads of the workgroup must call this; `flag` is a word of LDS that nothing else uses from here on.
-// The counter is zero again when the set is complete.
+// The counter wraps to zero when the set is complete.
+// The sets' counters lie on cache lines of their own: the chip performs atomics on one line one after another.  Workgroups that
+// only store, count and leave, all at the same time: 8 sets of 7 splits 2.7 us a launch with the counters side by side and a
+// store that clears them, 2.0 like this; 20 of 8 3.6, 2.1; 8 of 16 3.4, 2.1 (an empty launch 1.65).
+constexpr int FATTN_COUNTERS = 16384;              // a set number's own line below 512, shared by 32 at most beyond
+static __device__ __forceinline__ uint32_t fattn_counter_of(int64_t group) {
+    constexpr uint32_t LINE = 32, LINES = FATTN_COUNTERS / LINE;
+    return (uint32_t)group % LINES * LINE + (uint32_t)group / LINES;
+}
 static __device__ __forceinline__ bool fattn_last_of_set(const FattnArgs & a, int64_t group, int n, int * flag, bool wrote_plain) {
     if (wrote_plain) __threadfence();
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (threadIdx.x == 0) {
-        const unsigned old = __hip_atomic_fetch_add(a.counters + group, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const bool     all = old == (unsigned)(n - 1);
-        if (all) __hip_atomic_store(a.counters + group, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        *flag = all;
-    }
+    if (threadIdx.x == 0) *flag = atomicInc(a.counters + fattn_counter_of(group), (unsigned)(n - 1)) == (unsigned)(n - 1);
     __syncthreads();
     return *flag != 0;
 }
