@@ -469,6 +469,70 @@ void use_f16_copies(FattnArgs & a, void * ws) {
 // A K and a V of different storage types (CRISPASR_KV_QUANT_K / _V, src/core/attention.h:132-137) are both rounded to f16
 // copies first, whatever the kernel: the call is then planned and run as an F16 one.
 
+// Whether the decode kernel's keys are cut into ranges at all (two to `most` of them): where that prices within a tenth of the
+// uncut call.  An uncut call uses no scratch, so that it may be the first one to be captured and overlap any other; which calls
+// those are stays as it is, also where the pricing below would cut them (it counts the merge at the 1 us and more a range that
+// it once took).  Price, in us: the longer of the cache's pass through HBM and a wave's chain of 32-key steps - four of them 0.7
+// on 64-wide heads, 1.3 on wider ones, more where workgroups share a CU - and the merge.
+bool decode_is_cut(const FattnArgs & a, int ktype, int vtype, int64_t groups, int most) {
+    const double rows  = (double)(a.Nq * a.gqa < 16 ? a.Nq * a.gqa : 16);
+    const double bytes = (double)a.Hkv * a.B * a.Nkv *
+                         (double)(a.D / block_size(ktype) * type_size(ktype) + a.D / block_size(vtype) * type_size(vtype));
+    const double t_hbm = bytes > 8.0e6 ? (bytes - 8.0e6) / 5.0e6 : 0.0;      // (the first megabytes are a matter of latency, which the chain prices)
+    auto price = [&](int n, int keys) {
+        const double per_cu = (double)groups * n / a.n_cus, chain = (keys > 128 ? keys / 128.0 : 1.0) * (a.D <= 64 ? 0.7 : 1.3) * (per_cu > 1.0 ? per_cu : 1.0);
+        return (chain > t_hbm ? chain : t_hbm) + (n > 1 ? 1.0 + n * (0.25 + 0.017 * rows) : 0.0);
+    };
+    const double limit = price(1, (a.Nkv + 31) / 32 * 32) * 1.10;
+    for (int n = 2; n <= most && n <= 256; n++) {
+        const int keys = ((a.Nkv + n - 1) / n + 31) / 32 * 32;
+        if ((a.Nkv + keys - 1) / keys == n && price(n, keys) <= limit) return true;
+    }
+    return false;
+}
+
+// Into how many ranges: the count of least price.  In us: the longest of
+//  - a workgroup's chain of four 32-key steps at a time, its waves side by side: 0.9 on 64-wide heads and 1.5 on 128-wide ones over
+//    f16, by type otherwise; workgroups that share a CU, 4 and 2 of them at once, add 0.62 of a chain each, the next ones start over;
+//  - what a CU's workgroups pull through its one port, 31 GB/s;
+//  - the cache's pass through HBM, 8 TB/s beyond the first 8 MB;
+// with 0.3 of the other two, and 2.25 for the hand-over, more where it goes in batches of 8 and 16 ranges (fattn_merge_row), by the
+// rows and ranges, and where 16 ranges are not enough.  A masked token is taken to see 0.8 of its cache.  The constants were fitted on 460 shapes timed at up to 15
+// forced counts each, K/V cold (steps, batches of ragged and of full length, beams, cross-attention, several rows; f16, Q8_0, Q4_0,
+// Q5_1; 20 to 4096 keys): 2.1% off the best count in the geometric mean, the calls that stay uncut included, where the pricing
+// above, which also chose the count, is 5.0% off: 5 rows x 20 heads of 64 against 560 keys 7.5 -> 6.8 us in 7 ranges instead of
+// 4, 2048 Q8_0 entries under 8 heads of 128 9.5 -> 8.6 in 16 instead of 11, 10 sequences of up to 1025 f16 entries x 8 heads of
+// 128 16.4 -> 14.0 in 3 instead of 6.
+// The partials of a count past two take no more than 4 MiB with what the call needs beside them: half of the smallest scratch block.
+int decode_ranges(const FattnArgs & a, int type, int64_t groups, size_t beside) {
+    const bool   wide  = a.D > 64, narrow = type != MI355X_TYPE_F16 && type != MI355X_TYPE_Q8_0;
+    const double step  = (wide ? 1.5 : 0.9) * (narrow ? (wide ? 1.5 : 1.6) : type == MI355X_TYPE_Q8_0 ? (wide ? 0.95 : 0.77) : 1.0);
+    const double seen  = a.masked && a.Nq == 1 ? 0.8 : 1.0;
+    const double key   = 2.0 * (double)(a.D / block_size(type) * type_size(type)) * seen;      // bytes of a key's K and V rows
+    const double bytes = (double)a.Hkv * a.B * a.Nkv * key;
+    const double t_hbm = bytes > 8.0e6 ? (bytes - 8.0e6) / 8.0e6 : 0.0;
+    const double rows  = (double)(a.Nq * a.gqa < 16 ? a.Nq * a.gqa : 16);
+    const int    slots = wide ? 2 : 4;
+    const size_t part  = (size_t)a.Nq * a.Hq * a.B * (a.D + 2) * sizeof(float);
+    int    best   = 1;
+    double lowest = 1e30;
+    for (int n = 1; n <= 64 && n * 32 <= a.Nkv + 31; n += n < 16 ? 1 : n < 32 ? 4 : 16) {
+        const int keys = ((a.Nkv + n - 1) / n + 31) / 32 * 32;
+        if ((a.Nkv + keys - 1) / keys != n) continue;                   // not a count that whole steps give
+        if (!wide && a.Nkv < 512 && a.Nq * a.gqa == 1 && n * 128 > a.Nkv) break;
+        if (n > 2 && beside + part * n > ((size_t)4 << 20)) break;
+        const int    per_cu = (int)((groups * n + a.n_cus - 1) / a.n_cus), rounds = per_cu / slots, rest = per_cu % slots;
+        const double shared = rounds * (1.0 + 0.62 * (slots - 1)) + (rest ? 1.0 + 0.62 * (rest - 1) : 0.0);
+        const double chain  = (1.0 + ((keys + 127) / 128 - 1) * seen) * step * shared + (per_cu > slots ? 4.5 * (per_cu - slots) : 0.0);
+        const double port   = per_cu * keys * key / 31.0e3;
+        const double most   = chain > port ? (chain > t_hbm ? chain : t_hbm) : port > t_hbm ? port : t_hbm;
+        const double merge  = n == 1 ? 0.0 : (n <= 4 ? 2.25 : n <= 8 ? 2.5 : 3.65 + 12.0 * ((n + 15) / 16 - 1)) + 0.0035 * n * rows;
+        const double price  = most + 0.3 * (chain + port + t_hbm - most) + merge;
+        if (price <= lowest) { lowest = price; best = n; }
+    }
+    return best;
+}
+
 // (padded: a0.D is the padded head size and the copies are needed whatever the types)
 void make_plan_core(const FattnArgs & a0, int ktype, int vtype, const mi355x_fattn_params * p, bool padded, Plan & plan) {
     FattnArgs a = a0;
@@ -625,9 +689,7 @@ void make_plan_core(const FattnArgs & a0, int ktype, int vtype, const mi355x_fat
         const int64_t rows = (int64_t)a.Nq * a.Hq * a.B;
         // workgroups that exist before splitting, and the fewest keys worth a split
         const int64_t groups   = kernel == MI355X_FATTN_VEC ? rows : (int64_t)a.Hkv * a.B * a.q_chunks;
-        // decode kernel: a split must be worth the merge launch (about 2.5 us): measured on Whisper cross-attention
-        // (64-wide heads, 1500 keys: best at 8 splits) and a Q8_0 LLM cache (128-wide, 663 keys: best at 6 to 8),
-        // while 224 keys are fastest unsplit
+        // decode kernel: the bounds within which a cut is weighed at all
         // vector kernel (one workgroup per row and range; sweep of 1 and 2 queries x 8 .. 128 heads x sequences against 224 ..
         // 4096 F32 keys, twelve forced counts each, also with K/V that no cache holds): 1.5 workgroups per CU in all, a power
         // of two per row; ranges of at least 128 keys, for heads wider than 64 of 56 keys up to 448 keys and 112 beyond;
@@ -640,8 +702,6 @@ void make_plan_core(const FattnArgs & a0, int ktype, int vtype, const mi355x_fat
             // whole splits only while they still fit the target: past it a split doubles the grid and adds the merge
             ns = kernel == MI355X_FATTN_VEC ? (int)((target + groups - 1) / (groups > 0 ? groups : 1))
                                             : (int)(target / (groups > 0 ? groups : 1));
-            // (decode kernel: to the nearest count - 1500 keys are faster in 8 ranges of 192 than in 7 of 224, 663 in 7 of 96
-            //  than in 6 of 128, by 2-3%)
             const int max_by_keys = kernel == MI355X_FATTN_VEC ? (a.Nkv < 2 * min_keys ? 1 : (a.Nkv + min_keys - 1) / min_keys)
                                                                : (a.Nkv + min_keys / 2) / min_keys;
             if (ns > max_by_keys) ns = max_by_keys;
@@ -654,38 +714,8 @@ void make_plan_core(const FattnArgs & a0, int ktype, int vtype, const mi355x_fat
                 const int cap = a.Nkv >= 4096 ? 16 : 8;
                 if (ns > cap) ns = cap;
             }
-            // Decode kernel, long caches under few heads: those bounds alone give 40 to 64 ranges, and every range costs the
-            // set's merge (0.2 us each for one row, 0.45 us for sixteen: 4096 f16 keys x 8 heads of 128 took 16 us in
-            // 43 ranges and 12 us in 16).  Of the counts up to that bound, take the one a small model likes best -
-            // the longer of the cache's pass through HBM (at 5 TB/s) and a wave's chain of 32-key steps (four of them 0.7 us
-            // on 64-wide heads, 1.3 us on wider ones, more where workgroups share a CU), plus 1 us for the merge and a
-            // share for every range - and the larger count among near-equals (663 keys stay at 7 ranges, 1500 at 8).
-            // With K/V that no cache holds, 2 ranges were almost never the best count and up to 384 keys (256 under
-            // 128-wide heads) no split was: the fixed microsecond is what keeps those whole.  Against the best of ten forced counts on 192 shapes (1024 .. 8192 keys, 8 .. 40 KV
-            // heads x sequences, 1 .. 64 rows each, f16 and Q8_0) this is 5% off in the geometric mean, 35% at worst;
-            // the bounds alone were 20% and 2x.
-            if (kernel == MI355X_FATTN_DECODE_MMA && ns > 1) {
-                const double rows   = (double)(a.Nq * a.gqa < 16 ? a.Nq * a.gqa : 16);
-                const double per    = 0.25 + 0.017 * rows;
-                double t_hbm = ((double)a.Hkv * a.B * a.Nkv *
-                                (double)(a.D / block_size(ktype) * type_size(ktype) + a.D / block_size(vtype) * type_size(vtype)) - 8.0e6) / 5.0e6;
-                if (t_hbm < 0.0) t_hbm = 0.0;       // (the first megabytes are a matter of latency, which the chain prices)
-                double best = 1e30, est[257];
-                if (ns > 256) ns = 256;
-                for (int n = 1; n <= ns; n++) {
-                    const int kps_n = ((a.Nkv + n - 1) / n + 31) / 32 * 32;
-                    est[n] = 2e30;
-                    if ((a.Nkv + kps_n - 1) / kps_n != n) continue;             // not a count that whole steps give
-                    double chain = kps_n / 128.0;
-                    if (chain < 1.0) chain = 1.0;
-                    chain *= a.D <= 64 ? 0.7 : 1.3;
-                    const double per_cu = (double)groups * n / a.n_cus;     // workgroups sharing a CU share its steps
-                    if (per_cu > 1.0) chain *= per_cu;
-                    est[n] = (chain > t_hbm ? chain : t_hbm) + (n > 1 ? 1.0 + n * per : 0.0);
-                    if (est[n] < best) best = est[n];
-                }
-                while (ns > 1 && est[ns] > best * 1.10) ns--;
-            }
+            if (kernel == MI355X_FATTN_DECODE_MMA && ns > 1)
+                ns = decode_is_cut(a, ktype, vtype, groups, ns) ? decode_ranges(a, ktype, groups, plan.workspace) : 1;
         }
         if (ns > a.Nkv) ns = a.Nkv;
         if (ns < 1) ns = 1;
