@@ -20,6 +20,12 @@
 // Against the tile-wise kernel it replaced for these forms, per launch: 20 x 64 x 1500^2 in batches of 4 60.2 -> 56.8 us
 // (0.81 PFLOP/s), 8 x 64 x 1500 against 1536 keys 14.4 -> 12.8, 8 x 128 x 1500^2 x 4 55.2 -> 52.6, 10 x 128 x 1500^2 31.2 ->
 // 23.6, 64 x 128 x 300^2 14.9 -> 12.5, 30 x 64 x 300^2 8.8 -> 7.7.
+// Workgroups of eight waves, twice the queries (W = 8), bring a CU every block of K and V once instead of twice: the requests,
+// timed without them, were 12% of the first of these launches and 15% of the third.  Taken where they fill the CUs as evenly:
+// 20 x 64 x 1500^2 x 4 60.6 -> 59.4 us (one box), 12 x 64 x 1500^2 x 4 46.4 -> 42.9, 20 x 64 x 1000^2 x 4 37.2 -> 35.4, 8 x 128 x
+// 1500^2 x 4 55.8 -> 53.4, 8 x 128 x 750^2 x 8 33.6 -> 32.0; where they leave more CUs empty they lose (10 x 128 x 1500^2 x 2
+// 37.2 -> 44.6).  Eight waves that share the queries of two or four (the keys in turn), for a grid that leaves CUs to one
+// workgroup of four, changed nothing at 1500 keys (8 x 64 16.0 us either way) and lost 1 us below 1000.
 // What is left above the MFMAs of a wave alone on its SIMD is instruction issue (about 5 cycles an instruction).  Where two
 // share a SIMD nothing is full: by the counters of the first of these launches the matrix cores are busy for 49% of it (at
 // 1.85 GHz) and the vector ALU for 38%, and a wave stands ready for another instruction to end for 39% of its cycles and
@@ -38,8 +44,6 @@ typedef float    float4v __attribute__((ext_vector_type(4)));
 typedef short    short4v __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
 
-constexpr int   PIPE_WAVES   = 4;
-constexpr int   PIPE_THREADS = PIPE_WAVES * 64;
 constexpr int   RING         = 4;                  // slots per tensor (a power of two)
 constexpr float LOG2E        = 1.4426950408889634f;
 
@@ -54,17 +58,20 @@ typedef __attribute__((address_space(3))) short4v     lds_short4;
 // instructions stay on their side of it
 #define PIPE_FENCE() __builtin_amdgcn_sched_barrier(0)
 
-constexpr int pipe_lds_bytes(int D, int NQB, int KSP) {
+constexpr int pipe_lds_bytes(int D, int NQB, int KSP, int W) {
     const int ring  = 2 * RING * KSP * 32 * D * 2;
-    const int stage = PIPE_WAVES * 32 * D * 4;                                  // result rows / the pairs' partial results
+    const int stage = W * 32 * D * 4;                                           // result rows / the waves' partial results
     return ring > stage ? ring : stage;
 }
 
-// NQB: 32-query blocks per wave.  KSP = 2: waves w and w + 2 share their queries and take alternate 32-key blocks.
+// NQB: 32-query blocks per wave.  KSP = 2: the second half of the W waves shares the queries of the first and takes alternate
+// 32-key blocks.
 // PAD: heads of a.Dv elements (a multiple of 8 below D) on copies of K and V whose rows are zero-padded to D.
-template <int D, int NQB, int KSP, bool PAD>
-__global__ void __launch_bounds__(PIPE_THREADS, 2) fattn_pipe_kernel(const FattnArgs a, const int n_qtiles) {
+template <int D, int NQB, int KSP, int W, bool PAD>
+__global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a, const int n_qtiles) {
     static_assert(NQB == 1 || (NQB == 2 && D == 64 && KSP == 1 && !PAD), "forms");
+    constexpr int PIPE_THREADS = W * 64;
+    constexpr int QG   = W / KSP;                                 // waves that take different queries
     constexpr int KS   = D / 16;                                  // reduction steps of Q.K^T
     constexpr int DB   = D / 32;                                  // 32-wide blocks of the output's d
     constexpr int CH   = D / 8;                                   // 16-byte chunks per row
@@ -72,13 +79,17 @@ __global__ void __launch_bounds__(PIPE_THREADS, 2) fattn_pipe_kernel(const Fattn
     constexpr int BLKB = 32 * ROWB;                               // bytes of a block
     constexpr int STEPB = KSP * BLKB;                             // ... of a step: one block for every wave of a pair
     constexpr int SKEYS = KSP * 32;
-    constexpr int NLD  = STEPB / 1024 / PIPE_WAVES;               // loads per wave, step and tensor
+    // A step of one tensor is STEPB / 1024 load instructions.  Every wave makes its share of K's and of V's, NLD each, or (HALVES,
+    // where there are fewer of them than waves) the first half of the waves K's and the second V's.
+    constexpr bool HALVES = STEPB / 1024 < W;
+    constexpr int  NLD  = HALVES ? STEPB / 512 / W : STEPB / 1024 / W;
+    constexpr int  NLS  = HALVES ? NLD : 2 * NLD;                 // loads per wave and step
     constexpr int R    = RING;
     // steps ahead of the current one that its start requests, and loads that may still be under way then
     constexpr int DK   = R, DV = NQB == 2 ? R - 1 : R - 2;
-    constexpr int OPEN = (NQB == 2 ? R - 2 : R - 3) * 2 * NLD;
+    constexpr int OPEN = (NQB == 2 ? R - 2 : R - 3) * NLS;
     constexpr int BMW  = 32 * NQB;
-    constexpr int BMG  = BMW * PIPE_WAVES / KSP;
+    constexpr int BMG  = BMW * QG;
     constexpr int NM   = KS + 2 * DB;                             // MFMAs of a region
     constexpr int EPS  = 16 / NM;                                 // exponentials per MFMA
     // The reference m enters the scores as the C operand of their first MFMA, 16 registers of one value, and the exponentials
@@ -93,8 +104,8 @@ __global__ void __launch_bounds__(PIPE_THREADS, 2) fattn_pipe_kernel(const Fattn
     const int lane = tid & 63;
     const int l32  = lane & 31;
     const int hh   = lane >> 5;
-    const int qgroup = KSP == 2 ? wave & 1 : wave;
-    const int kgroup = KSP == 2 ? wave >> 1 : 0;
+    const int qgroup = wave % QG;
+    const int kgroup = wave / QG;
 
     // Workgroups go to the 8 XCDs round-robin; renumbered so that the query tiles of one (head, batch), which share K/V, sit
     // on one XCD and meet in its L2.
@@ -136,30 +147,45 @@ __global__ void __launch_bounds__(PIPE_THREADS, 2) fattn_pipe_kernel(const Fattn
     const uint64_t vbase = (uint64_t)(a.v + (int64_t)hk * a.nbv2 + (int64_t)bk * a.nbv3 + (int64_t)k_begin * a.nbv1);
 
     // ---- global -> LDS: slot L = (wave * NLD + j) * 64 + lane of a step holds chunk (L % CH) ^ swizzle of row L / CH ------
+    const int  lwave = HALVES ? wave % (W / 2) : wave;
+    const bool ofv   = HALVES && wave >= W / 2;                   // a wave that loads V alone
     int      row[NLD];
     uint32_t kch[NLD], vch[NLD];
 #pragma unroll
     for (int j = 0; j < NLD; j++) {
-        const int L = (wave * NLD + j) * 64 + lane, c = L % CH;
+        const int L = (lwave * NLD + j) * 64 + lane, c = L % CH;
         row[j] = L / CH;
         kch[j] = (uint32_t)((c ^ pipe_swz_k<D>(row[j] & 31)) * 16);
         vch[j] = (uint32_t)((c ^ pipe_swz_v<D>(row[j] & 31)) * 16);
     }
-    const uint32_t lds0 = wave * (NLD * 1024);
+    if (ofv)
+#pragma unroll
+        for (int j = 0; j < NLD; j++) kch[j] = vch[j];
+    const uint32_t lds0 = lwave * (NLD * 1024);
     // Requests go step by step; behind the last step they go on with its rows, and rows past its end repeat the last one
     // (their scores are excluded, or nobody looks), so that the waits can count.
     struct Stream {
         uint64_t at;          // first row of the next step to be requested
         int      left;        // its last row, counted from there
     };
-    Stream kst = {kbase, n_keys - 1}, vst = {vbase, n_keys - 1};
-    const uint32_t nb1k = (uint32_t)a.nbk1, nb1v = (uint32_t)a.nbv1;          // (below 2^24)
+    Stream kst = {ofv ? vbase : kbase, n_keys - 1}, vst = {vbase, n_keys - 1};
+    const uint32_t nb1v = (uint32_t)a.nbv1, nb1k = ofv ? nb1v : (uint32_t)a.nbk1;          // (below 2^24)
     auto request = [&](Stream & st, uint32_t nb1, const uint32_t (&ch)[NLD], uint32_t slot) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < NLD; j++) load_to_lds16<false>(st.at, __umul24((uint32_t)min(row[j], st.left), nb1) + ch[j], lds0 + slot + j * 1024);
         const bool more = st.left >= SKEYS;
         st.at   += more ? (uint64_t)SKEYS * nb1 : 0;
         st.left -= more ? SKEYS : 0;
+    };
+
+    // the requests of a step's start: K's DK steps ahead, V's DV
+    auto request_step = [&](uint32_t slot) __attribute__((always_inline)) {
+        if constexpr (HALVES) {
+            request(kst, nb1k, kch, ofv ? VRING + ((slot + DV * STEPB) & RMASK) : (slot + DK * STEPB) & RMASK);
+        } else {
+            request(kst, nb1k, kch, (slot + DK * STEPB) & RMASK);
+            request(vst, nb1v, vch, VRING + ((slot + DV * STEPB) & RMASK));
+        }
     };
 
     // Operand reads inside this wave's block of a slot: the address of reduction step 0 (of d block 0); step ks (block db) is
@@ -174,8 +200,12 @@ __global__ void __launch_bounds__(PIPE_THREADS, 2) fattn_pipe_kernel(const Fattn
     }
 #pragma unroll
     for (int j = 0; j < DK; j++) {
-        request(kst, nb1k, kch, j * STEPB);
-        if (j >= DK - DV) request(vst, nb1v, vch, VRING + (j - (DK - DV)) * STEPB);
+        if constexpr (HALVES) {
+            if (!ofv || j >= DK - DV) request(kst, nb1k, kch, ofv ? VRING + (j - (DK - DV)) * STEPB : j * STEPB);
+        } else {
+            request(kst, nb1k, kch, j * STEPB);
+            if (j >= DK - DV) request(vst, nb1v, vch, VRING + (j - (DK - DV)) * STEPB);
+        }
     }
 
     half8 qreg[NQB][KS];                       // f16 B operands in log2 units
@@ -242,7 +272,7 @@ __global__ void __launch_bounds__(PIPE_THREADS, 2) fattn_pipe_kernel(const Fattn
         for (int i = 0; i < STEPB / 16 / PIPE_THREADS; i++) *(float4 *)(lds + VRING + (R - 1) * STEPB + (i * PIPE_THREADS + tid) * 16) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
     // the first two blocks of K have landed
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((DK - 2 + DV) * NLD) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(HALVES ? (DK - 2) * NLD : (DK - 2 + DV) * NLD) : "memory");
     __builtin_amdgcn_s_barrier();
     auto exclude_past_end = [&](float16v & x, int step) __attribute__((always_inline)) {
         int lim = n_keys - step * SKEYS - kgroup * 32 - hh * 4;
@@ -292,8 +322,7 @@ __global__ void __launch_bounds__(PIPE_THREADS, 2) fattn_pipe_kernel(const Fattn
             // what was requested OPEN loads ago and earlier has landed, in every wave's share
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(OPEN) : "memory");
             __builtin_amdgcn_s_barrier();
-            request(kst, nb1k, kch, (cur + DK * STEPB) & RMASK);
-            request(vst, nb1v, vch, VRING + ((cur + DV * STEPB) & RMASK));
+            request_step(cur);
         }
         if (__builtin_expect((step + 1) * SKEYS > n_keys, 0)) exclude_past_end(s[U], step);
         // (one query block) operands of this region's second half
@@ -407,9 +436,9 @@ __global__ void __launch_bounds__(PIPE_THREADS, 2) fattn_pipe_kernel(const Fattn
 
     __syncthreads();                                   // every wave is done with the ring
     // ---- the pairs' second waves hand their state to the first ones through LDS -------------------------------------------
-    if (KSP == 2) {
+    if constexpr (KSP > 1) {
         constexpr int XREGS = DB * 16 + 2;                 // accumulators, reference, sum: one dword per lane each
-        static_assert(2 * XREGS * 256 <= pipe_lds_bytes(D, NQB, KSP), "hand-over");
+        static_assert(KSP == 2 && QG * XREGS * 256 <= pipe_lds_bytes(D, NQB, KSP, W), "hand-over");
         float * xs = (float *)lds + qgroup * (XREGS * 64) + lane;
         if (kgroup == 1) {
 #pragma unroll
@@ -507,16 +536,16 @@ __global__ void __launch_bounds__(PIPE_THREADS, 2) fattn_pipe_kernel(const Fattn
     }
 }
 
-template <int D, int NQB, int KSP, bool PAD>
+template <int D, int NQB, int KSP, int W, bool PAD>
 int launch(const FattnArgs & a, hipStream_t stream) {
-    constexpr int bmg = 32 * NQB * PIPE_WAVES / KSP, lds = pipe_lds_bytes(D, NQB, KSP);
+    constexpr int bmg = 32 * NQB * W / KSP, lds = pipe_lds_bytes(D, NQB, KSP, W);
     const int     n_qtiles = (a.Nq + bmg - 1) / bmg;
     const int64_t wgs = (int64_t)n_qtiles * a.Hq * a.B * a.n_splits;
     if (wgs > 0x7fffffff) return (int)hipErrorInvalidValue;
     static std::atomic<uint64_t> lds_allowed{0};
-    const hipError_t e = fattn_allow_lds((const void *)fattn_pipe_kernel<D, NQB, KSP, PAD>, lds, lds_allowed);
+    const hipError_t e = fattn_allow_lds((const void *)fattn_pipe_kernel<D, NQB, KSP, W, PAD>, lds, lds_allowed);
     if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL((fattn_pipe_kernel<D, NQB, KSP, PAD>), dim3((unsigned)wgs), dim3(PIPE_THREADS), (size_t)lds, stream, a, n_qtiles);
+    hipLaunchKernelGGL((fattn_pipe_kernel<D, NQB, KSP, W, PAD>), dim3((unsigned)wgs), dim3(W * 64), (size_t)lds, stream, a, n_qtiles);
     return (int)hipGetLastError();
 }
 
@@ -524,11 +553,20 @@ int launch(const FattnArgs & a, hipStream_t stream) {
 
 int fattn_pipe_launch(const FattnArgs & a, int query_blocks, int key_split, hipStream_t stream) {
     const bool pad = a.Dv != a.D;
+    // Eight waves a workgroup where that leaves no CU with more of them than workgroups of four do: more of those than CUs, and their
+    // number per CU even once rounded up.  (A caller who names the form gets four.)
+    auto groups = [&](int q) { return (int64_t)((a.Nq + q - 1) / q) * a.Hq * a.B * a.n_splits; };
+    auto fill   = [&](int64_t wgs) { return (wgs + a.n_cus - 1) / a.n_cus; };
+    auto eight  = [&](int q4) { return a.tile_variant == 0 && groups(q4) > a.n_cus && 2 * fill(groups(2 * q4)) <= fill(groups(q4)); };
+    if (query_blocks == 2) {
+        if (pad || a.D != 64) return (int)hipErrorInvalidValue;
+        return eight(256) ? launch<64, 2, 1, 8, false>(a, stream) : launch<64, 2, 1, 4, false>(a, stream);
+    }
     if (a.D == 64) {
-        if (query_blocks == 2) return pad ? (int)hipErrorInvalidValue : launch<64, 2, 1, false>(a, stream);
-        if (key_split == 2) return pad ? launch<64, 1, 2, true>(a, stream) : launch<64, 1, 2, false>(a, stream);
-        return pad ? launch<64, 1, 1, true>(a, stream) : launch<64, 1, 1, false>(a, stream);
+        if (key_split == 2) return pad ? launch<64, 1, 2, 4, true>(a, stream) : launch<64, 1, 2, 4, false>(a, stream);
+        return pad ? launch<64, 1, 1, 4, true>(a, stream) : launch<64, 1, 1, 4, false>(a, stream);
     }
     if (key_split == 2) return (int)hipErrorInvalidValue;         // (not a form of this kernel: see fattn_mma_launch)
-    return pad ? launch<128, 1, 1, true>(a, stream) : launch<128, 1, 1, false>(a, stream);
+    if (eight(128)) return pad ? launch<128, 1, 1, 8, true>(a, stream) : launch<128, 1, 1, 8, false>(a, stream);
+    return pad ? launch<128, 1, 1, 4, true>(a, stream) : launch<128, 1, 1, 4, false>(a, stream);
 }
