@@ -174,6 +174,14 @@ static __device__ __forceinline__ void load_to_lds16(uint64_t base, uint32_t off
     }
 }
 
+// the same with 4 bytes a lane
+static __device__ __forceinline__ void load_to_lds4(uint64_t base, uint32_t off, uint32_t to) {
+    const uint64_t p = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(base >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)base);
+    const uint32_t t = (uint32_t)__builtin_amdgcn_readfirstlane((int)to);
+    uint64_t q;
+    asm volatile("s_mov_b64 %0, %2\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %0" : "=&s"(q) : "v"(off), "s"(p), "s"(t) : "memory", "m0");
+}
+
 // lane l's and lane (l ^ 32)'s values, the lower lane's first, without the LDS crossbar (whose traffic would blur the waits of
 // a loop, and whose addresses cost registers)
 static __device__ __forceinline__ float2 both_halves(float x) {
@@ -435,6 +443,7 @@ int fattn_vec_launch(const FattnArgs & a, int ktype, hipStream_t stream);
 int fattn_merge_launch(const FattnArgs & a, hipStream_t stream);
 int fattn_mma_launch(const FattnArgs & a, int ktype, hipStream_t stream);
 int fattn_pipe_launch(const FattnArgs & a, int query_blocks, int key_split, hipStream_t stream);
+bool fattn_pipe_masked(const FattnArgs & a, int query_blocks, int key_split);
 // the instantiation of the tile kernel a call takes
 struct FattnMmaVariant {
     int  query_blocks;            // 32-query blocks per wave (1 or 2)

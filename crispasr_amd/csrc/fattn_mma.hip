@@ -1094,6 +1094,8 @@ int fattn_mma_launch(const FattnArgs & a, int ktype, hipStream_t stream) {
     // x 20 and 800 x 8 within 2%).
     if (ktype == MI355X_TYPE_F16 && v.direct && !a.masked && a.softcap == 0.0f && !(a.D == 128 && v.key_split == 2))
         return fattn_pipe_launch(a, v.query_blocks, v.key_split, stream);
+    if (ktype == MI355X_TYPE_F16 && v.direct && a.masked && fattn_pipe_masked(a, v.query_blocks, v.key_split))
+        return fattn_pipe_launch(a, v.query_blocks, v.key_split, stream);
     switch (ktype) {
         case MI355X_TYPE_F16:  return launch_type<MI355X_TYPE_F16>(a, v, stream);
         case MI355X_TYPE_F32:  return launch_type<MI355X_TYPE_F32>(a, v, stream);

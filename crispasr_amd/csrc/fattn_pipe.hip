@@ -26,6 +26,12 @@
 // 1500^2 x 4 55.8 -> 53.4, 8 x 128 x 750^2 x 8 33.6 -> 32.0; where they leave more CUs empty they lose (10 x 128 x 1500^2 x 2
 // 37.2 -> 44.6).  Eight waves that share the queries of two or four (the keys in turn), for a grid that leaves CUs to one
 // workgroup of four, changed nothing at 1500 keys (8 x 64 16.0 us either way) and lost 1 us below 1000.
+// Masked calls of 128-wide heads: a wave brings the mask of its next two blocks to LDS as it does K and V, so that the waits
+// go on counting, and adds it ahead of the exponentials; the last block is the last 32 keys of the range, whole.  Against the tile
+// kernel, whole calls: 2048 causal tokens behind 2048, 32 query and 8 KV heads, 162 -> 147 us (132 of them this kernel), 1000 causal
+// tokens 42.5 -> 37.5, 407 (rows that start between dwords, the pairs' form) 21.4 -> 20.1; under per-head masks 750 x 8 heads x 8
+// 45.7 -> 38.8, 1000 x 8 x 4 38.1 -> 32.7, 751 x 8 22.0 -> 19.2.  The 407-token launch (16 us) is 4.5 us until the first scores, 0.65
+// a step - 32 KB through a CU's port - and 3 for the hand-over and the stores.
 // What is left above the MFMAs of a wave alone on its SIMD is instruction issue (about 5 cycles an instruction).  Where two
 // share a SIMD nothing is full: by the counters of the first of these launches the matrix cores are busy for 49% of it (at
 // 1.85 GHz) and the vector ALU for 38%, and a wave stands ready for another instruction to end for 39% of its cycles and
@@ -58,8 +64,10 @@ typedef __attribute__((address_space(3))) short4v     lds_short4;
 // instructions stay on their side of it
 #define PIPE_FENCE() __builtin_amdgcn_sched_barrier(0)
 
-constexpr int pipe_lds_bytes(int D, int NQB, int KSP, int W) {
-    const int ring  = 2 * RING * KSP * 32 * D * 2;
+// A wave's mask block: 32 queries x 32 keys of f16, and for rows that start between dwords the one behind each row's last
+constexpr int pipe_mask_slot(int MASK) { return MASK == 2 ? 32 * 64 + 256 : MASK ? 32 * 64 : 0; }
+constexpr int pipe_lds_bytes(int D, int NQB, int KSP, int W, int MASK) {
+    const int ring  = 2 * RING * KSP * 32 * D * 2 + W * 2 * pipe_mask_slot(MASK);
     const int stage = W * 32 * D * 4;                                           // result rows / the waves' partial results
     return ring > stage ? ring : stage;
 }
@@ -67,9 +75,11 @@ constexpr int pipe_lds_bytes(int D, int NQB, int KSP, int W) {
 // NQB: 32-query blocks per wave.  KSP = 2: the second half of the W waves shares the queries of the first and takes alternate
 // 32-key blocks.
 // PAD: heads of a.Dv elements (a multiple of 8 below D) on copies of K and V whose rows are zero-padded to D.
-template <int D, int NQB, int KSP, int W, bool PAD>
+// MASK: 1 where rows start on dwords and Nkv is even, 2 where not; 128-wide heads, no slopes.
+template <int D, int NQB, int KSP, int W, bool PAD, int MASK>
 __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a, const int n_qtiles) {
     static_assert(NQB == 1 || (NQB == 2 && D == 64 && KSP == 1 && !PAD), "forms");
+    static_assert(!MASK || (D == 128 && NQB == 1 && W == 4 && !PAD), "masked forms");
     constexpr int PIPE_THREADS = W * 64;
     constexpr int QG   = W / KSP;                                 // waves that take different queries
     constexpr int KS   = D / 16;                                  // reduction steps of Q.K^T
@@ -87,7 +97,8 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     constexpr int R    = RING;
     // steps ahead of the current one that its start requests, and loads that may still be under way then
     constexpr int DK   = R, DV = NQB == 2 ? R - 1 : R - 2;
-    constexpr int OPEN = (NQB == 2 ? R - 2 : R - 3) * NLS;
+    constexpr int NML  = MASK == 2 ? 3 : MASK ? 2 : 0;            // ... of its own mask block
+    constexpr int OPEN = (NQB == 2 ? R - 2 : R - 3) * (NLS + NML);
     constexpr int BMW  = 32 * NQB;
     constexpr int BMG  = BMW * QG;
     constexpr int NM   = KS + 2 * DB;                             // MFMAs of a region
@@ -110,18 +121,27 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     // Workgroups go to the 8 XCDs round-robin; renumbered so that the query tiles of one (head, batch), which share K/V, sit
     // on one XCD and meet in its L2.
     int bid = blockIdx.x;
-    {
-        const int nb = gridDim.x;
-        const int per = nb / 8;
-        if (bid < per * 8) bid = (bid % 8) * per + bid / 8;
-    }
+    const int nb = gridDim.x, per = nb / 8;
+    if (bid < per * 8) bid = (bid % 8) * per + bid / 8;
     const int split = bid % a.n_splits;
     bid /= a.n_splits;
     const int k_begin = split * a.keys_per_split;
     const int k_end   = min(a.Nkv, k_begin + a.keys_per_split);
-    const int qt = bid % n_qtiles;
-    const int h  = (bid / n_qtiles) % a.Hq;
-    const int b  = bid / (n_qtiles * a.Hq);
+    int qt = bid % n_qtiles, pair = bid / n_qtiles;
+    if (MASK && a.n_splits == 1 && per * 8 == nb && per % n_qtiles == 0) {
+        // Masked workgroups differ in length (causal rows, padded sequences): an XCD's are ordered from the last query tile to the
+        // first, and every second group of n_cus / 8 - the ones that join the group before on its CUs - backwards, so that a CU's
+        // two add up to about the same.
+        const int cus = a.n_cus >= 8 ? a.n_cus / 8 : 32, heads = per / n_qtiles;
+        int i = blockIdx.x / 8;
+        const int seg = i / cus * cus;
+        if ((i / cus) & 1) i = seg + min(cus, per - seg) - 1 - (i - seg);
+        qt   = n_qtiles - 1 - i / heads;
+        pair = (int)(blockIdx.x % 8) * heads + i % heads;
+    }
+    // (masked: the batch runs faster than the head, or the longest sequence of a padded batch would be one XCD's alone)
+    const int h  = MASK ? pair / a.B : pair % a.Hq;
+    const int b  = MASK ? pair % a.B : pair / a.Hq;
     const int hk = h / a.gqa;
     const int bk = b / a.bq;
     const int q0 = qt * BMG + qgroup * BMW;
@@ -142,7 +162,7 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     }
 
     const int n_keys  = k_end - k_begin;
-    const int n_steps = (n_keys + SKEYS - 1) / SKEYS;
+    int       n_steps = (n_keys + SKEYS - 1) / SKEYS;
     const uint64_t kbase = (uint64_t)(a.k + (int64_t)hk * a.nbk2 + (int64_t)bk * a.nbk3 + (int64_t)k_begin * a.nbk1);
     const uint64_t vbase = (uint64_t)(a.v + (int64_t)hk * a.nbv2 + (int64_t)bk * a.nbv3 + (int64_t)k_begin * a.nbv1);
 
@@ -163,16 +183,28 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
         for (int j = 0; j < NLD; j++) kch[j] = vch[j];
     const uint32_t lds0 = lwave * (NLD * 1024);
     // Requests go step by step; behind the last step they go on with its rows, and rows past its end repeat the last one
-    // (their scores are excluded, or nobody looks), so that the waits can count.
+    // (their scores are excluded, or nobody looks), so that the waits can count.  Masked: a wave's loads of a step are rows of the
+    // block that its own products take, and the last block is the last 32 keys of the range (and keys before it, where a range
+    // has fewer), so that the mask's rows are read inside their ends; what the block before has had is excluded.
     struct Stream {
         uint64_t at;          // first row of the next step to be requested
         int      left;        // its last row, counted from there
     };
-    Stream kst = {ofv ? vbase : kbase, n_keys - 1}, vst = {vbase, n_keys - 1};
     const uint32_t nb1v = (uint32_t)a.nbv1, nb1k = ofv ? nb1v : (uint32_t)a.nbk1;          // (below 2^24)
+    const int      key0 = MASK ? min(32 * kgroup, n_keys - 32) : 0;             // the first block's first key
+    Stream kst = {ofv ? vbase : kbase + (int64_t)key0 * a.nbk1, MASK ? n_keys - 32 - key0 : n_keys - 1};
+    Stream vst = {vbase + (int64_t)key0 * a.nbv1, MASK ? n_keys - 32 - key0 : n_keys - 1};
     auto request = [&](Stream & st, uint32_t nb1, const uint32_t (&ch)[NLD], uint32_t slot) __attribute__((always_inline)) {
+        if constexpr (MASK) {
 #pragma unroll
-        for (int j = 0; j < NLD; j++) load_to_lds16<false>(st.at, __umul24((uint32_t)min(row[j], st.left), nb1) + ch[j], lds0 + slot + j * 1024);
+            for (int j = 0; j < NLD; j++) load_to_lds16<(MASK != 0)>(st.at, __umul24((uint32_t)(row[j] & 31), nb1) + ch[j], lds0 + slot + j * 1024);
+            const int by = min(st.left, SKEYS);
+            st.at   += (uint64_t)(uint32_t)by * nb1;
+            st.left -= by;
+            return;
+        }
+#pragma unroll
+        for (int j = 0; j < NLD; j++) load_to_lds16<(MASK != 0)>(st.at, __umul24((uint32_t)min(row[j], st.left), nb1) + ch[j], lds0 + slot + j * 1024);
         const bool more = st.left >= SKEYS;
         st.at   += more ? (uint64_t)SKEYS * nb1 : 0;
         st.left -= more ? SKEYS : 0;
@@ -198,6 +230,81 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
         const int c = ((lane >> 4) & 1) * 2 + ((i16 & 3) >> 1);
         vaddr = (uint32_t)((kr0 * CH + (c ^ pipe_swz_v<D>(kr0))) * 16 + 8 * (i16 & 1) + VRING + kgroup * BLKB);
     }
+    // ---- the mask: 32 rows of 64 bytes a block, their 16-byte chunks XOR-swizzled by row, two blocks per wave -----------------
+    constexpr uint32_t MSLOT = pipe_mask_slot(MASK);
+    const uint32_t m_lds = 2 * R * STEPB + wave * (2 * MSLOT);
+    const char * const plane = MASK ? a.mask + (int64_t)(h % a.Hm) * a.nbm2 + (int64_t)(b % a.Bm) * a.nbm3 : nullptr;
+    auto row_at = [&](int r) __attribute__((always_inline)) { return (uint32_t)min(q0 + r, a.Nq - 1) * (uint32_t)a.nbm1; };      // (below 2^31)
+    uint32_t moff[MASK ? 2 : 1];
+    const uint32_t mrow = MASK == 2 ? row_at(l32) : 0;
+#pragma unroll
+    for (int j = 0; j < (MASK ? 2 : 0); j++) moff[j] = row_at(j * 16 + (lane >> 2)) + (uint32_t)(((lane & 3) ^ ((lane >> 4) & 3)) * 16);
+    Stream mst = {MASK ? (uint64_t)plane + (uint64_t)((int64_t)(k_begin + key0) * 2) : 0, MASK ? n_keys - 32 - key0 : 0};
+    auto request_mask = [&](int slot) __attribute__((always_inline)) {
+        if constexpr (MASK != 0) {
+            // (rows that start between dwords: from the dword that holds their first key on, and the one that holds their last)
+            const uint32_t odd = MASK == 2 ? (uint32_t)mst.at & 2 : 0;
+#pragma unroll
+            for (int j = 0; j < 2; j++) load_to_lds16<(MASK != 0)>(mst.at - odd, MASK == 2 ? (moff[j] + odd) & ~3u : moff[j], m_lds + slot * MSLOT + j * 1024);
+            if (MASK == 2) load_to_lds4(mst.at - odd, (mrow + odd + 62) & ~3u, m_lds + slot * MSLOT + 2048);
+            const int by = min(mst.left, SKEYS);
+            mst.at   += (uint64_t)(2 * by);
+            mst.left -= by;
+        }
+    };
+    // adds the block in `slot` to scores x of block `block` in log2 units, or (the last block) excludes keys of the one before
+    auto add_mask = [&](float16v & x, int slot, int block) __attribute__((always_inline)) {
+        const uint32_t at = m_lds + slot * MSLOT + (uint32_t)(l32 * 64 + ((l32 >> 2) & 3) * 16);
+        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+        typedef __attribute__((address_space(3))) const u32x2 lds_u2;
+        typedef __attribute__((address_space(3))) const uint32_t lds_u1;
+        u32x2 w[4];
+#pragma unroll
+        for (int g = 0; g < 4; g++) w[g] = *(lds_u2 *)(uintptr_t)((at ^ (uint32_t)(g * 16)) + 8 * hh);
+        if constexpr (MASK == 2) {
+            uint32_t next[4];                                     // the dword behind each
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+                next[g] = *(lds_u1 *)(uintptr_t)(hh ? (g < 3 ? at ^ (uint32_t)((g + 1) * 16) : m_lds + slot * MSLOT + 2048 + l32 * 4)
+                                                    : (at ^ (uint32_t)(g * 16)) + 8);
+            // (where the block starts: its row's first key in the low or the high half of a dword)
+            const uint32_t start = (uint32_t)(uint64_t)plane + (uint32_t)(k_begin + min(32 * block, n_keys - 32)) * 2;
+            const uint32_t sh    = ((mrow + start) & 2) * 8;
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                w[g][0] = __builtin_amdgcn_alignbit(w[g][1], w[g][0], sh);
+                w[g][1] = __builtin_amdgcn_alignbit(next[g], w[g][1], sh);
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                x[4 * g + c] = fmaf((float)__builtin_bit_cast(_Float16, (uint16_t)(w[g][c >> 1] >> (16 * (c & 1)))), LOG2E, x[4 * g + c]);
+        if (__builtin_expect(32 * block + 32 > n_keys, 0)) {
+            int had = 32 * block + 32 - n_keys - hh * 4;
+            asm volatile("" : "+v"(had));
+#pragma unroll
+            for (int r = 0; r < 16; r++) x[r] = (r >> 2) * 8 + (r & 3) < had ? -INFINITY : x[r];
+        }
+    };
+    // A wave looks at the last 64 keys of its last 8 queries with the first requests; if none of them is seen, at the rows of all its
+    // queries, 256 keys at a time from the end on, until it meets a visible key: what lies behind is not walked.  Requests stay
+    // inside the rows by moving the last ones back: at worst a block is kept because the one before it is seen.
+    typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+    const int n_tiles = (n_keys + 63) / 64;
+    auto mask_keys = [&](int r, int key) __attribute__((always_inline)) {
+        return *(const u32x4_a2 *)(plane + (int64_t)min(q0 + r, a.Nq - 1) * a.nbm1 + (int64_t)min(k_begin + key, k_end - 8) * 2);
+    };
+    auto any_seen = [&](const u32x4_a2 & w) __attribute__((always_inline)) {                   // (0xFC00: a masked-out key)
+        return (w[0] ^ 0xFC00FC00u) | (w[1] ^ 0xFC00FC00u) | (w[2] ^ 0xFC00FC00u) | (w[3] ^ 0xFC00FC00u);
+    };
+    u32x4_a2 end_keys = {0u, 0u, 0u, 0u};
+    if constexpr (MASK != 0) {
+        end_keys = mask_keys(24 + (lane >> 3), (n_tiles - 1) * 64 + (lane & 7) * 8);
+        request_mask(0);
+        request_mask(1);
+    }
 #pragma unroll
     for (int j = 0; j < DK; j++) {
         if constexpr (HALVES) {
@@ -218,6 +325,31 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
 #pragma unroll
             for (int e = 0; e < 8; e++) qreg[qb][ks][e] = (_Float16)(qraw[qb][ks][e >> 2][e & 3] * qs);
         }
+
+    // (in the slot of V's that the first region asks for; read behind the barrier below)
+    int * const ends = (int *)(lds + VRING + (R - 2) * STEPB);
+    if constexpr (MASK != 0) {
+        int nt = n_tiles;
+        if (__builtin_amdgcn_ballot_w64(any_seen(end_keys) != 0) == 0) {
+            nt = 1;
+            for (int hi = n_tiles; hi > 0; hi -= 4) {
+                const int lo = max(hi - 4, 0);
+                u32x4_a2  w[16 / KSP];                            // (the two waves of a pair share the rows)
+                uint32_t  any = 0;
+#pragma unroll
+                for (int i = 0; i < 16 / KSP; i++) w[i] = mask_keys(kgroup * 16 + i * 2 + (lane >> 5), lo * 64 + (lane & 31) * 8);
+#pragma unroll
+                for (int i = 0; i < 16 / KSP; i++) any |= any_seen(w[i]);
+                const uint64_t v2 = __builtin_amdgcn_ballot_w64(any != 0);
+                const uint32_t v  = (uint32_t)v2 | (uint32_t)(v2 >> 32);
+                if (v) {
+                    nt = min(hi, lo + (31 - __builtin_clz(v)) / 8 + 1);
+                    break;
+                }
+            }
+        }
+        if (lane == 0) ends[wave] = nt;
+    }
 
     float16v oacc[NQB][DB], negm[SPLAT ? NQB : 1], s[2];
     half8    p[2][2];
@@ -274,6 +406,7 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     // the first two blocks of K have landed
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(HALVES ? (DK - 2) * NLD : (DK - 2 + DV) * NLD) : "memory");
     __builtin_amdgcn_s_barrier();
+    if constexpr (MASK != 0) n_steps = min(n_steps, max(max(ends[0], ends[1]), max(ends[2], ends[3])) * 64 / SKEYS);
     auto exclude_past_end = [&](float16v & x, int step) __attribute__((always_inline)) {
         int lim = n_keys - step * SKEYS - kgroup * 32 - hh * 4;
         asm volatile("" : "+v"(lim));            // (nothing of this is worth a register in the loop)
@@ -291,12 +424,15 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
             for (int r = 0; r < 16; r++) s[0][r] = 0.0f;
 #pragma unroll
             for (int ks = 0; ks < KS; ks++) s[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ks < 4 ? ka[ks & 3] : k1[ks & 3], qreg[qb][ks], s[0], 0, 0, 0);
-            if (n_keys < SKEYS) exclude_past_end(s[0], 0);
-            float mx = s[0][0];
+            float16v first = s[0];
+            if constexpr (MASK != 0)  add_mask(first, 0, kgroup);       // (its own turn comes with the first region)
+            else if (n_keys < SKEYS) { exclude_past_end(s[0], 0); first = s[0]; }
+            float mx = first[0];
 #pragma unroll
-            for (int r = 1; r < 16; r++) mx = fmaxf(mx, s[0][r]);
+            for (int r = 1; r < 16; r++) mx = fmaxf(mx, first[r]);
             mx = max_of_halves(mx);
-            m[qb] = mx > -INFINITY ? mx : 0.0f;
+            // (masked rows that see nothing yet stand on -inf: their exponentials are NaN, and the rare path below takes over)
+            m[qb] = MASK || mx > -INFINITY ? mx : 0.0f;
             if (SPLAT) {
 #pragma unroll
                 for (int r = 0; r < 16; r++) negm[SPLAT ? qb : 0][r] = -m[qb];
@@ -324,7 +460,11 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
             __builtin_amdgcn_s_barrier();
             request_step(cur);
         }
-        if (__builtin_expect((step + 1) * SKEYS > n_keys, 0)) exclude_past_end(s[U], step);
+        if constexpr (MASK != 0) {
+            add_mask(s[U], U, KSP * step + kgroup);
+            PIPE_FENCE();
+            request_mask(U);
+        } else if (__builtin_expect((step + 1) * SKEYS > n_keys, 0)) exclude_past_end(s[U], step);
         // (one query block) operands of this region's second half
         if (TURNS)          read_k(va, (cur + STEPB) & RMASK, KS - 4);
         else if (NQB == 1)  read_v(va, (cur - STEPB) & RMASK, 0);
@@ -380,10 +520,18 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
             float mx = s[U][0];
 #pragma unroll
             for (int r = 1; r < 16; r++) mx = fmaxf(mx, s[U][r]);
-            const float delta = fmaxf(max_of_halves(mx) - (SPLAT ? 0.0f : m[QB]), 0.0f);
-            const float f = __builtin_amdgcn_exp2f(-delta);
-            const float base = SPLAT ? delta : m[QB] + delta;      // what the scores at hand still have to come down by
-            m[QB] += delta;
+            float delta = 0.0f, f, base;                           // base: what the scores at hand still have to come down by
+            if constexpr (MASK != 0) {
+                base  = fmaxf(max_of_halves(mx), m[QB]);
+                f     = base == m[QB] ? 1.0f : __builtin_amdgcn_exp2f(m[QB] - base);
+                m[QB] = base;
+                if (base == -INFINITY) base = 0.0f;                // (no key seen: exponentials of -inf)
+            } else {
+                delta = fmaxf(max_of_halves(mx) - (SPLAT ? 0.0f : m[QB]), 0.0f);
+                f     = __builtin_amdgcn_exp2f(-delta);
+                base  = SPLAT ? delta : m[QB] + delta;
+                m[QB] += delta;
+            }
 #pragma unroll
             for (int r = 0; r < 4; r++) lacc[QB][r] = lprev * f;
 #pragma unroll
@@ -435,32 +583,51 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // (what was requested behind the last step)
 
     __syncthreads();                                   // every wave is done with the ring
-    // ---- the pairs' second waves hand their state to the first ones through LDS -------------------------------------------
-    if constexpr (KSP > 1) {
-        constexpr int XREGS = DB * 16 + 2;                 // accumulators, reference, sum: one dword per lane each
-        static_assert(KSP == 2 && QG * XREGS * 256 <= pipe_lds_bytes(D, NQB, KSP, W), "hand-over");
-        float * xs = (float *)lds + qgroup * (XREGS * 64) + lane;
-        if (kgroup == 1) {
-#pragma unroll
-            for (int db = 0; db < DB; db++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) xs[(db * 16 + r) * 64] = oacc[0][db][r];
-            xs[(DB * 16) * 64]     = m[0];
-            xs[(DB * 16 + 1) * 64] = lacc[0][0];
-        }
-        __syncthreads();
-        if (kgroup == 1) return;
-        // (a wave without a key of its own has a sum of zero and stands on reference 0)
-        const float mo = xs[(DB * 16) * 64], lo = xs[(DB * 16 + 1) * 64];
-        const float mn = lo == 0.0f ? m[0] : lacc[0][0] == 0.0f ? mo : fmaxf(m[0], mo);
-        const float fa = lacc[0][0] == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(m[0] - mn);
-        const float fo = lo == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(mo - mn);
-        lacc[0][0] = lacc[0][0] * fa + lo * fo;
+    // Excluded keys were multiplied by probabilities of zero, not skipped: the same for finite K/V, NaN otherwise.  Queries whose
+    // result is not finite are left out below and computed at the end, excluded keys unread, as the CPU op does it.
+    uint32_t bad = 0;                                      // (lanes l and l + 32 hold the same query)
+    if constexpr (MASK != 0) {
+        float chk = lacc[0][0] * 0.0f;
 #pragma unroll
         for (int db = 0; db < DB; db++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) oacc[0][db][r] = oacc[0][db][r] * fa + xs[(db * 16 + r) * 64] * fo;
-        m[0] = mn;
+            for (int r = 0; r < 16; r++) chk = fmaf(oacc[0][db][r], 0.0f, chk);
+        const uint64_t bits = __builtin_amdgcn_ballot_w64(chk != 0.0f);
+        bad = (uint32_t)bits | (uint32_t)(bits >> 32);
+    }
+
+    // ---- the two waves of a pair hand each other half of the result's columns through LDS ----------------------------------
+    if constexpr (KSP == 2) {
+        constexpr int HB    = DB / 2;
+        constexpr int XREGS = HB * 16 + 3;                 // accumulators, reference, sum, bad rows: one dword per lane each
+        static_assert(W * XREGS * 256 <= pipe_lds_bytes(D, NQB, KSP, W, MASK), "hand-over");
+        auto trade = [&](auto first) __attribute__((always_inline)) {
+            constexpr int MINE = decltype(first)::value * HB, THEIRS = HB - MINE;
+            float * const out = (float *)lds + wave * (XREGS * 64) + lane;
+            const float * const in = (const float *)lds + (wave ^ QG) * (XREGS * 64) + lane;
+#pragma unroll
+            for (int db = 0; db < HB; db++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) out[(db * 16 + r) * 64] = oacc[0][THEIRS + db][r];
+            out[(HB * 16) * 64]     = m[0];
+            out[(HB * 16 + 1) * 64] = lacc[0][0];
+            out[(HB * 16 + 2) * 64] = __uint_as_float(bad);
+            __syncthreads();
+            // (a wave without a key of its own has a sum of zero)
+            const float mo = in[(HB * 16) * 64], lo = in[(HB * 16 + 1) * 64];
+            const float mn = lo == 0.0f ? m[0] : lacc[0][0] == 0.0f ? mo : fmaxf(m[0], mo);
+            const float fa = lacc[0][0] == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(m[0] - mn);
+            const float fo = lo == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(mo - mn);
+            lacc[0][0] = lacc[0][0] * fa + lo * fo;
+#pragma unroll
+            for (int db = 0; db < HB; db++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) oacc[0][db][r] = oacc[0][MINE + db][r] * fa + in[(db * 16 + r) * 64] * fo;
+            m[0] = mn;
+            bad |= (uint32_t)__builtin_amdgcn_readfirstlane(__float_as_int(in[(HB * 16 + 2) * 64]));
+        };
+        if (kgroup == 0) trade(I0{});
+        else             trade(I1{});
     }
 
     // ---- normalise and write dst[D, Hq, Nq, B], or hand the unnormalised partial to the merge kernel -----------------------
@@ -497,11 +664,11 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
                 const int row = k * RPI + lane / CPR, c = lane % CPR;
                 const float4 o = *(const float4 *)(stg + row * D + ((c ^ (row & (CPR - 1))) * 4));
                 typedef float f32x4 __attribute__((ext_vector_type(4)));
-                if (q_first + row < a.Nq && (!PAD || a.n_splits > 1 || c * 4 < a.Dv))
+                if (q_first + row < a.Nq && (!PAD || a.n_splits > 1 || c * 4 < a.Dv) && (!MASK || !(bad >> row & 1)))
                     __builtin_nontemporal_store(f32x4{o.x, o.y, o.z, o.w}, (f32x4 *)(out0 + row * row_stride + c * 4));
             }
             __builtin_amdgcn_wave_barrier();               // the next query block reuses the staging rows
-            if (a.n_splits > 1 && hh == 0 && qi < a.Nq) {
+            if (a.n_splits > 1 && hh == 0 && qi < a.Nq && (!MASK || !(bad >> l32 & 1))) {
                 // (reference, sum) in natural-log units; a range with no visible key contributes nothing
                 float * pm = a.part_ml + ((((int64_t)b * a.Nq + qi) * a.Hq + h) * a.n_splits + split) * 2;
                 pm[0] = ltot == 0.0f ? -INFINITY : m[qb] * 0.6931471805599453f;
@@ -513,46 +680,71 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
         const float ltot = lacc[0][0];
         const float inv  = a.n_splits > 1 ? 1.0f : (ltot > 0.0f ? 1.0f / ltot : 0.0f);
         const int   qi   = q0 + l32;
-        if (qi < a.Nq) {
+        if (qi < a.Nq && (!MASK || !(bad >> l32 & 1))) {
             const int64_t row = ((int64_t)b * a.Nq + qi) * a.Hq + h;
             float * out = a.n_splits > 1 ? a.part_acc + (row * a.n_splits + split) * D : a.dst + row * dv;
 #pragma unroll
-            for (int db = 0; db < DB; db++)
+            for (int i = 0; i < DB / 2; i++)
 #pragma unroll
                 for (int g = 0; g < 4; g++) {
                     float4 o;
-                    o.x = oacc[0][db][g * 4 + 0] * inv;
-                    o.y = oacc[0][db][g * 4 + 1] * inv;
-                    o.z = oacc[0][db][g * 4 + 2] * inv;
-                    o.w = oacc[0][db][g * 4 + 3] * inv;
-                    if (!PAD || a.n_splits > 1 || db * 32 + g * 8 + hh * 4 < a.Dv) *(float4 *)(out + db * 32 + g * 8 + hh * 4) = o;
+                    o.x = oacc[0][i][g * 4 + 0] * inv;
+                    o.y = oacc[0][i][g * 4 + 1] * inv;
+                    o.z = oacc[0][i][g * 4 + 2] * inv;
+                    o.w = oacc[0][i][g * 4 + 3] * inv;
+                    const int d = (kgroup * (DB / 2) + i) * 32 + g * 8 + hh * 4;
+                    if (!PAD || a.n_splits > 1 || d < a.Dv) *(float4 *)(out + d) = o;
                 }
-            if (a.n_splits > 1 && hh == 0) {
+            if (a.n_splits > 1 && hh == 0 && kgroup == 0) {
                 float * pm = a.part_ml + (row * a.n_splits + split) * 2;
                 pm[0] = ltot == 0.0f ? -INFINITY : m[0] * 0.6931471805599453f;
                 pm[1] = ltot;
             }
         }
     }
+    if constexpr (MASK != 0) {
+        if (bad != 0 && kgroup == 0) {
+            for (; bad != 0; bad &= bad - 1) {
+                const int qi = q0 + __builtin_ctz(bad);
+                if (qi < a.Nq) attn_row_redo<MI355X_TYPE_F16, D>(a, qi, h, b, split, k_begin, k_end);
+            }
+        }
+    }
 }
 
-template <int D, int NQB, int KSP, int W, bool PAD>
+template <int D, int NQB, int KSP, int W, bool PAD, int MASK = 0>
 int launch(const FattnArgs & a, hipStream_t stream) {
-    constexpr int bmg = 32 * NQB * W / KSP, lds = pipe_lds_bytes(D, NQB, KSP, W);
+    constexpr int bmg = 32 * NQB * W / KSP, lds = pipe_lds_bytes(D, NQB, KSP, W, MASK);
     const int     n_qtiles = (a.Nq + bmg - 1) / bmg;
     const int64_t wgs = (int64_t)n_qtiles * a.Hq * a.B * a.n_splits;
     if (wgs > 0x7fffffff) return (int)hipErrorInvalidValue;
     static std::atomic<uint64_t> lds_allowed{0};
-    const hipError_t e = fattn_allow_lds((const void *)fattn_pipe_kernel<D, NQB, KSP, W, PAD>, lds, lds_allowed);
+    const hipError_t e = fattn_allow_lds((const void *)fattn_pipe_kernel<D, NQB, KSP, W, PAD, MASK>, lds, lds_allowed);
     if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL((fattn_pipe_kernel<D, NQB, KSP, W, PAD>), dim3((unsigned)wgs), dim3(W * 64), (size_t)lds, stream, a, n_qtiles);
+    hipLaunchKernelGGL((fattn_pipe_kernel<D, NQB, KSP, W, PAD, MASK>), dim3((unsigned)wgs), dim3(W * 64), (size_t)lds, stream, a, n_qtiles);
     return (int)hipGetLastError();
 }
 
 }  // namespace
 
+// The masked calls among those over f16 rows: whole 128-wide heads, no slopes, blocks of 32 keys that end inside the rows.
+// Rows that start between dwords need LDS that two workgroups of the unsplit form do not have on one CU.  Shorter key ranges
+// stay with the tile kernel, whose prologue is shorter (128 causal tokens x 32 heads 14.0 us there with their row writes, 15.3 here;
+// 100 x 64 heads under per-head masks 10.2, 11.5; 300 x 16 12.9, 13.6; 400 x 16 15.7, 15.4).
+bool fattn_pipe_masked(const FattnArgs & a, int query_blocks, int key_split) {
+    return a.D == 128 && a.Dv == 128 && query_blocks == 1 && a.max_bias <= 0.0f && a.softcap == 0.0f &&
+           (a.n_splits > 1 ? a.keys_per_split : a.Nkv) >= 384 && (uint64_t)a.Nq * (uint64_t)a.nbm1 < (1ull << 31) &&
+           (key_split == 2 || (a.mask_al4 && !(a.Nkv & 1)));
+}
+
 int fattn_pipe_launch(const FattnArgs & a, int query_blocks, int key_split, hipStream_t stream) {
     const bool pad = a.Dv != a.D;
+    if (a.masked) {
+        if (!fattn_pipe_masked(a, query_blocks, key_split)) return (int)hipErrorInvalidValue;
+        const bool dwords = a.mask_al4 && !(a.Nkv & 1);
+        if (key_split == 2) return dwords ? launch<128, 1, 2, 4, false, 1>(a, stream) : launch<128, 1, 2, 4, false, 2>(a, stream);
+        return launch<128, 1, 1, 4, false, 1>(a, stream);
+    }
     // Eight waves a workgroup where that leaves no CU with more of them than workgroups of four do: more of those than CUs, and their
     // number per CU even once rounded up.  (A caller who names the form gets four.)
     auto groups = [&](int q) { return (int64_t)((a.Nq + q - 1) / q) * a.Hq * a.B * a.n_splits; };

@@ -1,0 +1,81 @@
+"""The pipelined tile kernel under masks (128-wide heads, 384 keys of a range and more): last blocks of every length, rows on and between
+dwords, rows that see nothing at first or at all, bias values, ranges, references that climb, hidden rows of NaN bits."""
+import numpy as np
+import pytest
+
+import oracle as ora
+from cases import make_case, to_f32
+from crispasr_amd import ggml
+from gpu_util import assert_parity, run_gpu, run_oracle
+
+pytestmark = pytest.mark.gpu
+
+FORMS = [0x11, 0x21]
+
+
+def _masked(values, seed, **kw):
+    """values: float32 [Bm, Hm, Nq, Nkv]"""
+    case = make_case(seed=seed, D=128, Nq=values.shape[2], Nkv=values.shape[3], **kw)
+    case["mask"] = ora.from_f32(values.astype(np.float32), ora.F16)
+    return case
+
+
+def _run(case, variant, what, ranges=(1,)):
+    print("case", hex(variant), what, flush=True)
+    ref = run_oracle(case)
+    for ns in ranges:
+        assert_parity(run_gpu(case, kernel=ggml.KERNEL_MMA, tile_variant=variant, n_splits=ns), ref, "%s, %d ranges" % (what, ns))
+
+
+@pytest.mark.parametrize("variant", FORMS)
+@pytest.mark.parametrize("Nq,Nkv", [(1, 384), (33, 385), (64, 386), (65, 399), (129, 400), (70, 415), (128, 416), (40, 417), (66, 431), (31, 447),
+                                    (97, 448), (130, 449), (200, 479), (63, 480), (34, 511), (35, 514)])
+def test_last_blocks(variant, Nq, Nkv):
+    j, i = np.arange(Nkv), np.arange(Nq)[:, None]
+    causal = np.where(j <= i + Nkv - Nq, 0.0, -np.inf)
+    bias = np.random.default_rng(Nkv).normal(size=(2, 4, Nq, Nkv)) * 2.0
+    bias[1, :, :, Nkv - 37:] = -np.inf
+    _run(_masked(causal[None, None], 3300 + Nkv, Hq=4, Hkv=2, B=2, kv_layout="thd" if Nkv % 3 else "gap"), variant, "causal %d x %d" % (Nq, Nkv))
+    _run(_masked(bias, 3400 + Nkv, Hq=4, Hkv=4, B=2), variant, "bias %d x %d" % (Nq, Nkv))
+
+
+@pytest.mark.parametrize("variant", FORMS)
+@pytest.mark.parametrize("Nkv", [400, 451])
+def test_rows_that_start_late(variant, Nkv):
+    """first visible keys in every block, by row; rows without any; a far larger score at the end of what a row sees"""
+    Nq = 150
+    j, i = np.arange(Nkv), np.arange(Nq)[:, None]
+    late = (j >= (i * 37) % Nkv) & (i % 11 != 5)
+    case = _masked(np.where(late, 0.0, -np.inf)[None, None], 3500 + Nkv, Hq=2, B=2)
+    q, k = to_f32(case["q"]), to_f32(case["k"])
+    k[..., 0] = np.sqrt(np.linspace(0.0, 1.0, Nkv, dtype=np.float32)) * 4.0
+    q[..., 0] = 60.0 / 4.0 / case["scale"]
+    q[:, :, ::3, 0] *= -1.0
+    case["q"], case["k"] = ora.from_f32(q, ora.F32), ora.from_f32(k, ora.F16)
+    _run(case, variant, "late rows %d" % Nkv)
+
+
+@pytest.mark.parametrize("variant", FORMS)
+@pytest.mark.parametrize("Nkv", [900, 1013])
+def test_ranges(variant, Nkv):
+    """two ranges, the second shorter than the first: causal rows that end in either, and one length"""
+    Nq = 140
+    j, i = np.arange(Nkv), np.arange(Nq)[:, None]
+    for name, seen in (("causal", j <= i * 7), ("one length", (j < 130) & (i >= 0)), ("second range alone", j >= 600)):
+        _run(_masked(np.where(seen & (i >= 0), 0.0, -np.inf)[None, None], 3600 + Nkv, Hq=4, Hkv=2), variant, "%s %d" % (name, Nkv), (1, 2))
+
+
+@pytest.mark.parametrize("variant", FORMS)
+@pytest.mark.parametrize("Nkv", [500, 777])
+def test_hidden_nan_rows(variant, Nkv):
+    """excluded keys that hold NaN bits, scattered and at the end, by row: such rows are computed again, the others are not touched"""
+    Nq = 100
+    j, i = np.arange(Nkv), np.arange(Nq)[:, None]
+    holes = (j % 97 == 13) | (j > Nkv - 30)
+    seen = ~holes & (i >= 0)
+    case = _masked(np.where(seen, 0.0, -np.inf)[None, None], 3700 + Nkv, Hq=4, Hkv=2)
+    ref = run_oracle(case)
+    for t in (case["k"], case["v"]):
+        t.buf[t.offset:].reshape(2, Nkv, -1)[:, holes] = 0xFF
+    print("case", hex(variant), "hidden NaN rows", Nkv, flush=True)
+    assert_parity(run_gpu(case, kernel=ggml.KERNEL_MMA, tile_variant=variant, n_splits=1), ref)
