@@ -131,6 +131,13 @@ __device__ __forceinline__ half8 q8_dequant_keys(uint32_t q0, uint32_t q1, half8
     return r * d;
 }
 
+// a unit of a streamed row (aux 2: non-temporal, as stream_load)
+template <typename T>
+__device__ __forceinline__ T buffer_stream(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    if constexpr (sizeof(T) == 8) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 2));
+    else                          return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 2));
+}
+
 // raw global data of one 8-element chunk
 struct Chunk {
     uint4 v;         // f16: the 8 halves; q8_0: x,y = quants, z = scale bits
@@ -441,8 +448,8 @@ fattn_decode_kernel(const FattnArgs a) {
     uint32_t vdst[V8 ? NU : 1][V8 ? PCS / 2 : 1];
     // mask values of the lane's eight keys of the step, in the order of its scores
     u32x2_a2 mraw[2][MASK ? 2 : 1];
-    // a partial last step: its loads are clamped to the last valid row or unit (branch-free, in bounds) and the
-    // keys they stand for are excluded in the step
+    // a partial last step: its loads are clamped to the last valid row (branch-free, in bounds) or give zeros behind it, and
+    // the keys they stand for are excluded in the step
     auto issue = [&](int it, auto stage) __attribute__((always_inline)) {
         constexpr int s = decltype(stage)::value;
         const int j0 = k_begin + it * STEP;
@@ -473,15 +480,17 @@ fattn_decode_kernel(const FattnArgs a) {
             }
         }
         if (RAW) {
-            // one coalesced stream per tensor
-            const int last = min(STEP, k_end - j0) * (RS / UNIT) - 1;
-            const char * kp = kbase + (int64_t)j0 * RS;
-            const char * vp = vbase + (int64_t)j0 * RS;
+            // One coalesced stream per tensor, through a buffer that ends with the step's last valid row: what lies behind it are
+            // zeros, scales and minima among them, and the 2 * NU loads share one offset (its lane number through an asm, or
+            // each of the loop's would have its own).
+            const uint32_t bytes = (uint32_t)min(STEP, k_end - j0) * RS;
+            const auto     kb = fattn_buffer(kbase + (int64_t)j0 * RS, bytes), vb = fattn_buffer(vbase + (int64_t)j0 * RS, bytes);
+            uint32_t ln = (uint32_t)lane;
+            asm volatile("" : "+v"(ln));
 #pragma unroll
             for (int i = 0; i < NU; i++) {
-                const uint32_t off = (uint32_t)min(i * 64 + lane, last) * UNIT;
-                kun[ONE ? 0 : s][i] = stream_load<unit_t>(kp + off);
-                vun[ONE ? 0 : s][i] = stream_load<unit_t>(vp + off);
+                kun[ONE ? 0 : s][i] = buffer_stream<unit_t>(kb, (ln + i * 64) * UNIT);
+                vun[ONE ? 0 : s][i] = buffer_stream<unit_t>(vb, (ln + i * 64) * UNIT);
             }
             return;
         }
@@ -538,28 +547,8 @@ fattn_decode_kernel(const FattnArgs a) {
                         *(uint16_t *)(wave_mem + dst) = (uint16_t)(k % 2 ? w[k / 2] >> 16 : w[k / 2]);
                     }
                 }
-                // rows past k_end hold bytes of other rows: a zero scale makes exact zeros of them (the LDS runs a wave's
-                // writes in order)
-                if (tail) {
-#pragma unroll
-                    for (int t = 0; t < STEP * KS / 64; t++) {
-                        const int idx = t * 64 + lane, row = idx / KS;
-                        if (j0 + row >= k_end) *(uint16_t *)(vsc_stage + ((idx % KS) * STEP + row) * 2) = 0;
-                    }
-                }
             }
             if (ONE && nxt < walk_end) issue(nxt, stage);
-            if (!V8 && tail) {
-                // rows past k_end hold bytes of no row: a zero scale keeps what is made of them finite
-#pragma unroll
-                for (int t = 0; t < STEP * KS / 64; t++) {
-                    const int idx = t * 64 + lane;
-                    if (j0 + idx / KS >= k_end) {
-                        *(uint16_t *)(v_rawst + (idx / KS) * RS + (idx % KS) * BB) = 0;
-                        if (TYPE == MI355X_TYPE_Q4_1 || TYPE == MI355X_TYPE_Q5_1) *(uint16_t *)(v_rawst + (idx / KS) * RS + (idx % KS) * BB + 2) = 0;
-                    }
-                }
-            }
             __builtin_amdgcn_wave_barrier();
         }
         // ---- S^T = K . Q^T ------------------------------------------------------------------
