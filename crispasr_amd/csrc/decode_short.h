@@ -1,0 +1,86 @@
+// The decode kernel's arguments in 112 bytes (internal).  With them a workgroup finds its place without a division and has half the
+// scalar loads ahead of its first request; calls inside a graph, us, 376 bytes and these: 5 rows x 20 heads of 64 against 560
+// masked entries 6.95 -> 6.27, against 1500 7.0 -> 6.8, 8 heads of 128 against 2048 masked Q8_0 entries 9.1 -> 8.55, 663 entries
+// 7.4 -> 7.25.  A launch also costs the host 0.9 us less than one with 376 bytes (three launches of which one does 9.4 -> 8.5 us).
+#pragma once
+
+#include "fattn_common.h"
+
+// A step's call as the runtimes make it: up to 16 rows per KV head, K and V alike in their strides, no slopes, a mask that is one
+// head's or every head's own and one sequence's or every sequence's own.  Extents that one value stands for have a stride of zero.
+struct DecodeShort {
+    const char * q;
+    const char * k;
+    const char * v;
+    const char * mask;
+    float *      dst;
+    float *      part_acc;            // the (max, sum) pairs lie right behind it
+    unsigned *   counters;
+    uint32_t     nbq1, nbq2, nbq3;
+    uint32_t     nbk1, nbk2, nbk3;    // and V's
+    uint32_t     nbm1, nbm2, nbm3;
+    float        scale;
+    uint32_t     Nkv;
+    uint32_t     rows;                // Nq | gqa << 5 | n_splits << 10 | keys_per_split / 32 << 17 (0: not cut)
+    uint32_t     heads;               // Hkv | B << 16
+    uint32_t     Dv;
+};
+static_assert(sizeof(DecodeShort) <= 112, "see above");
+
+// false: the call needs the wide form
+static inline bool decode_shorten(const FattnArgs & a, DecodeShort & p) {
+    const int64_t nb[12] = {a.nbq1, a.nbq2, a.nbq3, a.nbk1, a.nbk2, a.nbk3, a.nbv1, a.nbv2, a.nbv3, a.nbm1, a.nbm2, a.nbm3};
+    for (int i = 0; i < (a.mask ? 12 : 9); i++)
+        if ((uint64_t)nb[i] > 0xFFFFFFFFull) return false;
+    const bool    one_sequence = a.Bk == 1;
+    const int64_t rows = (int64_t)a.Nq * a.Hq * a.B;
+    if (a.q_chunks != 1 || a.Nq < 1 || a.gqa < 1 || (int64_t)a.Nq * a.gqa > 16 || a.max_bias > 0.0f || a.softcap != 0.0f) return false;
+    if (!(one_sequence || a.Bk == a.B) || a.nbk1 != a.nbv1 || a.nbk2 != a.nbv2 || (!one_sequence && a.nbk3 != a.nbv3)) return false;
+    if (a.mask && (!(a.Hm == 1 || a.Hm == a.Hq) || !(a.Bm == 1 || a.Bm == a.B))) return false;
+    if (a.Hkv > 0xFFFF || a.B > 0xFFFF || a.Hq != a.Hkv * a.gqa) return false;
+    if (a.n_splits > 127 || (a.n_splits > 1 && (a.keys_per_split % 32 || a.keys_per_split / 32 < 1 || a.keys_per_split / 32 > 0x7FFF))) return false;
+    if (a.n_splits > 1 && a.part_ml != a.part_acc + rows * a.n_splits * a.D) return false;
+    if (a.n_splits == 1 && a.keys_per_split < a.Nkv) return false;
+    p.q = a.q; p.k = a.k; p.v = a.v; p.mask = a.mask; p.dst = a.dst;
+    p.part_acc = a.n_splits > 1 ? a.part_acc : nullptr;
+    p.counters = a.n_splits > 1 ? a.counters : nullptr;
+    p.nbq1 = (uint32_t)a.nbq1; p.nbq2 = (uint32_t)a.nbq2; p.nbq3 = (uint32_t)a.nbq3;
+    p.nbk1 = (uint32_t)a.nbk1; p.nbk2 = (uint32_t)a.nbk2; p.nbk3 = one_sequence ? 0 : (uint32_t)a.nbk3;
+    p.nbm1 = a.mask ? (uint32_t)a.nbm1 : 0;
+    p.nbm2 = a.mask && a.Hm > 1 ? (uint32_t)a.nbm2 : 0;
+    p.nbm3 = a.mask && a.Bm > 1 ? (uint32_t)a.nbm3 : 0;
+    p.scale = a.scale;
+    p.Nkv   = (uint32_t)a.Nkv;
+    p.rows  = (uint32_t)a.Nq | (uint32_t)a.gqa << 5 | (uint32_t)a.n_splits << 10 | (a.n_splits > 1 ? (uint32_t)(a.keys_per_split / 32) << 17 : 0);
+    p.heads = (uint32_t)a.Hkv | (uint32_t)a.B << 16;
+    p.Dv    = (uint32_t)a.Dv;
+    return true;
+}
+
+// what the kernel reads of the wide form (a stride of zero for the extents that one value stands for)
+static __host__ __device__ __forceinline__ FattnArgs decode_expand(const DecodeShort & p, int D) {
+    FattnArgs a = {};
+    a.q = p.q; a.k = p.k; a.v = p.v; a.mask = p.mask; a.dst = p.dst;
+    a.D  = D;
+    a.Dv = (int)p.Dv;
+    a.Nq = (int)(p.rows & 31u);
+    a.gqa = (int)(p.rows >> 5 & 31u);
+    a.n_splits = (int)(p.rows >> 10 & 127u);
+    a.Nkv = (int)p.Nkv;
+    a.keys_per_split = a.n_splits > 1 ? (int)(p.rows >> 17) * 32 : a.Nkv;
+    a.Hkv = (int)(p.heads & 0xFFFFu);
+    a.B = a.Bk = (int)(p.heads >> 16);
+    a.Hq = a.Hkv * a.gqa;
+    a.bq = a.q_chunks = 1;
+    a.Hm = p.nbm2 ? a.Hq : 1;
+    a.Bm = p.nbm3 ? a.B : 1;
+    a.masked = p.mask != nullptr;
+    a.nbq1 = p.nbq1; a.nbq2 = p.nbq2; a.nbq3 = p.nbq3;
+    a.nbk1 = a.nbv1 = p.nbk1; a.nbk2 = a.nbv2 = p.nbk2; a.nbk3 = a.nbv3 = p.nbk3;
+    a.nbm1 = p.nbm1; a.nbm2 = p.nbm2; a.nbm3 = p.nbm3;
+    a.scale = p.scale;
+    a.part_acc = p.part_acc;
+    a.part_ml  = p.part_acc + (int64_t)a.Nq * a.Hq * a.B * a.n_splits * D;
+    a.counters = p.counters;
+    return a;
+}

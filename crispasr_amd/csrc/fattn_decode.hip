@@ -32,6 +32,7 @@
 // requested with its K and V: one step for 64 sequences of 500 to 4096 Q8_0 entries (32 query, 8 KV heads of 128) 115 -> 81 us,
 // 3.8 TB/s over the entries seen; the bound is the bytes in flight of the longest sequences' splits.
 #include "fattn_row.h"
+#include "decode_short.h"
 
 #include <stdlib.h>
 #include <type_traits>
@@ -319,9 +320,9 @@ template <int D> __device__ const V8Places<D> v8_places_table = v8_places<D>();
 // first K/V request: computing the 36 of them costs more instructions than a 32-key step).
 // PAD: f16 rows of a.Dv elements (a multiple of 8 below D) read in place: the chunks of a row behind Dv are zeros in the
 // registers, q is read and dst written up to Dv.  An instantiation of its own: the others stay the code they were.
-template <int D, int TYPE, bool MASK, bool RAW, bool V8, bool PAD = false>
-__global__ void __launch_bounds__(DEC_THREADS) __attribute__((amdgpu_waves_per_eu((decode_waves_min<D, TYPE, RAW>()), (decode_waves_max<D, RAW, V8>()))))
-fattn_decode_kernel(const FattnArgs a) {
+// SHORT: the arguments came as DecodeShort, the grid is (split, KV head, batch), and there is one chunk of rows.
+template <int D, int TYPE, bool MASK, bool RAW, bool V8, bool PAD, bool SHORT>
+__device__ __forceinline__ void decode_body(const FattnArgs & a) {
     static_assert(!PAD || (TYPE == MI355X_TYPE_F16 && !RAW && !V8), "other head sizes: f16 rows, read per lane");
     static_assert(!V8 || RAW, "the int8 V stage belongs to the streamed Q8_0 path");
     constexpr int KS  = D / 32;                    // reduction steps of Q.K^T (one Q8_0 block each)
@@ -370,28 +371,40 @@ fattn_decode_kernel(const FattnArgs a) {
     int     split, chunk, hk, b;
     int64_t set;                                   // index of (chunk, KV head, batch): the merge's counter
     // (divisions by multiply and shift: a call that is one or two steps long spends 0.3 us on five ordinary ones)
-    uint32_t pair = blockIdx.x;
     chunk = 0;
-    if (a.q_chunks != 1) {
-        const uint32_t w  = blockIdx.x >> 3;
-        const uint32_t wc = divide(w, a.by_chunks);
-        pair  = wc * 8u + (blockIdx.x & 7u);
-        chunk = (int)(w - wc * (uint32_t)a.q_chunks);
-        if (pair >= (uint32_t)a.n_splits * (uint32_t)a.Hkv * (uint32_t)a.B) return;      // (<= the grid)
+    if constexpr (SHORT) {
+        split = (int)blockIdx.x;
+        hk    = (int)blockIdx.y;
+        b     = (int)blockIdx.z;
+        set   = (int64_t)b * a.Hkv + hk;
+    } else {
+        uint32_t pair = blockIdx.x;
+        if (a.q_chunks != 1) {
+            const uint32_t w  = blockIdx.x >> 3;
+            const uint32_t wc = divide(w, a.by_chunks);
+            pair  = wc * 8u + (blockIdx.x & 7u);
+            chunk = (int)(w - wc * (uint32_t)a.q_chunks);
+            if (pair >= (uint32_t)a.n_splits * (uint32_t)a.Hkv * (uint32_t)a.B) return;      // (<= the grid)
+        }
+        const uint32_t head = divide(pair, a.by_splits);
+        b     = (int)divide(head, a.by_hkv);
+        split = (int)(pair - head * (uint32_t)a.n_splits);
+        hk    = (int)head - b * a.Hkv;
+        set   = (int64_t)head * a.q_chunks + chunk;
     }
-    const uint32_t head = divide(pair, a.by_splits);
-    b     = (int)divide(head, a.by_hkv);
-    split = (int)(pair - head * (uint32_t)a.n_splits);
-    hk    = (int)head - b * a.Hkv;
-    set   = (int64_t)head * a.q_chunks + chunk;
-    const int bk    = (int)divide((uint32_t)b, a.by_bq);
+    const int bk = SHORT ? b : (int)divide((uint32_t)b, a.by_bq);
+    // row / gqa (SHORT: both at most 16, and (row + 1/2) / gqa is never near a whole number)
+    const float per_row = SHORT ? __builtin_amdgcn_rcpf((float)a.gqa) : 0.0f;
+    auto query_of = [&](int row) __attribute__((always_inline)) {
+        return SHORT ? (int)(((float)row + 0.5f) * per_row) : (int)divide((uint32_t)row, a.by_gqa);
+    };
 
     // row r = iq1 * gqa + gg of this KV head  <->  query iq1 of q head hk*gqa + gg; column j is row chunk*16 + j
     const int  R      = a.Nq * a.gqa;
     const int  row0   = chunk * 16;
     const bool col_ok = row0 + j < R;
     const int  jc     = col_ok ? row0 + j : row0;
-    const int  iq1    = (int)divide((uint32_t)jc, a.by_gqa);
+    const int  iq1    = query_of(jc);
     const int  h      = hk * a.gqa + jc - iq1 * a.gqa;
 
     const int k_begin = split * a.keys_per_split;
@@ -400,8 +413,8 @@ fattn_decode_kernel(const FattnArgs a) {
     half8 qreg[KS];
     const char * kbase = a.k + (int64_t)hk * a.nbk2 + (int64_t)bk * a.nbk3;
     const char * vbase = a.v + (int64_t)hk * a.nbv2 + (int64_t)bk * a.nbv3;
-    const char * mhead = MASK ? a.mask + (int64_t)(h - (int)divide((uint32_t)h, a.by_hm) * a.Hm) * a.nbm2 +
-                                (int64_t)(b - (int)divide((uint32_t)b, a.by_bm) * a.Bm) * a.nbm3
+    const char * mhead = MASK ? a.mask + (int64_t)(SHORT ? h : h - (int)divide((uint32_t)h, a.by_hm) * a.Hm) * a.nbm2 +
+                                (int64_t)(SHORT ? b : b - (int)divide((uint32_t)b, a.by_bm) * a.Bm) * a.nbm3
                               : nullptr;
     const uint16_t * mrow = (const uint16_t *)(mhead + (int64_t)iq1 * a.nbm1);
     const float mslope = MASK ? fattn_slope(a, h) * LOG2E : 0.0f;
@@ -424,8 +437,8 @@ fattn_decode_kernel(const FattnArgs a) {
     // are written, 16 query, 8 KV heads of 128, 10.3, 9.2 and 9.9 us.  Splits of one step a wave never look.
     const uint32_t EXCLUDED2 = 0xFC00FC00u;                 // two masked-out keys
     int        walk = wave, walk_end = n_steps;             // the steps that the wave walks
-    const int  iq_0    = MASK ? (int)divide((uint32_t)row0, a.by_gqa) : 0;
-    const int  iq_1    = MASK ? (int)divide((uint32_t)min(row0 + 15, R - 1), a.by_gqa) : 0;
+    const int  iq_0    = MASK ? query_of(row0) : 0;
+    const int  iq_1    = MASK ? query_of(min(row0 + 15, R - 1)) : 0;
     const bool one_row = iq_1 == iq_0;
     const bool looking = MASK && n_steps > DEC_WAVES && (one_row ? n_steps <= 128 : n_steps <= 16 && iq_1 - iq_0 < 8) && (a.Hm == 1 || R == 1) &&
                          __builtin_amdgcn_ballot_w64(!(mslope > 0.0f)) == 0;
@@ -775,7 +788,7 @@ fattn_decode_kernel(const FattnArgs a) {
             L += red_ml[w][col][1] * f[w];
         }
         bad = not_finite(L);
-        const int     ciq1 = (int)divide((uint32_t)(row0 + col), a.by_gqa);
+        const int     ciq1 = query_of(row0 + col);
         const int     ch   = hk * a.gqa + row0 + col - ciq1 * a.gqa;
         const int64_t row  = ((int64_t)b * a.Nq + ciq1) * a.Hq + ch;
         const int dv = PAD ? a.Dv : D;              // dst rows are dv floats; partial rows stay D apart
@@ -844,14 +857,45 @@ fattn_decode_kernel(const FattnArgs a) {
         constexpr int LPR = D / 4;                  // lanes per row: 8 or 4 rows per pass
         for (int c = tid / LPR; c < 16 && row0 + c < R; c += DEC_THREADS / LPR) {
             const int r = row0 + c;
-            const int riq = (int)divide((uint32_t)r, a.by_gqa);
+            const int riq = query_of(r);
             fattn_merge_row<true>(a, ((int64_t)b * a.Nq + riq) * a.Hq + hk * a.gqa + r - riq * a.gqa, tid % LPR);
         }
     }
 }
 
+template <int D, int TYPE, bool MASK, bool RAW, bool V8, bool PAD = false>
+__global__ void __launch_bounds__(DEC_THREADS) __attribute__((amdgpu_waves_per_eu((decode_waves_min<D, TYPE, RAW>()), (decode_waves_max<D, RAW, V8>()))))
+fattn_decode_kernel(const FattnArgs a) {
+    decode_body<D, TYPE, MASK, RAW, V8, PAD, false>(a);
+}
+
+template <int D, int TYPE, bool MASK, bool RAW, bool V8, bool PAD>
+__global__ void __launch_bounds__(DEC_THREADS)
+__attribute__((amdgpu_waves_per_eu((D == 64 && TYPE == MI355X_TYPE_F16 && !MASK ? 4 : decode_waves_min<D, TYPE, RAW>()), (decode_waves_max<D, RAW, V8>()))))
+fattn_decode_short_kernel(const DecodeShort p) {
+    FattnArgs a = decode_expand(p, D);
+    if (!PAD) a.Dv = D;
+    decode_body<D, TYPE, MASK, RAW, V8, PAD, true>(a);
+}
+
 template <int D, int TYPE, bool MASK, bool RAW, bool V8 = false, bool PAD = false>
 int launch_one(FattnArgs a, hipStream_t stream) {
+    const int64_t pairs = (int64_t)a.n_splits * a.Hkv * a.B;
+    const int64_t wgs   = a.q_chunks == 1 ? pairs : (pairs + 7) / 8 * 8 * a.q_chunks;      // as the kernel numbers them
+    if (wgs > 0x7fffffff || a.q_chunks != (a.Nq * a.gqa + 15) / 16) return (int)hipErrorInvalidValue;
+    const dim3 grid((unsigned)wgs);
+    constexpr int lds = decode_lds_bytes<D, TYPE, RAW, V8>();
+    if constexpr (TYPE == MI355X_TYPE_F16 || V8 || (RAW && TYPE != MI355X_TYPE_Q8_0)) {      // (the rows of a cache as they usually lie)
+        DecodeShort p;
+        if (decode_shorten(a, p)) {
+            static std::atomic<uint64_t> short_lds_allowed{0};
+            const hipError_t e = fattn_allow_lds((const void *)fattn_decode_short_kernel<D, TYPE, MASK, RAW, V8, PAD>, lds, short_lds_allowed);
+            if (e != hipSuccess) return (int)e;
+            hipLaunchKernelGGL((fattn_decode_short_kernel<D, TYPE, MASK, RAW, V8, PAD>), dim3((unsigned)a.n_splits, (unsigned)a.Hkv, (unsigned)a.B),
+                               dim3(DEC_THREADS), lds, stream, p);
+            return (int)hipGetLastError();
+        }
+    }
     a.by_splits = fast_div((uint32_t)a.n_splits);
     a.by_chunks = fast_div((uint32_t)a.q_chunks);
     a.by_hkv    = fast_div((uint32_t)a.Hkv);
@@ -859,11 +903,6 @@ int launch_one(FattnArgs a, hipStream_t stream) {
     a.by_bq     = fast_div((uint32_t)a.bq);
     a.by_hm     = fast_div((uint32_t)a.Hm);
     a.by_bm     = fast_div((uint32_t)a.Bm);
-    const int64_t pairs = (int64_t)a.n_splits * a.Hkv * a.B;
-    const int64_t wgs   = a.q_chunks == 1 ? pairs : (pairs + 7) / 8 * 8 * a.q_chunks;      // as the kernel numbers them
-    if (wgs > 0x7fffffff || a.q_chunks != (a.Nq * a.gqa + 15) / 16) return (int)hipErrorInvalidValue;
-    const dim3 grid((unsigned)wgs);
-    constexpr int lds = decode_lds_bytes<D, TYPE, RAW, V8>();
     static std::atomic<uint64_t> lds_allowed{0};
     const hipError_t e = fattn_allow_lds((const void *)fattn_decode_kernel<D, TYPE, MASK, RAW, V8, PAD>, lds, lds_allowed);
     if (e != hipSuccess) return (int)e;
