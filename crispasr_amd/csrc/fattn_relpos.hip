@@ -135,11 +135,18 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
         } else {
             const int      first = min(max(row0, 0), last_row);
             const uint64_t at    = (uint64_t)(base + (int64_t)first * nb1);
-#pragma unroll (FIRST ? NDM : 1)
-            for (int j = 0; j < NDM; j++) {
+            auto instruction = [&](int j) __attribute__((always_inline)) {
                 const uint32_t ins = min((uint32_t)(j * NW + wave), (uint32_t)TI - 1);
                 const uint32_t rr  = (uint32_t)(min(max(row0 + (int)ins * RPI + lr, 0), last_row) - first);
                 load_to_lds16<true>(at, rr * nb + (V ? cv : ck ^ ((ins & (16 / RPI - 1)) * 64)), to + ins * 1024);
+            };
+            // (two loops: the compiler has crashed over an unroll count that depends on the instantiation)
+            if constexpr (FIRST) {
+#pragma unroll
+                for (int j = 0; j < NDM; j++) instruction(j);
+            } else {
+#pragma unroll 1
+                for (int j = 0; j < NDM; j++) instruction(j);
             }
         }
     };
