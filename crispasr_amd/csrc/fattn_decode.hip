@@ -26,7 +26,8 @@
 // product - to be widened and multiplied by those keys' scales in registers: same values, half the LDS bytes, one
 // register stage instead of two.  Q4_0 / Q4_1 / Q5_0 / Q5_1 rows are streamed the same way into raw K and V stages and
 // dequantised out of LDS (V into the f16 stage).  Streams and f16 rows are loaded non-temporal: they are read once.
-// Loads of the next step are in flight while the current one is consumed.  Waves are merged through LDS, splits by fattn_merge_kernel.
+// Loads of the next step are in flight while the current one is consumed.  Waves are merged through LDS, splits by the last
+// workgroup of a set where the call has counters for it (fattn_last_of_set), by fattn_merge_kernel otherwise.
 //
 // Masked calls walk the steps between the first and the last that one of their rows sees, and a step's mask values are
 // requested with its K and V: one step for 64 sequences of 500 to 4096 Q8_0 entries (32 query, 8 KV heads of 128) 115 -> 81 us,
