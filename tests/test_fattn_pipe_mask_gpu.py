@@ -79,3 +79,25 @@ def test_hidden_nan_rows(variant, Nkv):
         t.buf[t.offset:].reshape(2, Nkv, -1)[:, holes] = 0xFF
     print("case", hex(variant), "hidden NaN rows", Nkv, flush=True)
     assert_parity(run_gpu(case, kernel=ggml.KERNEL_MMA, tile_variant=variant, n_splits=1), ref)
+
+
+@pytest.mark.parametrize("variant", FORMS)
+@pytest.mark.parametrize("Nkv", [384, 511, 640])
+def test_extreme_mask_values(variant, Nkv):
+    """the type's lowest and largest finite value in place of -inf and 0: rows of nothing else, at the start, at the end, scattered, among
+    excluded keys.  V climbs from 0 to 4 with the key, so a row's result tells which keys it took.  A sum of a score and +-65504 is rounded to
+    2^-8 (natural) in the oracle and to 2^-7 (log2) here, twice: no probability is off by more than 2^-6 of itself, no mean by 4 * 2^-6."""
+    Nq = 70
+    j, i = np.arange(Nkv), np.arange(Nq)[:, None] % 7
+    low, high = -65504.0, 65504.0
+    seen = j * (i + 1) % 5 < 3
+    for name, m in (("lowest", np.where(i == 0, low, np.where(i == 1, np.where(j < 200, low, 0.0), np.where(i == 2, np.where(j < 200, 0.0, low),
+                                np.where(i == 3, np.where(seen, low, -np.inf), np.where(i == 4, np.where(j > 300, low, -np.inf), np.where(seen, 0.0, low))))))),
+                    ("largest", np.where(i < 3, np.where(j > 100 * i, high, 0.0), np.where(i < 5, np.where(seen, high, low), np.where(seen, high, -np.inf))))):
+        case = _masked(np.broadcast_to(m, (1, 1, Nq, Nkv)), 3800 + Nkv, Hq=4, Hkv=2)
+        case["q"] = ora.from_f32(np.clip(to_f32(case["q"]), -3, 3) * 0.05, ora.F32)
+        case["v"] = ora.from_f32(np.broadcast_to((4.0 * j / Nkv)[:, None], to_f32(case["v"]).shape), ora.F16)
+        ref = run_oracle(case)
+        print("case", hex(variant), name, Nkv, flush=True)
+        out = run_gpu(case, kernel=ggml.KERNEL_MMA, tile_variant=variant, n_splits=1)
+        assert np.isfinite(out).all() and np.abs(out - ref).max() <= 4 * 2.0 ** -6, (name, np.abs(out - ref).max())
