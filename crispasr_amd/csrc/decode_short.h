@@ -23,11 +23,30 @@ struct DecodeShort {
     uint32_t     Nkv;
     uint32_t     rows;                // Nq | gqa << 5 | n_splits << 10 | keys_per_split / 32 << 17 (0: not cut)
     uint32_t     heads;               // Hkv | B << 16
-    uint32_t     Dv;
+    uint32_t     Dv;                  // | sequences in the first round << 16 (0: in their own order, see decode_turns)
 };
 static_assert(sizeof(DecodeShort) <= 112, "see above");
 
 // false: the call needs the wide form
+// Sequences of different lengths in one call (a mask of every sequence's own ends each), more workgroups than CUs: a CU that gets the
+// workgroups of two long ones is the last.  Workgroup n_cus + i comes to the CU of workgroup i, so the sequences of the first round (a
+// workgroup on every CU) go in their own order, and those behind them by length (sequence_of_turn): the longest beside the shortest.
+// In graphs, 32 query, 8 KV heads of 128, lengths spread evenly and shuffled, us: 64 sequences of 500 to 4096 Q8_0 entries 81 -> 71, of
+// 200 to 2048 f16 entries 69 -> 55, 40 of these 64 -> 52, 128 of 300 to 2048 Q8_0 entries 77 -> 68, 64 of 100 to 512 16.9 -> 15.9;
+// of one length 99.9 -> 99.9 (4096), 19.6 -> 19.6 (36 x 600).  (The first round by length as well, from the middle to the longest, is
+// better yet where few CUs get a second workgroup, 40 f16 sequences 44, but its look is in nobody's shadow: +1.2 us.)
+// Not where the look has nothing to hide behind: below 64 kB of a head's K (64 sequences of 512 Q8_0 entries have 70), and for rows that
+// are bound by their dequantising (all but f16 and Q8_0 of 128) below 128 kB and where the second round is not whole: 48 sequences of
+// 1000 Q4_0 entries 24.1 -> 25.1, of 2048 Q8_0 entries of 64 26.4 -> 27.2; 64 of 400 to 4000 Q4_0 entries of 64 44.3 -> 42.5.
+// Returns the sequences in the first round, or 0: their own order.
+static inline uint32_t decode_turns(const FattnArgs & a, int row_bytes) {
+    if (!a.mask || a.n_splits != 1 || a.Bm != a.B || a.B < 2 || a.B > 128 || a.Hkv > a.n_cus || (int64_t)a.Hkv * a.B <= a.n_cus) return 0;
+    const int  first = a.n_cus / a.Hkv;            // (below B)
+    const bool wide  = row_bytes >= 128;
+    if ((int64_t)a.Nkv * row_bytes < (wide ? 64 : 128) * 1024 || (!wide && a.B < 2 * first)) return 0;
+    return (uint32_t)first;
+}
+
 static inline bool decode_shorten(const FattnArgs & a, DecodeShort & p) {
     const int64_t nb[12] = {a.nbq1, a.nbq2, a.nbq3, a.nbk1, a.nbk2, a.nbk3, a.nbv1, a.nbv2, a.nbv3, a.nbm1, a.nbm2, a.nbm3};
     for (int i = 0; i < (a.mask ? 12 : 9); i++)
@@ -62,7 +81,7 @@ static __host__ __device__ __forceinline__ FattnArgs decode_expand(const DecodeS
     FattnArgs a = {};
     a.q = p.q; a.k = p.k; a.v = p.v; a.mask = p.mask; a.dst = p.dst;
     a.D  = D;
-    a.Dv = (int)p.Dv;
+    a.Dv = (int)(p.Dv & 0xFFFFu);
     a.Nq = (int)(p.rows & 31u);
     a.gqa = (int)(p.rows >> 5 & 31u);
     a.n_splits = (int)(p.rows >> 10 & 127u);

@@ -31,7 +31,7 @@
 //
 // Masked calls walk the steps between the first and the last that one of their rows sees, and a step's mask values are
 // requested with its K and V: one step for 64 sequences of 500 to 4096 Q8_0 entries (32 query, 8 KV heads of 128) 115 -> 81 us,
-// 3.8 TB/s over the entries seen; the bound is the bytes in flight of the longest sequences' splits.
+// 71 with the sequences paired by length on the CUs (sequence_of_turn), 4.5 TB/s over the entries seen; the bound is what a CU's port brings.
 #include "fattn_row.h"
 #include "decode_short.h"
 
@@ -313,6 +313,64 @@ constexpr V8Places<D> v8_places() {
 }
 template <int D> __device__ const V8Places<D> v8_places_table = v8_places<D>();
 
+// The sequence whose turn it is where they go by length (decode_turns; at most 128).  Lengths are counted in eighths: eight keys of
+// every sequence's mask, two a wave, in the last query's row (what a count is off by, or a mask that does not end a sequence, costs
+// balance and nothing else: every workgroup counts the same, and the places are a permutation).  A look costs 1.3 us where nothing else
+// runs on the CU, so the first round takes the sequences in their own order, and the next ones, whose look hides behind it, make up for that.
+__device__ __forceinline__ int sequence_of_turn(const FattnArgs & a, int turn, int first, char * lds) {
+    if (turn < first) return turn;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    int * counts = (int *)lds;                     // [wave][128]
+    const bool more = a.B > 64;
+#pragma unroll
+    for (int g = 0; g < 2; g++)
+        if (g == 0 || more) {
+            const int        b   = min(g * 64 + lane, a.B - 1);
+            const uint16_t * row = (const uint16_t *)(a.mask + (int64_t)b * a.nbm3 + (int64_t)(a.Nq - 1) * a.nbm1);
+            const uint16_t v0 = row[(int)((int64_t)(wave * 4 + 1) * a.Nkv >> 4)], v1 = row[(int)((int64_t)(wave * 4 + 3) * a.Nkv >> 4)];
+            counts[wave * 128 + g * 64 + lane] = (v0 != 0xFC00u) + (v1 != 0xFC00u);
+        }
+    __syncthreads();
+    int seen[2] = {0, -1};
+#pragma unroll
+    for (int w = 0; w < DEC_WAVES; w++) seen[0] += counts[w * 128 + lane];
+    if (lane >= a.B) seen[0] = -1;
+    if (more && 64 + lane < a.B) {
+        seen[1] = 0;
+#pragma unroll
+        for (int w = 0; w < DEC_WAVES; w++) seen[1] += counts[w * 128 + 64 + lane];
+    }
+    __syncthreads();                               // the stages of the key loop lie where the counts do
+
+    // places by length, the longest first, among the sequences [from, to): of sequence `lane` and of 64 + lane
+    int place[2];
+    auto rank = [&](int from, int to) __attribute__((always_inline)) {
+        place[0] = place[1] = -1;
+        int n = 0;
+#pragma unroll
+        for (int eighths = 8; eighths >= 0; eighths--)
+#pragma unroll
+            for (int g = 0; g < 2; g++)
+                if (g == 0 || more) {
+                    const bool     one   = seen[g] == eighths && g * 64 + lane >= from && g * 64 + lane < to;
+                    const uint64_t those = __ballot(one);
+                    const int      at    = n + __builtin_amdgcn_mbcnt_hi((uint32_t)(those >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)those, 0));
+                    if (one) place[g] = at;
+                    n += __popcll(those);
+                }
+    };
+    const int behind = turn - first, pairs = min(first, a.B - first);      // (pairs <= 64)
+    int want = behind;
+    if (behind < pairs) {                          // beside sequence `behind`: the longest of those gets the shortest of these
+        rank(0, pairs);
+        want = pairs - 1 - __builtin_amdgcn_readlane(place[0], behind);
+    }
+    rank(first, a.B);
+    const uint64_t low = __ballot(place[0] == want), high = __ballot(place[1] == want);
+    return low ? __builtin_ctzll(low) : high ? 64 + __builtin_ctzll(high) : 0;
+}
+
 // V8 (with RAW): V's quants go to LDS as bytes and come back through ds_read_b64_tr_b8 already in operand layout
 // (8 consecutive keys of one column per lane).  The transposing read ignores the low three address bits and the quants
 // of block b start at byte 34 b + 2 of a row, so the rows cannot stay as they are in memory: V arrives as the same
@@ -321,9 +379,9 @@ template <int D> __device__ const V8Places<D> v8_places_table = v8_places<D>();
 // first K/V request: computing the 36 of them costs more instructions than a 32-key step).
 // PAD: f16 rows of a.Dv elements (a multiple of 8 below D) read in place: the chunks of a row behind Dv are zeros in the
 // registers, q is read and dst written up to Dv.  An instantiation of its own: the others stay the code they were.
-// SHORT: the arguments came as DecodeShort, the grid is (split, KV head, batch), and there is one chunk of rows.
+// SHORT: the arguments came as DecodeShort, the grid is (split, KV head, batch), and there is one chunk of rows; `first`: decode_turns.
 template <int D, int TYPE, bool MASK, bool RAW, bool V8, bool PAD, bool SHORT>
-__device__ __forceinline__ void decode_body(const FattnArgs & a) {
+__device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
     static_assert(!PAD || (TYPE == MI355X_TYPE_F16 && !RAW && !V8), "other head sizes: f16 rows, read per lane");
     static_assert(!V8 || RAW, "the int8 V stage belongs to the streamed Q8_0 path");
     constexpr int KS  = D / 32;                    // reduction steps of Q.K^T (one Q8_0 block each)
@@ -376,7 +434,7 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a) {
     if constexpr (SHORT) {
         split = (int)blockIdx.x;
         hk    = (int)blockIdx.y;
-        b     = (int)blockIdx.z;
+        b     = MASK && first ? sequence_of_turn(a, (int)blockIdx.z, first, smem) : (int)blockIdx.z;
         set   = (int64_t)b * a.Hkv + hk;
     } else {
         uint32_t pair = blockIdx.x;
@@ -867,7 +925,7 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a) {
 template <int D, int TYPE, bool MASK, bool RAW, bool V8, bool PAD = false>
 __global__ void __launch_bounds__(DEC_THREADS) __attribute__((amdgpu_waves_per_eu((decode_waves_min<D, TYPE, RAW>()), (decode_waves_max<D, RAW, V8>()))))
 fattn_decode_kernel(const FattnArgs a) {
-    decode_body<D, TYPE, MASK, RAW, V8, PAD, false>(a);
+    decode_body<D, TYPE, MASK, RAW, V8, PAD, false>(a, 0);
 }
 
 template <int D, int TYPE, bool MASK, bool RAW, bool V8, bool PAD>
@@ -876,7 +934,7 @@ __attribute__((amdgpu_waves_per_eu((D == 64 && TYPE == MI355X_TYPE_F16 && !MASK 
 fattn_decode_short_kernel(const DecodeShort p) {
     FattnArgs a = decode_expand(p, D);
     if (!PAD) a.Dv = D;
-    decode_body<D, TYPE, MASK, RAW, V8, PAD, true>(a);
+    decode_body<D, TYPE, MASK, RAW, V8, PAD, true>(a, (int)(p.Dv >> 16));
 }
 
 template <int D, int TYPE, bool MASK, bool RAW, bool V8 = false, bool PAD = false>
@@ -889,6 +947,7 @@ int launch_one(FattnArgs a, hipStream_t stream) {
     if constexpr (TYPE == MI355X_TYPE_F16 || V8 || (RAW && TYPE != MI355X_TYPE_Q8_0)) {      // (the rows of a cache as they usually lie)
         DecodeShort p;
         if (decode_shorten(a, p)) {
+            if (MASK) p.Dv |= decode_turns(a, TYPE == MI355X_TYPE_F16 ? D * 2 : D / 32 * raw_block_bytes<TYPE>()) << 16;
             static std::atomic<uint64_t> short_lds_allowed{0};
             const hipError_t e = fattn_allow_lds((const void *)fattn_decode_short_kernel<D, TYPE, MASK, RAW, V8, PAD>, lds, short_lds_allowed);
             if (e != hipSuccess) return (int)e;
