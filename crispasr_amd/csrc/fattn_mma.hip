@@ -1055,9 +1055,10 @@ void fattn_mma_variant(const FattnArgs & a, int ktype, FattnMmaVariant & v) {
     // whole one when the key loop is long enough to carry its merge.
     const int64_t slots1 = (int64_t)(a.Nq + 127) / 128 * 128, slots2 = (int64_t)(a.Nq + 255) / 256 * 256;
     const bool two_auto = wg2 >= cus && slots2 * 10 <= slots1 * 11;
-    // (With a mask the split form, which skips excluded blocks, carries its merge from 512 keys on; and a mask whose rows
-    // cannot go through LDS costs the unsplit forms a quarter of their speed: there the split form wins up to 1.6
-    // workgroups per CU.)
+    // (With a mask the split form carries its merge from 512 keys on; and a mask whose rows cannot go through LDS costs the
+    // unsplit forms a quarter of their speed: there the split form wins up to 1.6 workgroups per CU.  Both were measured on 64-wide
+    // heads, whose split form skips excluded blocks; 128-wide heads have one rule with and without a mask, and from 384 keys on
+    // the pipelined kernel, which leaves out the keys ahead of the first visible one and behind the last.)
     // (a zero-padded head exists in the direct forms only: its K/V are the call's own f16 copies)
     const bool direct = ktype == MI355X_TYPE_F16 && (!no_direct || a.Dv != a.D) && a.nbk1 < (1u << 24) && a.nbv1 < (1u << 24);
     const bool mdma_ok = a.masked && a.softcap == 0.0f && direct && !no_mdma && a.mask_al4 && a.Nkv >= 64 && !(a.Nkv & 1) &&

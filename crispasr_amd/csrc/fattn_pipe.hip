@@ -32,6 +32,15 @@
 // tokens 42.5 -> 37.5, 407 (rows that start between dwords, the pairs' form) 21.4 -> 20.1; under per-head masks 750 x 8 heads x 8
 // 45.7 -> 38.8, 1000 x 8 x 4 38.1 -> 32.7, 751 x 8 22.0 -> 19.2.  The 407-token launch (16 us) is 4.5 us until the first scores, 0.65
 // a step - 32 KB through a CU's port - and 3 for the hand-over and the stores.
+// Hidden keys: the walk ends behind the last 64 that a query of the workgroup sees, starts at the first ones (ranges of 12 tiles and
+// more, where that leaves out four), and between the two a hidden block is walked like a visible one - the pairs' form is bound by
+// its K and V bytes, which the tile kernel, which skips the block's products, fetches as well.  A row that has seen nothing yet
+// stands on a reference below every score: while it stood on -inf its sums were NaN and the wave took the rare path in every step.
+// us a call, tile kernel / on -inf and from the first key on / as it is, 8 heads: 1000 causal tokens in a window of 256 21.4 / 24.4 /
+// 17.7, four sequences in 900 tokens 20.9 / 24.4 / 17.4, 768 tokens whose first half is hidden 19.1 / 19.1 / 14.7, 500 causal tokens x 4
+// padded on the left 16.9 / 18.2 / 16.6, 407 tokens in four sequences (odd rows) 15.55 / 17.3 / 15.6, the middle half of 2048 hidden
+// 45.5 / 32.5 / 32.9; 32 heads, 2048 tokens in a window of 256 77 / 66 / 42.  What it costs where no key is hidden: nothing
+// (2048 x 8 heads 35.0 -> 35.3, 1024 x 32 30.7 -> 31.1, 407 x 32 16.55 -> 16.15; these differ by 1% from run to run).
 // What is left above the MFMAs of a wave alone on its SIMD is instruction issue (about 5 cycles an instruction).  Where two
 // share a SIMD nothing is full: by the counters of the first of these launches the matrix cores are busy for 49% of it (at
 // 1.85 GHz) and the vector ALU for 38%, and a wave stands ready for another instruction to end for 39% of its cycles and
@@ -290,7 +299,8 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     };
     // A wave looks at the last 64 keys of its last 8 queries with the first requests; if none of them is seen, at the rows of all its
     // queries, 256 keys at a time from the end on, until it meets a visible key: what lies behind is not walked.  Requests stay
-    // inside the rows by moving the last ones back: at worst a block is kept because the one before it is seen.
+    // inside the rows by moving the last ones back: at worst a block is kept because the one before it is seen.  The first 64 keys
+    // of its first 8 queries tell it likewise whether to look for the first key that one of them sees (`first_tile`, below).
     typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
     const int n_tiles = (n_keys + 63) / 64;
     auto mask_keys = [&](int r, int key) __attribute__((always_inline)) {
@@ -299,21 +309,30 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     auto any_seen = [&](const u32x4_a2 & w) __attribute__((always_inline)) {                   // (0xFC00: a masked-out key)
         return (w[0] ^ 0xFC00FC00u) | (w[1] ^ 0xFC00FC00u) | (w[2] ^ 0xFC00FC00u) | (w[3] ^ 0xFC00FC00u);
     };
-    u32x4_a2 end_keys = {0u, 0u, 0u, 0u};
-    if constexpr (MASK != 0) {
-        end_keys = mask_keys(24 + (lane >> 3), (n_tiles - 1) * 64 + (lane & 7) * 8);
-        request_mask(0);
-        request_mask(1);
-    }
-#pragma unroll
-    for (int j = 0; j < DK; j++) {
-        if constexpr (HALVES) {
-            if (!ofv || j >= DK - DV) request(kst, nb1k, kch, ofv ? VRING + (j - (DK - DV)) * STEPB : j * STEPB);
-        } else {
-            request(kst, nb1k, kch, j * STEPB);
-            if (j >= DK - DV) request(vst, nb1v, vch, VRING + (j - (DK - DV)) * STEPB);
+    u32x4_a2 end_keys = {0u, 0u, 0u, 0u}, first_keys = {0u, 0u, 0u, 0u};
+    // (the look at the first keys costs 0.4 us where they are visible; below 12 tiles that is what it could save: 640 tokens x 8 heads,
+    //  all visible 15.2 us without it and 15.6 with it, in four sequences 15.9 and 14.9)
+    const bool from_first = MASK && n_tiles >= 12;
+    auto first_requests = [&]() __attribute__((always_inline)) {
+        if constexpr (MASK != 0) {
+            request_mask(0);
+            request_mask(1);
         }
+#pragma unroll
+        for (int j = 0; j < DK; j++) {
+            if constexpr (HALVES) {
+                if (!ofv || j >= DK - DV) request(kst, nb1k, kch, ofv ? VRING + (j - (DK - DV)) * STEPB : j * STEPB);
+            } else {
+                request(kst, nb1k, kch, j * STEPB);
+                if (j >= DK - DV) request(vst, nb1v, vch, VRING + (j - (DK - DV)) * STEPB);
+            }
+        }
+    };
+    if constexpr (MASK != 0) {
+        end_keys   = mask_keys(24 + (lane >> 3), (n_tiles - 1) * 64 + (lane & 7) * 8);
+        if (from_first) first_keys = mask_keys(lane >> 3, (lane & 7) * 8);
     }
+    first_requests();
 
     half8 qreg[NQB][KS];                       // f16 B operands in log2 units
 #pragma unroll
@@ -329,26 +348,45 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     // (in the slot of V's that the first region asks for; read behind the barrier below)
     int * const ends = (int *)(lds + VRING + (R - 2) * STEPB);
     if constexpr (MASK != 0) {
-        int nt = n_tiles;
+        // which of the 32 runs of 8 keys from tile `lo` on some query of the wave sees
+        auto runs_seen = [&](int lo) __attribute__((always_inline)) {
+            u32x4_a2 w[16 / KSP];                                 // (the two waves of a pair share the rows)
+            uint32_t any = 0;
+#pragma unroll
+            for (int i = 0; i < 16 / KSP; i++) w[i] = mask_keys(kgroup * 16 + i * 2 + (lane >> 5), lo * 64 + (lane & 31) * 8);
+#pragma unroll
+            for (int i = 0; i < 16 / KSP; i++) any |= any_seen(w[i]);
+            const uint64_t v = __builtin_amdgcn_ballot_w64(any != 0);
+            return (uint32_t)v | (uint32_t)(v >> 32);
+        };
+        int nt = n_tiles, ft = 0;
         if (__builtin_amdgcn_ballot_w64(any_seen(end_keys) != 0) == 0) {
             nt = 1;
+#pragma unroll 1
             for (int hi = n_tiles; hi > 0; hi -= 4) {
-                const int lo = max(hi - 4, 0);
-                u32x4_a2  w[16 / KSP];                            // (the two waves of a pair share the rows)
-                uint32_t  any = 0;
-#pragma unroll
-                for (int i = 0; i < 16 / KSP; i++) w[i] = mask_keys(kgroup * 16 + i * 2 + (lane >> 5), lo * 64 + (lane & 31) * 8);
-#pragma unroll
-                for (int i = 0; i < 16 / KSP; i++) any |= any_seen(w[i]);
-                const uint64_t v2 = __builtin_amdgcn_ballot_w64(any != 0);
-                const uint32_t v  = (uint32_t)v2 | (uint32_t)(v2 >> 32);
+                const int      lo = max(hi - 4, 0);
+                const uint32_t v  = runs_seen(lo);
                 if (v) {
                     nt = min(hi, lo + (31 - __builtin_clz(v)) / 8 + 1);
                     break;
                 }
             }
         }
-        if (lane == 0) ends[wave] = nt;
+        if (from_first && __builtin_amdgcn_ballot_w64(any_seen(first_keys) != 0) == 0) {
+            ft = nt;
+#pragma unroll 1
+            for (int lo = 0; lo < nt; lo += 4) {
+                const uint32_t v = runs_seen(lo);
+                if (v) {
+                    ft = lo + __builtin_ctz(v) / 8;
+                    break;
+                }
+            }
+        }
+        if (lane == 0) {
+            ends[wave]     = nt;
+            ends[W + wave] = ft;
+        }
     }
 
     float16v oacc[NQB][DB], negm[SPLAT ? NQB : 1], s[2];
@@ -404,9 +442,30 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
         for (int i = 0; i < STEPB / 16 / PIPE_THREADS; i++) *(float4 *)(lds + VRING + (R - 1) * STEPB + (i * PIPE_THREADS + tid) * 16) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
     // the first two blocks of K have landed
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(HALVES ? (DK - 2) * NLD : (DK - 2 + DV) * NLD) : "memory");
-    __builtin_amdgcn_s_barrier();
-    if constexpr (MASK != 0) n_steps = min(n_steps, max(max(ends[0], ends[1]), max(ends[2], ends[3])) * 64 / SKEYS);
+    auto first_landed = [&]() __attribute__((always_inline)) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(HALVES ? (DK - 2) * NLD : (DK - 2 + DV) * NLD) : "memory");
+        __builtin_amdgcn_s_barrier();
+    };
+    first_landed();
+    int step = 0;
+    if constexpr (MASK != 0) {
+        n_steps = min(n_steps, max(max(ends[0], ends[1]), max(ends[2], ends[3])) * 64 / SKEYS);
+        // Keys that no query of the workgroup sees before the first one (windows, padding on the left, several sequences in a row):
+        // the requests start again behind them, where that leaves out four tiles or more (2.6 us for 1.5).
+        const int first_tile = __builtin_amdgcn_readfirstlane(min(min(ends[W], ends[W + 1]), min(ends[W + 2], ends[W + 3])));
+        if (first_tile >= 4 && first_tile * 64 / SKEYS < n_steps) {
+            step = first_tile * 64 / SKEYS;
+            // every wave has read `ends`, and nothing is on its way into the slots
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            const int key = min(first_tile * 64 + 32 * kgroup, n_keys - 32), left = n_keys - 32 - key;
+            kst = {kbase + (int64_t)key * a.nbk1, left};
+            vst = {vbase + (int64_t)key * a.nbv1, left};
+            mst = {(uint64_t)plane + (uint64_t)((int64_t)(k_begin + key) * 2), left};
+            first_requests();
+            first_landed();
+        }
+    }
     auto exclude_past_end = [&](float16v & x, int step) __attribute__((always_inline)) {
         int lim = n_keys - step * SKEYS - kgroup * 32 - hh * 4;
         asm volatile("" : "+v"(lim));            // (nothing of this is worth a register in the loop)
@@ -425,14 +484,15 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
 #pragma unroll
             for (int ks = 0; ks < KS; ks++) s[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ks < 4 ? ka[ks & 3] : k1[ks & 3], qreg[qb][ks], s[0], 0, 0, 0);
             float16v first = s[0];
-            if constexpr (MASK != 0)  add_mask(first, 0, kgroup);       // (its own turn comes with the first region)
+            if constexpr (MASK != 0)  add_mask(first, 0, KSP * step + kgroup);       // (its own turn comes with the first region)
             else if (n_keys < SKEYS) { exclude_past_end(s[0], 0); first = s[0]; }
             float mx = first[0];
 #pragma unroll
             for (int r = 1; r < 16; r++) mx = fmaxf(mx, first[r]);
             mx = max_of_halves(mx);
-            // (masked rows that see nothing yet stand on -inf: their exponentials are NaN, and the rare path below takes over)
-            m[qb] = MASK || mx > -INFINITY ? mx : 0.0f;
+            // (masked rows that see nothing yet stand below every score: the exponentials of hidden keys are zeros, and the first key
+            //  that such a row sees leaves f16's range, so that the rare path below gives it a reference)
+            m[qb] = mx > -INFINITY ? mx : MASK ? -3.0e38f : 0.0f;
             if (SPLAT) {
 #pragma unroll
                 for (int r = 0; r < 16; r++) negm[SPLAT ? qb : 0][r] = -m[qb];
@@ -445,8 +505,7 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
         if (NQB == 1) read_k(ka, STEPB, 0);      // (of a single step: what the slot holds, multiplied and not used)
     }
 
-    int      step = 0;
-    uint32_t cur  = 0;                                            // slot of the current step
+    uint32_t cur = 0;                                             // slot of the current step
 
     // One unit: the softmax of s[U] (query block QB), with the scores of the next unit into s[1 - U] and V^T.P^T of the one
     // before on the matrix cores.
@@ -525,7 +584,6 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
                 base  = fmaxf(max_of_halves(mx), m[QB]);
                 f     = base == m[QB] ? 1.0f : __builtin_amdgcn_exp2f(m[QB] - base);
                 m[QB] = base;
-                if (base == -INFINITY) base = 0.0f;                // (no key seen: exponentials of -inf)
             } else {
                 delta = fmaxf(max_of_halves(mx) - (SPLAT ? 0.0f : m[QB]), 0.0f);
                 f     = __builtin_amdgcn_exp2f(-delta);
@@ -534,10 +592,12 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
             }
 #pragma unroll
             for (int r = 0; r < 4; r++) lacc[QB][r] = lprev * f;
+            if (!MASK || __builtin_amdgcn_ballot_w64(lprev != 0.0f && f != 1.0f) != 0) {       // (not where rows see their first keys)
 #pragma unroll
-            for (int db = 0; db < DB; db++)
+                for (int db = 0; db < DB; db++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) oacc[QB][db][r] *= f;
+                    for (int r = 0; r < 16; r++) oacc[QB][db][r] *= f;
+            }
             if (SPLAT) {
 #pragma unroll
                 for (int r = 0; r < 16; r++) negm[SPLAT ? QB : 0][r] -= delta;
