@@ -103,7 +103,8 @@ struct Scratch {
 };
 Scratch g_scratch[64];
 
-int get_scratch(size_t bytes, void ** out, hipStream_t st) {
+// room: the caller can do with less while the block may not grow - what it holds instead of a refusal
+int get_scratch(size_t bytes, void ** out, hipStream_t st, size_t * room = nullptr) {
     int dev = 0;
     HIP_TRY(hipGetDevice(&dev));
     if (dev < 0 || dev >= 64) return fail(MI355X_ERR_HIP, "device index %d out of range", dev);
@@ -113,7 +114,11 @@ int get_scratch(size_t bytes, void ** out, hipStream_t st) {
         // growing means hipMalloc: not while the stream is being recorded into a graph
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(st, &cs) != hipSuccess) (void)hipGetLastError();
-        else if (cs != hipStreamCaptureStatusNone)
+        else if (cs != hipStreamCaptureStatusNone && room && s.ptr) {
+            *out  = s.ptr;
+            *room = s.size;
+            return MI355X_OK;
+        } else if (cs != hipStreamCaptureStatusNone)
             return fail(MI355X_ERR_WORKSPACE, "this call needs %zu bytes of workspace and the library holds %zu: pass one, or make the call "
                         "once before capturing", bytes, s.size);
         size_t want = s.size ? s.size : (size_t)(8u << 20);
@@ -124,6 +129,7 @@ int get_scratch(size_t bytes, void ** out, hipStream_t st) {
         s.size = want;
     }
     *out = s.ptr;
+    if (room) *room = s.size;
     return MI355X_OK;
 }
 
@@ -474,21 +480,45 @@ void use_f16_copies(FattnArgs & a, void * ws) {
 // those are stays as it is, also where the pricing below would cut them (it counts the merge at the 1 us and more a range that
 // it once took).  Price, in us: the longer of the cache's pass through HBM and a wave's chain of 32-key steps - four of them 0.7
 // on 64-wide heads, 1.3 on wider ones, more where workgroups share a CU - and the merge.
-bool decode_is_cut(const FattnArgs & a, int ktype, int vtype, int64_t groups, int most) {
-    const double rows  = (double)(a.Nq * a.gqa < 16 ? a.Nq * a.gqa : 16);
-    const double bytes = (double)a.Hkv * a.B * a.Nkv *
-                         (double)(a.D / block_size(ktype) * type_size(ktype) + a.D / block_size(vtype) * type_size(vtype));
-    const double t_hbm = bytes > 8.0e6 ? (bytes - 8.0e6) / 5.0e6 : 0.0;      // (the first megabytes are a matter of latency, which the chain prices)
-    auto price = [&](int n, int keys) {
+struct DecodeCut {
+    const FattnArgs & a;
+    int64_t groups;
+    double  rows, t_hbm;
+    DecodeCut(const FattnArgs & a_, int ktype, int vtype, int64_t groups_) : a(a_), groups(groups_) {
+        rows = (double)(a.Nq * a.gqa < 16 ? a.Nq * a.gqa : 16);
+        const double bytes = (double)a.Hkv * a.B * a.Nkv *
+                             (double)(a.D / block_size(ktype) * type_size(ktype) + a.D / block_size(vtype) * type_size(vtype));
+        t_hbm = bytes > 8.0e6 ? (bytes - 8.0e6) / 5.0e6 : 0.0;      // (the first megabytes are a matter of latency, which the chain prices)
+    }
+    // 0: not a count that whole steps give
+    int keys(int n) const {
+        const int k = ((a.Nkv + n - 1) / n + 31) / 32 * 32;
+        return (a.Nkv + k - 1) / k == n ? k : 0;
+    }
+    double price(int n, int keys) const {
         const double per_cu = (double)groups * n / a.n_cus, chain = (keys > 128 ? keys / 128.0 : 1.0) * (a.D <= 64 ? 0.7 : 1.3) * (per_cu > 1.0 ? per_cu : 1.0);
         return (chain > t_hbm ? chain : t_hbm) + (n > 1 ? 1.0 + n * (0.25 + 0.017 * rows) : 0.0);
-    };
-    const double limit = price(1, (a.Nkv + 31) / 32 * 32) * 1.10;
-    for (int n = 2; n <= most && n <= 256; n++) {
-        const int keys = ((a.Nkv + n - 1) / n + 31) / 32 * 32;
-        if ((a.Nkv + keys - 1) / keys == n && price(n, keys) <= limit) return true;
     }
-    return false;
+    bool cut(int most) const {
+        const double limit = price(1, keys(1)) * 1.10;
+        for (int n = 2; n <= most && n <= 256; n++)
+            if (keys(n) && price(n, keys(n)) <= limit) return true;
+        return false;
+    }
+    // the largest count within a tenth of the least price: as many ranges as a caller's workspace has to hold (fit_plan)
+    int fewest(int most) const {
+        if (most > 256) most = 256;
+        double least = price(1, keys(1));
+        for (int n = 2; n <= most; n++)
+            if (keys(n) && price(n, keys(n)) < least) least = price(n, keys(n));
+        while (most > 1 && !(keys(most) && price(most, keys(most)) <= least * 1.10)) most--;
+        return most;
+    }
+};
+// two workgroups a CU, ranges of 128 or 64 keys: no more than that are weighed
+int decode_most(const FattnArgs & a, int64_t groups) {
+    const int64_t by_cus = (int64_t)a.n_cus * 2 / (groups > 0 ? groups : 1), min_keys = a.D <= 64 ? 128 : 64, by_keys = (a.Nkv + min_keys / 2) / min_keys;
+    return (int)(by_cus < by_keys ? by_cus : by_keys);
 }
 
 // Into how many ranges: the count of least price.  In us: the longest of
@@ -689,33 +719,26 @@ void make_plan_core(const FattnArgs & a0, int ktype, int vtype, const mi355x_fat
         const int64_t rows = (int64_t)a.Nq * a.Hq * a.B;
         // workgroups that exist before splitting, and the fewest keys worth a split
         const int64_t groups   = kernel == MI355X_FATTN_VEC ? rows : (int64_t)a.Hkv * a.B * a.q_chunks;
-        // decode kernel: the bounds within which a cut is weighed at all
         // vector kernel (one workgroup per row and range; sweep of 1 and 2 queries x 8 .. 128 heads x sequences against 224 ..
         // 4096 F32 keys, twelve forced counts each, also with K/V that no cache holds): 1.5 workgroups per CU in all, a power
         // of two per row; ranges of at least 128 keys, for heads wider than 64 of 56 keys up to 448 keys and 112 beyond;
         // at most 8 ranges (16 from 4096 keys on: every range costs its row's merge 0.5 us)
         // (32 heads of 128 against 4096 keys: 29.0 us in 32 ranges, 21.9 in 16; 2 x 128 rows against 1024 keys: 32.8 us in 4, 29.5 in 2)
-        const int     min_keys = kernel == MI355X_FATTN_VEC ? (a.D > 64 ? (a.Nkv > 448 ? 112 : 56) : 128) : (a.D <= 64 ? 128 : 64);
         int ns = p->n_splits;
-        if (ns <= 0) {
-            const int64_t target = kernel == MI355X_FATTN_VEC ? (int64_t)a.n_cus * 3 / 2 : (int64_t)a.n_cus * 2;
-            // whole splits only while they still fit the target: past it a split doubles the grid and adds the merge
-            ns = kernel == MI355X_FATTN_VEC ? (int)((target + groups - 1) / (groups > 0 ? groups : 1))
-                                            : (int)(target / (groups > 0 ? groups : 1));
-            const int max_by_keys = kernel == MI355X_FATTN_VEC ? (a.Nkv < 2 * min_keys ? 1 : (a.Nkv + min_keys - 1) / min_keys)
-                                                               : (a.Nkv + min_keys / 2) / min_keys;
-            if (ns > max_by_keys) ns = max_by_keys;
-            if (kernel == MI355X_FATTN_VEC) {
-                // the workgroup budget rounds down to a power of two
-                int by_wgs = 1;
-                const int64_t streams = groups / a.gqa > 0 ? groups / a.gqa : 1;      // the rows of a GQA group read the same keys
-                while (by_wgs * 2 <= (int)((target + streams - 1) / streams)) by_wgs *= 2;
-                ns = by_wgs < max_by_keys ? by_wgs : max_by_keys;
-                const int cap = a.Nkv >= 4096 ? 16 : 8;
-                if (ns > cap) ns = cap;
-            }
-            if (kernel == MI355X_FATTN_DECODE_MMA && ns > 1)
-                ns = decode_is_cut(a, ktype, vtype, groups, ns) ? decode_ranges(a, ktype, groups, plan.workspace) : 1;
+        if (ns <= 0 && kernel == MI355X_FATTN_VEC) {
+            const int     min_keys    = a.D > 64 ? (a.Nkv > 448 ? 112 : 56) : 128;
+            const int64_t target      = (int64_t)a.n_cus * 3 / 2;
+            const int     max_by_keys = a.Nkv < 2 * min_keys ? 1 : (a.Nkv + min_keys - 1) / min_keys;
+            // the workgroup budget rounds down to a power of two
+            int by_wgs = 1;
+            const int64_t streams = groups / a.gqa > 0 ? groups / a.gqa : 1;      // the rows of a GQA group read the same keys
+            while (by_wgs * 2 <= (int)((target + streams - 1) / streams)) by_wgs *= 2;
+            ns = by_wgs < max_by_keys ? by_wgs : max_by_keys;
+            const int cap = a.Nkv >= 4096 ? 16 : 8;
+            if (ns > cap) ns = cap;
+        } else if (ns <= 0) {
+            const int most = decode_most(a, groups);
+            ns = most > 1 && DecodeCut(a, ktype, vtype, groups).cut(most) ? decode_ranges(a, ktype, groups, plan.workspace) : 1;
         }
         if (ns > a.Nkv) ns = a.Nkv;
         if (ns < 1) ns = 1;
@@ -731,6 +754,23 @@ void make_plan_core(const FattnArgs & a0, int ktype, int vtype, const mi355x_fat
         //  4 GiB of the first one's - with 128-wide heads, 16384 heads in 128 ranges are too many)
         if (ns > 1 && groups <= MERGE_COUNTERS && (int64_t)a.Hq * ns * a.D * 16 < 0xFFF00000LL) plan.merge_sets = groups;
     }
+}
+
+// A plan that has to do with `room` bytes: a decode call that AUTO cut takes as many ranges as its partials fit there, down to those
+// that the price of whole steps and merges asks for (`fewest`, which was once the count itself: workspaces that programs sized by it
+// stay large enough).  plan.workspace stays what the call would use at best.  False: the call does not fit.
+bool fit_plan(FattnArgs a, int ktype, int vtype, const mi355x_fattn_params * p, size_t room, Plan & plan) {
+    if (plan.workspace <= room) return true;
+    if (plan.kernel != MI355X_FATTN_DECODE_MMA || p->n_splits > 0 || plan.n_splits < 2 || room < plan.ws_partials) return false;
+    if (a.D != plan.pad) apply_pad(a, plan);
+    if (plan.kv_to_f16) ktype = vtype = MI355X_TYPE_F16;
+    const int64_t groups = (int64_t)a.Hkv * a.B * a.q_chunks;
+    const size_t  part   = (size_t)a.Nq * a.Hq * a.B * (a.D + 2) * sizeof(float);
+    const size_t  n      = (room - plan.ws_partials) / part;                  // (below plan.n_splits)
+    if (n < (size_t)DecodeCut(a, ktype, vtype, groups).fewest(decode_most(a, groups))) return false;
+    plan.keys_per_split = ((a.Nkv + (int)n - 1) / (int)n + 31) / 32 * 32;
+    plan.n_splits       = (a.Nkv + plan.keys_per_split - 1) / plan.keys_per_split;
+    return true;
 }
 
 // Head sizes the MFMA kernels have no form for (multiples of 8 below 128 other than 64: 32 and 48, 80 and 96 of other
@@ -944,6 +984,7 @@ int mi355x_fattn_plan(const mi355x_tensor * q, const mi355x_tensor * k, const mi
     fill_args(a, q, k, v, mask, nullptr, params);
     Plan plan;
     make_plan(a, k->type, v->type, params, plan);
+    if (params->workspace) fit_plan(a, k->type, v->type, params, params->workspace_size, plan);
     if (kernel) *kernel = plan.kernel;
     if (n_splits) *n_splits = plan.n_splits;
     return MI355X_OK;
@@ -959,6 +1000,7 @@ int mi355x_fattn_plan_details(const mi355x_tensor * q, const mi355x_tensor * k, 
     fill_args(a, q, k, v, mask, nullptr, params);
     Plan plan;
     make_plan(a, k->type, v->type, params, plan);
+    if (params->workspace) fit_plan(a, k->type, v->type, params, params->workspace_size, plan);
     memset(info, 0, sizeof(*info));
     info->kernel         = plan.kernel;
     info->n_splits       = plan.n_splits;
@@ -1003,6 +1045,16 @@ int mi355x_fattn_workspace_size(const mi355x_tensor * q, const mi355x_tensor * k
     return MI355X_OK;
 }
 
+// whether the call proper (no q_quant) can be made with `room` bytes of workspace
+static bool call_fits(const mi355x_tensor * q, const mi355x_tensor * k, const mi355x_tensor * v, const mi355x_tensor * mask,
+                      const mi355x_fattn_params * params, size_t room) {
+    FattnArgs a;
+    fill_args(a, q, k, v, mask, nullptr, params);
+    Plan plan;
+    make_plan(a, k->type, v->type, params, plan);
+    return fit_plan(a, k->type, v->type, params, room, plan);
+}
+
 // counter_set: which of the library's counter sets a launch that merges its splits in the kernel may use (-1: none)
 static int flash_attn_run(const mi355x_tensor * q, const mi355x_tensor * k, const mi355x_tensor * v,
                           const mi355x_tensor * mask, const mi355x_tensor * dst,
@@ -1022,8 +1074,11 @@ static int flash_attn_run(const mi355x_tensor * q, const mi355x_tensor * k, cons
         if (rc) return rc;
         void * ws = params->workspace;
         if (ws) {
-            if (params->workspace_size < qb + need)
-                return fail(MI355X_ERR_WORKSPACE, "workspace %zu < %zu bytes", params->workspace_size, qb + need);
+            if (params->workspace_size < qb + need) {
+                if (params->workspace_size < qb || !call_fits(q, k, v, mask, &inner, params->workspace_size - qb))
+                    return fail(MI355X_ERR_WORKSPACE, "workspace %zu < %zu bytes", params->workspace_size, qb + need);
+                need = params->workspace_size - qb;
+            }
             if ((uintptr_t)ws % 16) return fail(MI355X_ERR_WORKSPACE, "workspace must be 16-byte aligned");
         } else {
             rc = get_scratch(qb + need, &ws, (hipStream_t)stream);
@@ -1075,7 +1130,7 @@ static int flash_attn_run(const mi355x_tensor * q, const mi355x_tensor * k, cons
     if (plan.workspace) {
         ws = params->workspace;
         if (ws) {
-            if (params->workspace_size < plan.workspace)
+            if (!fit_plan(a, k->type, v->type, params, params->workspace_size, plan))
                 return fail(MI355X_ERR_WORKSPACE, "workspace %zu < %zu bytes", params->workspace_size, plan.workspace);
             if ((uintptr_t)ws % 16) return fail(MI355X_ERR_WORKSPACE, "workspace must be 16-byte aligned");
         } else {
@@ -1488,14 +1543,16 @@ int mi355x_flash_attn_relpos(const mi355x_tensor * q_u, const mi355x_tensor * q_
         return relpos_fused_run(q_u, q_v, k, v, r, add, dst, params, f, ws, (hipStream_t)stream);
     }
     void * ws = params->workspace;
-    if (ws) {
-        if (params->workspace_size < mb + ib)
-            return fail(MI355X_ERR_WORKSPACE, "workspace %zu < %zu bytes", params->workspace_size, mb + ib);
-        if ((uintptr_t)ws % 16) return fail(MI355X_ERR_WORKSPACE, "workspace must be 16-byte aligned");
-    } else {
-        rc = get_scratch(mb + ib, &ws, (hipStream_t)stream);
+    size_t room = params->workspace_size;
+    if (!ws) {
+        rc = get_scratch(mb + ib, &ws, (hipStream_t)stream, &room);
         if (rc) return rc;
     }
+    if (room < mb + ib) {
+        if (room < mb || !call_fits(q_u, k, v, &m, params, room - mb)) return fail(MI355X_ERR_WORKSPACE, "workspace %zu < %zu bytes", room, mb + ib);
+        ib = room - mb;
+    }
+    if ((uintptr_t)ws % 16) return fail(MI355X_ERR_WORKSPACE, "workspace must be 16-byte aligned");
     m.data = ws;
     rc = relpos_run(q_v, r, add, &m, params->scale, (char *)ws + mb - relpos_table_bytes(r), (hipStream_t)stream);
     if (rc) return rc;

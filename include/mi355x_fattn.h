@@ -92,7 +92,11 @@ typedef struct mi355x_fattn_params {
                               * to finish a set of key ranges does it - where a call on a caller's workspace, which may overlap
                               * others, uses a second launch: same arithmetic, same bits.)
                               * Else 16-byte aligned.  With a caller's workspace of mi355x_fattn_workspace_size bytes the call allocates nothing
-                              * and launches kernels only (no memset or copy nodes): it may be recorded into a HIP graph. */
+                              * and launches kernels only (no memset or copy nodes): it may be recorded into a HIP graph.
+                              * The number is not monotonic in the keys (a longer cache may be cut into fewer ranges): a
+                              * workspace for a growing cache takes the largest one.  A decode call that AUTO cuts into more
+                              * ranges than the workspace holds takes as many as fit; one too small for the few it cannot do
+                              * without is refused with MI355X_ERR_WORKSPACE. */
     size_t  workspace_size;
     int32_t q_quant;         /* 0 = the query rows as they are.  MI355X_TYPE_Q8_0 = round every query row to Q8_0 blocks first
                               * (d = amax/127 per 32 values), which is what ggml-cpu is recalled to do when K is Q8_0 (the

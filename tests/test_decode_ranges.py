@@ -61,3 +61,35 @@ def test_uncut_calls_stay_uncut(seed):
         assert ns == 1 or need >= ns * part
         uncut += before == 1
     assert 50 < uncut < 250
+
+
+def _plan_in(room, ktype, hd, hq, hkv, B, nq, nkv):
+    """the ranges of the call on a caller's workspace of `room` bytes"""
+    p = ggml._params(0.1, 0.0, 0.0, 0, ggml.KERNEL_DECODE_MMA, 0, None)
+    p.workspace, p.workspace_size = 4096, room
+    q, k = _tensor(ggml.F32, (hd, nq, hq, B)), _tensor(TYPES[ktype][0], (hd, nkv, hkv, B))
+    info = ggml.CPlanInfo()
+    assert ggml.lib().mi355x_fattn_plan_details(ctypes.byref(q), ctypes.byref(k), ctypes.byref(k), None, ctypes.byref(p), ctypes.byref(info)) == ggml.OK
+    return info
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_workspaces_of_the_former_sizes_still_do(seed):
+    """a caller's workspace that holds the ranges a call was once cut into, and fewer than it is cut into now, takes as many as fit"""
+    r = random.Random(100 + seed)
+    held = 0
+    for _ in range(300):
+        hd, hq, hkv = r.choice([(128, 32, 8), (128, 16, 8), (64, 16, 16), (64, 32, 8), (64, 20, 20), (64, 6, 6)])
+        call = (r.choice(sorted(TYPES)), hd, hq, hkv, r.choice([1, 2, 8, 17, 40]), r.choice([1, 1, 5, 16]), int(2 ** r.uniform(8, 14)))
+        ns, need = _plan(*call, masked=False)
+        before, part = _was_cut(*call), call[2] * call[4] * call[5] * (hd + 2) * 4
+        for room in (before * part, before * part + part // 2, need - 1, need):
+            info = _plan_in(room, *call)
+            assert info.workspace == need
+            if ns == 1 or room >= need:
+                assert info.n_splits == ns, (call, room, info.n_splits, ns)
+            elif room >= before * part:
+                assert 2 <= info.n_splits < ns and info.n_splits * part <= room, (call, room, info.n_splits, ns)
+                assert info.n_splits * info.keys_per_split >= call[6] > (info.n_splits - 1) * info.keys_per_split and info.keys_per_split % 32 == 0
+                held += 1
+    assert held > 50
