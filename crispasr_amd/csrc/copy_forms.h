@@ -16,6 +16,7 @@ struct NarrowCopy {
     uint32_t     n;                        // units
     FastDiv      div[3];
     uint32_t     snb[3], dnb[3];           // pitches of counts 1 .. 3
+    uint32_t     whole;                    // see whole_pieces
     typedef uint32_t index, offset;
 };
 static_assert(sizeof(NarrowCopy) <= 112, "arguments of a cheap launch");
@@ -87,6 +88,16 @@ static Walk walk_of(const int64_t (&ne)[4], const int64_t (&nb)[4], int64_t unit
     return w;
 }
 
+// What the runs of a destination's units are whole pieces of, the end of a contiguous destination aside: 128-byte lines 2, 32-byte
+// sectors 1, neither 0.
+static int whole_pieces(const char * dst, const Walk & t, int64_t dstep) {
+    const int first = t.n && t.pitch[0] == dstep ? 1 : 0;          // (units that lie behind one another)
+    uint64_t  bits  = (uint64_t)(uintptr_t)dst;
+    if (t.n > first) bits |= (uint64_t)(first ? t.count[0] * dstep : dstep);
+    for (int i = first; i < t.n; i++) bits |= (uint64_t)t.pitch[i];
+    return bits % 128 == 0 ? 2 : bits % 32 == 0 ? 1 : 0;
+}
+
 // The narrow form, where there is one: the two sides cut into the same counts, the first of them units that are adjacent on both.
 static bool narrow_copy(const CpyArgs & a, int64_t unit0, int64_t sstep, int64_t dstep, int64_t threads, NarrowCopy & v) {
     if (threads + 256 >= ((int64_t)1 << 31)) return false;
@@ -110,6 +121,7 @@ static bool narrow_copy(const CpyArgs & a, int64_t unit0, int64_t sstep, int64_t
     v.dst    = a.dst;
     v.mirror = a.mirror;
     v.n      = (uint32_t)a.n;
+    v.whole  = (uint32_t)whole_pieces(a.dst, t, dstep);
     int64_t sspan = sstep, dspan = dstep;
     sp[0] = sstep;
     dp[0] = dstep;

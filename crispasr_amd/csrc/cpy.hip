@@ -75,16 +75,21 @@ template <typename T, typename I> __device__ __forceinline__ int64_t element_pit
 // both: F32 -> F16 rows of 128, 663 x 8 2.40 / 2.29 / 2.29, 2048 x 64 24.1 / 23.2 / 22.6; Q8_0 -> F32, 663 x 8 2.32 / 2.15 / 2.15, 2048 x 8
 // 3.84 / 3.88 / 2.78, 2048 x 64 17.9 / 17.7 / 11.4.  So dequantised reads, which outgrow the caches, are both; what the next
 // launch reads is written through only (six encoder layers whose K and V are copied to F16 first: 119 us plain, 118 written
-// through, 124 both).  Pieces of lines written through cost up to twice the plain stores: other kernels keep plain ones.
+// through, 124 both).  Pieces of lines written through cost up to twice the plain stores: other kernels keep plain ones, and so do
+// these where the destination's rows are not whole 32-byte sectors; non-temporal ones need whole 128-byte lines.  2048 x 64 rows into a
+// token-major destination, plain / written through / non-temporal as well: F16 rows of 48 bytes 3.8 / 4.6, of 80 6.7 / 7.7; F32 rows of 96
+// bytes 5.7 / 4.5, of 160 7.1 / 5.3, F16 rows of 128 at 192 7.15 / 5.6; Q8_0 -> F32 rows of 512 at 544 15.0 / 13.6 / 22.1, at 512 13.0 (all).
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 template <bool STREAM, typename T> __device__ __forceinline__ void store16(const NarrowCopy & a, uint32_t to, T x) {
-    // (a buffer store, because only its builtin takes the cache bits: 2 = non-temporal, 16 = write through)
+    // (buffer stores, because only their builtin takes the cache bits: 2 = non-temporal, 16 = write through)
     const auto r = __builtin_amdgcn_make_buffer_rsrc(a.dst, 0, -1, 0x00020000);
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), r, (int)to, 0, STREAM ? 18 : 16);
+    if (STREAM && a.whole == 2) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), r, (int)to, 0, 18);
+    else if (a.whole)           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), r, (int)to, 0, 16);
+    else                        *(T *)(a.dst + to) = x;
 }
 template <bool STREAM, typename I, typename T> __device__ __forceinline__ void store16(const WideCopy<I> & a, int64_t to, T x) {
-    if (STREAM) __builtin_nontemporal_store(x, (T *)(a.dst + to));
-    else        *(T *)(a.dst + to) = x;
+    if (STREAM && a.whole == 2) __builtin_nontemporal_store(x, (T *)(a.dst + to));
+    else                        *(T *)(a.dst + to) = x;
 }
 
 template <typename A, typename TS, typename TD>
@@ -571,8 +576,9 @@ static bool prepare_index(CpyArgs & a, int64_t unit0, int64_t threads) {
 }
 
 // a kernel of this file over `threads` lanes for units of `unit0` elements, a.n of them: in the narrow form where `narrow` filled
-// it in, else in the wide one, with 32-bit indices where they do.  walked: its 64-bit form goes on from the grid's end.
-#define FORM_LAUNCH(a, unit0, threads, walked, narrow, v, KERNEL, ...)                                                         \
+// it in, else in the wide one, with 32-bit indices where they do.  walked: its 64-bit form goes on from the grid's end.  pieces: of the
+// wide form, whole_pieces.
+#define FORM_LAUNCH(a, unit0, threads, walked, narrow, v, pieces, KERNEL, ...)                                                 \
     do {                                                                                                                  \
         const dim3 g_((unsigned)(((threads) + 255) / 256));                                                               \
         if (narrow) {                                                                                                     \
@@ -581,6 +587,7 @@ static bool prepare_index(CpyArgs & a, int64_t unit0, int64_t threads) {
         }                                                                                                                 \
         WideCopy<uint32_t> w_;                                                                                            \
         (CpyArgs &)w_ = a;                                                                                                \
+        w_.whole = (pieces);                                                                                              \
         if (prepare_index(w_, unit0, threads)) {                                                                          \
             hipLaunchKernelGGL((KERNEL<WideCopy<uint32_t>, __VA_ARGS__>), g_, dim3(256), 0, stream, w_);                  \
         } else {                                                                                                          \
@@ -595,13 +602,13 @@ static bool prepare_index(CpyArgs & a, int64_t unit0, int64_t threads) {
     do {                                                                                                                  \
         NarrowCopy v_;                                                                                                    \
         const bool n_ = (a).snb[0] == (int64_t)(es) && narrow_copy(a, unit0, sstep, dstep, threads, v_);                  \
-        FORM_LAUNCH(a, unit0, threads, walked, n_, v_, KERNEL, __VA_ARGS__);                                                      \
+        FORM_LAUNCH(a, unit0, threads, walked, n_, v_, whole_pieces((a).dst, walk_of((a).dne, (a).dnb, unit0, dstep), dstep), KERNEL, __VA_ARGS__); \
     } while (0)
 #define ROWS_LAUNCH(a, unit0, threads, ...)                                                                               \
     do {                                                                                                                  \
         NarrowRows v_;                                                                                                    \
         const bool n_ = narrow_rows(a, unit0, threads, v_);                                                               \
-        FORM_LAUNCH(a, unit0, threads, false, n_, v_, set_rows_kernel, __VA_ARGS__);                                             \
+        FORM_LAUNCH(a, unit0, threads, false, n_, v_, 0, set_rows_kernel, __VA_ARGS__);                               \
     } while (0)
 
 template <typename TS, typename TD>

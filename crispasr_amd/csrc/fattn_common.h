@@ -403,6 +403,7 @@ struct CpyArgs {
     int32_t same_shape;        // sne == dne (likewise)
     int64_t n;                 // elements (or blocks of 32 when a side is a block type)
     int64_t mirror;            // 0, or the distance in bytes from dst to a second copy that gets the same stores
+    int32_t whole;             // what the destination is whole pieces of: 128-byte lines 2, 32-byte sectors 1, else 0 (filled in by the launcher)
     // SET_ROWS only
     const char * idx;
     int32_t idx_is_i64;
