@@ -37,10 +37,10 @@
 // its K and V bytes, which the tile kernel, which skips the block's products, fetches as well.  A row that has seen nothing yet
 // stands on a reference below every score: while it stood on -inf its sums were NaN and the wave took the rare path in every step.
 // us a call, tile kernel / on -inf and from the first key on / as it is, 8 heads: 1000 causal tokens in a window of 256 21.4 / 24.4 /
-// 17.7, four sequences in 900 tokens 20.9 / 24.4 / 17.4, 768 tokens whose first half is hidden 19.1 / 19.1 / 14.7, 500 causal tokens x 4
-// padded on the left 16.9 / 18.2 / 16.6, 407 tokens in four sequences (odd rows) 15.55 / 17.3 / 15.6, the middle half of 2048 hidden
-// 45.5 / 32.5 / 32.9; 32 heads, 2048 tokens in a window of 256 77 / 66 / 42.  What it costs where no key is hidden: nothing
-// (2048 x 8 heads 35.0 -> 35.3, 1024 x 32 30.7 -> 31.1, 407 x 32 16.55 -> 16.15; these differ by 1% from run to run).
+// 17.7, four sequences in 900 tokens 20.9 / 24.4 / 16.7, 768 tokens whose first half is hidden 19.0 / 19.0 / 14.6, 500 causal tokens x 4
+// padded on the left 16.8 / 18.1 / 16.3, 407 tokens in four sequences (odd rows) 15.5 / 17.3 / 15.3, the middle half of 2048 hidden
+// 45.7 / 32.3 / 32.8; 32 heads, 1024 tokens in a window of 256 40.9 / 35.9 / 23.1.  Where no key is hidden ahead of the first: 2048 x 8
+// heads, all visible 34.3 -> 34.9 (runs differ by 2%), 1024 x 32 30.1 -> 30.0, causal 29.6 -> 28.6, 407 x 32 16.2 -> 15.75.
 // What is left above the MFMAs of a wave alone on its SIMD is instruction issue (about 5 cycles an instruction).  Where two
 // share a SIMD nothing is full: by the counters of the first of these launches the matrix cores are busy for 49% of it (at
 // 1.85 GHz) and the vector ALU for 38%, and a wave stands ready for another instruction to end for 39% of its cycles and
@@ -88,7 +88,7 @@ constexpr int pipe_lds_bytes(int D, int NQB, int KSP, int W, int MASK) {
 template <int D, int NQB, int KSP, int W, bool PAD, int MASK>
 __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a, const int n_qtiles) {
     static_assert(NQB == 1 || (NQB == 2 && D == 64 && KSP == 1 && !PAD), "forms");
-    static_assert(!MASK || (D == 128 && NQB == 1 && W == 4 && !PAD), "masked forms");
+    static_assert(!MASK || (D == 128 && NQB == 1 && W == 4 && !PAD), "masked forms");       // (none of them HALVES)
     constexpr int PIPE_THREADS = W * 64;
     constexpr int QG   = W / KSP;                                 // waves that take different queries
     constexpr int KS   = D / 16;                                  // reduction steps of Q.K^T
@@ -304,7 +304,7 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
     const int n_tiles = (n_keys + 63) / 64;
     auto mask_keys = [&](int r, int key) __attribute__((always_inline)) {
-        return *(const u32x4_a2 *)(plane + (int64_t)min(q0 + r, a.Nq - 1) * a.nbm1 + (int64_t)min(k_begin + key, k_end - 8) * 2);
+        return *(const u32x4_a2 *)(plane + (row_at(r) + (uint32_t)min(k_begin + key, k_end - 8) * 2));      // (below 2^32)
     };
     auto any_seen = [&](const u32x4_a2 & w) __attribute__((always_inline)) {                   // (0xFC00: a masked-out key)
         return (w[0] ^ 0xFC00FC00u) | (w[1] ^ 0xFC00FC00u) | (w[2] ^ 0xFC00FC00u) | (w[3] ^ 0xFC00FC00u);
@@ -313,26 +313,21 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     // (the look at the first keys costs 0.4 us where they are visible; below 12 tiles that is what it could save: 640 tokens x 8 heads,
     //  all visible 15.2 us without it and 15.6 with it, in four sequences 15.9 and 14.9)
     const bool from_first = MASK && n_tiles >= 12;
-    auto first_requests = [&]() __attribute__((always_inline)) {
-        if constexpr (MASK != 0) {
-            request_mask(0);
-            request_mask(1);
-        }
-#pragma unroll
-        for (int j = 0; j < DK; j++) {
-            if constexpr (HALVES) {
-                if (!ofv || j >= DK - DV) request(kst, nb1k, kch, ofv ? VRING + (j - (DK - DV)) * STEPB : j * STEPB);
-            } else {
-                request(kst, nb1k, kch, j * STEPB);
-                if (j >= DK - DV) request(vst, nb1v, vch, VRING + (j - (DK - DV)) * STEPB);
-            }
-        }
-    };
     if constexpr (MASK != 0) {
-        end_keys   = mask_keys(24 + (lane >> 3), (n_tiles - 1) * 64 + (lane & 7) * 8);
+        end_keys = mask_keys(24 + (lane >> 3), (n_tiles - 1) * 64 + (lane & 7) * 8);
         if (from_first) first_keys = mask_keys(lane >> 3, (lane & 7) * 8);
+        request_mask(0);
+        request_mask(1);
     }
-    first_requests();
+#pragma unroll
+    for (int j = 0; j < DK; j++) {
+        if constexpr (HALVES) {
+            if (!ofv || j >= DK - DV) request(kst, nb1k, kch, ofv ? VRING + (j - (DK - DV)) * STEPB : j * STEPB);
+        } else {
+            request(kst, nb1k, kch, j * STEPB);
+            if (j >= DK - DV) request(vst, nb1v, vch, VRING + (j - (DK - DV)) * STEPB);
+        }
+    }
 
     half8 qreg[NQB][KS];                       // f16 B operands in log2 units
 #pragma unroll
@@ -348,40 +343,36 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     // (in the slot of V's that the first region asks for; read behind the barrier below)
     int * const ends = (int *)(lds + VRING + (R - 2) * STEPB);
     if constexpr (MASK != 0) {
-        // which of the 32 runs of 8 keys from tile `lo` on some query of the wave sees
-        auto runs_seen = [&](int lo) __attribute__((always_inline)) {
-            u32x4_a2 w[16 / KSP];                                 // (the two waves of a pair share the rows)
-            uint32_t any = 0;
-#pragma unroll
-            for (int i = 0; i < 16 / KSP; i++) w[i] = mask_keys(kgroup * 16 + i * 2 + (lane >> 5), lo * 64 + (lane & 31) * 8);
-#pragma unroll
-            for (int i = 0; i < 16 / KSP; i++) any |= any_seen(w[i]);
-            const uint64_t v = __builtin_amdgcn_ballot_w64(any != 0);
-            return (uint32_t)v | (uint32_t)(v >> 32);
-        };
-        int nt = n_tiles, ft = 0;
-        if (__builtin_amdgcn_ballot_w64(any_seen(end_keys) != 0) == 0) {
-            nt = 1;
+        int  nt = n_tiles, ft = 0, at = 0;                       // at: tiles looked at from the end in question
+        bool last  = __builtin_amdgcn_ballot_w64(any_seen(end_keys) != 0) == 0;
+        bool first = from_first && __builtin_amdgcn_ballot_w64(any_seen(first_keys) != 0) == 0;
+        // (One loop for both ends, the last one first, in line: a launch behind other kernels fetches the code anew, and what lies out of
+        //  line costs a jump to it.  Four layers of 407 tokens with their row writes and conversions, the same inputs each pass: 91.0 us
+        //  with the look at the end alone, 94 with two loops or with this one out of line, 91.5 like this; five inputs in turn 100 and 96.)
+        if (last || first) {
 #pragma unroll 1
-            for (int hi = n_tiles; hi > 0; hi -= 4) {
-                const int      lo = max(hi - 4, 0);
-                const uint32_t v  = runs_seen(lo);
-                if (v) {
-                    nt = min(hi, lo + (31 - __builtin_clz(v)) / 8 + 1);
-                    break;
+            do {
+                const int hi = n_tiles - at, lo = last ? max(hi - 4, 0) : at;
+                u32x4_a2  w[16 / KSP];             // (the two waves of a pair share the rows)
+                uint32_t  any = 0;
+#pragma unroll
+                for (int i = 0; i < 16 / KSP; i++) w[i] = mask_keys(kgroup * 16 + i * 2 + (lane >> 5), lo * 64 + (lane & 31) * 8);
+#pragma unroll
+                for (int i = 0; i < 16 / KSP; i++) any |= any_seen(w[i]);
+                asm volatile("" : "+v"(any));      // (one word: else the compiler keeps 32 compares' results in scalar registers)
+                const uint64_t v2 = __builtin_amdgcn_ballot_w64(any != 0);
+                const uint32_t v  = (uint32_t)v2 | (uint32_t)(v2 >> 32);        // runs of 8 keys
+                if (v == 0 && (last ? hi > 4 : at + 4 < nt)) {
+                    at += 4;
+                } else if (last) {
+                    nt   = v ? min(hi, lo + (31 - __builtin_clz(v)) / 8 + 1) : 1;
+                    last = false;
+                    at   = 0;
+                } else {
+                    ft    = v ? lo + __builtin_ctz(v) / 8 : nt;
+                    first = false;
                 }
-            }
-        }
-        if (from_first && __builtin_amdgcn_ballot_w64(any_seen(first_keys) != 0) == 0) {
-            ft = nt;
-#pragma unroll 1
-            for (int lo = 0; lo < nt; lo += 4) {
-                const uint32_t v = runs_seen(lo);
-                if (v) {
-                    ft = lo + __builtin_ctz(v) / 8;
-                    break;
-                }
-            }
+            } while (last || first);
         }
         if (lane == 0) {
             ends[wave]     = nt;
@@ -447,22 +438,28 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
         __builtin_amdgcn_s_barrier();
     };
     first_landed();
-    int step = 0;
+    int first_step = 0;
     if constexpr (MASK != 0) {
         n_steps = min(n_steps, max(max(ends[0], ends[1]), max(ends[2], ends[3])) * 64 / SKEYS);
         // Keys that no query of the workgroup sees before the first one (windows, padding on the left, several sequences in a row):
         // the requests start again behind them, where that leaves out four tiles or more (2.6 us for 1.5).
         const int first_tile = __builtin_amdgcn_readfirstlane(min(min(ends[W], ends[W + 1]), min(ends[W + 2], ends[W + 3])));
         if (first_tile >= 4 && first_tile * 64 / SKEYS < n_steps) {
-            step = first_tile * 64 / SKEYS;
+            first_step = first_tile * 64 / SKEYS;
             // every wave has read `ends`, and nothing is on its way into the slots
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
-            const int key = min(first_tile * 64 + 32 * kgroup, n_keys - 32), left = n_keys - 32 - key;
-            kst = {kbase + (int64_t)key * a.nbk1, left};
-            vst = {vbase + (int64_t)key * a.nbv1, left};
-            mst = {(uint64_t)plane + (uint64_t)((int64_t)(k_begin + key) * 2), left};
-            first_requests();
+            const int left = max(n_keys - 32 - (first_tile * 64 + 32 * kgroup), 0);
+            kst = {kst.at + (int64_t)(kst.left - left) * nb1k, left};
+            vst = {vst.at + (int64_t)(vst.left - left) * nb1v, left};
+            mst = {mst.at + (int64_t)(mst.left - left) * 2, left};
+            request_mask(0);
+            request_mask(1);
+#pragma unroll
+            for (int j = 0; j < DK; j++) {
+                request(kst, nb1k, kch, j * STEPB);
+                if (j >= DK - DV) request(vst, nb1v, vch, VRING + (j - (DK - DV)) * STEPB);
+            }
             first_landed();
         }
     }
@@ -484,7 +481,7 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
 #pragma unroll
             for (int ks = 0; ks < KS; ks++) s[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ks < 4 ? ka[ks & 3] : k1[ks & 3], qreg[qb][ks], s[0], 0, 0, 0);
             float16v first = s[0];
-            if constexpr (MASK != 0)  add_mask(first, 0, KSP * step + kgroup);       // (its own turn comes with the first region)
+            if constexpr (MASK != 0)  add_mask(first, 0, KSP * first_step + kgroup);       // (its own turn comes with the first region)
             else if (n_keys < SKEYS) { exclude_past_end(s[0], 0); first = s[0]; }
             float mx = first[0];
 #pragma unroll
@@ -505,7 +502,8 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
         if (NQB == 1) read_k(ka, STEPB, 0);      // (of a single step: what the slot holds, multiplied and not used)
     }
 
-    uint32_t cur = 0;                                             // slot of the current step
+    int      step = first_step;
+    uint32_t cur  = 0;                                            // slot of the current step
 
     // One unit: the softmax of s[U] (query block QB), with the scores of the next unit into s[1 - U] and V^T.P^T of the one
     // before on the matrix cores.
