@@ -129,7 +129,8 @@ def bench_encoder(args, ca, ora, torch):
     except OSError:
         pass
     pd = ca.ggml.flash_attn_plan_details(layers[0]["q"], layers[0]["k"], layers[0]["v"], None, scale)
-    kname = (f"fattn_pipe_kernel<D={D}, query_blocks={pd['query_blocks']}, key_split={pd['key_split']}, F16, "
+    waves = ca.ggml.flash_attn_plan_form(layers[0]["q"], layers[0]["k"], layers[0]["v"], None, scale)["waves"]
+    kname = (f"fattn_pipe_kernel<D={D}, query_blocks={pd['query_blocks']}, key_split={pd['key_split']}, waves={waves}, F16, "
              f"direct={pd['direct']}>" if pd["kernel"] == ca.ggml.KERNEL_MMA else f"kernel {pd['kernel']}")
     res = {
         "value": value, "ms_per_step": ms_per_step,
@@ -138,7 +139,7 @@ def bench_encoder(args, ca, ora, torch):
                      "traffic_source": "profiles/fattn_pipe_whisper_encoders.txt: rocprofv3 FETCH_SIZE + WRITE_SIZE of this "
                                        "command in runs of their own, scaled by a plain copy; a constant of that profile, not "
                                        "measured by this run",
-                     "kernel": kname, "queries_per_workgroup": pd["queries_per_workgroup"], "n_splits": pd["n_splits"],
+                     "kernel": kname, "queries_per_workgroup": pd["queries_per_workgroup"] * waves // 4, "n_splits": pd["n_splits"],
                      "us_per_launch": kernel_ms * 1e3, "flops_per_launch": flops_layer},
         "parity": {"max_abs": max_abs, "rel_l2": rel, "ok": bool(parity_ok), "rows_checked": 50,
                    "oracle": "oracle/fattn_oracle.c exact mode"},

@@ -990,6 +990,41 @@ int mi355x_fattn_plan(const mi355x_tensor * q, const mi355x_tensor * k, const mi
     return MI355X_OK;
 }
 
+// the tile kernel's variant of a planned call, in the order of the call itself: the f16 copies first, then the question whether that
+// kernel takes the shape.  waves: a workgroup's in the pipelined kernel, or 0
+static bool tile_plan(FattnArgs a, int ktype, const Plan & plan, FattnMmaVariant & var, int & waves) {
+    if (plan.kernel != MI355X_FATTN_MMA) return false;
+    apply_pad(a, plan);
+    if (plan.kv_to_f16) {
+        use_f16_copies(a, nullptr);
+        ktype = MI355X_TYPE_F16;
+    }
+    if (!fattn_mma_supported(a, ktype)) return false;
+    a.n_splits = plan.n_splits;
+    a.keys_per_split = plan.keys_per_split;
+    fattn_mma_variant(a, ktype, var);
+    waves = fattn_pipe_waves(a, ktype, var);
+    return true;
+}
+
+int mi355x_fattn_plan_form(const mi355x_tensor * q, const mi355x_tensor * k, const mi355x_tensor * v,
+                           const mi355x_tensor * mask, const mi355x_fattn_params * params,
+                           int32_t * pipelined, int32_t * waves) {
+    if (!pipelined || !waves) return fail(MI355X_ERR_INVALID, "null argument");
+    const int rc = check(q, k, v, mask, nullptr, params);
+    if (rc) return rc;
+    FattnArgs a;
+    fill_args(a, q, k, v, mask, nullptr, params);
+    Plan plan;
+    make_plan(a, k->type, v->type, params, plan);
+    FattnMmaVariant var;
+    int        w    = 0;
+    const bool tile = tile_plan(a, k->type, plan, var, w);
+    *pipelined = w > 0 ? 1 : 0;
+    *waves     = tile ? (w > 0 ? w : 4) : 0;
+    return MI355X_OK;
+}
+
 int mi355x_fattn_plan_details(const mi355x_tensor * q, const mi355x_tensor * k, const mi355x_tensor * v,
                               const mi355x_tensor * mask, const mi355x_fattn_params * params,
                               mi355x_fattn_plan_info * info) {
@@ -1009,19 +1044,9 @@ int mi355x_fattn_plan_details(const mi355x_tensor * q, const mi355x_tensor * k, 
     info->workspace      = plan.workspace;
     info->head_pad       = plan.pad;
     info->merge_in_kernel = plan.merge_sets > 0 && !params->workspace && !g_no_fused_merge ? 1 : 0;
-    if (plan.kernel == MI355X_FATTN_MMA) {
-        // the order of the call itself: the f16 copies first, then the question whether the tile kernel takes the shape
-        int ktype = k->type;
-        apply_pad(a, plan);
-        if (plan.kv_to_f16) {
-            use_f16_copies(a, nullptr);
-            ktype = MI355X_TYPE_F16;
-        }
-        if (!fattn_mma_supported(a, ktype)) return MI355X_OK;
-        a.n_splits = plan.n_splits;
-        a.keys_per_split = plan.keys_per_split;
-        FattnMmaVariant var;
-        fattn_mma_variant(a, ktype, var);
+    FattnMmaVariant var;
+    int waves = 0;
+    if (tile_plan(a, k->type, plan, var, waves)) {
         info->queries_per_workgroup = var.queries_per_workgroup;
         info->query_blocks = var.query_blocks;
         info->key_split    = var.key_split;

@@ -443,17 +443,18 @@ struct FattnRelposArgs {
 int fattn_vec_launch(const FattnArgs & a, int ktype, hipStream_t stream);
 int fattn_merge_launch(const FattnArgs & a, hipStream_t stream);
 int fattn_mma_launch(const FattnArgs & a, int ktype, hipStream_t stream);
-int fattn_pipe_launch(const FattnArgs & a, int query_blocks, int key_split, hipStream_t stream);
-bool fattn_pipe_masked(const FattnArgs & a, int query_blocks, int key_split);
 // the instantiation of the tile kernel a call takes
 struct FattnMmaVariant {
     int  query_blocks;            // 32-query blocks per wave (1 or 2)
     int  key_split;               // 2: the waves of a workgroup pair up over the two halves of every key tile
-    int  queries_per_workgroup;
+    int  queries_per_workgroup;   // of four waves
     bool direct;                  // K/V tiles move global -> LDS without passing registers
     bool mask_dma;                // so does the mask
 };
 void fattn_mma_variant(const FattnArgs & a, int ktype, FattnMmaVariant & v);
+// waves of a workgroup of the pipelined kernel, which takes the variant's place, or 0: the tile kernel's (four)
+int fattn_pipe_waves(const FattnArgs & a, int ktype, const FattnMmaVariant & v);
+int fattn_pipe_launch(const FattnArgs & a, const FattnMmaVariant & v, int waves, hipStream_t stream);
 bool fattn_mma_supported(const FattnArgs & a, int ktype);
 int fattn_decode_launch(const FattnArgs & a, int ktype, hipStream_t stream);
 bool fattn_decode_supported(const FattnArgs & a, int ktype);

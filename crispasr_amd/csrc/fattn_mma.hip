@@ -1031,7 +1031,7 @@ int launch_type(const FattnArgs & a, const FattnMmaVariant & v, hipStream_t stre
 
 }  // namespace
 
-// Which instantiation a call takes (also what mi355x_fattn_plan_info reports):
+// Which instantiation a call takes (also what mi355x_fattn_plan_info reports; whether in the pipelined kernel: fattn_pipe_waves):
 //  - two query blocks per wave (256 queries per workgroup) halve the LDS operand traffic per MFMA; one block keeps
 //    more workgroups in flight when there are few queries;
 //  - the key-split form (64 queries per workgroup) when 128-query workgroups leave CUs empty or alone;
@@ -1090,13 +1090,8 @@ bool fattn_mma_supported(const FattnArgs & a, int ktype) {
 int fattn_mma_launch(const FattnArgs & a, int ktype, hipStream_t stream) {
     FattnMmaVariant v;
     fattn_mma_variant(a, ktype, v);
-    // Plain attention over f16 rows is the pipelined kernel's, but for the key-split form of 128-wide heads: there a wave has
-    // few blocks, and the longer prologue costs what the loop gains (300 tokens x 30 heads 10.8 against 11.9 us a launch, 500
-    // x 20 and 800 x 8 within 2%).
-    if (ktype == MI355X_TYPE_F16 && v.direct && !a.masked && a.softcap == 0.0f && !(a.D == 128 && v.key_split == 2))
-        return fattn_pipe_launch(a, v.query_blocks, v.key_split, stream);
-    if (ktype == MI355X_TYPE_F16 && v.direct && a.masked && fattn_pipe_masked(a, v.query_blocks, v.key_split))
-        return fattn_pipe_launch(a, v.query_blocks, v.key_split, stream);
+    const int waves = fattn_pipe_waves(a, ktype, v);
+    if (waves) return fattn_pipe_launch(a, v, waves, stream);
     switch (ktype) {
         case MI355X_TYPE_F16:  return launch_type<MI355X_TYPE_F16>(a, v, stream);
         case MI355X_TYPE_F32:  return launch_type<MI355X_TYPE_F32>(a, v, stream);

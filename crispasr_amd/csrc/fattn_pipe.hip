@@ -789,34 +789,42 @@ int launch(const FattnArgs & a, hipStream_t stream) {
 // Rows that start between dwords need LDS that two workgroups of the unsplit form do not have on one CU.  Shorter key ranges
 // stay with the tile kernel, whose prologue is shorter (128 causal tokens x 32 heads 14.0 us there with their row writes, 15.3 here;
 // 100 x 64 heads under per-head masks 10.2, 11.5; 300 x 16 12.9, 13.6; 400 x 16 15.7, 15.4).
-bool fattn_pipe_masked(const FattnArgs & a, int query_blocks, int key_split) {
-    return a.D == 128 && a.Dv == 128 && query_blocks == 1 && a.max_bias <= 0.0f && a.softcap == 0.0f &&
+static bool pipe_masked(const FattnArgs & a, const FattnMmaVariant & v) {
+    return a.D == 128 && a.Dv == 128 && v.query_blocks == 1 && a.max_bias <= 0.0f &&
            (a.n_splits > 1 ? a.keys_per_split : a.Nkv) >= 384 && (uint64_t)a.Nq * (uint64_t)a.nbm1 < (1ull << 31) &&
-           (key_split == 2 || (a.mask_al4 && !(a.Nkv & 1)));
+           (v.key_split == 2 || (a.mask_al4 && !(a.Nkv & 1)));
 }
 
-int fattn_pipe_launch(const FattnArgs & a, int query_blocks, int key_split, hipStream_t stream) {
+// Plain attention over f16 rows is this kernel's, but for the key-split form of 128-wide heads: there a wave has few blocks, and
+// the longer prologue costs what the loop gains (300 tokens x 30 heads 10.8 against 11.9 us a launch, 500 x 20 and 800 x 8 within 2%).
+// Eight waves a workgroup where that leaves no CU with more of them than workgroups of four do: more of those than CUs, and their
+// number per CU even once rounded up.  (A caller who names the form gets four.)
+int fattn_pipe_waves(const FattnArgs & a, int ktype, const FattnMmaVariant & v) {
+    if (ktype != MI355X_TYPE_F16 || !v.direct || a.softcap != 0.0f) return 0;
+    if (a.masked) return pipe_masked(a, v) ? 4 : 0;
+    if (v.key_split == 2) return a.D == 128 ? 0 : 4;
+    if (a.tile_variant != 0 || (a.D == 64 && v.query_blocks != 2)) return 4;
+    const int q4 = v.queries_per_workgroup;
+    auto groups  = [&](int q) { return (int64_t)((a.Nq + q - 1) / q) * a.Hq * a.B * a.n_splits; };
+    auto fill    = [&](int64_t wgs) { return (wgs + a.n_cus - 1) / a.n_cus; };
+    return groups(q4) > a.n_cus && 2 * fill(groups(2 * q4)) <= fill(groups(q4)) ? 8 : 4;
+}
+
+int fattn_pipe_launch(const FattnArgs & a, const FattnMmaVariant & v, int waves, hipStream_t stream) {
     const bool pad = a.Dv != a.D;
     if (a.masked) {
-        if (!fattn_pipe_masked(a, query_blocks, key_split)) return (int)hipErrorInvalidValue;
         const bool dwords = a.mask_al4 && !(a.Nkv & 1);
-        if (key_split == 2) return dwords ? launch<128, 1, 2, 4, false, 1>(a, stream) : launch<128, 1, 2, 4, false, 2>(a, stream);
+        if (v.key_split == 2) return dwords ? launch<128, 1, 2, 4, false, 1>(a, stream) : launch<128, 1, 2, 4, false, 2>(a, stream);
         return launch<128, 1, 1, 4, false, 1>(a, stream);
     }
-    // Eight waves a workgroup where that leaves no CU with more of them than workgroups of four do: more of those than CUs, and their
-    // number per CU even once rounded up.  (A caller who names the form gets four.)
-    auto groups = [&](int q) { return (int64_t)((a.Nq + q - 1) / q) * a.Hq * a.B * a.n_splits; };
-    auto fill   = [&](int64_t wgs) { return (wgs + a.n_cus - 1) / a.n_cus; };
-    auto eight  = [&](int q4) { return a.tile_variant == 0 && groups(q4) > a.n_cus && 2 * fill(groups(2 * q4)) <= fill(groups(q4)); };
-    if (query_blocks == 2) {
+    if (v.query_blocks == 2) {
         if (pad || a.D != 64) return (int)hipErrorInvalidValue;
-        return eight(256) ? launch<64, 2, 1, 8, false>(a, stream) : launch<64, 2, 1, 4, false>(a, stream);
+        return waves == 8 ? launch<64, 2, 1, 8, false>(a, stream) : launch<64, 2, 1, 4, false>(a, stream);
     }
     if (a.D == 64) {
-        if (key_split == 2) return pad ? launch<64, 1, 2, 4, true>(a, stream) : launch<64, 1, 2, 4, false>(a, stream);
+        if (v.key_split == 2) return pad ? launch<64, 1, 2, 4, true>(a, stream) : launch<64, 1, 2, 4, false>(a, stream);
         return pad ? launch<64, 1, 1, 4, true>(a, stream) : launch<64, 1, 1, 4, false>(a, stream);
     }
-    if (key_split == 2) return (int)hipErrorInvalidValue;         // (not a form of this kernel: see fattn_mma_launch)
-    if (eight(128)) return pad ? launch<128, 1, 1, 8, true>(a, stream) : launch<128, 1, 1, 8, false>(a, stream);
+    if (waves == 8) return pad ? launch<128, 1, 1, 8, true>(a, stream) : launch<128, 1, 1, 8, false>(a, stream);
     return pad ? launch<128, 1, 1, 4, true>(a, stream) : launch<128, 1, 1, 4, false>(a, stream);
 }

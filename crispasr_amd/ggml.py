@@ -90,7 +90,7 @@ class CDeviceInfo(ctypes.Structure):
 EXPORTS = [
     "mi355x_api_version", "mi355x_status_string", "mi355x_last_error",
     "mi355x_device_count", "mi355x_device_get_info", "mi355x_set_device", "mi355x_stream_synchronize",
-    "mi355x_fattn_supports", "mi355x_flash_attn_ext", "mi355x_flash_attn_ext_noalloc", "mi355x_fattn_workspace_size", "mi355x_fattn_plan", "mi355x_fattn_plan_details",
+    "mi355x_fattn_supports", "mi355x_flash_attn_ext", "mi355x_flash_attn_ext_noalloc", "mi355x_fattn_workspace_size", "mi355x_fattn_plan", "mi355x_fattn_plan_details", "mi355x_fattn_plan_form",
     "mi355x_relpos_bias_supports", "mi355x_relpos_bias", "mi355x_relpos_bias_workspace_size", "mi355x_flash_attn_relpos", "mi355x_fattn_relpos_workspace_size",
     "mi355x_cpy_supports", "mi355x_cpy", "mi355x_set_rows", "mi355x_set_rows_supports",
     "mi355x_buffer_alloc", "mi355x_buffer_free", "mi355x_host_buffer_alloc", "mi355x_host_buffer_free", "mi355x_host_buffer_mirror_stats", "mi355x_host_buffer_invalidate", "mi355x_buffer_memset", "mi355x_buffer_set",
@@ -123,6 +123,7 @@ def lib() -> ctypes.CDLL:
         L.mi355x_flash_attn_ext_noalloc.argtypes = [PT, PT, PT, PT, PT, PP, ctypes.c_void_p]
         L.mi355x_fattn_workspace_size.argtypes = [PT, PT, PT, PT, PP, ctypes.POINTER(ctypes.c_size_t)]
         L.mi355x_fattn_plan.argtypes = [PT, PT, PT, PT, PP, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)]
+        L.mi355x_fattn_plan_form.argtypes = [PT, PT, PT, PT, PP, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)]
         L.mi355x_fattn_plan_details.argtypes = [PT, PT, PT, PT, PP, ctypes.POINTER(CPlanInfo)]
         L.mi355x_relpos_bias_supports.argtypes = [PT, PT, PT, PT]
         L.mi355x_relpos_bias.argtypes = [PT, PT, PT, PT, ctypes.c_float, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
@@ -339,6 +340,17 @@ def flash_attn_plan_details(q: Tensor, k: Tensor, v: Tensor, mask: Optional[Tens
     _check(lib().mi355x_fattn_plan_details(q.ref(), k.ref(), v.ref(), mask.ref() if mask is not None else None,
                                            ctypes.byref(p), ctypes.byref(info)))
     return {f: getattr(info, f) for f, _ in CPlanInfo._fields_}
+
+
+def flash_attn_plan_form(q: Tensor, k: Tensor, v: Tensor, mask: Optional[Tensor] = None, scale: float = 1.0,
+                         max_bias: float = 0.0, logit_softcap: float = 0.0, kernel: int = KERNEL_AUTO,
+                         n_splits: int = 0, tile_variant: int = 0) -> dict:
+    """{"pipelined": whether the pipelined kernel takes the tile kernel's call, "waves": of a workgroup (0: not the tile kernel's)}"""
+    p = _params(scale, max_bias, logit_softcap, PREC_DEFAULT, kernel, n_splits, None, 0, tile_variant)
+    pipelined, waves = ctypes.c_int32(), ctypes.c_int32()
+    _check(lib().mi355x_fattn_plan_form(q.ref(), k.ref(), v.ref(), mask.ref() if mask is not None else None,
+                                        ctypes.byref(p), ctypes.byref(pipelined), ctypes.byref(waves)))
+    return {"pipelined": pipelined.value, "waves": waves.value}
 
 
 def flash_attn_workspace_size(q: Tensor, k: Tensor, v: Tensor, mask: Optional[Tensor] = None, scale: float = 1.0,

@@ -216,11 +216,11 @@ typedef struct mi355x_fattn_plan_info {
     int32_t kv_to_f16;               /* 1: F32 / quantised K and V are rounded to f16 copies in the workspace first */
     size_t  workspace;               /* bytes, as mi355x_fattn_workspace_size reports (without the q_quant part) */
     /* tile kernel only (0 otherwise) */
-    int32_t queries_per_workgroup;   /* 256, 128 or 64 */
+    int32_t queries_per_workgroup;   /* 256, 128 or 64, of four waves (a workgroup of eight takes twice as many: mi355x_fattn_plan_form) */
     int32_t query_blocks;            /* 32-query blocks per wave: 1 or 2 */
     int32_t key_split;               /* 2: the waves of a workgroup pair up over the two halves of every 64-key tile */
     int32_t direct;                  /* K/V tiles move global -> LDS without passing registers */
-    int32_t mask_dma;                /* the mask takes the same road */
+    int32_t mask_dma;                /* the mask takes the same road (of the tile-wise kernel; the pipelined one's always does) */
     int32_t merge_in_kernel;         /* 1: the split-KV partials are merged by the last workgroup to finish each set of ranges (no
                                       * merge launch): calls on the library's scratch (params->workspace == NULL); the
                                       * allocation-free entry point does the same for the same shapes */
@@ -231,6 +231,12 @@ typedef struct mi355x_fattn_plan_info {
 int mi355x_fattn_plan_details(const mi355x_tensor * q, const mi355x_tensor * k, const mi355x_tensor * v,
                               const mi355x_tensor * mask, const mi355x_fattn_params * params,
                               mi355x_fattn_plan_info * info);
+
+/* Which of the two kernels behind that plan runs, and its workgroups: pipelined 1 where the software-pipelined kernel takes the tile-wise
+ * one's place; waves 4 or 8, 0 where the plan is not the tile kernel's. */
+int mi355x_fattn_plan_form(const mi355x_tensor * q, const mi355x_tensor * k, const mi355x_tensor * v,
+                           const mi355x_tensor * mask, const mi355x_fattn_params * params,
+                           int32_t * pipelined, int32_t * waves);
 
 /* ---- FastConformer relative-position attention (src/core/fastconformer.h:876-935) ---------- */
 

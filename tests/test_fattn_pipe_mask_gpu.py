@@ -6,7 +6,7 @@ import pytest
 import oracle as ora
 from cases import make_case, to_f32
 from crispasr_amd import ggml
-from gpu_util import assert_parity, run_gpu, run_oracle
+from gpu_util import assert_parity, run_gpu, run_oracle, upload
 
 pytestmark = pytest.mark.gpu
 
@@ -20,10 +20,18 @@ def _masked(values, seed, **kw):
     return case
 
 
+def _is_pipelined(case, variant, ns=1):
+    """rows between dwords and odd key counts: the pairs' form alone"""
+    t = [upload(case[n]) for n in ("q", "k", "v", "mask")]
+    form = ggml.flash_attn_plan_form(*t, case["scale"], kernel=ggml.KERNEL_MMA, tile_variant=variant, n_splits=ns)
+    assert form == {"pipelined": int(variant == 0x21 or t[1].ne[1] % 2 == 0), "waves": 4}, form
+
+
 def _run(case, variant, what, ranges=(1,)):
     print("case", hex(variant), what, flush=True)
     ref = run_oracle(case)
     for ns in ranges:
+        _is_pipelined(case, variant, ns)
         assert_parity(run_gpu(case, kernel=ggml.KERNEL_MMA, tile_variant=variant, n_splits=ns), ref, "%s, %d ranges" % (what, ns))
 
 
@@ -101,3 +109,19 @@ def test_extreme_mask_values(variant, Nkv):
         print("case", hex(variant), name, Nkv, flush=True)
         out = run_gpu(case, kernel=ggml.KERNEL_MMA, tile_variant=variant, n_splits=1)
         assert np.isfinite(out).all() and np.abs(out - ref).max() <= 4 * 2.0 ** -6, (name, np.abs(out - ref).max())
+
+
+@pytest.mark.parametrize("variant", FORMS)
+@pytest.mark.parametrize("Nkv", [1921, 1922, 1925, 1951, 1952])
+def test_a_last_range_of_fewer_keys_than_a_block(variant, Nkv):
+    """six ranges of 384 keys, the sixth of 1, 2, 5, 31 and 32: its block begins in the range before, where the keys hold NaN bits and are excluded"""
+    Nq = 70
+    j, i = np.arange(Nkv), np.arange(Nq)[:, None]
+    hidden = (j >= 1880) & (j < 1920)
+    case = _masked(np.where(~hidden & (j >= i * 25) & ((j < 1920) | (i % 3 != 1)), 0.0, -np.inf)[None, None], 3900 + Nkv, Hq=4, Hkv=2)
+    ref = run_oracle(case)
+    for t in (case["k"], case["v"]):
+        t.buf[t.offset:].reshape(2, Nkv, -1)[:, hidden] = 0xFF
+    print("case", hex(variant), Nkv, "in six ranges", flush=True)
+    _is_pipelined(case, variant, 6)
+    assert_parity(run_gpu(case, kernel=ggml.KERNEL_MMA, tile_variant=variant, n_splits=6), ref)

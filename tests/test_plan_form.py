@@ -1,0 +1,34 @@
+"""Which kernel runs a tile kernel's call, and with how many waves a workgroup, planned without a GPU."""
+import pytest
+
+import crispasr_amd as ca
+from crispasr_amd import ggml
+
+
+def _t(type_, ne):
+    return ca.Tensor(None, type_, ne)
+
+
+def _form(D, Nq, Nkv, H, B=1, ktype=ggml.F16, mask=None, **kw):
+    q, k = _t(ggml.F32, (D, Nq, H, B)), _t(ktype, (D, Nkv, H, B))
+    kw.setdefault("kernel", ggml.KERNEL_MMA)
+    return tuple(ggml.flash_attn_plan_form(q, k, k, _t(ggml.F16, (Nkv, Nq, mask, 1)) if mask else None, 0.1, **kw).values())
+
+
+@pytest.mark.parametrize("D,Nq,B", [(64, 1500, 4), (64, 1000, 4), (128, 750, 4)])
+def test_eight_waves_where_they_fill_the_cus_as_evenly(D, Nq, B):
+    assert _form(D, Nq, Nq, 20, B) == (1, 8)
+    assert _form(D, Nq, Nq, 20, B, tile_variant=0x12 if D == 64 else 0x11) == (1, 4)      # (a form by name has four)
+    assert _form(D, Nq, Nq, 20, B, logit_softcap=30.0) == (0, 4)
+    assert _form(D, Nq, Nq, 10, 1) in ((1, 4), (0, 4))
+
+
+def test_masked_calls():
+    for Nkv, variant, pipelined in ((384, 0x11, 1), (383, 0x11, 0), (382, 0x11, 0), (384, 0x21, 1), (385, 0x21, 1), (385, 0x11, 0), (383, 0x21, 0)):
+        assert _form(128, 200, Nkv, 8, mask=1, tile_variant=variant) == (pipelined, 4), (Nkv, variant)
+    assert _form(128, 200, 1024, 8, mask=1, tile_variant=0x21, n_splits=2) == (1, 4)
+    assert _form(128, 200, 1024, 8, mask=1, tile_variant=0x21, n_splits=4) == (0, 4)       # (ranges of 256 keys)
+    assert _form(128, 200, 1024, 8, mask=1, max_bias=8.0) == (0, 4)
+    assert _form(64, 1500, 1500, 20, 4, mask=1) == (0, 4)
+    assert _form(64, 200, 1024, 8, ktype=ggml.F32) == (1, 4)                               # (on f16 copies)
+    assert _form(128, 1, 1024, 8, kernel=ggml.KERNEL_AUTO) == (0, 0)
