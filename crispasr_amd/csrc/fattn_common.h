@@ -182,6 +182,19 @@ static __device__ __forceinline__ void load_to_lds4(uint64_t base, uint32_t off,
     asm volatile("s_mov_b64 %0, %2\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %0" : "=&s"(q) : "v"(off), "s"(p), "s"(t) : "memory", "m0");
 }
 
+// Workgroups of a masked call differ in length (causal rows, padded sequences): an XCD's are ordered from the last query tile to the
+// first, and every second group of n_cus / 8 - the ones that join the group before on its CUs - backwards, so that a CU's two add
+// up to about the same.  In the tile-wise kernel, us a layer without it, without the turn and with it: 2048 causal tokens, 32 heads of
+// 128 89, 79 and 76; 16 heads of 64 56 and 51 (plain and with it).  For grids of whole heads an XCD (per = workgroups of one).
+static __device__ __forceinline__ void masked_order(int per, int n_qtiles, int n_cus, int & qt, int & pair) {
+    const int cus = n_cus >= 8 ? n_cus / 8 : 32, heads = per / n_qtiles;
+    int i = blockIdx.x / 8;
+    const int seg = i / cus * cus;
+    if ((i / cus) & 1) i = seg + min(cus, per - seg) - 1 - (i - seg);
+    qt   = n_qtiles - 1 - i / heads;
+    pair = (int)(blockIdx.x % 8) * heads + i % heads;
+}
+
 // lane l's and lane (l ^ 32)'s values, the lower lane's first, without the LDS crossbar (whose traffic would blur the waits of
 // a loop, and whose addresses cost registers)
 static __device__ __forceinline__ float2 both_halves(float x) {

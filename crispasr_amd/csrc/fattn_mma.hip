@@ -199,19 +199,7 @@ __global__ void __launch_bounds__(MMA_THREADS, 2) fattn_mma_kernel(const FattnAr
     const int k_begin = split * a.keys_per_split;
     const int k_end   = min(a.Nkv, k_begin + a.keys_per_split);
     int qt = bid % n_qtiles, pair = bid / n_qtiles;
-    if (MASK && a.n_splits == 1 && per * 8 == nb && per % n_qtiles == 0) {
-        // Workgroups of a masked call differ in length (causal rows, padded sequences).  An XCD's are ordered from the last
-        // query tile to the first, and every second group of n_cus / 8 - the ones that join the group before on its CUs -
-        // backwards, so that a CU's two add up to about the same (2048 causal tokens, 32 heads of 128, with what `trim`
-        // saves: 76 us a layer against 79 without the turn and 89 in the plain order; 16 heads of 64, which skip block by
-        // block instead: 56 -> 51).
-        const int cus = a.n_cus >= 8 ? a.n_cus / 8 : 32, heads = per / n_qtiles;
-        int i = blockIdx.x / 8;
-        const int seg = i / cus * cus;
-        if ((i / cus) & 1) i = seg + min(cus, per - seg) - 1 - (i - seg);
-        qt   = n_qtiles - 1 - i / heads;
-        pair = (int)(blockIdx.x % 8) * heads + i % heads;
-    }
+    if (MASK && a.n_splits == 1 && per * 8 == nb && per % n_qtiles == 0) masked_order(per, n_qtiles, a.n_cus, qt, pair);
     // (masked: the batch runs faster than the head, or the longest sequence of a padded batch would be one XCD's alone)
     const int h = MASK ? pair / a.B : pair % a.Hq;
     const int b = MASK ? pair % a.B : pair / a.Hq;

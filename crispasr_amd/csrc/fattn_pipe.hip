@@ -137,17 +137,7 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     const int k_begin = split * a.keys_per_split;
     const int k_end   = min(a.Nkv, k_begin + a.keys_per_split);
     int qt = bid % n_qtiles, pair = bid / n_qtiles;
-    if (MASK && a.n_splits == 1 && per * 8 == nb && per % n_qtiles == 0) {
-        // Masked workgroups differ in length (causal rows, padded sequences): an XCD's are ordered from the last query tile to the
-        // first, and every second group of n_cus / 8 - the ones that join the group before on its CUs - backwards, so that a CU's
-        // two add up to about the same.
-        const int cus = a.n_cus >= 8 ? a.n_cus / 8 : 32, heads = per / n_qtiles;
-        int i = blockIdx.x / 8;
-        const int seg = i / cus * cus;
-        if ((i / cus) & 1) i = seg + min(cus, per - seg) - 1 - (i - seg);
-        qt   = n_qtiles - 1 - i / heads;
-        pair = (int)(blockIdx.x % 8) * heads + i % heads;
-    }
+    if (MASK && a.n_splits == 1 && per * 8 == nb && per % n_qtiles == 0) masked_order(per, n_qtiles, a.n_cus, qt, pair);
     // (masked: the batch runs faster than the head, or the longest sequence of a padded batch would be one XCD's alone)
     const int h  = MASK ? pair / a.B : pair % a.Hq;
     const int b  = MASK ? pair % a.B : pair / a.Hq;
