@@ -250,7 +250,10 @@ constexpr uint32_t FATTN_NO_ADDRESS = 0xFFFFFFF0u;          // an offset behind 
 // up to 16 splits.  What counts beside that round trip is the number of requests: they take 16 bytes (two pairs, or four values)
 // and ask memory for nothing behind the last split.  Against batches of 8 in 8-byte requests, the next batch behind a branch
 // (for which the compiler waited as if for both), with the counters below, us a call inside a graph: 5 rows x 20 heads of 64,
-// 8 splits 7.83 -> 7.0; 8 heads of 128, 7 splits of Q8_0 7.8 -> 7.45, 13 splits of f16 9.9 -> 9.1, 16 of Q4_0 9.9 -> 8.8.
+// 8 splits 7.83 -> 7.0; 8 heads of 128, 7 splits of Q8_0 7.8 -> 7.45, 13 splits of f16 9.9 -> 9.1, 16 of Q4_0 9.9 -> 8.8.  More than 16 splits
+// are batches of 16 one after another, without the next one ahead: 8 heads of 128 against 8192 keys in 32 splits 15.2 -> 11.85, in 64 20.8 ->
+// 14.55.  In a launch of its own, whose requests past the end are not free, up to 8 that are left over are a batch of 8: the tile kernel's
+// 22 ranges of 64 x 4 heads 12.3 in batches of 8, 12.65 in two of 16, 12.2 like this; 32 ranges 12.75 -> 12.6, 64 16.5 -> 16.0.
 template <bool DEVICE>
 static __device__ __forceinline__ void fattn_merge_row(const FattnArgs & a, int64_t row, int d4) {
     typedef uint32_t u4 __attribute__((ext_vector_type(4)));
@@ -314,7 +317,10 @@ static __device__ __forceinline__ void fattn_merge_row(const FattnArgs & a, int6
     if (n <= 4)      fold(std::integral_constant<int, 4>{}, 0);
     else if (n <= 8) fold(std::integral_constant<int, 8>{}, 0);
     else
-        for (int s0 = 0; s0 < n; s0 += 16) fold(std::integral_constant<int, 16>{}, s0);
+        for (int s0 = 0; s0 < n; s0 += 16) {
+            if (!DEVICE && n - s0 <= 8) fold(std::integral_constant<int, 8>{}, s0);
+            else                        fold(std::integral_constant<int, 16>{}, s0);
+        }
     const float inv = L > 0.0f ? 1.0f / L : 0.0f;
     out.x *= inv; out.y *= inv; out.z *= inv; out.w *= inv;
     // (dst rows are Dv floats - the head size - also where the partial rows are those of a head zero-padded to D)

@@ -20,7 +20,7 @@ CASES = {
 }
 
 
-@pytest.mark.parametrize("ranges", [2, 4, 5, 8, 9, 16, 17, 33])
+@pytest.mark.parametrize("ranges", [2, 4, 5, 8, 9, 16, 17, 24, 25, 33])
 @pytest.mark.parametrize("name", sorted(CASES))
 def test_ranges_are_merged(name, ranges):
     case = make_case(**CASES[name])
