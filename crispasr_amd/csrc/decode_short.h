@@ -27,7 +27,6 @@ struct DecodeShort {
 };
 static_assert(sizeof(DecodeShort) <= 112, "see above");
 
-// false: the call needs the wide form
 // Sequences of different lengths in one call (a mask of every sequence's own ends each), more workgroups than CUs: a CU that gets the
 // workgroups of two long ones is the last.  Workgroup n_cus + i comes to the CU of workgroup i, so the sequences of the first round (a
 // workgroup on every CU) go in their own order, and those behind them by length (sequence_of_turn): the longest beside the shortest.
@@ -47,6 +46,7 @@ static inline uint32_t decode_turns(const FattnArgs & a, int row_bytes) {
     return (uint32_t)first;
 }
 
+// false: the call needs the wide form
 static inline bool decode_shorten(const FattnArgs & a, DecodeShort & p) {
     const int64_t nb[12] = {a.nbq1, a.nbq2, a.nbq3, a.nbk1, a.nbk2, a.nbk3, a.nbv1, a.nbv2, a.nbv3, a.nbm1, a.nbm2, a.nbm3};
     for (int i = 0; i < (a.mask ? 12 : 9); i++)

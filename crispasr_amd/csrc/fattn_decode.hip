@@ -31,7 +31,8 @@
 //
 // Masked calls walk the steps between the first and the last that one of their rows sees, and a step's mask values are
 // requested with its K and V: one step for 64 sequences of 500 to 4096 Q8_0 entries (32 query, 8 KV heads of 128) 115 -> 81 us,
-// 71 with the sequences paired by length on the CUs (sequence_of_turn), 4.5 TB/s over the entries seen; the bound is what a CU's port brings.
+// 71 with the sequences paired by length on the CUs (sequence_of_turn), 4.5 TB/s over the entries seen; the bound is what a CU's port
+// brings.  (Calls inside a graph.  By box and inputs 65 to 71 us, 4.5 to 4.9 TB/s.)
 #include "fattn_row.h"
 #include "decode_short.h"
 
@@ -928,6 +929,9 @@ fattn_decode_kernel(const FattnArgs a) {
     decode_body<D, TYPE, MASK, RAW, V8, PAD, false>(a, 0);
 }
 
+// (unmasked 64-wide f16 rows: 128 registers instead of 138, for four waves a SIMD.  That pays where workgroups share a CU and walk long
+//  ranges - 16 heads against 4000 keys, 8 sequences 28.1 -> 26.1 us, 16 of them 45.5 -> 44.5 - and costs 1 to 2% elsewhere, 5 rows x
+//  20 heads against 1500 keys 7.00 -> 7.07, 64 sequences of them 79.3 -> 80.8)
 template <int D, int TYPE, bool MASK, bool RAW, bool V8, bool PAD>
 __global__ void __launch_bounds__(DEC_THREADS)
 __attribute__((amdgpu_waves_per_eu((D == 64 && TYPE == MI355X_TYPE_F16 && !MASK ? 4 : decode_waves_min<D, TYPE, RAW>()), (decode_waves_max<D, RAW, V8>()))))

@@ -28,7 +28,7 @@
 // workgroup of four, changed nothing at 1500 keys (8 x 64 16.0 us either way) and lost 1 us below 1000.
 // Masked calls of 128-wide heads: a wave brings the mask of its next two blocks to LDS as it does K and V, so that the waits
 // go on counting, and adds it ahead of the exponentials; the last block is the last 32 keys of the range, whole.  Against the tile
-// kernel, whole calls: 2048 causal tokens behind 2048, 32 query and 8 KV heads, 162 -> 147 us (132 of them this kernel), 1000 causal
+// kernel, whole calls: 2048 causal tokens behind 2048, 32 query and 8 KV heads, with their row writes 146.8 -> 133.4 us, 1000 causal
 // tokens 42.5 -> 37.5, 407 (rows that start between dwords, the pairs' form) 21.4 -> 20.1; under per-head masks 750 x 8 heads x 8
 // 45.7 -> 38.8, 1000 x 8 x 4 38.1 -> 32.7, 751 x 8 22.0 -> 19.2.  The 407-token launch (16 us) is 4.5 us until the first scores, 0.65
 // a step - 32 KB through a CU's port - and 3 for the hand-over and the stores.
@@ -41,7 +41,8 @@
 // padded on the left 16.8 / 18.1 / 16.3, 407 tokens in four sequences (odd rows) 15.5 / 17.3 / 15.3, the middle half of 2048 hidden
 // 45.7 / 32.3 / 32.8; 32 heads, 1024 tokens in a window of 256 40.9 / 35.9 / 23.1.  Where no key is hidden ahead of the first: 2048 x 8
 // heads, all visible 34.3 -> 34.9 (runs differ by 2%), 1024 x 32 30.1 -> 30.0, causal 29.6 -> 28.6, 407 x 32 16.2 -> 15.75.
-// What is left above the MFMAs of a wave alone on its SIMD is instruction issue (about 5 cycles an instruction).  Where two
+// What is left above the MFMAs of a wave alone on its SIMD is not known: its instructions take about 5 cycles each, but a second wave
+// that takes half of them changed nothing (above).  Where two
 // share a SIMD nothing is full: by the counters of the first of these launches the matrix cores are busy for 49% of it (at
 // 1.85 GHz) and the vector ALU for 38%, and a wave stands ready for another instruction to end for 39% of its cycles and
 // waits at a counter or barrier for 21%.
@@ -241,7 +242,9 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     Stream mst = {MASK ? (uint64_t)plane + (uint64_t)((int64_t)(k_begin + key0) * 2) : 0, MASK ? n_keys - 32 - key0 : 0};
     auto request_mask = [&](int slot) __attribute__((always_inline)) {
         if constexpr (MASK != 0) {
-            // (rows that start between dwords: from the dword that holds their first key on, and the one that holds their last)
+            // (rows that start between dwords: from the dword that holds their first key on, and the one that holds their last.  Of a mask's
+            //  first and last row that can be the two bytes ahead of its first element or behind its last one, in the same dword, so in
+            //  mapped memory; they are shifted out.)
             const uint32_t odd = MASK == 2 ? (uint32_t)mst.at & 2 : 0;
 #pragma unroll
             for (int j = 0; j < 2; j++) load_to_lds16<(MASK != 0)>(mst.at - odd, MASK == 2 ? (moff[j] + odd) & ~3u : moff[j], m_lds + slot * MSLOT + j * 1024);

@@ -144,7 +144,8 @@ int mi355x_stream_synchronize(void * stream);
  *        (Q4_0 .. Q5_1: up to 16 query rows per KV head read the blocks in the decode kernel (head sizes 64 and 128, no
  *         soft cap; other shapes in the vector kernel); more rows go through one conversion of K and V to f16 in the
  *         workspace and the tile kernel)
- *   mask NULL, or F16 [>=Nkv, >=Nq, Hm, Bm], rows contiguous; head h reads h % Hm,
+ *   mask NULL, or F16 [>=Nkv, >=Nq, Hm, Bm], rows contiguous (read by dwords: of one that starts or ends between two of
+ *                    them, the two bytes beside it are fetched and not used); head h reads h % Hm,
  *        batch b reads b % Bm; -inf entries exclude the key
  *   Hq % Hkv == 0 (query head h reads KV head h / (Hq/Hkv)), B % Bk == 0.
  *   D: a multiple of 4 up to 256.  64 and 128 run on the MFMA kernels.  So do the other multiples of 8 below 128 (32, 48,
