@@ -243,6 +243,18 @@ static __device__ __forceinline__ __amdgpu_buffer_rsrc_t fattn_buffer(const void
 }
 constexpr uint32_t FATTN_NO_ADDRESS = 0xFFFFFFF0u;          // an offset behind every buffer's end
 
+// 16 bytes a lane from a buffer (fattn_buffer) to LDS address to + at + 16 * lane: `off` moves on by `inc` and is where they lie.  The add
+// stands between the write of m0 and the load that reads it, which have to be an instruction apart.  In asm for load_to_lds16's reason.
+static __device__ __forceinline__ void buffer_to_lds16(__amdgpu_buffer_rsrc_t buf, uint32_t & off, uint32_t inc, uint32_t to, uint32_t at) {
+    asm volatile("s_add_i32 m0, %3, %4\n\tv_add_u32 %0, %2, %0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
+                 : "+v"(off) : "s"(buf), "s"(inc), "s"(to), "s"(at) : "memory", "m0", "scc");
+}
+// the same with 4 bytes a lane
+static __device__ __forceinline__ void buffer_to_lds4(__amdgpu_buffer_rsrc_t buf, uint32_t & off, uint32_t inc, uint32_t to, uint32_t at) {
+    asm volatile("s_add_i32 m0, %3, %4\n\tv_add_u32 %0, %2, %0\n\tbuffer_load_dword %0, %1, 0 offen lds"
+                 : "+v"(off) : "s"(buf), "s"(inc), "s"(to), "s"(at) : "memory", "m0", "scc");
+}
+
 // out[row] = sum_s acc_s * exp(m_s - M) / sum_s l_s * exp(m_s - M), for the four values d4*4 .. d4*4+3 of the row, folded in in
 // split order.  DEVICE: the partials come from other workgroups of this launch (and the rows of a wave rise with its lanes, all
 // their partials within 4 GiB).

@@ -13,9 +13,14 @@
 // behind it), waits on loads just issued.  Matrix instructions and what reads their results are the compiler's, none of them
 // inline assembly: it puts the wait states between the two, and leaves them out around instructions it does not know.
 //
-// K and V blocks of 32 keys go global -> LDS (global_load_lds_dwordx4, chunks XOR-swizzled) into a ring of 4 slots each, one
+// K and V blocks of 32 keys go global -> LDS (16 bytes a lane, chunks XOR-swizzled) into a ring of 4 slots each, one
 // barrier per block; what a block's start requests is needed two or three blocks later (8 slots are no faster: a CU's path
-// from L2 into LDS gives 53 B/clk from two blocks ahead on).
+// from L2 into LDS gives 53 B/clk from two blocks ahead on).  A request is three instructions: a tensor is a buffer that ends with the
+// range's last row, so that nothing has to hold a request back inside it, and K's and V's slots have one number.  With clamped row
+// numbers and moving bases a request took six and 6 to 12 scalar ones more a step; together with a wait for LDS reads that the
+// compiler could not count across the loop's head (a scalar load was on its way), us a pass, in turn on one box: 6 layers of 8 x 64 x
+// 1500 against 1536 with their copies 114.7 -> 111.2, 4 of 20 x 64 x 1500^2 x 4 214.7 -> 212.6, 750 x 8 heads of 128 x 8 under a bias
+// 43.5 -> 43.1, causal 407 and 2048 behind 2048 as before (90.7, 133.6: two waves a SIMD fill these gaps).
 //
 // Against the tile-wise kernel it replaced for these forms, per launch: 20 x 64 x 1500^2 in batches of 4 60.2 -> 56.8 us
 // (0.81 PFLOP/s), 8 x 64 x 1500 against 1536 keys 14.4 -> 12.8, 8 x 128 x 1500^2 x 4 55.2 -> 52.6, 10 x 128 x 1500^2 31.2 ->
@@ -116,7 +121,10 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     // The reference m enters the scores as the C operand of their first MFMA, 16 registers of one value, and the exponentials
     // need no subtraction.  128-wide heads have vector instructions to spare and no registers: they subtract.
     constexpr bool SPLAT = D == 64;
+    // Slot s of the ring holds the K of steps s, s + R, ... and the V of steps s + DV, ...: what a step's start requests goes into one slot
     constexpr uint32_t VRING = R * STEPB, RMASK = R * STEPB - 1;
+    auto k_slot = [](uint32_t cur, int ahead) __attribute__((always_inline)) { return (cur + (uint32_t)(ahead + R) * STEPB) & RMASK; };
+    auto v_slot = [](uint32_t cur, int ahead) __attribute__((always_inline)) { return (cur + (uint32_t)(ahead + R - DV) * STEPB) & RMASK; };
 
     extern __shared__ __attribute__((aligned(16))) char lds[];
 
@@ -167,56 +175,51 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     const uint64_t vbase = (uint64_t)(a.v + (int64_t)hk * a.nbv2 + (int64_t)bk * a.nbv3 + (int64_t)k_begin * a.nbv1);
 
     // ---- global -> LDS: slot L = (wave * NLD + j) * 64 + lane of a step holds chunk (L % CH) ^ swizzle of row L / CH ------
-    const int  lwave = HALVES ? wave % (W / 2) : wave;
-    const bool ofv   = HALVES && wave >= W / 2;                   // a wave that loads V alone
-    int      row[NLD];
-    uint32_t kch[NLD], vch[NLD];
-#pragma unroll
-    for (int j = 0; j < NLD; j++) {
-        const int L = (lwave * NLD + j) * 64 + lane, c = L % CH;
-        row[j] = L / CH;
-        kch[j] = (uint32_t)((c ^ pipe_swz_k<D>(row[j] & 31)) * 16);
-        vch[j] = (uint32_t)((c ^ pipe_swz_v<D>(row[j] & 31)) * 16);
-    }
-    if (ofv)
-#pragma unroll
-        for (int j = 0; j < NLD; j++) kch[j] = vch[j];
-    const uint32_t lds0 = lwave * (NLD * 1024);
-    // Requests go step by step; behind the last step they go on with its rows, and rows past its end repeat the last one
-    // (their scores are excluded, or nobody looks), so that the waits can count.  Masked: a wave's loads of a step are rows of the
-    // block that its own products take, and the last block is the last 32 keys of the range (and keys before it, where a range
-    // has fewer), so that the mask's rows are read inside their ends; what the block before has had is excluded.
-    struct Stream {
-        uint64_t at;          // first row of the next step to be requested
-        int      left;        // its last row, counted from there
-    };
+    // Each tensor is a buffer that ends with the range's last row, each request's address one register that a step moves on: what is
+    // requested behind the end is zeros and reaches no memory (its scores are excluded, or nobody looks), and the waits can count.
+    const int      lwave = HALVES ? wave % (W / 2) : wave;
+    const bool     ofv   = HALVES && wave >= W / 2;               // a wave that loads V alone
     const uint32_t nb1v = (uint32_t)a.nbv1, nb1k = ofv ? nb1v : (uint32_t)a.nbk1;          // (below 2^24)
-    const int      key0 = MASK ? min(32 * kgroup, n_keys - 32) : 0;             // the first block's first key
-    Stream kst = {ofv ? vbase : kbase + (int64_t)key0 * a.nbk1, MASK ? n_keys - 32 - key0 : n_keys - 1};
-    Stream vst = {vbase + (int64_t)key0 * a.nbv1, MASK ? n_keys - 32 - key0 : n_keys - 1};
-    auto request = [&](Stream & st, uint32_t nb1, const uint32_t (&ch)[NLD], uint32_t slot) __attribute__((always_inline)) {
-        if constexpr (MASK) {
+    const uint32_t inck = SKEYS * nb1k, incv = SKEYS * nb1v;
+    const auto     kbuf = fattn_buffer((const void *)(ofv ? vbase : kbase), (uint32_t)(n_keys - 1) * nb1k + ROWB);       // (below 2^31)
+    const auto     vbuf = fattn_buffer((const void *)vbase, (uint32_t)(n_keys - 1) * nb1v + ROWB);
+    uint32_t kof[NLD], vof[NLD];                                  // (of the request before the next one)
+    auto start_at = [&](uint32_t key) __attribute__((always_inline)) {
 #pragma unroll
-            for (int j = 0; j < NLD; j++) load_to_lds16<(MASK != 0)>(st.at, __umul24((uint32_t)(row[j] & 31), nb1) + ch[j], lds0 + slot + j * 1024);
-            const int by = min(st.left, SKEYS);
-            st.at   += (uint64_t)(uint32_t)by * nb1;
-            st.left -= by;
-            return;
+        for (int j = 0; j < NLD; j++) {
+            const int L = (lwave * NLD + j) * 64 + lane, c = L % CH, row = L / CH;
+            const uint32_t ck = (uint32_t)((c ^ pipe_swz_k<D>(row & 31)) * 16), cv = (uint32_t)((c ^ pipe_swz_v<D>(row & 31)) * 16);
+            kof[j] = __umul24((uint32_t)row, nb1k) + (ofv ? cv : ck) + key * nb1k - inck;
+            vof[j] = __umul24((uint32_t)row, nb1v) + cv + key * nb1v - incv;
         }
-#pragma unroll
-        for (int j = 0; j < NLD; j++) load_to_lds16<(MASK != 0)>(st.at, __umul24((uint32_t)min(row[j], st.left), nb1) + ch[j], lds0 + slot + j * 1024);
-        const bool more = st.left >= SKEYS;
-        st.at   += more ? (uint64_t)SKEYS * nb1 : 0;
-        st.left -= more ? SKEYS : 0;
     };
-
-    // the requests of a step's start: K's DK steps ahead, V's DV
+    start_at(0);
+    uint32_t lds0[NLD];
+#pragma unroll
+    for (int j = 0; j < NLD; j++) lds0[j] = (lwave * NLD + j) * 1024 + (ofv ? VRING : 0);
+    auto request_k = [&](uint32_t slot) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < NLD; j++) buffer_to_lds16(kbuf, kof[j], inck, lds0[j], slot);
+    };
+    auto request_v = [&](uint32_t slot) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < NLD; j++) buffer_to_lds16(vbuf, vof[j], incv, lds0[j] + VRING, slot);
+    };
+    // the requests of the start of a step: K's DK steps ahead, V's DV
     auto request_step = [&](uint32_t slot) __attribute__((always_inline)) {
-        if constexpr (HALVES) {
-            request(kst, nb1k, kch, ofv ? VRING + ((slot + DV * STEPB) & RMASK) : (slot + DK * STEPB) & RMASK);
-        } else {
-            request(kst, nb1k, kch, (slot + DK * STEPB) & RMASK);
-            request(vst, nb1v, vch, VRING + ((slot + DV * STEPB) & RMASK));
+        request_k(slot);
+        if (!HALVES) request_v(slot);
+    };
+    // ... and ahead of the first step, as if of the steps before it (a wave that loads V alone leaves out the first DK - DV)
+    auto request_first = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < DK; j++) {
+            if constexpr (HALVES) {
+                if (!ofv || j >= DK - DV) request_k(j * STEPB);
+            } else {
+                request_k(j * STEPB);
+                if (j >= DK - DV) request_v(j * STEPB);
+            }
         }
     };
 
@@ -235,26 +238,31 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     const uint32_t m_lds = 2 * R * STEPB + wave * (2 * MSLOT);
     const char * const plane = MASK ? a.mask + (int64_t)(h % a.Hm) * a.nbm2 + (int64_t)(b % a.Bm) * a.nbm3 : nullptr;
     auto row_at = [&](int r) __attribute__((always_inline)) { return (uint32_t)min(q0 + r, a.Nq - 1) * (uint32_t)a.nbm1; };      // (below 2^31)
-    uint32_t moff[MASK ? 2 : 1];
-    const uint32_t mrow = MASK == 2 ? row_at(l32) : 0;
-#pragma unroll
-    for (int j = 0; j < (MASK ? 2 : 0); j++) moff[j] = row_at(j * 16 + (lane >> 2)) + (uint32_t)(((lane & 3) ^ ((lane >> 4) & 3)) * 16);
-    Stream mst = {MASK ? (uint64_t)plane + (uint64_t)((int64_t)(k_begin + key0) * 2) : 0, MASK ? n_keys - 32 - key0 : 0};
-    auto request_mask = [&](int slot) __attribute__((always_inline)) {
+    // (Rows that start between dwords: from the dword that holds the block's first key on, and the one that holds its last.  Of the mask's
+    //  first and last row that can be the two bytes ahead of its first element or behind its last one, in the same dword, so in mapped
+    //  memory; they are shifted out.)
+    const uint32_t m_odd = MASK == 2 ? (uint32_t)(uint64_t)plane & 2 : 0;
+    const auto     mbuf  = fattn_buffer(plane - m_odd, MASK ? (m_odd + (uint32_t)(a.Nq - 1) * (uint32_t)a.nbm1 + (uint32_t)a.Nkv * 2 + 3) & ~3u : 0u);
+    uint32_t       mof[MASK ? 3 : 1], m_shift = 0;                // (m_shift: bits from a row's first dword to the block's first key)
+    auto start_mask_at = [&](int key) __attribute__((always_inline)) {
         if constexpr (MASK != 0) {
-            // (rows that start between dwords: from the dword that holds their first key on, and the one that holds their last.  Of a mask's
-            //  first and last row that can be the two bytes ahead of its first element or behind its last one, in the same dword, so in
-            //  mapped memory; they are shifted out.)
-            const uint32_t odd = MASK == 2 ? (uint32_t)mst.at & 2 : 0;
+            const uint32_t at = m_odd + (uint32_t)(k_begin + 32 * kgroup + key) * 2;
 #pragma unroll
-            for (int j = 0; j < 2; j++) load_to_lds16<(MASK != 0)>(mst.at - odd, MASK == 2 ? (moff[j] + odd) & ~3u : moff[j], m_lds + slot * MSLOT + j * 1024);
-            if (MASK == 2) load_to_lds4(mst.at - odd, (mrow + odd + 62) & ~3u, m_lds + slot * MSLOT + 2048);
-            const int by = min(mst.left, SKEYS);
-            mst.at   += (uint64_t)(2 * by);
-            mst.left -= by;
+            for (int j = 0; j < 2; j++)
+                mof[j] = ((at + row_at(j * 16 + (lane >> 2))) & ~3u) + (uint32_t)(((lane & 3) ^ ((lane >> 4) & 3)) * 16) - SKEYS * 2;
+            mof[2]  = MASK == 2 ? ((at + row_at(l32) + 62) & ~3u) - SKEYS * 2 : 0;
+            m_shift = MASK == 2 ? ((at + row_at(l32)) & 2) * 8 : 0;
         }
     };
-    // adds the block in `slot` to scores x of block `block` in log2 units, or (the last block) excludes keys of the one before
+    start_mask_at(0);
+    auto request_mask = [&](int slot) __attribute__((always_inline)) {
+        if constexpr (MASK != 0) {
+#pragma unroll
+            for (int j = 0; j < 2; j++) buffer_to_lds16(mbuf, mof[j], SKEYS * 2, m_lds + (slot * MSLOT + j * 1024), 0);
+            if (MASK == 2) buffer_to_lds4(mbuf, mof[2], SKEYS * 2, m_lds + (slot * MSLOT + 2048), 0);
+        }
+    };
+    // adds the block in `slot` to scores x of block `block` in log2 units and excludes keys past the end
     auto add_mask = [&](float16v & x, int slot, int block) __attribute__((always_inline)) {
         const uint32_t at = m_lds + slot * MSLOT + (uint32_t)(l32 * 64 + ((l32 >> 2) & 3) * 16);
         typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -269,13 +277,10 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
             for (int g = 0; g < 4; g++)
                 next[g] = *(lds_u1 *)(uintptr_t)(hh ? (g < 3 ? at ^ (uint32_t)((g + 1) * 16) : m_lds + slot * MSLOT + 2048 + l32 * 4)
                                                     : (at ^ (uint32_t)(g * 16)) + 8);
-            // (where the block starts: its row's first key in the low or the high half of a dword)
-            const uint32_t start = (uint32_t)(uint64_t)plane + (uint32_t)(k_begin + min(32 * block, n_keys - 32)) * 2;
-            const uint32_t sh    = ((mrow + start) & 2) * 8;
 #pragma unroll
             for (int g = 0; g < 4; g++) {
-                w[g][0] = __builtin_amdgcn_alignbit(w[g][1], w[g][0], sh);
-                w[g][1] = __builtin_amdgcn_alignbit(next[g], w[g][1], sh);
+                w[g][0] = __builtin_amdgcn_alignbit(w[g][1], w[g][0], m_shift);
+                w[g][1] = __builtin_amdgcn_alignbit(next[g], w[g][1], m_shift);
             }
         }
 #pragma unroll
@@ -284,10 +289,10 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
             for (int c = 0; c < 4; c++)
                 x[4 * g + c] = fmaf((float)__builtin_bit_cast(_Float16, (uint16_t)(w[g][c >> 1] >> (16 * (c & 1)))), LOG2E, x[4 * g + c]);
         if (__builtin_expect(32 * block + 32 > n_keys, 0)) {
-            int had = 32 * block + 32 - n_keys - hh * 4;
-            asm volatile("" : "+v"(had));
+            int lim = n_keys - 32 * block - hh * 4;
+            asm volatile("" : "+v"(lim));            // (nothing of this is worth a register in the loop)
 #pragma unroll
-            for (int r = 0; r < 16; r++) x[r] = (r >> 2) * 8 + (r & 3) < had ? -INFINITY : x[r];
+            for (int r = 0; r < 16; r++) x[r] = (r >> 2) * 8 + (r & 3) < lim ? x[r] : -INFINITY;
         }
     };
     // A wave looks at the last 64 keys of its last 8 queries with the first requests; if none of them is seen, at the rows of all its
@@ -312,15 +317,7 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
         request_mask(0);
         request_mask(1);
     }
-#pragma unroll
-    for (int j = 0; j < DK; j++) {
-        if constexpr (HALVES) {
-            if (!ofv || j >= DK - DV) request(kst, nb1k, kch, ofv ? VRING + (j - (DK - DV)) * STEPB : j * STEPB);
-        } else {
-            request(kst, nb1k, kch, j * STEPB);
-            if (j >= DK - DV) request(vst, nb1v, vch, VRING + (j - (DK - DV)) * STEPB);
-        }
-    }
+    request_first();
 
     half8 qreg[NQB][KS];                       // f16 B operands in log2 units
 #pragma unroll
@@ -334,7 +331,7 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
         }
 
     // (in the slot of V's that the first region asks for; read behind the barrier below)
-    int * const ends = (int *)(lds + VRING + (R - 2) * STEPB);
+    int * const ends = (int *)(lds + VRING + v_slot(0, DV));
     if constexpr (MASK != 0) {
         int  nt = n_tiles, ft = 0, at = 0;                       // at: tiles looked at from the end in question
         bool last  = __builtin_amdgcn_ballot_w64(any_seen(end_keys) != 0) == 0;
@@ -423,7 +420,7 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     if (NQB == 1) {
         // the first unit multiplies the V of a step before the first one by zeros: it must be finite
 #pragma unroll
-        for (int i = 0; i < STEPB / 16 / PIPE_THREADS; i++) *(float4 *)(lds + VRING + (R - 1) * STEPB + (i * PIPE_THREADS + tid) * 16) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        for (int i = 0; i < STEPB / 16 / PIPE_THREADS; i++) *(float4 *)(lds + VRING + v_slot(0, -1) + (i * PIPE_THREADS + tid) * 16) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
     // the first two blocks of K have landed
     auto first_landed = [&]() __attribute__((always_inline)) {
@@ -442,17 +439,11 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
             // every wave has read `ends`, and nothing is on its way into the slots
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
-            const int left = max(n_keys - 32 - (first_tile * 64 + 32 * kgroup), 0);
-            kst = {kst.at + (int64_t)(kst.left - left) * nb1k, left};
-            vst = {vst.at + (int64_t)(vst.left - left) * nb1v, left};
-            mst = {mst.at + (int64_t)(mst.left - left) * 2, left};
+            start_at((uint32_t)first_tile * 64);
+            start_mask_at(first_tile * 64);
             request_mask(0);
             request_mask(1);
-#pragma unroll
-            for (int j = 0; j < DK; j++) {
-                request(kst, nb1k, kch, j * STEPB);
-                if (j >= DK - DV) request(vst, nb1v, vch, VRING + (j - (DK - DV)) * STEPB);
-            }
+            request_first();
             first_landed();
         }
     }
@@ -500,11 +491,11 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
 
     // One unit: the softmax of s[U] (query block QB), with the scores of the next unit into s[1 - U] and V^T.P^T of the one
     // before on the matrix cores.
-    auto region = [&](auto u_tag, auto start_tag) __attribute__((always_inline)) {
+    auto region = [&](auto u_tag) __attribute__((always_inline)) {
         constexpr int  U     = decltype(u_tag)::value;
-        constexpr bool START = decltype(start_tag)::value;        // the first unit of a step
+        constexpr bool START = NQB == 1 || U == 0;                // the first unit of a step
         constexpr int  QB    = NQB == 2 ? U : 0, NX = NQB == 2 ? 1 - U : 0;
-        if (START) {
+        if constexpr (START) {
             // what was requested OPEN loads ago and earlier has landed, in every wave's share
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(OPEN) : "memory");
             __builtin_amdgcn_s_barrier();
@@ -516,8 +507,8 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
             request_mask(U);
         } else if (__builtin_expect((step + 1) * SKEYS > n_keys, 0)) exclude_past_end(s[U], step);
         // (one query block) operands of this region's second half
-        if (TURNS)          read_k(va, (cur + STEPB) & RMASK, KS - 4);
-        else if (NQB == 1)  read_v(va, (cur - STEPB) & RMASK, 0);
+        if (TURNS)          read_k(va, k_slot(cur, 1), KS - 4);
+        else if (NQB == 1)  read_v(va, v_slot(cur, -1), 0);
         PIPE_FENCE();
         float e[16];
         float lprev = lacc[QB][0];                                // (a copy by force: else all four old sums stay in registers)
@@ -531,11 +522,11 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
 #pragma unroll
         for (int j = 0; j < NM; j++) {
             // operands that take the place of those that the MFMA before has read for the last time
-            if (TURNS && j == 4)                         read_v(ka, (cur - STEPB) & RMASK, 0);
-            if (TURNS && j == 8)                         read_v(va, (cur - STEPB) & RMASK, 4);
-            if (TURNS && j == 12)                        read_k(ka, (cur + 2 * STEPB) & RMASK, 0);
-            if (!TURNS && NQB == 1 && j == KS)           read_k(ka, (cur + 2 * STEPB) & RMASK, 0);
-            if (NQB == 2 && U == 0 && j == KS)           read_k(ka, (cur + STEPB) & RMASK, 0);
+            if (TURNS && j == 4)                         read_v(ka, v_slot(cur, -1), 0);
+            if (TURNS && j == 8)                         read_v(va, v_slot(cur, -1), 4);
+            if (TURNS && j == 12)                        read_k(ka, k_slot(cur, 2), 0);
+            if (!TURNS && NQB == 1 && j == KS)           read_k(ka, k_slot(cur, 2), 0);
+            if (NQB == 2 && U == 0 && j == KS)           read_k(ka, k_slot(cur, 1), 0);
             PIPE_FENCE();
             if (j == 0) {
                 if (SPLAT) {
@@ -558,11 +549,11 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
             if (j == NM - 2) add_sums(0);
             PIPE_FENCE();
         }
-        if (NQB == 2 && U == 0) read_v(va, cur, 0);
+        if (NQB == 2 && U == 0) read_v(va, v_slot(cur, 0), 0);
 #pragma unroll
         for (; packed < 8; packed++) pack(packed);
         add_sums(1);
-        if (NQB == 1 || U == 1) cur = (cur + STEPB) & RMASK;
+        if (NQB == 1 || U == 1) cur = k_slot(cur, 1);
         PIPE_FENCE();
         // A probability that left f16's range (inf, or NaN from an infinite score) shows in the row's sum: the reference has
         // fallen 16 binary orders behind.  Wave-uniform and rare.
@@ -617,17 +608,18 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
         for (int k2 = 0; k2 < 2; k2++)
 #pragma unroll
             for (int db = 0; db < DB; db++) {
-                const half8 v = NQB == 2 ? va[(k2 * DB + db) % (2 * DB)] : read_v1((cur - STEPB) & RMASK, k2, db);
+                const half8 v = NQB == 2 ? va[(k2 * DB + db) % (2 * DB)] : read_v1(v_slot(cur, -1), k2, db);
                 oacc[QB][db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, p[U][k2], oacc[QB][db], 0, 0, 0);
             }
     };
     // (One query block: an odd number of steps is made even by one whose keys all lie past the end.  Leaving the loop in the
     //  middle would cost the accumulators' 64 registers a copy in every turn.)
+    __builtin_amdgcn_s_waitcnt(0xC07F);                          // lgkmcnt(0), known to the compiler: scalar loads on their way are not counted
 #pragma unroll 1
     while (step < n_steps) {
-        region(I0{}, std::true_type{});
+        region(I0{});
         if (NQB == 1) step++;
-        region(I1{}, std::integral_constant<bool, NQB == 1>{});
+        region(I1{});
         step++;
     }
     last_pv(I1{});
@@ -792,8 +784,11 @@ static bool pipe_masked(const FattnArgs & a, const FattnMmaVariant & v) {
 // the longer prologue costs what the loop gains (300 tokens x 30 heads 10.8 against 11.9 us a launch, 500 x 20 and 800 x 8 within 2%).
 // Eight waves a workgroup where that leaves no CU with more of them than workgroups of four do: more of those than CUs, and their
 // number per CU even once rounded up.  (A caller who names the form gets four.)
+// Request addresses are 32-bit numbers inside a range of a head's keys, up to 8 steps of 64 behind its end: longer ones are the tile kernel's.
 int fattn_pipe_waves(const FattnArgs & a, int ktype, const FattnMmaVariant & v) {
     if (ktype != MI355X_TYPE_F16 || !v.direct || a.softcap != 0.0f) return 0;
+    const int64_t keys = (a.n_splits > 1 ? a.keys_per_split : a.Nkv) + 8 * 64;
+    if (keys * a.nbk1 >= ((int64_t)1 << 31) || keys * a.nbv1 >= ((int64_t)1 << 31)) return 0;
     if (a.masked) return pipe_masked(a, v) ? 4 : 0;
     if (v.key_split == 2) return a.D == 128 ? 0 : 4;
     if (a.tile_variant != 0 || (a.D == 64 && v.query_blocks != 2)) return 4;
