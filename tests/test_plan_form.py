@@ -37,7 +37,7 @@ def test_masked_calls():
 @pytest.mark.parametrize("mask", [None, 1])
 def test_ranges_longer_than_request_addresses(mask):
     """1000 rows 2 MiB apart lie beyond 2^31 bytes: the tile kernel's, with 64-bit addresses"""
-    def pipelined(pitch, **kw):
+    def pipelined(pitch, ns=1):
         q, k = _t(ggml.F32, (128, 100, 4, 1)), ca.Tensor(None, ggml.F16, (128, 1000, 4, 1), (2, pitch, 256, pitch * 1000))
-        return ggml.flash_attn_plan_form(q, k, k, _t(ggml.F16, (1000, 100, mask, 1)) if mask else None, 0.1, kernel=ggml.KERNEL_MMA, tile_variant=0x11, **kw)["pipelined"]
-    assert pipelined(1 << 20) == 1 and pipelined(1 << 21) == 0 and (mask or pipelined(1 << 21, n_splits=3) == 1)
+        return ggml.flash_attn_plan_form(q, k, k, _t(ggml.F16, (1000, 100, mask, 1)) if mask else None, 0.1, kernel=ggml.KERNEL_MMA, tile_variant=0x11, n_splits=ns)["pipelined"]
+    assert pipelined(1 << 20) == 1 and pipelined(1 << 21) == 0 and (mask or pipelined(1 << 21, 3) == 1)
