@@ -20,7 +20,15 @@
 // numbers and moving bases a request took six and 6 to 12 scalar ones more a step; together with a wait for LDS reads that the
 // compiler could not count across the loop's head (a scalar load was on its way), us a pass, in turn on one box: 6 layers of 8 x 64 x
 // 1500 against 1536 with their copies 114.7 -> 111.2, 4 of 20 x 64 x 1500^2 x 4 214.7 -> 212.6, 750 x 8 heads of 128 x 8 under a bias
-// 43.5 -> 43.1, causal 407 and 2048 behind 2048 as before (90.7, 133.6: two waves a SIMD fill these gaps).
+// 43.5 -> 43.1, causal 407 and 2048 behind 2048 as before (90.7, 133.6: two waves a SIMD fill these gaps).  A step's requests go out one
+// behind each of its first matrix instructions (a wave alone on its SIMD waits for each to be taken), the last of the prologue's behind
+// the first scores: 8 x 64 x 1500 against 1536, K and V from memory, 12.9 -> 12.5 us a launch.
+//
+// Waves that share queries (KSP > 1) get them through LDS: the workgroup's rows are brought once, along the rows.  A wave's own loads
+// of its operands, 32 rows an instruction, took 1.1 us for each 32 queries.  Launches, us, with their own loads and like this: 8 x 64 x
+// 1500 against 1536 13.4 -> 12.6, 8 x 64 x 300^2 6.9 -> 6.4; whole passes with both changes, in turn with the code before them: 6 of the
+// first layers 111.2 -> 104, four causal layers of 407 tokens, 32 heads of 128, with their row writes 90.8 -> 80.6.  (Eight waves of
+// their own 64 queries each: 216.9 and 218.3 us, memory gives the rows no faster.)
 //
 // Against the tile-wise kernel it replaced for these forms, per launch: 20 x 64 x 1500^2 in batches of 4 60.2 -> 56.8 us
 // (0.81 PFLOP/s), 8 x 64 x 1500 against 1536 keys 14.4 -> 12.8, 8 x 128 x 1500^2 x 4 55.2 -> 52.6, 10 x 128 x 1500^2 31.2 ->
@@ -34,9 +42,9 @@
 // Masked calls of 128-wide heads: a wave brings the mask of its next two blocks to LDS as it does K and V, so that the waits
 // go on counting, and adds it ahead of the exponentials; the last block is the last 32 keys of the range, whole.  Against the tile
 // kernel, whole calls: 2048 causal tokens behind 2048, 32 query and 8 KV heads, with their row writes 146.8 -> 133.4 us, 1000 causal
-// tokens 42.5 -> 37.5, 407 (rows that start between dwords, the pairs' form) 21.4 -> 20.1; under per-head masks 750 x 8 heads x 8
-// 45.7 -> 38.8, 1000 x 8 x 4 38.1 -> 32.7, 751 x 8 22.0 -> 19.2.  The 407-token launch (16 us) is 4.5 us until the first scores, 0.65
-// a step - 32 KB through a CU's port - and 3 for the hand-over and the stores.
+// tokens 42.5 -> 37.5, 407 (rows that start between dwords, the pairs' form) 21.4 -> 20.1 (now 17.6); under per-head masks 750 x 8 heads x 8
+// 45.7 -> 38.8, 1000 x 8 x 4 38.1 -> 32.7, 751 x 8 22.0 -> 19.2.  A step of the 407-token launch is 0.65 us, 32 KB through a CU's
+// port; the hand-over and the stores are 3 us of it.
 // Hidden keys: the walk ends behind the last 64 that a query of the workgroup sees, starts at the first ones (ranges of 12 tiles and
 // more, where that leaves out four), and between the two a hidden block is walked like a visible one - the pairs' form is bound by
 // its K and V bytes, which the tile kernel, which skips the block's products, fetches as well.  A row that has seen nothing yet
@@ -82,7 +90,7 @@ typedef __attribute__((address_space(3))) short4v     lds_short4;
 // A wave's mask block: 32 queries x 32 keys of f16, and for rows that start between dwords the one behind each row's last
 constexpr int pipe_mask_slot(int MASK) { return MASK == 2 ? 32 * 64 + 256 : MASK ? 32 * 64 : 0; }
 constexpr int pipe_lds_bytes(int D, int NQB, int KSP, int W, int MASK) {
-    const int ring  = 2 * RING * KSP * 32 * D * 2 + W * 2 * pipe_mask_slot(MASK);
+    const int ring  = 2 * RING * KSP * 32 * D * 2 + W * 2 * pipe_mask_slot(MASK) + (MASK && KSP > 1 ? 2 * W * 4 : 0);
     const int stage = W * 32 * D * 4;                                           // result rows / the waves' partial results
     return ring > stage ? ring : stage;
 }
@@ -111,9 +119,10 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     constexpr int  NLS  = HALVES ? NLD : 2 * NLD;                 // loads per wave and step
     constexpr int R    = RING;
     // steps ahead of the current one that its start requests, and loads that may still be under way then
-    constexpr int DK   = R, DV = NQB == 2 ? R - 1 : R - 2;
+    constexpr int DK   = R, DV = NQB == 2 ? DK - 1 : DK - 2;
     constexpr int NML  = MASK == 2 ? 3 : MASK ? 2 : 0;            // ... of its own mask block
-    constexpr int OPEN = (NQB == 2 ? R - 2 : R - 3) * (NLS + NML);
+    constexpr int AHEAD = DK - 1;                                 // ... of which the last go out behind the first scores
+    constexpr int OPEN = (DV - 1) * (NLS + NML);
     constexpr int BMW  = 32 * NQB;
     constexpr int BMG  = BMW * QG;
     constexpr int NM   = KS + 2 * DB;                             // MFMAs of a region
@@ -121,10 +130,10 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     // The reference m enters the scores as the C operand of their first MFMA, 16 registers of one value, and the exponentials
     // need no subtraction.  128-wide heads have vector instructions to spare and no registers: they subtract.
     constexpr bool SPLAT = D == 64;
-    // Slot s of the ring holds the K of steps s, s + R, ... and the V of steps s + DV, ...: what a step's start requests goes into one slot
+    // Slot s of the ring holds the K of steps s, s + R, ... and the V of the steps DK - DV before: what a step's start requests goes into one slot
     constexpr uint32_t VRING = R * STEPB, RMASK = R * STEPB - 1;
     auto k_slot = [](uint32_t cur, int ahead) __attribute__((always_inline)) { return (cur + (uint32_t)(ahead + R) * STEPB) & RMASK; };
-    auto v_slot = [](uint32_t cur, int ahead) __attribute__((always_inline)) { return (cur + (uint32_t)(ahead + R - DV) * STEPB) & RMASK; };
+    auto v_slot = [](uint32_t cur, int ahead) __attribute__((always_inline)) { return (cur + (uint32_t)(ahead + R + DK - DV) * STEPB) & RMASK; };
 
     extern __shared__ __attribute__((aligned(16))) char lds[];
 
@@ -155,17 +164,34 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     const int q0 = qt * BMG + qgroup * BMW;
 
     // ---- Q rows: requested first, converted behind the first requests of K and V, so that all of them are one round trip ---
-    float4v qraw[NQB][KS][2];
+    // Where waves share queries the workgroup brings its 64 rows once, to LDS as they are, 16 bytes a lane along the rows (chunks
+    // XOR-swizzled), into slots of V's ring that nothing is requested into yet.
+    constexpr bool     QLDS  = KSP > 1;
+    constexpr int      QCH   = D / 4;                             // 16-byte chunks of a row
+    constexpr int      NQL   = BMG * QCH / PIPE_THREADS;          // ... of a lane
+    constexpr uint32_t QAT   = VRING;
+    static_assert(!QLDS || BMG * D * 4 <= (DK - DV) * STEPB, "the slots ahead of the first V");
+    float4v qraw[NQB][QLDS ? 1 : KS][2];
+    if constexpr (QLDS) {
+        const uint64_t q64  = (uint64_t)(a.q + (int64_t)(qt * BMG) * a.nbq1 + (int64_t)h * a.nbq2 + (int64_t)b * a.nbq3);
+        const int      rows = min(BMG, a.Nq - qt * BMG) - 1;
 #pragma unroll
-    for (int qb = 0; qb < NQB; qb++) {
+        for (int i = 0; i < NQL; i++) {
+            const int L = (wave * NQL + i) * 64 + lane, row = L / QCH, c = (L % QCH) ^ (row & 15);
+            // (padded: a lane with nothing behind Dv reads the row's first chunk, and its values are scaled by zero)
+            load_to_lds16<(MASK != 0)>(q64, (uint32_t)min(row, rows) * (uint32_t)a.nbq1 + (!PAD || c * 4 < a.Dv ? c * 16 : 0), QAT + (wave * NQL + i) * 1024);
+        }
+    }
+#pragma unroll
+    for (int qb = 0; qb < (QLDS ? 0 : NQB); qb++) {
         const int qi = min(q0 + qb * 32 + l32, a.Nq - 1);
         const float * qrow = (const float *)(a.q + (int64_t)qi * a.nbq1 + (int64_t)h * a.nbq2 + (int64_t)b * a.nbq3);
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
             // (padded: a lane with nothing behind Dv reads the row's first 8 elements and scales them by zero)
             const float * q8 = qrow + (!PAD || ks * 16 + hh * 8 < a.Dv ? ks * 16 + hh * 8 : 0);
-            qraw[qb][ks][0] = *(const float4v *)q8;
-            qraw[qb][ks][1] = *(const float4v *)(q8 + 4);
+            qraw[qb][QLDS ? 0 : ks][0] = *(const float4v *)q8;
+            qraw[qb][QLDS ? 0 : ks][1] = *(const float4v *)(q8 + 4);
         }
     }
 
@@ -205,15 +231,15 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
 #pragma unroll
         for (int j = 0; j < NLD; j++) buffer_to_lds16(vbuf, vof[j], incv, lds0[j] + VRING, slot);
     };
-    // the requests of the start of a step: K's DK steps ahead, V's DV
-    auto request_step = [&](uint32_t slot) __attribute__((always_inline)) {
-        request_k(slot);
-        if (!HALVES) request_v(slot);
+    // request i < NLS of a step: K's DK steps ahead, V's DV
+    auto request_step = [&](uint32_t slot, int i) __attribute__((always_inline)) {
+        if (i < NLD) buffer_to_lds16(kbuf, kof[i], inck, lds0[i], slot);
+        else         buffer_to_lds16(vbuf, vof[i - NLD], incv, lds0[i - NLD] + VRING, slot);
     };
     // ... and ahead of the first step, as if of the steps before it (a wave that loads V alone leaves out the first DK - DV)
-    auto request_first = [&]() __attribute__((always_inline)) {
+    auto request_first = [&](int from, int to) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < DK; j++) {
+        for (int j = from; j < to; j++) {
             if constexpr (HALVES) {
                 if (!ofv || j >= DK - DV) request_k(j * STEPB);
             } else {
@@ -317,21 +343,36 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
         request_mask(0);
         request_mask(1);
     }
-    request_first();
+    request_first(0, AHEAD);
 
     half8 qreg[NQB][KS];                       // f16 B operands in log2 units
+    if constexpr (QLDS) {
+        // (the loads behind Q's and the looks at the mask)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NML + (2 * AHEAD - (DK - DV)) * NLD) : "memory");
+        __builtin_amdgcn_s_barrier();
+    }
 #pragma unroll
     for (int qb = 0; qb < NQB; qb++)
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
-            asm volatile("" : "+v"(qraw[qb][ks][0]), "+v"(qraw[qb][ks][1]));          // (not before here)
+            float4v x[2];
+            if constexpr (QLDS) {
+                typedef __attribute__((address_space(3))) const float4v lds_float4;
+                const int row = (qgroup * NQB + qb) * 32 + l32;
+#pragma unroll
+                for (int e = 0; e < 2; e++) x[e] = *(lds_float4 *)(uintptr_t)(QAT + row * (D * 4) + (((ks * 4 + hh * 2 + e) ^ (row & 15)) * 16));
+            } else {
+                asm volatile("" : "+v"(qraw[qb][QLDS ? 0 : ks][0]), "+v"(qraw[qb][QLDS ? 0 : ks][1]));          // (not before here)
+                x[0] = qraw[qb][QLDS ? 0 : ks][0];
+                x[1] = qraw[qb][QLDS ? 0 : ks][1];
+            }
             const float qs = !PAD || ks * 16 + hh * 8 < a.Dv ? a.scale * LOG2E : 0.0f;
 #pragma unroll
-            for (int e = 0; e < 8; e++) qreg[qb][ks][e] = (_Float16)(qraw[qb][ks][e >> 2][e & 3] * qs);
+            for (int e = 0; e < 8; e++) qreg[qb][ks][e] = (_Float16)(x[e >> 2][e & 3] * qs);
         }
 
-    // (in the slot of V's that the first region asks for; read behind the barrier below)
-    int * const ends = (int *)(lds + VRING + v_slot(0, DV));
+    // (in the slot of V's that the first region asks for, or behind the masks where Q is in that; read behind the barrier below)
+    int * const ends = (int *)(lds + (QLDS ? 2 * R * STEPB + W * 2 * MSLOT : VRING + v_slot(0, DV)));
     if constexpr (MASK != 0) {
         int  nt = n_tiles, ft = 0, at = 0;                       // at: tiles looked at from the end in question
         bool last  = __builtin_amdgcn_ballot_w64(any_seen(end_keys) != 0) == 0;
@@ -417,17 +458,19 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
         for (int i = 0; i < 4; i++) to[i] = read_v1(slot, (i0 + i) / DB, (i0 + i) % DB);
     };
 
-    if (NQB == 1) {
+    // the first two blocks of K have landed
+    auto first_landed = [&]() __attribute__((always_inline)) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(HALVES ? (AHEAD - 2) * NLD : (2 * AHEAD - 2 - (DK - DV)) * NLD) : "memory");
+        __builtin_amdgcn_s_barrier();
+    };
+    auto clear_first_v = [&]() __attribute__((always_inline)) {
         // the first unit multiplies the V of a step before the first one by zeros: it must be finite
 #pragma unroll
         for (int i = 0; i < STEPB / 16 / PIPE_THREADS; i++) *(float4 *)(lds + VRING + v_slot(0, -1) + (i * PIPE_THREADS + tid) * 16) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
-    // the first two blocks of K have landed
-    auto first_landed = [&]() __attribute__((always_inline)) {
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(HALVES ? (DK - 2) * NLD : (DK - 2 + DV) * NLD) : "memory");
-        __builtin_amdgcn_s_barrier();
     };
+    if (NQB == 1 && !QLDS) clear_first_v();
     first_landed();
+    if (NQB == 1 && QLDS) clear_first_v();             // (every wave has read Q there)
     int first_step = 0;
     if constexpr (MASK != 0) {
         n_steps = min(n_steps, max(max(ends[0], ends[1]), max(ends[2], ends[3])) * 64 / SKEYS);
@@ -443,7 +486,7 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
             start_mask_at(first_tile * 64);
             request_mask(0);
             request_mask(1);
-            request_first();
+            request_first(0, AHEAD);
             first_landed();
         }
     }
@@ -499,13 +542,12 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
             // what was requested OPEN loads ago and earlier has landed, in every wave's share
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(OPEN) : "memory");
             __builtin_amdgcn_s_barrier();
-            request_step(cur);
         }
         if constexpr (MASK != 0) {
             add_mask(s[U], U, KSP * step + kgroup);
             PIPE_FENCE();
             request_mask(U);
-        } else if (__builtin_expect((step + 1) * SKEYS > n_keys, 0)) exclude_past_end(s[U], step);
+        } else if (__builtin_expect(step * SKEYS > n_keys - 32 * kgroup - 32, 0)) exclude_past_end(s[U], step);
         // (one query block) operands of this region's second half
         if (TURNS)          read_k(va, k_slot(cur, 1), KS - 4);
         else if (NQB == 1)  read_v(va, v_slot(cur, -1), 0);
@@ -543,6 +585,7 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
                 const int i = j - KS, k2 = i / DB, db = i % DB;
                 oacc[NX][db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(TURNS ? (k2 ? va[db & 3] : ka[db & 3]) : va[i % (2 * DB)], p[1 - U][k2], oacc[NX][db], 0, 0, 0);
             }
+            if (START && j < NLS) request_step(k_slot(cur, DK), j);
 #pragma unroll
             for (int k = 0; k < EPS; k++) { e[done] = __builtin_amdgcn_exp2f(SPLAT ? s[U][done] : s[U][done] - m[QB]); done++; }
             while (packed * 2 + 2 <= done - EPS) { pack(packed); packed++; }
@@ -614,6 +657,7 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     };
     // (One query block: an odd number of steps is made even by one whose keys all lie past the end.  Leaving the loop in the
     //  middle would cost the accumulators' 64 registers a copy in every turn.)
+    request_first(AHEAD, DK);
     __builtin_amdgcn_s_waitcnt(0xC07F);                          // lgkmcnt(0), known to the compiler: scalar loads on their way are not counted
 #pragma unroll 1
     while (step < n_steps) {
@@ -789,6 +833,7 @@ int fattn_pipe_waves(const FattnArgs & a, int ktype, const FattnMmaVariant & v) 
     if (ktype != MI355X_TYPE_F16 || !v.direct || a.softcap != 0.0f) return 0;
     const int64_t keys = (a.n_splits > 1 ? a.keys_per_split : a.Nkv) + 8 * 64;
     if (keys * a.nbk1 >= ((int64_t)1 << 31) || keys * a.nbv1 >= ((int64_t)1 << 31)) return 0;
+    if (v.key_split > 1 && (a.nbq1 < 0 || a.nbq1 >= 1 << 25)) return 0;        // (64 rows of Q likewise)
     if (a.masked) return pipe_masked(a, v) ? 4 : 0;
     if (v.key_split == 2) return a.D == 128 ? 0 : 4;
     if (a.tile_variant != 0 || (a.D == 64 && v.query_blocks != 2)) return 4;
