@@ -24,6 +24,11 @@
 // behind each of its first matrix instructions (a wave alone on its SIMD waits for each to be taken), the last of the prologue's behind
 // the first scores: 8 x 64 x 1500 against 1536, K and V from memory, 12.9 -> 12.5 us a launch.
 //
+// KSP = W: each wave takes two blocks of queries, all that its workgroup has, and every fourth block of keys, which it fetches for itself:
+// LDS gives an operand for two products instead of one, and nothing in the loop waits for another wave.  A unit's 0.33 us become 0.27,
+// the prologue (its rings are filled by four times as many loads) and the hand-over of four results cost 0.7 us more: 8 x 64 x 1500
+// against 1536 12.5 -> 11.75 us a launch, 6 layers with their copies 104 -> 98.
+//
 // Waves that share queries (KSP > 1) get them through LDS: the workgroup's rows are brought once, along the rows.  A wave's own loads
 // of its operands, 32 rows an instruction, took 1.1 us for each 32 queries.  Launches, us, with their own loads and like this: 8 x 64 x
 // 1500 against 1536 13.4 -> 12.6, 8 x 64 x 300^2 6.9 -> 6.4; whole passes with both changes, in turn with the code before them: 6 of the
@@ -96,12 +101,12 @@ constexpr int pipe_lds_bytes(int D, int NQB, int KSP, int W, int MASK) {
 }
 
 // NQB: 32-query blocks per wave.  KSP = 2: the second half of the W waves shares the queries of the first and takes alternate
-// 32-key blocks.
+// 32-key blocks.  KSP = W: see above.
 // PAD: heads of a.Dv elements (a multiple of 8 below D) on copies of K and V whose rows are zero-padded to D.
 // MASK: 1 where rows start on dwords and Nkv is even, 2 where not; 128-wide heads, no slopes.
 template <int D, int NQB, int KSP, int W, bool PAD, int MASK>
 __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a, const int n_qtiles) {
-    static_assert(NQB == 1 || (NQB == 2 && D == 64 && KSP == 1 && !PAD), "forms");
+    static_assert(NQB == 1 || (NQB == 2 && D == 64 && (KSP == 1 || KSP == W) && !PAD && !MASK), "forms");
     static_assert(!MASK || (D == 128 && NQB == 1 && W == 4 && !PAD), "masked forms");       // (none of them HALVES)
     constexpr int PIPE_THREADS = W * 64;
     constexpr int QG   = W / KSP;                                 // waves that take different queries
@@ -119,7 +124,8 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     constexpr int  NLS  = HALVES ? NLD : 2 * NLD;                 // loads per wave and step
     constexpr int R    = RING;
     // steps ahead of the current one that its start requests, and loads that may still be under way then
-    constexpr int DK   = R, DV = NQB == 2 ? DK - 1 : DK - 2;
+    constexpr bool ALONE = KSP == W;                              // a wave fetches the blocks it takes, all of them, and nobody else reads them
+    constexpr int DK   = ALONE ? R - 1 : R, DV = NQB == 2 ? DK - 1 : DK - 2;
     constexpr int NML  = MASK == 2 ? 3 : MASK ? 2 : 0;            // ... of its own mask block
     constexpr int AHEAD = DK - 1;                                 // ... of which the last go out behind the first scores
     constexpr int OPEN = (DV - 1) * (NLS + NML);
@@ -196,7 +202,7 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     }
 
     const int n_keys  = k_end - k_begin;
-    int       n_steps = (n_keys + SKEYS - 1) / SKEYS;
+    int       n_steps = ALONE ? ((n_keys + 31) / 32 + KSP - 1 - kgroup) / KSP : (n_keys + SKEYS - 1) / SKEYS;      // (ALONE: the wave's own, 0 at worst)
     const uint64_t kbase = (uint64_t)(a.k + (int64_t)hk * a.nbk2 + (int64_t)bk * a.nbk3 + (int64_t)k_begin * a.nbk1);
     const uint64_t vbase = (uint64_t)(a.v + (int64_t)hk * a.nbv2 + (int64_t)bk * a.nbv3 + (int64_t)k_begin * a.nbv1);
 
@@ -541,7 +547,7 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
         if constexpr (START) {
             // what was requested OPEN loads ago and earlier has landed, in every wave's share
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(OPEN) : "memory");
-            __builtin_amdgcn_s_barrier();
+            if (!ALONE) __builtin_amdgcn_s_barrier();
         }
         if constexpr (MASK != 0) {
             add_mask(s[U], U, KSP * step + kgroup);
@@ -717,6 +723,45 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
         else             trade(I1{});
     }
 
+    // ---- ... and the four that have its keys among them: wave 2 qb + db gets block db of the columns of query block qb --------
+    float16v part = {};
+    if constexpr (ALONE) {
+        static_assert(!ALONE || (W == 4 && NQB * DB == W), "a block for every wave");
+        static_assert(!ALONE || W * W * 4096 + W * NQB * 512 <= pipe_lds_bytes(D, NQB, KSP, W, MASK), "hand-over");
+        float4v * const box = (float4v *)lds + lane;                             // [wave][block][quarter][lane]
+        float2 * const  ml  = (float2 *)(lds + W * W * 4096) + lane;             // [wave][query block][lane]
+#pragma unroll
+        for (int i = 0; i < W; i++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const float16v & o = oacc[i / DB][i % DB];
+                box[((wave * W + i) * 4 + g) * 64] = float4v{o[4 * g], o[4 * g + 1], o[4 * g + 2], o[4 * g + 3]};
+            }
+#pragma unroll
+        for (int qb = 0; qb < NQB; qb++) ml[(wave * NQB + qb) * 64] = make_float2(m[qb], lacc[qb][0]);
+        __syncthreads();
+        // (a wave without a key of its own has a sum of zero)
+        float2 of[W];
+        float  M = -INFINITY, L = 0.0f;
+#pragma unroll
+        for (int w = 0; w < W; w++) of[w] = ml[(w * NQB + wave / DB) * 64];
+#pragma unroll
+        for (int w = 0; w < W; w++) M = of[w].y == 0.0f ? M : fmaxf(M, of[w].x);
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+            const float f = of[w].y == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(of[w].x - M);
+            L += of[w].y * f;
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const float4v o = box[((w * W + wave) * 4 + g) * 64];
+#pragma unroll
+                for (int e = 0; e < 4; e++) part[4 * g + e] += o[e] * f;
+            }
+        }
+        m[0]       = M;
+        lacc[0][0] = L;
+    }
+
     // ---- normalise and write dst[D, Hq, Nq, B], or hand the unnormalised partial to the merge kernel -----------------------
     const int dv = PAD ? a.Dv : D;                      // dst rows are dv floats; partial rows are D apart
     if constexpr (KSP == 1) {
@@ -766,7 +811,7 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
         // (short launches: straight from the accumulators, the detour would cost them a round trip)
         const float ltot = lacc[0][0];
         const float inv  = a.n_splits > 1 ? 1.0f : (ltot > 0.0f ? 1.0f / ltot : 0.0f);
-        const int   qi   = q0 + l32;
+        const int   qi   = q0 + (ALONE ? wave / DB * 32 : 0) + l32;
         if (qi < a.Nq && (!MASK || !(bad >> l32 & 1))) {
             const int64_t row = ((int64_t)b * a.Nq + qi) * a.Hq + h;
             float * out = a.n_splits > 1 ? a.part_acc + (row * a.n_splits + split) * D : a.dst + row * dv;
@@ -774,15 +819,16 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
             for (int i = 0; i < DB / 2; i++)
 #pragma unroll
                 for (int g = 0; g < 4; g++) {
+                    const float16v & x = ALONE ? part : oacc[0][i];
                     float4 o;
-                    o.x = oacc[0][i][g * 4 + 0] * inv;
-                    o.y = oacc[0][i][g * 4 + 1] * inv;
-                    o.z = oacc[0][i][g * 4 + 2] * inv;
-                    o.w = oacc[0][i][g * 4 + 3] * inv;
-                    const int d = (kgroup * (DB / 2) + i) * 32 + g * 8 + hh * 4;
+                    o.x = x[g * 4 + 0] * inv;
+                    o.y = x[g * 4 + 1] * inv;
+                    o.z = x[g * 4 + 2] * inv;
+                    o.w = x[g * 4 + 3] * inv;
+                    const int d = ((ALONE ? wave % DB : kgroup * (DB / 2)) + i) * 32 + g * 8 + hh * 4;
                     if (!PAD || a.n_splits > 1 || d < a.Dv) *(float4 *)(out + d) = o;
                 }
-            if (a.n_splits > 1 && hh == 0 && kgroup == 0) {
+            if (a.n_splits > 1 && hh == 0 && (ALONE ? wave % DB : kgroup) == 0) {
                 float * pm = a.part_ml + (row * a.n_splits + split) * 2;
                 pm[0] = ltot == 0.0f ? -INFINITY : m[0] * 0.6931471805599453f;
                 pm[1] = ltot;
@@ -843,6 +889,15 @@ int fattn_pipe_waves(const FattnArgs & a, int ktype, const FattnMmaVariant & v) 
     return groups(q4) > a.n_cus && 2 * fill(groups(2 * q4)) <= fill(groups(q4)) ? 8 : 4;
 }
 
+// Calls of the pairs' form whose four waves rather take different keys of the same 64 queries (KSP = W): a CU holds one such workgroup,
+// and its waves have to have keys enough for the longer hand-over.  us a call, pairs and like this, in graphs: 8 heads x 1500 13.2, 12.6,
+// x 1000 10.4, 10.1, x 768 8.9, 8.9, x 500 7.4, 7.7; 4 x 1500 12.7, 12.0, 4 x 800 9.7, 9.25.  Nearly every CU with one (all ask L2 for
+// their keys at once): 12 x 1300 14.05, 13.5, 16 x 1000 11.5, 11.8.
+static bool pipe_alone(const FattnArgs & a) {
+    const int64_t wgs = (int64_t)((a.Nq + 63) / 64) * a.Hq * a.B * a.n_splits;
+    return a.tile_variant == 0 && wgs <= a.n_cus && (a.n_splits > 1 ? a.keys_per_split : a.Nkv) >= (wgs * 8 <= (int64_t)a.n_cus * 7 ? 768 : 1152);
+}
+
 int fattn_pipe_launch(const FattnArgs & a, const FattnMmaVariant & v, int waves, hipStream_t stream) {
     const bool pad = a.Dv != a.D;
     if (a.masked) {
@@ -855,6 +910,7 @@ int fattn_pipe_launch(const FattnArgs & a, const FattnMmaVariant & v, int waves,
         return waves == 8 ? launch<64, 2, 1, 8, false>(a, stream) : launch<64, 2, 1, 4, false>(a, stream);
     }
     if (a.D == 64) {
+        if (v.key_split == 2 && !pad && pipe_alone(a)) return launch<64, 2, 4, 4, false>(a, stream);
         if (v.key_split == 2) return pad ? launch<64, 1, 2, 4, true>(a, stream) : launch<64, 1, 2, 4, false>(a, stream);
         return pad ? launch<64, 1, 1, 4, true>(a, stream) : launch<64, 1, 1, 4, false>(a, stream);
     }
