@@ -498,7 +498,7 @@ int fill_launch(void * ptr, int value, size_t size, hipStream_t stream) {
     const size_t tail = size - head - n16 * 16;
     const size_t threads = n16 > 16 ? n16 : 16;                    // head and tail are below 16 bytes each
     if ((threads + 255) / 256 > 0x7fffffffu) return (int)hipErrorInvalidValue;
-    hipLaunchKernelGGL(fill_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream,
+    fattn_launch(fill_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream,
                        (unsigned char *)ptr, (unsigned)(value & 0xff), head, n16, tail);
     return (int)hipGetLastError();
 }
@@ -524,15 +524,15 @@ int kv_to_f16_launch(const FattnArgs & a, int ktype, int vtype, void * dst, hipS
     const bool small = n + 256 < ((int64_t)1 << 31);             // 32-bit indices do
     if (ktype != vtype || a.Dv != a.D) {
         if (rider) return (int)hipErrorInvalidValue;
-        if (small) hipLaunchKernelGGL(kv_to_f16_mixed_kernel<uint32_t>, g, dim3(256), 0, stream, a, ktype, vtype, (char *)dst, v);
-        else       hipLaunchKernelGGL(kv_to_f16_mixed_kernel<int64_t>, g, dim3(256), 0, stream, a, ktype, vtype, (char *)dst, v);
+        if (small) fattn_launch(kv_to_f16_mixed_kernel<uint32_t>, g, dim3(256), 0, stream, a, ktype, vtype, (char *)dst, v);
+        else       fattn_launch(kv_to_f16_mixed_kernel<int64_t>, g, dim3(256), 0, stream, a, ktype, vtype, (char *)dst, v);
         return (int)hipGetLastError();
     }
     switch (ktype) {
 #define KV16(T)                                                                                                         \
     case T:                                                                                                             \
-        if (small) hipLaunchKernelGGL((kv_to_f16_kernel<uint32_t, T>), g, dim3(256), 0, stream, a, (char *)dst, x, v);    \
-        else       hipLaunchKernelGGL((kv_to_f16_kernel<int64_t, T>), g, dim3(256), 0, stream, a, (char *)dst, x, v);     \
+        if (small) fattn_launch((kv_to_f16_kernel<uint32_t, T>), g, dim3(256), 0, stream, a, (char *)dst, x, v);    \
+        else       fattn_launch((kv_to_f16_kernel<int64_t, T>), g, dim3(256), 0, stream, a, (char *)dst, x, v);     \
         break
         KV16(MI355X_TYPE_F32);
         KV16(MI355X_TYPE_Q8_0);
@@ -582,19 +582,19 @@ static bool prepare_index(CpyArgs & a, int64_t unit0, int64_t threads) {
     do {                                                                                                                  \
         const dim3 g_((unsigned)(((threads) + 255) / 256));                                                               \
         if (narrow) {                                                                                                     \
-            hipLaunchKernelGGL((KERNEL<decltype(v), __VA_ARGS__>), g_, dim3(256), 0, stream, v);                          \
+            fattn_launch((KERNEL<decltype(v), __VA_ARGS__>), g_, dim3(256), 0, stream, v);                          \
             break;                                                                                                        \
         }                                                                                                                 \
         WideCopy<uint32_t> w_;                                                                                            \
         (CpyArgs &)w_ = a;                                                                                                \
         w_.whole = (pieces);                                                                                              \
         if (prepare_index(w_, unit0, threads)) {                                                                          \
-            hipLaunchKernelGGL((KERNEL<WideCopy<uint32_t>, __VA_ARGS__>), g_, dim3(256), 0, stream, w_);                  \
+            fattn_launch((KERNEL<WideCopy<uint32_t>, __VA_ARGS__>), g_, dim3(256), 0, stream, w_);                  \
         } else {                                                                                                          \
             WideCopy<int64_t> l_;                                                                                         \
             (CpyArgs &)l_ = w_;                                                                                           \
             const dim3 lg_((unsigned)((((walked) && (threads) > MAX_WALKED ? MAX_WALKED : (threads)) + 255) / 256));      \
-            hipLaunchKernelGGL((KERNEL<WideCopy<int64_t>, __VA_ARGS__>), lg_, dim3(256), 0, stream, l_);                  \
+            fattn_launch((KERNEL<WideCopy<int64_t>, __VA_ARGS__>), lg_, dim3(256), 0, stream, l_);                  \
         }                                                                                                                 \
     } while (0)
 // (es: bytes of a source element, whole blocks counted as one)

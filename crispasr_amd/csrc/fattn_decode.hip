@@ -955,7 +955,7 @@ int launch_one(FattnArgs a, hipStream_t stream) {
             static std::atomic<uint64_t> short_lds_allowed{0};
             const hipError_t e = fattn_allow_lds((const void *)fattn_decode_short_kernel<D, TYPE, MASK, RAW, V8, PAD>, lds, short_lds_allowed);
             if (e != hipSuccess) return (int)e;
-            hipLaunchKernelGGL((fattn_decode_short_kernel<D, TYPE, MASK, RAW, V8, PAD>), dim3((unsigned)a.n_splits, (unsigned)a.Hkv, (unsigned)a.B),
+            fattn_launch((fattn_decode_short_kernel<D, TYPE, MASK, RAW, V8, PAD>), dim3((unsigned)a.n_splits, (unsigned)a.Hkv, (unsigned)a.B),
                                dim3(DEC_THREADS), lds, stream, p);
             return (int)hipGetLastError();
         }
@@ -970,7 +970,7 @@ int launch_one(FattnArgs a, hipStream_t stream) {
     static std::atomic<uint64_t> lds_allowed{0};
     const hipError_t e = fattn_allow_lds((const void *)fattn_decode_kernel<D, TYPE, MASK, RAW, V8, PAD>, lds, lds_allowed);
     if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL((fattn_decode_kernel<D, TYPE, MASK, RAW, V8, PAD>), grid, dim3(DEC_THREADS), lds, stream, a);
+    fattn_launch((fattn_decode_kernel<D, TYPE, MASK, RAW, V8, PAD>), grid, dim3(DEC_THREADS), lds, stream, a);
     return (int)hipGetLastError();
 }
 

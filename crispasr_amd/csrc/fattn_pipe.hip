@@ -854,7 +854,7 @@ int launch(const FattnArgs & a, hipStream_t stream) {
     static std::atomic<uint64_t> lds_allowed{0};
     const hipError_t e = fattn_allow_lds((const void *)fattn_pipe_kernel<D, NQB, KSP, W, PAD, MASK>, lds, lds_allowed);
     if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL((fattn_pipe_kernel<D, NQB, KSP, W, PAD, MASK>), dim3((unsigned)wgs), dim3(W * 64), (size_t)lds, stream, a, n_qtiles);
+    fattn_launch((fattn_pipe_kernel<D, NQB, KSP, W, PAD, MASK>), dim3((unsigned)wgs), dim3(W * 64), (size_t)lds, stream, a, n_qtiles);
     return (int)hipGetLastError();
 }
 

@@ -487,7 +487,7 @@ int launch_d(const FattnRelposArgs & a, hipStream_t stream) {
         static std::atomic<uint64_t> lds_allowed{0};                                                                          \
         const hipError_t e = fattn_allow_lds((const void *)fattn_relpos_kernel<D, NW, ADD, F16>, lds, lds_allowed);           \
         if (e != hipSuccess) return (int)e;                                                                                   \
-        hipLaunchKernelGGL((fattn_relpos_kernel<D, NW, ADD, F16>), dim3((unsigned)grid), dim3(NW * 64), lds, stream, a);    \
+        fattn_launch((fattn_relpos_kernel<D, NW, ADD, F16>), dim3((unsigned)grid), dim3(NW * 64), lds, stream, a);    \
     } while (0)
     if (!a.add)          FR_LAUNCH(false, false);
     else if (a.add_f16)  FR_LAUNCH(true, true);

@@ -104,10 +104,10 @@ int launch_typed(const FattnArgs & a, hipStream_t stream) {
     const dim3 grid((unsigned)(rows * a.n_splits));
     const dim3 block(VEC_THREADS);
     const int  lanes = (a.D + 7) / 8;
-    if (lanes <= 4)       hipLaunchKernelGGL((fattn_vec_kernel<TYPE, 4>),  grid, block, 0, stream, a);
-    else if (lanes <= 8)  hipLaunchKernelGGL((fattn_vec_kernel<TYPE, 8>),  grid, block, 0, stream, a);
-    else if (lanes <= 16) hipLaunchKernelGGL((fattn_vec_kernel<TYPE, 16>), grid, block, 0, stream, a);
-    else                  hipLaunchKernelGGL((fattn_vec_kernel<TYPE, 32>), grid, block, 0, stream, a);
+    if (lanes <= 4)       fattn_launch((fattn_vec_kernel<TYPE, 4>),  grid, block, 0, stream, a);
+    else if (lanes <= 8)  fattn_launch((fattn_vec_kernel<TYPE, 8>),  grid, block, 0, stream, a);
+    else if (lanes <= 16) fattn_launch((fattn_vec_kernel<TYPE, 16>), grid, block, 0, stream, a);
+    else                  fattn_launch((fattn_vec_kernel<TYPE, 32>), grid, block, 0, stream, a);
     return (int)hipGetLastError();
 }
 
@@ -130,6 +130,6 @@ int fattn_merge_launch(const FattnArgs & a, hipStream_t stream) {
     const int rows = a.Nq * a.Hq * a.B;
     const int rows_per_block = 4 * (64 / (a.D / 4));          // D is a multiple of 8, at most 256
     const dim3 grid((unsigned)((rows + rows_per_block - 1) / rows_per_block));
-    hipLaunchKernelGGL(fattn_merge_kernel, grid, dim3(256), 0, stream, a, rows);
+    fattn_launch(fattn_merge_kernel, grid, dim3(256), 0, stream, a, rows);
     return (int)hipGetLastError();
 }

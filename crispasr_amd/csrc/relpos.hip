@@ -329,7 +329,7 @@ int launch_dt(const RelposArgs & a, hipStream_t stream) {
     if (ea != hipSuccess) return (int)ea;
     const int64_t groups = (int64_t)((a.n_qblocks + RP_WAVES - 1) / RP_WAVES) * a.B;
     const dim3 grid((unsigned)((groups + 7) / 8 * 8 * a.n_chunks * a.H));
-    hipLaunchKernelGGL((relpos_bias_kernel<D, RTYPE>), grid, dim3(RP_WAVES * 64), LDS, stream, a);
+    fattn_launch((relpos_bias_kernel<D, RTYPE>), grid, dim3(RP_WAVES * 64), LDS, stream, a);
     return (int)hipGetLastError();
 }
 
