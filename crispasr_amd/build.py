@@ -16,6 +16,8 @@ SOURCES = ["api.hip", "fattn_vec.hip", "fattn_mma.hip", "fattn_pipe.hip", "fattn
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # the first seven numbers among a kernel's parameters are in scalar registers when a wave starts
+    "-mllvm", "-amdgpu-kernarg-preload-count=7",
     "-Wall", "-Wno-unused-function",
 ]
 

@@ -4,22 +4,26 @@
 
 #include "fattn_common.h"
 
+#include <stddef.h>
+
 // The two forms a copy's arguments take.  Narrow: both sides walked by the same (at most) four counts, units of dimension 0
 // contiguous, spans below 4 GiB - what every cache write and read of the runtimes comes down to once adjacent dimensions that
 // lie behind one another are one.  It is what it is because of its size: a launch whose kernel arguments take more than 112
 // bytes costs the host 0.8 us more, 2 us on an idle queue (measured, bytes against us a launch in a chain of empty kernels: 16
 // 2.5, 64 2.6, 112 2.7, 120 3.5, 352 3.7), and the 60 copies of a decoder step were bound by that.  Wide: everything else.
+// The loads' addresses come from the first 56 bytes, so that a large copy's can be in registers when its waves start (see ArgTail).
 struct NarrowCopy {
     const char * src;
+    uint32_t     n;                        // units
+    uint32_t     d[3], m[3], shifts;       // divisions by counts 0 .. 2 (FastDiv, a byte for each shift); the fourth byte: whole_pieces
+    uint32_t     snb[3], dnb[3];           // pitches of counts 1 .. 3
     char *       dst;
     int64_t      mirror;
-    uint32_t     n;                        // units
-    FastDiv      div[3];
-    uint32_t     snb[3], dnb[3];           // pitches of counts 1 .. 3
-    uint32_t     whole;                    // see whole_pieces
     typedef uint32_t index, offset;
+    template <typename F> __host__ __device__ void pointers(F f) { f(src, dst); }
 };
-static_assert(sizeof(NarrowCopy) <= 112, "arguments of a cheap launch");
+static_assert(sizeof(NarrowCopy) <= 112 && offsetof(NarrowCopy, dnb) < 56, "arguments of a cheap launch");
+static __host__ __device__ __forceinline__ uint32_t whole_of(const NarrowCopy & a) { return a.shifts >> 24; }
 
 // The same two forms for SET_ROWS: narrow where rows, indices and pitches need 32 bits and nothing is mirrored.  Broadcast
 // indices have a pitch of zero in it (x1, x2: their pitches along dimensions 2 and 3).
@@ -44,9 +48,13 @@ static __host__ __device__ __forceinline__ Units units_of(uint32_t i, const Fast
     const uint32_t r1 = divide(i, div[0]), r2 = divide(r1, div[1]), i3 = divide(r2, div[2]);
     return {i - r1 * div[0].d, r1 - r2 * div[1].d, r2 - i3 * div[2].d, i3};
 }
+static __host__ __device__ __forceinline__ Units units_of(uint32_t i, const NarrowCopy & a) {
+    const uint32_t s = a.shifts;
+    return units_of(i, {FastDiv{a.d[0], a.m[0], s & 31}, FastDiv{a.d[1], a.m[1], s >> 8 & 31}, FastDiv{a.d[2], a.m[2], s >> 16 & 31}});
+}
 // byte offsets of unit i on both sides; sstep and dstep: bytes from one unit to the next along dimension 0
 static __host__ __device__ __forceinline__ void offsets(const NarrowCopy & a, uint32_t i, int, uint32_t sstep, uint32_t dstep, uint32_t & so, uint32_t & to) {
-    const Units u = units_of(i, a.div);
+    const Units u = units_of(i, a);
     so = u.i0 * sstep + u.i1 * a.snb[0] + u.i2 * a.snb[1] + u.i3 * a.snb[2];
     to = u.i0 * dstep + u.i1 * a.dnb[0] + u.i2 * a.dnb[1] + u.i3 * a.dnb[2];
 }
@@ -121,14 +129,17 @@ static bool narrow_copy(const CpyArgs & a, int64_t unit0, int64_t sstep, int64_t
     v.dst    = a.dst;
     v.mirror = a.mirror;
     v.n      = (uint32_t)a.n;
-    v.whole  = (uint32_t)whole_pieces(a.dst, t, dstep);
+    v.shifts = (uint32_t)whole_pieces(a.dst, t, dstep) << 24;
     int64_t sspan = sstep, dspan = dstep;
     sp[0] = sstep;
     dp[0] = dstep;
     for (int i = 0; i < 4; i++)
         if (!add_span(sspan, count[i], sp[i]) || !add_span(dspan, count[i], dp[i])) return false;
     for (int i = 0; i < 3; i++) {
-        v.div[i] = fast_div((uint32_t)count[i]);
+        const FastDiv f = fast_div((uint32_t)count[i]);
+        v.d[i] = f.d;
+        v.m[i] = f.m;
+        v.shifts |= f.s << (8 * i);
         v.snb[i] = (uint32_t)sp[i + 1];
         v.dnb[i] = (uint32_t)dp[i + 1];
     }

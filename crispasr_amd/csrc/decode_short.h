@@ -6,26 +6,31 @@
 
 #include "fattn_common.h"
 
+#include <stddef.h>
+
 // A step's call as the runtimes make it: up to 16 rows per KV head, K and V alike in their strides, no slopes, a mask that is one
 // head's or every head's own and one sequence's or every sequence's own.  Extents that one value stands for have a stride of zero.
+// The first requests of K, V and Q come from the first 56 bytes (see ArgTail).
 struct DecodeShort {
-    const char * q;
     const char * k;
     const char * v;
+    const char * q;
+    uint32_t     nbk1, nbk2, nbk3;    // and V's
+    uint32_t     nbq1, nbq2, nbq3;
+    uint32_t     Nkv;
+    uint32_t     rows;                // Nq | gqa << 5 | n_splits << 10 | keys_per_split / 32 << 17, or, not cut, the sequences in the first
+                                      // round << 17 (0: in their own order, see decode_turns)
     const char * mask;
+    uint32_t     nbm1, nbm2, nbm3;
+    uint32_t     heads;               // Hkv | B << 16
+    float        scale;
+    uint32_t     Dv;
     float *      dst;
     float *      part_acc;            // the (max, sum) pairs lie right behind it
     unsigned *   counters;
-    uint32_t     nbq1, nbq2, nbq3;
-    uint32_t     nbk1, nbk2, nbk3;    // and V's
-    uint32_t     nbm1, nbm2, nbm3;
-    float        scale;
-    uint32_t     Nkv;
-    uint32_t     rows;                // Nq | gqa << 5 | n_splits << 10 | keys_per_split / 32 << 17 (0: not cut)
-    uint32_t     heads;               // Hkv | B << 16
-    uint32_t     Dv;                  // | sequences in the first round << 16 (0: in their own order, see decode_turns)
+    template <typename F> __host__ __device__ void pointers(F f) { f(k, v, q, mask, dst, part_acc, counters); }
 };
-static_assert(sizeof(DecodeShort) <= 112, "see above");
+static_assert(sizeof(DecodeShort) == 112 && offsetof(DecodeShort, mask) == 56, "see above");
 
 // Sequences of different lengths in one call (a mask of every sequence's own ends each), more workgroups than CUs: a CU that gets the
 // workgroups of two long ones is the last.  Workgroup n_cus + i comes to the CU of workgroup i, so the sequences of the first round (a
@@ -81,7 +86,7 @@ static __host__ __device__ __forceinline__ FattnArgs decode_expand(const DecodeS
     FattnArgs a = {};
     a.q = p.q; a.k = p.k; a.v = p.v; a.mask = p.mask; a.dst = p.dst;
     a.D  = D;
-    a.Dv = (int)(p.Dv & 0xFFFFu);
+    a.Dv = (int)p.Dv;
     a.Nq = (int)(p.rows & 31u);
     a.gqa = (int)(p.rows >> 5 & 31u);
     a.n_splits = (int)(p.rows >> 10 & 127u);
