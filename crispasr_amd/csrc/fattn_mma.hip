@@ -1046,15 +1046,22 @@ void fattn_mma_variant(const FattnArgs & a, int ktype, FattnMmaVariant & v) {
     const bool two_auto = wg2 >= cus && slots2 * 10 <= slots1 * 11;
     // (With a mask the split form carries its merge from 512 keys on; and a mask whose rows cannot go through LDS costs the
     // unsplit forms a quarter of their speed: there the split form wins up to 1.6 workgroups per CU.  Both were measured on 64-wide
-    // heads, whose split form skips excluded blocks; 128-wide heads have one rule with and without a mask, and from 384 keys on
-    // the pipelined kernel, which leaves out the keys ahead of the first visible one and behind the last.)
+    // heads, whose split form skips excluded blocks; 128-wide heads have one rule with and without a mask, and from 64 or 128 keys
+    // on the pipelined kernel, which leaves out the keys ahead of the first visible one and behind the last.)
     // (a zero-padded head exists in the direct forms only: its K/V are the call's own f16 copies)
     const bool direct = ktype == MI355X_TYPE_F16 && (!no_direct || a.Dv != a.D) && a.nbk1 < (1u << 24) && a.nbv1 < (1u << 24);
     const bool mdma_ok = a.masked && a.softcap == 0.0f && direct && !no_mdma && a.mask_al4 && a.Nkv >= 64 && !(a.Nkv & 1) &&
                          (uint64_t)a.Nq * a.nbm1 < (1ull << 31);
     bool ksp_auto;
-    if (a.D == 128)           ksp_auto = wg1 * 2 <= cus || (wg1 <= cus && a.Nkv >= 2048);
-    else if (!a.masked)       ksp_auto = wg1 <= cus && (wg1 * 5 <= (int64_t)cus * 3 || a.Nkv >= 1024) && a.Nkv > 128;
+    // 128-wide pairs have a CU to themselves in the pipelined kernel, and pay as long as each has one: 300 tokens x 48 heads (240 of them)
+    // under per-head masks 18.0 -> 13.9 us, plain 12.1 -> 11.3; 290 x 56 (280) 15.75 and with pairs 21.95.  64-wide ones share CUs: 1000 tokens x 20
+    // heads 14.9 -> 13.5 us a layer, 900 x 20 14.6 -> 13.8, 780 x 20 12.6 either way, 250 x 20 x 4 8.1 and with pairs 8.7.
+    const int64_t wgp = (int64_t)((a.Nq + 63) / 64) * heads;
+    const bool pipes = direct && (!a.masked || (a.Dv == 128 && a.Nkv >= 64 && a.max_bias <= 0.0f));
+    // (Of 64 keys each wave of a pair has one block: its merge shows once a quarter of the CUs run one. 64 tokens x 32 heads 4.9 us a layer
+    // either way, x 96 7.5 and with pairs 7.7, x 200 7.7, 8.85.)
+    if (a.D == 128)           ksp_auto = wg1 * 4 <= cus || (a.Nkv > 64 && (wg1 * 2 <= cus || (pipes && wgp <= cus))) || (wg1 <= cus && a.Nkv >= 2048);
+    else if (!a.masked)       ksp_auto = wg1 <= cus && (wg1 * 5 <= (int64_t)cus * 3 || (a.Nkv >= 768 && wg1 * 3 <= (int64_t)cus * 2) || a.Nkv >= 1024) && a.Nkv > 128;
     else if (!mdma_ok && a.Nkv >= 256) ksp_auto = wg1 * 5 <= (int64_t)cus * 8;
     else                      ksp_auto = wg1 <= cus && (wg1 * 5 <= (int64_t)cus * 3 || a.Nkv >= 512);
     // (a head zero-padded to 64 keeps to one query block: the two-block form stores whole rows of D floats)

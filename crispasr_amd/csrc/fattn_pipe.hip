@@ -860,18 +860,20 @@ int launch(const FattnArgs & a, hipStream_t stream) {
 
 }  // namespace
 
-// The masked calls among those over f16 rows: whole 128-wide heads, no slopes, blocks of 32 keys that end inside the rows.
-// Rows that start between dwords need LDS that two workgroups of the unsplit form do not have on one CU.  Shorter key ranges
-// stay with the tile kernel, whose prologue is shorter (128 causal tokens x 32 heads 14.0 us there with their row writes, 15.3 here;
-// 100 x 64 heads under per-head masks 10.2, 11.5; 300 x 16 12.9, 13.6; 400 x 16 15.7, 15.4).
+// The masked calls among those over f16 rows: whole 128-wide heads, no slopes.  Rows that start between dwords need LDS that two
+// workgroups of the unsplit form do not have on one CU.  Ranges from 64 keys on for pairs of waves, from 128 for the unsplit form (a caller
+// who names the form: 384, as ever).  us a call in a graph, tile kernel and this: pairs, four causal layers of 383 tokens x 32 heads with
+// their row writes 87.0, 69.9, of 256 66.3, 58.8, of 128 55.1, 51.4, of 100 52.4, 50.5; under per-head masks 100 x 8 heads 10.9, 9.5, 300 x 8
+// 14.1, 12.1; unsplit, 150 x 8 heads x 16 16.0, 14.3, 250 x 8 x 16 20.5, 17.4, 380 x 8 x 8 21.3, 17.9.
 static bool pipe_masked(const FattnArgs & a, const FattnMmaVariant & v) {
+    const int least = a.tile_variant ? 384 : v.key_split == 2 ? 64 : 128;
     return a.D == 128 && a.Dv == 128 && v.query_blocks == 1 && a.max_bias <= 0.0f &&
-           (a.n_splits > 1 ? a.keys_per_split : a.Nkv) >= 384 && (uint64_t)a.Nq * (uint64_t)a.nbm1 < (1ull << 31) &&
+           (a.n_splits > 1 ? a.keys_per_split : a.Nkv) >= least && (uint64_t)a.Nq * (uint64_t)a.nbm1 < (1ull << 31) &&
            (v.key_split == 2 || (a.mask_al4 && !(a.Nkv & 1)));
 }
 
-// Plain attention over f16 rows is this kernel's, but for the key-split form of 128-wide heads: there a wave has few blocks, and
-// the longer prologue costs what the loop gains (300 tokens x 30 heads 10.8 against 11.9 us a launch, 500 x 20 and 800 x 8 within 2%).
+// Plain attention over f16 rows is this kernel's.  (The pairs' form of 128-wide heads since queries come through LDS; us a layer, tile
+// kernel and this: 8 heads x 80 7.9, 6.9, x 300 11.0, 9.75, x 1500 25.6, 19.8, 10 x 1000 20.0, 15.45, 80-wide 8 x 1500 31.0, 24.9.)
 // Eight waves a workgroup where that leaves no CU with more of them than workgroups of four do: more of those than CUs, and their
 // number per CU even once rounded up.  (A caller who names the form gets four.)
 // Request addresses are 32-bit numbers inside a range of a head's keys, up to 8 steps of 64 behind its end: longer ones are the tile kernel's.
@@ -881,7 +883,7 @@ int fattn_pipe_waves(const FattnArgs & a, int ktype, const FattnMmaVariant & v) 
     if (keys * a.nbk1 >= ((int64_t)1 << 31) || keys * a.nbv1 >= ((int64_t)1 << 31)) return 0;
     if (v.key_split > 1 && (a.nbq1 < 0 || a.nbq1 >= 1 << 25)) return 0;        // (64 rows of Q likewise)
     if (a.masked) return pipe_masked(a, v) ? 4 : 0;
-    if (v.key_split == 2) return a.D == 128 ? 0 : 4;
+    if (v.key_split == 2) return 4;
     if (a.tile_variant != 0 || (a.D == 64 && v.query_blocks != 2)) return 4;
     const int q4 = v.queries_per_workgroup;
     auto groups  = [&](int q) { return (int64_t)((a.Nq + q - 1) / q) * a.Hq * a.B * a.n_splits; };
@@ -914,6 +916,7 @@ int fattn_pipe_launch(const FattnArgs & a, const FattnMmaVariant & v, int waves,
         if (v.key_split == 2) return pad ? launch<64, 1, 2, 4, true>(a, stream) : launch<64, 1, 2, 4, false>(a, stream);
         return pad ? launch<64, 1, 1, 4, true>(a, stream) : launch<64, 1, 1, 4, false>(a, stream);
     }
+    if (v.key_split == 2) return pad ? launch<128, 1, 2, 4, true>(a, stream) : launch<128, 1, 2, 4, false>(a, stream);
     if (waves == 8) return pad ? launch<128, 1, 1, 8, true>(a, stream) : launch<128, 1, 1, 8, false>(a, stream);
     return pad ? launch<128, 1, 1, 4, true>(a, stream) : launch<128, 1, 1, 4, false>(a, stream);
 }
