@@ -293,6 +293,10 @@ static __device__ __forceinline__ void buffer_to_lds16(__amdgpu_buffer_rsrc_t bu
     asm volatile("s_add_i32 m0, %3, %4\n\tv_add_u32 %0, %2, %0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
                  : "+v"(off) : "s"(buf), "s"(inc), "s"(to), "s"(at) : "memory", "m0", "scc");
 }
+// the same with an offset that stays as it is
+static __device__ __forceinline__ void buffer_to_lds16(__amdgpu_buffer_rsrc_t buf, uint32_t off, uint32_t to, uint32_t at) {
+    asm volatile("s_add_i32 m0, %2, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(buf), "s"(to), "s"(at) : "memory", "m0", "scc");
+}
 // the same with 4 bytes a lane
 static __device__ __forceinline__ void buffer_to_lds4(__amdgpu_buffer_rsrc_t buf, uint32_t & off, uint32_t inc, uint32_t to, uint32_t at) {
     asm volatile("s_add_i32 m0, %3, %4\n\tv_add_u32 %0, %2, %0\n\tbuffer_load_dword %0, %1, 0 offen lds"

@@ -29,10 +29,17 @@
 // for them: K and V have two halves each.  K, V and the table are f16 with 16-byte aligned rows (the caller rounds F32 ones
 // first, as the reference's own graph does for the mask product's operands).
 //
-// What bounds it: the chain of a step - operand reads, product, un-skew, exponentials, product - with 1 to 2 waves on a SIMD
-// (8 x 8 heads of 128 x 750: matrix cores busy 17%, vector ALU 25%, waves waiting 41% of their cycles; neither the
-// additive mask's loads nor the blocks' are what they wait for).  Against one half, two barriers a step and operand reads two
-// at a time: 8 heads x 128, calls of 1000 tokens x 4 78.4 -> 73.0 us, 750 x 8 90.9 -> 86.0; 8 x 64, 750 x 8 62.7 -> 56.9.
+// The vector work of a tile stands beside the matrix instructions of another: a step turns tile t's scores into probabilities beside
+// the two Q products of tile t + 1, and un-skews those beside P.V.  Q_u, Q_v and the result pass through the wave's square, so that
+// the memory sees them along the rows.
+//
+// What bounds it: the blocks of a step are requested one step ahead, and its waves walk the keys in phase, so that each waits for
+// its first reader's trip to memory (8 x 8 heads of 128 x 750, two workgroups of 3 waves a CU: 70 us, 61 without the loop's
+// requests, 57 without its mask either); 40 us are ahead of the second step and behind the last, 13 of them Q_u's and Q_v's.
+// Against all of a step in one chain, operands of Q fetched as they lie and requests of six instructions, us a call: 8 heads x
+// 128, 300 tokens 22.9 -> 19.6, 120 x 8 16.9 -> 14.7, 200 x 4 22.5 -> 20.6, 1000 x 2 55.2 -> 48.7, 750 x 8 (F32 K, V and table) 88.1 -> 85.6;
+// 8 x 64, 750 x 8 46.5 -> 45.9.  Registers are short in the 128-wide forms with a mask: one spilled operand is a load whose wait
+// takes the requests in with it (+5 us at 1000 x 2), which is why sums of addresses are kept from moving out of the loop.
 #include "fattn_row.h"
 
 #include <stdlib.h>
@@ -58,6 +65,9 @@ constexpr float FR_SUM_LIMIT = 4096.0f;               // a tile's 16 probabiliti
 template <int D> constexpr int fr_kp() { return 2 * D; }          // bytes per K / table row in LDS (chunks swizzled, no padding)
 template <int D> __device__ __forceinline__ int fr_swz(int r) { return D == 64 ? (r >> 1) & 7 : r & 15; }
 template <int D> __device__ __forceinline__ int fr_swz_v(int r) { return D == 64 ? r & 7 : (r & 3) << 2; }
+// what stands before it stays there, what stands behind it too
+#define FR_FENCE() __builtin_amdgcn_sched_barrier(0)
+constexpr int FR_RD = 3, FR_VD = 2;                   // operands of the two Q products and of P.V that are read ahead (four: scratch)
 // two K tiles, two V tiles, NW + 1 table blocks (NW in use, one being written), one un-skew square per wave
 template <int D, int NW> constexpr int fr_lds_bytes() { return (4 + NW + 1) * 32 * fr_kp<D>() + NW * 32 * FR_SQP * 4; }
 
@@ -117,93 +127,95 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     const int      lr = lane / CH, lc = lane % CH;
     const uint32_t ck = (uint32_t)((lc ^ fr_swz<D>(lr)) * 16), cv = (uint32_t)((lc ^ fr_swz_v<D>(lr)) * 16);
     static_assert(RPI == 4 || RPI == 8, "the swizzles of rows r and r + RPI * ins differ by 4 * (ins % (16 / RPI)) (K) or not at all (V)");
-    // Rows row0 .. row0 + 31 of a tensor, in one of two layouts.  (NW = 3: the last wave repeats an instruction of the one before.)
-    auto dma_rows = [&](char * dst, const char * base, int64_t nb1, int row0, int last_row, auto is_v, auto is_first) __attribute__((always_inline)) {
-        constexpr bool V      = decltype(is_v)::value;
-        constexpr bool FIRST  = decltype(is_first)::value;            // before the loop: one form for all, instructions are cold
-        const uint32_t to     = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)dst;
-        const uint32_t nb     = (uint32_t)nb1;                        // (row offsets inside a tile are 32-bit)
-        uint32_t       lrow   = (uint32_t)lr;
-        asm volatile("" : "+v"(lrow));                                // (its products are not worth registers in the loop)
-        if (!FIRST && __builtin_expect(row0 >= 0 && row0 + 31 <= last_row, 1)) {
-            const uint64_t at = (uint64_t)(base + (int64_t)row0 * nb1);
+    // Rows row0 .. row0 + 31 of a tensor, in one of two layouts, before the loop.  (NW = 3: the last wave repeats an instruction of
+    // the one before.)
+    auto dma_rows = [&](char * dst, const char * base, int64_t nb1, int row0, int last_row, bool is_v) __attribute__((always_inline)) {
+        const uint32_t to    = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)dst;
+        const uint32_t nb    = (uint32_t)nb1;                         // (row offsets inside a tile are 32-bit)
+        const int      first = min(max(row0, 0), last_row);
+        const uint64_t at    = (uint64_t)(base + (int64_t)first * nb1);
 #pragma unroll
-            for (int j = 0; j < NDM; j++) {
-                const uint32_t ins = min((uint32_t)(j * NW + wave), (uint32_t)TI - 1);         // uniform
-                load_to_lds16<true>(at + ins * RPI * nb, lrow * nb + (V ? cv : ck ^ ((ins & (16 / RPI - 1)) * 64)), to + ins * 1024);
-            }
-        } else {
-            const int      first = min(max(row0, 0), last_row);
-            const uint64_t at    = (uint64_t)(base + (int64_t)first * nb1);
-            auto instruction = [&](int j) __attribute__((always_inline)) {
-                const uint32_t ins = min((uint32_t)(j * NW + wave), (uint32_t)TI - 1);
-                const uint32_t rr  = (uint32_t)(min(max(row0 + (int)ins * RPI + lr, 0), last_row) - first);
-                load_to_lds16<true>(at, rr * nb + (V ? cv : ck ^ ((ins & (16 / RPI - 1)) * 64)), to + ins * 1024);
-            };
-            // (two loops: the compiler has crashed over an unroll count that depends on the instantiation)
-            if constexpr (FIRST) {
-#pragma unroll
-                for (int j = 0; j < NDM; j++) instruction(j);
-            } else {
-#pragma unroll 1
-                for (int j = 0; j < NDM; j++) instruction(j);
-            }
+        for (int j = 0; j < NDM; j++) {
+            const uint32_t ins = min((uint32_t)(j * NW + wave), (uint32_t)TI - 1);             // uniform
+            const uint32_t rr  = (uint32_t)(min(max(row0 + (int)ins * RPI + lr, 0), last_row) - first);
+            load_to_lds16<true>(at, rr * nb + (is_v ? cv : ck ^ ((ins & (16 / RPI - 1)) * 64)), to + ins * 1024);
         }
     };
-    typedef std::integral_constant<bool, false> KLayout;
-    typedef std::integral_constant<bool, true>  VLayout;
-    auto dma_k = [&](int t, auto first) __attribute__((always_inline)) { dma_rows(kt + (t & 1) * 32 * KP, kbase, a.nbk1, 32 * t, a.Nkv - 1, KLayout{}, first); };
-    auto dma_v = [&](int t, auto first) __attribute__((always_inline)) { dma_rows(vt + (t & 1) * 32 * KP, vbase, a.nbv1, 32 * t, a.Nkv - 1, VLayout{}, first); };
+    auto dma_k = [&](int t) __attribute__((always_inline)) { dma_rows(kt + (t & 1) * 32 * KP, kbase, a.nbk1, 32 * t, a.Nkv - 1, false); };
+    auto dma_v = [&](int t) __attribute__((always_inline)) { dma_rows(vt + (t & 1) * 32 * KP, vbase, a.nbv1, 32 * t, a.Nkv - 1, true); };
     auto slot_of = [&](int beta) { return ring + ((beta + NW - 1) % FR_SLOTS) * 32 * KP; };   // beta >= 1 - NW
-    auto dma_r = [&](int beta, auto first) __attribute__((always_inline)) { dma_rows(slot_of(beta), rbase, a.nbr1, p_base0 + 32 * beta, NR - 1, KLayout{}, first); };
+    auto dma_r = [&](int beta, char * to) __attribute__((always_inline)) { dma_rows(to, rbase, a.nbr1, p_base0 + 32 * beta, NR - 1, false); };
 
-    // ---- prologue: table blocks 1 - NW .. 1, the first K and V tiles, Q_u and Q_v as B operands ---------------------
+    // ---- prologue: table blocks 1 - NW .. 2, the first K tiles and V tile, Q_u and Q_v as B operands -----------------
+    // (block 1 - NW, which only the last wave reads and only here, lies in V's second half: its slot has block 2 already)
+    char * const first_block = vt + 32 * KP;
+    dma_r(1 - NW, first_block);
 #pragma unroll 1
-    for (int beta = 1 - NW; beta <= 1; beta++) dma_r(beta, std::true_type{});
-    dma_k(0, std::true_type{});
-    dma_v(0, std::true_type{});
+    for (int beta = 2 - NW; beta <= 2; beta++) dma_r(beta, slot_of(beta));
+    dma_k(0);
+    dma_v(0);
+    dma_k(1);
+    // Q_u and Q_v come along the rows, 4 of 64 values an instruction, and turn into B operands in the wave's square, as f16: fetched as
+    // the operands lie an instruction takes 32 bytes of each of 32 rows
     half8 qu[KS], qv[KS];
     {
-        const float * pu = (const float *)(a.qu + (int64_t)iq * a.nbu1 + (int64_t)h * a.nbu2 + (int64_t)b * a.nbu3);
-        const float * pv = (const float *)(a.qv + (int64_t)iq * a.nbw1 + (int64_t)h * a.nbw2 + (int64_t)b * a.nbw3);
-        const float   qs = a.scale * FR_LOG2E;
+        constexpr int QP = D / 64;                                    // pieces of 64 values a row
+        const int     qr = lane >> 4, qc = lane & 15;
+        float4v       raw[2 * QP][8];
 #pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            const float4v u0 = *(const float4v *)(pu + ks * 16 + hh * 8), u1 = *(const float4v *)(pu + ks * 16 + hh * 8 + 4);
-            const float4v w0 = *(const float4v *)(pv + ks * 16 + hh * 8), w1 = *(const float4v *)(pv + ks * 16 + hh * 8 + 4);
+        for (int i = 0; i < 2 * QP; i++) {
+            const bool    u  = i < QP;
+            const char  * at = (u ? a.qu + (int64_t)h * a.nbu2 + (int64_t)b * a.nbu3 : a.qv + (int64_t)h * a.nbw2 + (int64_t)b * a.nbw3) + i % QP * 256 + qc * 16;
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                qu[ks][e] = (_Float16)(u0[e] * qs); qu[ks][e + 4] = (_Float16)(u1[e] * qs);
-                qv[ks][e] = (_Float16)w0[e];        qv[ks][e + 4] = (_Float16)w1[e];
+            for (int j = 0; j < 8; j++) raw[i][j] = *(const float4v *)(at + (int64_t)min(i0w + 4 * j + qr, a.Nq - 1) * (u ? a.nbu1 : a.nbw1));
+        }
+        const float qs = a.scale * FR_LOG2E;
+#pragma unroll
+        for (int i = 0; i < 2 * QP; i++) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                half4 x;
+#pragma unroll
+                for (int e = 0; e < 4; e++) x[e] = (_Float16)(i < QP ? raw[i][j][e] * qs : raw[i][j][e]);
+                *(half4 *)((char *)sq + (4 * j + qr) * (FR_SQP * 4) + qc * 8) = x;
             }
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int e = 0; e < 4; e++) (i < QP ? qu : qv)[i % QP * 4 + e] = *(const half8 *)((const char *)sq + il * (FR_SQP * 4) + e * 32 + hh * 16);
+            asm volatile("" ::: "memory");
         }
     }
     constexpr int AES = ADD_F16 ? 2 : 4;
-    const char * addrow = nullptr;                  // the query's row of the additive mask
+    uint32_t add_off = 0;                           // the query's row of the additive mask, from that of the wave's first query
     // (The head's and the sequence's offsets in scalar registers: the divisions leave theirs in vector ones, and the 128-wide
     //  forms held them through the loop in scratch, for the rows that are done again.  What is left of it, one register in the
     //  form of 3 waves and three in that of 2, belongs to the epilogue; a build without it is 1% slower at 750 tokens.)
-    const char * add_head = nullptr;
+    const char * add_head = nullptr, * add_wave = nullptr;
     if (ADD) {
         add_head = a.add + (int64_t)__builtin_amdgcn_readfirstlane(h % a.Ha) * a.nba2 + (int64_t)__builtin_amdgcn_readfirstlane(b % a.Ba) * a.nba3;
-        addrow   = add_head + (int64_t)iq * a.nba1;
+        add_wave = add_head + (int64_t)min(i0w, a.Nq - 1) * a.nba1;
+        add_off  = (uint32_t)(iq - min(i0w, a.Nq - 1)) * (uint32_t)a.nba1;
     }
     // the additive mask's values of a tile: requested when the tile before is done with its own, waited for with that
     // tile's blocks
     typedef typename std::conditional<ADD_F16, half4_a2, float4_a4>::type araw_t;
     araw_t araw[ADD ? 4 : 1];
     auto load_add = [&](int t) __attribute__((always_inline)) {
+        const char * tile = add_wave + (int64_t)32 * AES * t;                                 // uniform
+        uint32_t off = add_off;
+        int      key = 4 * hh;
+        asm volatile("" : "+v"(off), "+v"(key));              // (sums of them are not worth registers in the loop)
         if (__builtin_expect(32 * t + 32 <= a.Nkv, 1)) {
 #pragma unroll
-            for (int g = 0; g < 4; g++) araw[ADD ? g : 0] = *(const araw_t *)(addrow + ((int64_t)32 * t + 8 * g + 4 * hh) * AES);
+            for (int g = 0; g < 4; g++) araw[ADD ? g : 0] = *(const araw_t *)(tile + (off + key * AES) + 8 * g * AES);
         } else {
 #pragma unroll
             for (int g = 0; g < 4; g++)
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
-                    const int key = min(32 * t + 8 * g + 4 * hh + c, a.Nkv - 1);
-                    if constexpr (ADD_F16) araw[ADD ? g : 0][c] = *(const _Float16 *)(addrow + (int64_t)key * 2);
-                    else                   araw[ADD ? g : 0][c] = *(const float *)(addrow + (int64_t)key * 4);
+                    const uint32_t at = off + (uint32_t)min(8 * g + key + c, a.Nkv - 1 - 32 * t) * AES;
+                    if constexpr (ADD_F16) araw[ADD ? g : 0][c] = *(const _Float16 *)(tile + at);
+                    else                   araw[ADD ? g : 0][c] = *(const float *)(tile + at);
                 }
         }
     };
@@ -216,24 +228,26 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     // masked, scans backwards four tiles per round trip; the workgroup takes the largest count.
     int NTL = NT;
     if (ADD) {
+        const int tr = lane >> 3, tc = (lane & 7) * 4;                // (along the rows: 8 of them an instruction)
         auto tile_max = [&](int tt) __attribute__((always_inline)) {
             float v = -INFINITY;
 #pragma unroll
             for (int g = 0; g < 4; g++) {
-                const int key0 = 32 * tt + 8 * g + 4 * hh;
+                const char * row = add_head + (int64_t)min(i0w + 8 * g + tr, a.Nq - 1) * a.nba1;
+                const int key0 = 32 * tt + tc;
                 if (32 * tt + 32 <= a.Nkv) {
                     if (ADD_F16) {
-                        const half4_a2 x = *(const half4_a2 *)(addrow + (int64_t)key0 * 2);
+                        const half4_a2 x = *(const half4_a2 *)(row + (int64_t)key0 * 2);
                         v = fmaxf(fmaxf(v, fmaxf((float)x[0], (float)x[1])), fmaxf((float)x[2], (float)x[3]));
                     } else {
-                        const float4_a4 x = *(const float4_a4 *)(addrow + (int64_t)key0 * 4);
+                        const float4_a4 x = *(const float4_a4 *)(row + (int64_t)key0 * 4);
                         v = fmaxf(fmaxf(v, fmaxf(x[0], x[1])), fmaxf(x[2], x[3]));
                     }
                 } else {
 #pragma unroll
                     for (int c = 0; c < 4; c++) {
                         const int key = min(key0 + c, a.Nkv - 1);
-                        v = fmaxf(v, ADD_F16 ? (float)*(const _Float16 *)(addrow + (int64_t)key * 2) : *(const float *)(addrow + (int64_t)key * 4));
+                        v = fmaxf(v, ADD_F16 ? (float)*(const _Float16 *)(row + (int64_t)key * 2) : *(const float *)(row + (int64_t)key * 4));
                     }
                 }
             }
@@ -304,11 +318,6 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
         return acc;
     };
 
-    // the wave's block 0 (= block -wave in wave 0's numbering): its lower-right triangle is the first tile's
-    half8 ops[KS];
-    read_block(ops, slot_of(-wave));
-    float16v bd_prev = times_q(ops, qv);
-
     float16v oacc[DBO];
 #pragma unroll
     for (int db = 0; db < DBO; db++)
@@ -316,69 +325,146 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
         for (int r = 0; r < 16; r++) oacc[db][r] = 0.0f;
     float m = -INFINITY, l = 0.0f;
 
-
-    // un-skew constants: slot r of a lane sits at row k_r + 4 hh of its block, i.e. at key (x + k_r) mod 32 with
-    // x = il + 4 hh + 1, and belongs to the previous block exactly when that sum reaches 32
+    // un-skew: slot r of a lane sits at row k_r + 4 hh of its block, i.e. at key (x + k_r) mod 32 with x = il + 4 hh + 1, and
+    // belongs to the previous block exactly when that sum reaches 32
     const int x_lane = il + 4 * hh + 1;
-    const int sq_new = il * FR_SQP + x_lane, sq_prev = sq_new - 32;
+    int sq_new = il * FR_SQP + x_lane;
+    auto unskew = [&](int r, const float16v & older, const float16v & newer) __attribute__((always_inline)) {
+        const int  k_r  = 8 * (r >> 2) + (r & 3);
+        const bool prev = x_lane + k_r >= 32;
+        sq[(prev ? sq_new - 32 : sq_new) + k_r] = prev ? older[r] : newer[r];
+    };
+    float4v bd[4];                                     // a tile's position scores, back in the layout of S^T
+    auto read_square = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int g = 0; g < 4; g++) bd[g] = *(const float4v *)&sq[il * FR_SQP + 8 * g + 4 * hh];
+    };
+
+    // the first tile's products: the wave's blocks 0 (= block -wave in wave 0's numbering), whose lower-right triangle it takes, and 1
+    float16v bd_prev, s;
+    {
+        half8 ops[KS];
+        read_block(ops, wave == NW - 1 ? first_block : slot_of(-wave));
+        const float16v bd0 = times_q(ops, qv);
+        read_block(ops, slot_of(1 - wave));
+        bd_prev = times_q(ops, qv);
+        read_block(ops, kt);
+        s = times_q(ops, qu);
+#pragma unroll
+        for (int r = 0; r < 16; r++) unskew(r, bd0, bd_prev);
+        read_square();
+    }
 
     // (the compiler's wait for them belongs here, behind that of `meet`: further down it would wait for the blocks on their way)
     auto have_add = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int g = 0; g < 4; g++) asm volatile("" : "+v"(araw[ADD ? g : 0]));
     };
-    meet();                                            // block 1 - NW has been read: its slot takes the next one
+    meet();                                            // what was read here may be written over
     if (ADD) have_add();
 
+    // A step's requests, K tile t + 2, table block t + 3 and V tile t + 1: workgroups of 3 waves share them out by tensor, 8 or 4 to
+    // each, others by rows, so that a wave's are as many as any other's.  A tensor's rows of one step are a buffer that ends
+    // with the tensor's last row (rows behind it are zeros: excluded keys, or no key at all), its address moves on by 32 rows.
+    constexpr bool BY_TENSOR = NW == 3;
+    constexpr int  TPW = BY_TENSOR ? 1 : 3, IPT = BY_TENSOR ? TI : TI / NW;        // tensors of a wave, instructions of each
+    uint64_t rq_base[TPW];
+    uint32_t rq_nb[TPW], rq_row[TPW], rq_chunk[TPW];   // pitch; the lane's row and chunk in an instruction
+    int      rq_left[TPW];                             // rows from the step's first one on
+    const uint32_t rq_ins = BY_TENSOR ? 0 : (uint32_t)wave;
+    constexpr uint32_t RQ_STRIDE = BY_TENSOR ? 1 : NW;
+#pragma unroll
+    for (int i = 0; i < TPW; i++) {
+        const int      which = BY_TENSOR ? wave : i;
+        const int      row0  = which == 0 ? 64 : which == 1 ? p_base0 + 96 : 32;
+        const int64_t  nb1   = which == 0 ? a.nbk1 : which == 1 ? a.nbr1 : a.nbv1;
+        rq_base[i]  = (uint64_t)((which == 0 ? kbase : which == 1 ? rbase : vbase) + (int64_t)row0 * nb1);
+        rq_nb[i]    = (uint32_t)nb1;
+        rq_left[i]  = (which == 1 ? NR : a.Nkv) - row0;
+        rq_row[i]   = (uint32_t)lr * rq_nb[i];
+        rq_chunk[i] = which == 2 ? cv : ck;
+    }
+    constexpr int NRQ = TPW * IPT;
+    __amdgpu_buffer_rsrc_t rq_buf[TPW];
+    uint32_t rq_to[TPW];
+    const uint32_t lds_k = lds_at(kt), lds_v = lds_at(vt), lds_ring = lds_at(ring);
+    uint32_t ring_next = (uint32_t)(3 + NW - 1) % FR_SLOTS;                   // slot of block t + 3
+    auto requests_of = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < TPW; i++) {
+            const int      which = BY_TENSOR ? wave : i;
+            const int      rows  = min(rq_left[i], 32);
+            rq_buf[i]   = fattn_buffer((const void *)rq_base[i], rows > 0 ? (uint32_t)(rows - 1) * rq_nb[i] + 2 * D : 0);
+            rq_base[i] += (uint64_t)rq_nb[i] * 32;
+            rq_left[i] -= 32;
+            asm volatile("" : "+v"(rq_row[i]), "+v"(rq_chunk[i]));           // (their sums are not worth registers in the loop)
+            rq_to[i]    = which == 0 ? lds_k + (t & 1) * 32 * KP : which == 1 ? lds_ring + ring_next * 32 * KP : lds_v + ((t + 1) & 1) * 32 * KP;
+        }
+        ring_next = ring_next + 1 == FR_SLOTS ? 0 : ring_next + 1;
+    };
+    auto request = [&](int n) __attribute__((always_inline)) {
+        const int      i    = n / IPT, j = n % IPT;
+        const uint32_t ins  = rq_ins + j * RQ_STRIDE;
+        const uint32_t turn = (BY_TENSOR ? wave : i) == 2 ? 0 : (ins & (16 / RPI - 1)) * 64;
+        const uint32_t off  = (rq_chunk[i] ^ turn) + rq_row[i] + ins * RPI * rq_nb[i];
+        buffer_to_lds16(rq_buf[i], off, rq_to[i], ins * 1024);
+    };
+
+    // A step turns the scores of tile t, which the step before has left in registers, into probabilities beside the products of tile t + 1
+    // (the last step's are of no tile and not used), and un-skews those beside P.V: a matrix instruction is followed by its share of
+    // the vector work, its next operand and a request, and none of them moves (FR_FENCE).
+    uint32_t ring_at = (uint32_t)(2 - wave + NW - 1) % FR_SLOTS;              // slot of the wave's block t + 2
 #pragma unroll 1
     for (int t = 0; t < NTL; t++) {
-        const bool tail = 32 * t + 32 > a.Nkv;             // uniform
-        read_block(ops, slot_of(t + 1 - wave));
-        // the next step's blocks: into the halves and the slot that the step before this one has left
-        if (t + 1 < NTL) {
-            dma_k(t + 1, std::false_type{});
-            dma_r(t + 2, std::false_type{});
-            dma_v(t + 1, std::false_type{});
-        }
-        // ---- the position product against this step's table block, the content product against its K tile -------------
-        half8 kops[KS];
-        read_block(kops, kt + (t & 1) * 32 * KP);
-        const float16v bd_new = times_q(ops, qv);
-        const float16v s = times_q(kops, qu);
-        // (beside the second product) select per slot, un-skew through the square
+        requests_of(t);
+        constexpr int OPS = 2 * KS, RD = FR_RD, PER = 16 / OPS;               // products; operands read ahead; pairs of scores to each
+        const uint32_t r_at = lds_ring + ring_at * 32 * KP + op0, k_at = lds_k + ((t + 1) & 1) * 32 * KP + op0;
+        ring_at = ring_at + 1 == FR_SLOTS ? 0 : ring_at + 1;
+        auto operand = [&](int i) __attribute__((always_inline)) { return *(lds_half8 *)(uintptr_t)((i < KS ? r_at : k_at) ^ (i % KS * 32)); };
+        half8 ops[RD];
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int  k_r  = 8 * (r >> 2) + (r & 3);
-            const bool prev = x_lane + k_r >= 32;
-            sq[(prev ? sq_prev : sq_new) + k_r] = prev ? bd_prev[r] : bd_new[r];
-        }
-        bd_prev = bd_new;
-
+        for (int i = 0; i < RD; i++) ops[i] = operand(i);
+        FR_FENCE();
+        float16v acc;
+        auto product = [&](int i) __attribute__((always_inline)) {
+            if (i % KS == 0) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[r] = 0.0f;
+            }
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ops[i % RD], i < KS ? qv[i % KS] : qu[i % KS], acc, 0, 0, 0);
+            if (i + RD < OPS) ops[i % RD] = operand(i + RD);
+#pragma unroll
+            for (int n = NRQ * i / OPS; n < NRQ * (i + 1) / OPS; n++) request(n);
+        };
         // ---- mask = f16(scale * BD + add); scores in log2 units ------------------------------------------------------
         float s2[16];
+        auto mask_pair = [&](int r) __attribute__((always_inline)) {
+            float2v mk;
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const float4v bd = *(const float4v *)&sq[il * FR_SQP + 8 * g + 4 * hh];
+            for (int e = 0; e < 2; e++)                        // as the graph: scale, then add
+                mk[e] = ADD ? mul_then_add(bd[r >> 2][(r & 3) + e], a.scale, (float)araw[ADD ? r >> 2 : 0][(r & 3) + e]) : bd[r >> 2][(r & 3) + e] * a.scale;
+            uint32_t pk;                                       // rounded two at a time (the compiler converts one at a time)
+            asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(pk) : "v"(mk[0]), "v"(mk[1]));
+            const half2v mh = __builtin_bit_cast(half2v, pk);
 #pragma unroll
-            for (int c = 0; c < 4; c += 2) {
-                float2v mk;
+            for (int e = 0; e < 2; e++) s2[r + e] = fmaf((float)mh[e], FR_LOG2E, s[r + e]);
+        };
 #pragma unroll
-                for (int e = 0; e < 2; e++)                    // as the graph: scale, then add
-                    mk[e] = ADD ? mul_then_add(bd[c + e], a.scale, (float)araw[g][c + e]) : bd[c + e] * a.scale;
-                uint32_t pk;                                   // rounded two at a time (the compiler converts one at a time)
-                asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(pk) : "v"(mk[0]), "v"(mk[1]));
-                const half2v mh = __builtin_bit_cast(half2v, pk);
+        for (int i = 0; i < KS; i++) {
+            product(i);
 #pragma unroll
-                for (int e = 0; e < 2; e++) s2[4 * g + c + e] = fmaf((float)mh[e], FR_LOG2E, s[4 * g + c + e]);
-            }
+            for (int n = 0; n < PER; n++) mask_pair(2 * (i * PER + n));
+            FR_FENCE();
         }
+        const float16v bd_new = acc;
         if (ADD && t + 1 < NTL) load_add(t + 1);
-        if (__builtin_expect(tail, 0)) {                   // keys past the end of the last tile
+        if (__builtin_expect(32 * t + 32 > a.Nkv, 0)) {    // keys past the end of the last tile
+            int key = 4 * hh;
+            asm volatile("" : "+v"(key));
 #pragma unroll
             for (int r = 0; r < 16; r++)
-                if (32 * t + 8 * (r >> 2) + 4 * hh + (r & 3) >= a.Nkv) s2[r] = -INFINITY;
+                if (key + 8 * (r >> 2) + (r & 3) >= a.Nkv - 32 * t) s2[r] = -INFINITY;
         }
-        __builtin_amdgcn_wave_barrier();
 
         // ---- online softmax ----------------------------------------------------------------------------------------------
         // P = 2^(s2 - m) in f16 against the row's reference m as it stands; the row sum is taken over the rounded values
@@ -387,52 +473,71 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
         // with the reference raised to the tile's maximum.  Sums and accumulators are f32; a probability stays below
         // FR_SUM_LIMIT in f16.
         half8 p[2];
-        float lsum;
-        auto exp_tile = [&](float ref) __attribute__((always_inline)) {
+        float lsum = 0.0f;
+        auto exp_pair = [&](int r, float ref) __attribute__((always_inline)) {
             const half2v ones = {(_Float16)1.0f, (_Float16)1.0f};
-            float dsum = 0.0f;
-#pragma unroll
-            for (int r = 0; r < 16; r += 2) {
-                half2v p2;
-                p2[0] = (_Float16)__builtin_amdgcn_exp2f(s2[r] - ref);
-                p2[1] = (_Float16)__builtin_amdgcn_exp2f(s2[r + 1] - ref);
-                dsum = __builtin_amdgcn_fdot2(p2, ones, dsum, false);
-                p[r >> 3][r & 7]       = p2[0];
-                p[r >> 3][(r & 7) + 1] = p2[1];
-            }
-            lsum = dsum;
+            half2v p2;
+            p2[0] = (_Float16)__builtin_amdgcn_exp2f(s2[r] - ref);
+            p2[1] = (_Float16)__builtin_amdgcn_exp2f(s2[r + 1] - ref);
+            lsum = __builtin_amdgcn_fdot2(p2, ones, lsum, false);
+            p[r >> 3][r & 7]       = p2[0];
+            p[r >> 3][(r & 7) + 1] = p2[1];
         };
-        exp_tile(m == -INFINITY ? 0.0f : m);
+        {
+            const float ref = m == -INFINITY ? 0.0f : m;
+#pragma unroll
+            for (int i = 0; i < KS; i++) {
+                product(KS + i);
+#pragma unroll
+                for (int n = 0; n < PER; n++) exp_pair(2 * (i * PER + n), ref);
+                FR_FENCE();
+            }
+        }
+        s = acc;
+        // ---- O^T += V^T . P^T -------------------------------------------------------------------------------------------
+        constexpr int VOPS = 2 * DBO, VD = FR_VD;
+        const uint32_t v_at = lds_v + (t & 1) * 32 * KP + va0;
+        auto v_operand = [&](int i) __attribute__((always_inline)) {
+            const uint32_t p0 = (v_at ^ (i / 2 * 64)) + 16 * (i % 2) * KP;
+            const half4 lo = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)(uintptr_t)p0));
+            const half4 hi = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)(uintptr_t)(p0 + 8 * KP)));
+            return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        };
+        half8 vops[VD];
+#pragma unroll
+        for (int i = 0; i < VD; i++) vops[i] = v_operand(i);
         if (__builtin_amdgcn_ballot_w64(!(lsum <= FR_SUM_LIMIT) || m == -INFINITY) != 0) {     // wave-uniform; rare after the first step
             float tmax = s2[0];
 #pragma unroll
             for (int r = 1; r < 16; r++) tmax = fmaxf(tmax, s2[r]);
-            tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));      // both halves of a query must agree
+            tmax = max_of_halves(tmax);                        // both halves of a query must agree
             const float mn = tmax > m ? tmax : m;
             const float f  = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mn);     // m = -inf: nothing accumulated yet, f = 0
             l *= f;
 #pragma unroll
             for (int db = 0; db < DBO; db++) oacc[db] *= f;
             m = mn;
-            exp_tile(m == -INFINITY ? 0.0f : m);
-        }
-        l += lsum;
-
-        // ---- O^T += V^T . P^T -------------------------------------------------------------------------------------------
-        {
-            const uint32_t v_at = lds_at(vt + (t & 1) * 32 * KP) + va0;
+            const float ref = m == -INFINITY ? 0.0f : m;
+            lsum = 0.0f;
 #pragma unroll
-            for (int db = 0; db < DBO; db++) {
-#pragma unroll
-                for (int ks = 0; ks < 2; ks++) {
-                    const uint32_t p0 = (v_at ^ (db * 64)) + 16 * ks * KP;
-                    const half4 lo = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)(uintptr_t)p0));
-                    const half4 hi = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)(uintptr_t)(p0 + 8 * KP)));
-                    const half8 va = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-                    oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, p[ks], oacc[db], 0, 0, 0);
-                }
+            for (int r = 0; r < 16; r += 2) {
+                exp_pair(r, ref);
+                FR_FENCE();                                    // (a pair at a time: there are no registers for more)
             }
         }
+        l += lsum;
+        asm volatile("" : "+v"(sq_new));                   // (nor are the slots' addresses)
+        FR_FENCE();
+#pragma unroll
+        for (int i = 0; i < VOPS; i++) {
+            oacc[i / 2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vops[i % VD], p[i % 2], oacc[i / 2], 0, 0, 0);
+            if (i + VD < VOPS) vops[i % VD] = v_operand(i + VD);
+#pragma unroll
+            for (int r = 16 * i / VOPS; r < 16 * (i + 1) / VOPS; r++) unskew(r, bd_prev, bd_new);
+            FR_FENCE();
+        }
+        bd_prev = bd_new;
+        read_square();
         meet();
         if (ADD) have_add();
     }
@@ -450,18 +555,27 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
             for (int r = 0; r < 16; r++) chk = fmaf(oacc[db][r], 0.0f, chk);
         badbits = __builtin_amdgcn_ballot_w64(chk != 0.0f);
     }
-    if (i0w + il < a.Nq) {
+    {   // through the square, 32 values of d at a time: 8 rows of 128 bytes a store instead of 32 bytes of 32 rows
         const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-        float * orow = a.dst + (((int64_t)b * a.Nq + (i0w + il)) * a.H + h) * D;
+        int         at   = lane;
+        asm volatile("" : "+v"(at));                                  // (not worth registers in the loop)
+        const int   orow = at >> 3, ocol = (at & 7) * 4;
+        float * const out = a.dst + (((int64_t)b * a.Nq + i0w) * a.H + h) * D + ocol;
 #pragma unroll
-        for (int db = 0; db < DBO; db++)
+        for (int db = 0; db < DBO; db++) {
 #pragma unroll
             for (int g = 0; g < 4; g++) {
                 float4v o;
 #pragma unroll
                 for (int c = 0; c < 4; c++) o[c] = oacc[db][4 * g + c] * inv;
-                *(float4v *)(orow + 32 * db + 8 * g + 4 * hh) = o;
+                *(float4v *)&sq[il * FR_SQP + 8 * g + 4 * hh] = o;
             }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const float4v o = *(const float4v *)&sq[(8 * j + orow) * FR_SQP + ocol];
+                if (i0w + 8 * j + orow < a.Nq) *(float4v *)(out + (int64_t)(8 * j + orow) * a.H * D + 32 * db) = o;
+            }
+        }
     }
     if constexpr (ADD) {
         if (badbits != 0) {
