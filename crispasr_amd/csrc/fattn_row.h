@@ -47,6 +47,43 @@ static __device__ __forceinline__ void row_load8(const char * row, int d0, bool 
     }
 }
 
+// The same where the launch knows how the rows lie, from a buffer that holds them all.  PIECES 2: rows of whole 16-byte loads of each
+// type (head sizes that are multiples of 8); 1: rows of whole pieces of 4 elements, 16 bytes of F32 or 8 of F16.  The two pieces of the
+// lane's 8 elements lie at `at` and behind it; pieces that are not the row's are asked for at no address and are zeros.  (Element by
+// element a 36-wide F32 row is 8 loads a lane, and of two ways to load chosen at run time each stands in a branch of its own.)
+template <int TYPE, int PIECES>
+static __device__ __forceinline__ void row_load8_pieces(__amdgpu_buffer_rsrc_t rows, uint32_t at, bool in0, bool in1, float (&out)[8]) {
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+    constexpr uint32_t PIECE = TYPE == MI355X_TYPE_F32 ? 16 : 8;
+    const int at0 = (int)(in0 ? at : FATTN_NO_ADDRESS), at1 = (int)(in1 ? at + PIECE : FATTN_NO_ADDRESS);
+    if constexpr (TYPE == MI355X_TYPE_F32) {
+        const u4 a = __builtin_amdgcn_raw_buffer_load_b128(rows, at0, 0, 0);
+        const u4 b = __builtin_amdgcn_raw_buffer_load_b128(rows, at1, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            out[i]     = __uint_as_float(a[i]);
+            out[4 + i] = __uint_as_float(b[i]);
+        }
+    } else {
+        uint32_t w[4];
+        if constexpr (PIECES == 2) {
+            const u4 a = __builtin_amdgcn_raw_buffer_load_b128(rows, at0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) w[i] = a[i];
+        } else {
+            const u2 a = __builtin_amdgcn_raw_buffer_load_b64(rows, at0, 0, 0);
+            const u2 b = __builtin_amdgcn_raw_buffer_load_b64(rows, at1, 0, 0);
+            w[0] = a[0]; w[1] = a[1]; w[2] = b[0]; w[3] = b[1];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            out[2 * i]     = h2f_bits((uint16_t)(w[i] & 0xffffu));
+            out[2 * i + 1] = h2f_bits((uint16_t)(w[i] >> 16));
+        }
+    }
+}
+
 // online-softmax state of the lanes that share 8 elements of d: running maximum, sum, unnormalised accumulators
 struct RowPartial {
     float m, l;
@@ -62,6 +99,33 @@ static __device__ __forceinline__ void row_partial_merge(RowPartial & a, const R
 #pragma unroll
     for (int e = 0; e < 8; e++) a.acc[e] = a.acc[e] * fa + b.acc[e] * fb;
     a.m = mn;
+}
+
+// lane ^ OFF's value, for the merge of a wave's groups: 4 through the LDS crossbar; 8, 16 and 32 in the vector unit (a rotation of
+// a row by half, and swaps of which the lower lanes' partner is the second result: only lanes that have the bit OFF clear may use it)
+template <int OFF>
+static __device__ __forceinline__ float partner_above(float x) {
+    static_assert(OFF == 4 || OFF == 8 || OFF == 16 || OFF == 32, "a power of two that a group can be wide");
+    if constexpr (OFF == 4)  return xor_shuffle(x, 4);
+    if constexpr (OFF == 8)  return dpp_mov<0x128>(x);               // row_ror:8
+    if constexpr (OFF == 16) {
+        uint32_t a = __float_as_uint(x), b = a;
+        asm volatile("" : "+v"(b));                                  // (as in both_halves)
+        return __uint_as_float(__builtin_amdgcn_permlane16_swap(a, b, false, false)[1]);
+    }
+    return both_halves(x).y;
+}
+template <int OFF>
+static __device__ __forceinline__ void merge_groups(RowPartial & st) {
+    if constexpr (OFF < 64) {
+        RowPartial o;
+        o.m = partner_above<OFF>(st.m);
+        o.l = partner_above<OFF>(st.l);
+#pragma unroll
+        for (int e = 0; e < 8; e++) o.acc[e] = partner_above<OFF>(st.acc[e]);
+        row_partial_merge(st, o);
+        merge_groups<OFF * 2>(st);
+    }
 }
 
 constexpr int ROW_UNROLL = 4;
@@ -92,9 +156,15 @@ struct RowMaskTensor {
 // Keys [k_begin, k_end) of one row, visited by NWAVES waves: a K or V row is spread over LPR lanes (8 elements each), so a
 // wave takes 64 / LPR rows per load; every group of LPR lanes keeps its own state over the keys it visits.  q holds the
 // lane's 8 query elements (zeros where d0 is past D).  All 64 lanes must be active (DPP reductions).
-template <int TYPE_K, int TYPE_V, int LPR, int NWAVES, typename MaskFn>
+// The state of the whole wave ends in its lanes 0 .. LPR - 1.  PIECES above 0: F32 or f16 rows that lie as row_load8_pieces says, all of
+// them within 4 GiB, and a range that is not empty; `requested` is called when its first rows are on their way.
+struct RowNothing {
+    __device__ __forceinline__ void operator()() const {}
+};
+template <int TYPE_K, int TYPE_V, int LPR, int NWAVES, int PIECES = 0, typename MaskFn, typename RequestedFn = RowNothing>
 static __device__ __forceinline__ void row_scan(const RowScanArgs & a, const float (&q)[8], const char * kbase, const char * vbase,
-                                                const MaskFn & mask_at, int k_begin, int k_end, int wave, int lane, RowPartial & st) {
+                                                const MaskFn & mask_at, int k_begin, int k_end, int wave, int lane, RowPartial & st,
+                                                const RequestedFn & requested = RequestedFn()) {
     constexpr int G = 64 / LPR;                 // key rows per wave per load
     const int  grp    = lane / LPR;
     const int  d0     = (lane % LPR) * 8;
@@ -103,7 +173,14 @@ static __device__ __forceinline__ void row_scan(const RowScanArgs & a, const flo
     const bool al     = a.aligned16;
     const int  stride = NWAVES * G * ROW_UNROLL;
     // every lane runs the same trip count so that the DPP reductions see full groups
-    for (int j0 = k_begin; j0 < k_end; j0 += stride) {
+    constexpr int SIZE = TYPE_K == MI355X_TYPE_F32 ? 4 : 2;      // (PIECES > 0: K and V are of one type)
+    __amdgpu_buffer_rsrc_t krows, vrows;
+    if constexpr (PIECES > 0) {
+        static_assert(TYPE_K == TYPE_V && (TYPE_K == MI355X_TYPE_F32 || TYPE_K == MI355X_TYPE_F16), "rows of elements");
+        krows = fattn_buffer(kbase, (uint32_t)(k_end - 1) * (uint32_t)a.nbk1 + (uint32_t)a.D * SIZE);
+        vrows = fattn_buffer(vbase, (uint32_t)(k_end - 1) * (uint32_t)a.nbv1 + (uint32_t)a.D * SIZE);
+    }
+    const auto step = [&](int j0, const auto & asked) __attribute__((always_inline)) {
         float kf[ROW_UNROLL][8];
         float vf[ROW_UNROLL][8];
         float s[ROW_UNROLL];
@@ -112,14 +189,26 @@ static __device__ __forceinline__ void row_scan(const RowScanArgs & a, const flo
 #pragma unroll
         for (int u = 0; u < ROW_UNROLL; u++) {
             jj[u] = j0 + (u * NWAVES + wave) * G + grp;
-            const int jc = min(jj[u], k_end - 1);
-            row_load8<TYPE_K>(kbase + (size_t)jc * a.nbk1, d0c, al, nv, kf[u]);
+            if constexpr (PIECES > 0) {
+                const bool in = jj[u] < k_end;
+                row_load8_pieces<TYPE_K, PIECES>(krows, (uint32_t)jj[u] * (uint32_t)a.nbk1 + d0 * SIZE, in && d0 < a.D, in && d0 + 4 < a.D, kf[u]);
+            } else {
+                const int jc = min(jj[u], k_end - 1);
+                row_load8<TYPE_K>(kbase + (size_t)jc * a.nbk1, d0c, al, nv, kf[u]);
+            }
         }
 #pragma unroll
         for (int u = 0; u < ROW_UNROLL; u++) {
-            const int jc = min(jj[u], k_end - 1);
-            row_load8<TYPE_V>(vbase + (size_t)jc * a.nbv1, d0c, al, nv, vf[u]);
+            if constexpr (PIECES > 0) {
+                const bool in = jj[u] < k_end;
+                row_load8_pieces<TYPE_V, PIECES>(vrows, (uint32_t)jj[u] * (uint32_t)a.nbv1 + d0 * SIZE, in && d0 < a.D, in && d0 + 4 < a.D, vf[u]);
+            } else {
+                const int jc = min(jj[u], k_end - 1);
+                row_load8<TYPE_V>(vbase + (size_t)jc * a.nbv1, d0c, al, nv, vf[u]);
+            }
         }
+        if constexpr (PIECES > 0) __builtin_amdgcn_sched_barrier(0);         // (all requests ahead of the first use)
+        asked();
         float mloc = -INFINITY;
 #pragma unroll
         for (int u = 0; u < ROW_UNROLL; u++) {
@@ -140,6 +229,12 @@ static __device__ __forceinline__ void row_scan(const RowScanArgs & a, const flo
             // (a visible key with a NaN score makes the row NaN, as it does on the CPU: the maximum must not ignore it)
             mloc = fmaxf(mloc, s[u] == s[u] ? s[u] : INFINITY);
         }
+        if constexpr (PIECES > 0) {              // (or the compiler asks for V behind the branch below, when K has come)
+#pragma unroll
+            for (int u = 0; u < ROW_UNROLL; u++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) asm volatile("" : "+v"(vf[u][e]) : "v"(mloc));
+        }
         if (mloc > st.m) {                       // uniform within a group
             const float alpha = __expf(st.m - mloc);   // exp(-inf) = 0 on the first hit
             st.l *= alpha;
@@ -150,24 +245,25 @@ static __device__ __forceinline__ void row_scan(const RowScanArgs & a, const flo
         if (st.m > -INFINITY) {
 #pragma unroll
             for (int u = 0; u < ROW_UNROLL; u++) {
-                if (ex[u]) continue;             // nor is its V row: 0 * NaN would not be 0
+                // nor is its V row: 0 * NaN would not be 0 (without a mask excluded keys are those past the end, whose rows are zeros)
+                if ((PIECES == 0 || mask_at.present()) && ex[u]) continue;
                 const float p = __expf(s[u] - st.m);
                 st.l += p;
 #pragma unroll
                 for (int e = 0; e < 8; e++) st.acc[e] = fmaf(p, vf[u][e], st.acc[e]);
             }
         }
+    };
+    // (the first step of a range that is known to hold keys stands by itself: ahead of a loop's requests the compiler waits for all that
+    //  is on its way, q's rows among it)
+    int j0 = k_begin;
+    if constexpr (PIECES > 0) {
+        step(j0, requested);
+        j0 += stride;
     }
+    for (; j0 < k_end; j0 += stride) step(j0, RowNothing());
     // merge the G groups of this wave (lanes with equal position in their group)
-#pragma unroll
-    for (int off = LPR; off < 64; off <<= 1) {
-        RowPartial o;
-        o.m = xor_shuffle(st.m, off);
-        o.l = xor_shuffle(st.l, off);
-#pragma unroll
-        for (int e = 0; e < 8; e++) o.acc[e] = xor_shuffle(st.acc[e], off);
-        row_partial_merge(st, o);
-    }
+    merge_groups<LPR>(st);
 }
 
 // lanes 0 .. LPR-1 hold the row's final state: write dst, or this split's partial for the merge (natural-log units).
@@ -183,18 +279,21 @@ static __device__ __forceinline__ void row_store(const FattnArgs & a, const RowP
         for (int e = 0; e < 8; e++)
             if (e < 4 || d0 + e < a.Dv) out[e] = st.acc[e] * inv;       // (the head size is a multiple of 4)
     } else {
-        float * pa = a.part_acc + (row * a.n_splits + split) * a.D + d0;
+        float * pa = a.part_acc + (row * a.n_splits + split) * a.D + d0;          // (8-byte aligned: the head size is a multiple of 4)
 #pragma unroll
-        for (int e = 0; e < 8; e++)
+        for (int e = 0; e < 8; e += 2)
             if (e < 4 || d0 + e < a.D) {
-                if (COHERENT) device_store(pa + e, st.acc[e]);
-                else          pa[e] = st.acc[e];
+                if (COHERENT) {
+                    device_store2(pa + e, st.acc[e], st.acc[e + 1]);
+                } else {
+                    pa[e]     = st.acc[e];
+                    pa[e + 1] = st.acc[e + 1];
+                }
             }
         if (lane == 0) {
             float * pm = a.part_ml + (row * a.n_splits + split) * 2;
             if (COHERENT) {
-                device_store(pm, st.m);
-                device_store(pm + 1, st.l);
+                device_store2(pm, st.m, st.l);
             } else {
                 pm[0] = st.m;
                 pm[1] = st.l;
