@@ -18,13 +18,12 @@ struct DecodeShort {
     uint32_t     nbk1, nbk2, nbk3;    // and V's
     uint32_t     nbq1, nbq2, nbq3;
     uint32_t     Nkv;
-    uint32_t     rows;                // Nq | gqa << 5 | n_splits << 10 | keys_per_split / 32 << 17, or, not cut, the sequences in the first
-                                      // round << 17 (0: in their own order, see decode_turns)
+    uint32_t     rows;                // Nq | gqa << 5 | n_splits << 10 | keys_per_split / 32 << 17 (0: not cut)
     const char * mask;
     uint32_t     nbm1, nbm2, nbm3;
     uint32_t     heads;               // Hkv | B << 16
     float        scale;
-    uint32_t     Dv;
+    uint32_t     Dv;                  // | sequences in the first round << 16 (0: in their own order, see decode_turns)
     float *      dst;
     float *      part_acc;            // the (max, sum) pairs lie right behind it
     unsigned *   counters;
@@ -86,7 +85,7 @@ static __host__ __device__ __forceinline__ FattnArgs decode_expand(const DecodeS
     FattnArgs a = {};
     a.q = p.q; a.k = p.k; a.v = p.v; a.mask = p.mask; a.dst = p.dst;
     a.D  = D;
-    a.Dv = (int)p.Dv;
+    a.Dv = (int)(p.Dv & 0xFFFFu);
     a.Nq = (int)(p.rows & 31u);
     a.gqa = (int)(p.rows >> 5 & 31u);
     a.n_splits = (int)(p.rows >> 10 & 127u);

@@ -933,7 +933,7 @@ template <int D, bool MASK, int TYPE, bool RAW, bool V8, bool PAD>
 __device__ __forceinline__ void decode_short(const DecodeShort & p) {
     FattnArgs a = decode_expand(p, D);
     if (!PAD) a.Dv = D;
-    decode_body<D, TYPE, MASK, RAW, V8, PAD, true>(a, MASK && a.n_splits == 1 ? (int)(p.rows >> 17) : 0);
+    decode_body<D, TYPE, MASK, RAW, V8, PAD, true>(a, MASK ? (int)(p.Dv >> 16) : 0);
 }
 template <int D, int TYPE, bool RAW, bool V8, bool PAD>
 __global__ void __launch_bounds__(DEC_THREADS) __attribute__((amdgpu_waves_per_eu((decode_waves_min<D, TYPE, RAW>()), (decode_waves_max<D, RAW, V8>()))))
@@ -965,7 +965,7 @@ int launch_one(FattnArgs a, hipStream_t stream) {
     if constexpr (TYPE == MI355X_TYPE_F16 || V8 || (RAW && TYPE != MI355X_TYPE_Q8_0)) {      // (the rows of a cache as they usually lie)
         DecodeShort p;
         if (decode_shorten(a, p)) {
-            if (MASK) p.rows |= decode_turns(a, TYPE == MI355X_TYPE_F16 ? D * 2 : D / 32 * raw_block_bytes<TYPE>()) << 17;      // (of calls that are not cut)
+            if (MASK) p.Dv |= decode_turns(a, TYPE == MI355X_TYPE_F16 ? D * 2 : D / 32 * raw_block_bytes<TYPE>()) << 16;
             static std::atomic<uint64_t> short_lds_allowed{0};
             const dim3 short_grid((unsigned)a.n_splits, (unsigned)a.Hkv, (unsigned)a.B);
             if constexpr (MASK) {
