@@ -563,8 +563,23 @@ int decode_ranges(const FattnArgs & a, int type, int64_t groups, size_t beside) 
     return best;
 }
 
-// (padded: a0.D is the padded head size and the copies are needed whatever the types)
-void make_plan_core(const FattnArgs & a0, int ktype, int vtype, const mi355x_fattn_params * p, bool padded, Plan & plan) {
+// F32 K/V without a mask that the vector kernel's short form takes (fattn_vec.hip) and is done with before the tile kernel: its time goes
+// with the rows' passes over their keys, the tile kernel's starts at the depth of a tile's conversion.  us, vector and tile kernel,
+// 8, 12 and 20 heads x 2 to 48 queries x 40 to 1500 keys: 64-wide heads, 20 x 5 x 1500 9.0 and 10.6, 12 x 12 x 750 8.2 and 10.0, 12 x 12 x
+// 1500 11.2 and 10.3, 20 x 24 x 40 4.6 and 4.5, 20 x 32 x 40 5.1 and 4.5; 128-wide, 8 x 15 x 375 7.2 and 18.9, 20 x 8 x 750 11.3 and 18.1,
+// 20 x 48 x 200 12.7 and 15.0, 8 x 16 x 1500 14.4 and 13.9, 12 x 12 x 1500 17.3 and 14.5; other head sizes, which the tile kernel pads, 32,
+// 8 x 16 x 1500 7.4 and 13.5, 48, 12 x 24 x 750 10.1 and 11.8, 96, 8 x 16 x 750 9.6 and 14.9, 12 x 48 x 375 12.7 and 12.4.  (It also multiplies by the values as they are, where
+// the tile kernel rounds them to f16.)  Callers who name a number of ranges or a form of the tile kernel keep the rules without this.
+bool vec_takes_step(const FattnArgs & a, int ktype, int vtype, const mi355x_fattn_params * p) {
+    if (p->kernel != MI355X_FATTN_AUTO || p->n_splits > 0 || p->tile_variant) return false;
+    if (ktype != MI355X_TYPE_F32 || vtype != MI355X_TYPE_F32 || a.masked || a.softcap != 0.0f || a.gqa != 1 || (a.Nq != 1 && a.B != 1)) return false;
+    if (!a.aligned16 || a.Dv != a.D || a.nbk1 != a.nbv1 || a.nbk2 != a.nbv2 || (a.Bk > 1 && a.nbk3 != a.nbv3)) return false;
+    const int64_t rows = (int64_t)a.Nq * a.Hq * a.B, pairs = rows * a.Nkv;
+    return a.D < 64 ? rows <= 512 && pairs <= 220000 : a.D == 64 ? rows <= 512 && pairs <= 180000 : rows <= 1024 && pairs <= 190000;
+}
+
+// (padded: a0.D is the padded head size and the copies are needed whatever the types; steps: by vec_takes_step's rule too)
+void make_plan_core(const FattnArgs & a0, int ktype, int vtype, const mi355x_fattn_params * p, bool padded, Plan & plan, bool steps = true) {
     FattnArgs a = a0;
     const bool mixed = ktype != vtype || padded;
     if (mixed) {
@@ -627,6 +642,7 @@ void make_plan_core(const FattnArgs & a0, int ktype, int vtype, const mi355x_fat
                      : a.Nq >= 16 && (a.D == 64 || a.D == 128) && a.q_aligned16 ? MI355X_FATTN_MMA
                                                                                 : MI355X_FATTN_VEC;
         else if (fattn_decode_supported(a, ktype) && ((a.q_chunks <= 1 && !tile_rows) || chunked)) kernel = MI355X_FATTN_DECODE_MMA;
+        else if (steps && !mixed && vec_takes_step(a, ktype, vtype, p))      kernel = MI355X_FATTN_VEC;
         else if ((a.Nq >= 16 || tile_rows) && fattn_mma_supported(a, ktype)) kernel = MI355X_FATTN_MMA;
         // F32 K/V under 2 .. 15 queries (the decode kernel does not read F32): the vector kernel streams the keys once per
         // query row, the tile kernel once per head - worth its padding from about 40k (row, key) pairs on at 64-wide heads
@@ -756,23 +772,6 @@ void make_plan_core(const FattnArgs & a0, int ktype, int vtype, const mi355x_fat
     }
 }
 
-// A plan that has to do with `room` bytes: a decode call that AUTO cut takes as many ranges as its partials fit there, down to those
-// that the price of whole steps and merges asks for (`fewest`, which was once the count itself: workspaces that programs sized by it
-// stay large enough).  plan.workspace stays what the call would use at best.  False: the call does not fit.
-bool fit_plan(FattnArgs a, int ktype, int vtype, const mi355x_fattn_params * p, size_t room, Plan & plan) {
-    if (plan.workspace <= room) return true;
-    if (plan.kernel != MI355X_FATTN_DECODE_MMA || p->n_splits > 0 || plan.n_splits < 2 || room < plan.ws_partials) return false;
-    if (a.D != plan.pad) apply_pad(a, plan);
-    if (plan.kv_to_f16) ktype = vtype = MI355X_TYPE_F16;
-    const int64_t groups = (int64_t)a.Hkv * a.B * a.q_chunks;
-    const size_t  part   = (size_t)a.Nq * a.Hq * a.B * (a.D + 2) * sizeof(float);
-    const size_t  n      = (room - plan.ws_partials) / part;                  // (below plan.n_splits)
-    if (n < (size_t)DecodeCut(a, ktype, vtype, groups).fewest(decode_most(a, groups))) return false;
-    plan.keys_per_split = ((a.Nkv + (int)n - 1) / (int)n + 31) / 32 * 32;
-    plan.n_splits       = (a.Nkv + plan.keys_per_split - 1) / plan.keys_per_split;
-    return true;
-}
-
 // Head sizes the MFMA kernels have no form for (multiples of 8 below 128 other than 64: 32 and 48, 80 and 96 of other
 // Whisper-like towers, ...) can still run on them, as the next larger of 64 and 128 with zeros behind the head's own
 // elements: the products over the padding are exact zeros, so the result is what the head size itself would give.
@@ -781,7 +780,7 @@ bool fit_plan(FattnArgs a, int ktype, int vtype, const mi355x_fattn_params * p, 
 //  - The decode kernel, over F16 caches: it reads the rows where they lie and pads in its registers.  No copy.
 // The vector kernel, which takes any head size, keeps what neither takes: few query rows over F32 and quantised caches,
 // and calls too small to pay for the copy launch.
-void make_plan(const FattnArgs & a0, int ktype, int vtype, const mi355x_fattn_params * p, Plan & plan) {
+void make_plan(const FattnArgs & a0, int ktype, int vtype, const mi355x_fattn_params * p, Plan & plan, bool steps = true) {
     static const bool no_pad = getenv("MI355X_FATTN_NO_PAD") != nullptr;        // comparison runs
     const int pad = a0.D >= 8 && a0.D < 128 && a0.D != 64 && a0.D % 8 == 0 ? (a0.D < 64 ? 64 : 128) : 0;
     // The decode kernel reads f16 rows of such a head size where they lie (no copies): the chunks of a row behind the head's
@@ -837,7 +836,7 @@ void make_plan(const FattnArgs & a0, int ktype, int vtype, const mi355x_fattn_pa
         // (where the padded plan would take the decode kernel - 16 queries or more in 16-row chunks over F32 or quantised
         //  K/V, which that kernel does not pad - the tile kernel stands in: the vector kernel is 2 to 4 times slower there)
         bool want = p->kernel == MI355X_FATTN_MMA;
-        if (!want) {
+        if (!want && !(steps && vec_takes_step(a0, ktype, vtype, p))) {
             want = (pairs >= 100000 && (plan.kernel == MI355X_FATTN_MMA || (plan.kernel == MI355X_FATTN_DECODE_MMA && a0.Nq >= 16))) ||
                    (pad == 128 && a0.Nq >= 2 && a0.Nq < 16 && pairs >= 150000);
         }
@@ -857,7 +856,33 @@ void make_plan(const FattnArgs & a0, int ktype, int vtype, const mi355x_fattn_pa
             return;
         }
     }
-    make_plan_core(a0, ktype, vtype, p, false, plan);
+    make_plan_core(a0, ktype, vtype, p, false, plan, steps);
+}
+
+// A plan that has to do with `room` bytes: a decode call that AUTO cut takes as many ranges as its partials fit there, down to those
+// that the price of whole steps and merges asks for (`fewest`, which was once the count itself: workspaces that programs sized by it
+// stay large enough); a call that vec_takes_step moved to the vector kernel, whose partials do not fit, is the tile kernel's, which may
+// need none (64-wide, not padded: where it needs its copies these are larger).  plan.workspace stays what the call would use at best.
+// False: the call does not fit.
+bool fit_plan(FattnArgs a, int ktype, int vtype, const mi355x_fattn_params * p, size_t room, Plan & plan) {
+    if (plan.workspace <= room) return true;
+    if (plan.kernel == MI355X_FATTN_VEC && vec_takes_step(a, ktype, vtype, p)) {
+        Plan other;
+        make_plan(a, ktype, vtype, p, other, false);
+        if (other.kernel != MI355X_FATTN_MMA || other.pad || other.workspace > room) return false;
+        plan = other;
+        return true;
+    }
+    if (plan.kernel != MI355X_FATTN_DECODE_MMA || p->n_splits > 0 || plan.n_splits < 2 || room < plan.ws_partials) return false;
+    if (a.D != plan.pad) apply_pad(a, plan);
+    if (plan.kv_to_f16) ktype = vtype = MI355X_TYPE_F16;
+    const int64_t groups = (int64_t)a.Hkv * a.B * a.q_chunks;
+    const size_t  part   = (size_t)a.Nq * a.Hq * a.B * (a.D + 2) * sizeof(float);
+    const size_t  n      = (room - plan.ws_partials) / part;                  // (below plan.n_splits)
+    if (n < (size_t)DecodeCut(a, ktype, vtype, groups).fewest(decode_most(a, groups))) return false;
+    plan.keys_per_split = ((a.Nkv + (int)n - 1) / (int)n + 31) / 32 * 32;
+    plan.n_splits       = (a.Nkv + plan.keys_per_split - 1) / plan.keys_per_split;
+    return true;
 }
 
 // q_quant: the query rows rounded to Q8_0 and back, as contiguous F32 [D, Nq, Hq, B] at ws + q8_bytes
