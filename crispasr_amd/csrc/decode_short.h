@@ -55,6 +55,7 @@ static inline bool decode_shorten(const FattnArgs & a, DecodeShort & p) {
     const int64_t nb[12] = {a.nbq1, a.nbq2, a.nbq3, a.nbk1, a.nbk2, a.nbk3, a.nbv1, a.nbv2, a.nbv3, a.nbm1, a.nbm2, a.nbm3};
     for (int i = 0; i < (a.mask ? 12 : 9); i++)
         if ((uint64_t)nb[i] > 0xFFFFFFFFull) return false;
+    if (a.nbk1 > 1 << 26) return false;                       // (32 rows are within 4 GiB)
     const bool    one_sequence = a.Bk == 1;
     const int64_t rows = (int64_t)a.Nq * a.Hq * a.B;
     if (a.q_chunks != 1 || a.Nq < 1 || a.gqa < 1 || (int64_t)a.Nq * a.gqa > 16 || a.max_bias > 0.0f || a.softcap != 0.0f) return false;

@@ -137,8 +137,9 @@ __device__ __forceinline__ half8 q8_dequant_keys(uint32_t q0, uint32_t q1, half8
 // a unit of a streamed row (aux 2: non-temporal, as stream_load)
 template <typename T>
 __device__ __forceinline__ T buffer_stream(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-    if constexpr (sizeof(T) == 8) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 2));
-    else                          return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 2));
+    if constexpr (sizeof(T) == 16)     return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 2));
+    else if constexpr (sizeof(T) == 8) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 2));
+    else                               return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 2));
 }
 
 // raw global data of one 8-element chunk
@@ -381,10 +382,12 @@ __device__ __forceinline__ int sequence_of_turn(const FattnArgs & a, int turn, i
 // PAD: f16 rows of a.Dv elements (a multiple of 8 below D) read in place: the chunks of a row behind Dv are zeros in the
 // registers, q is read and dst written up to Dv.  An instantiation of its own: the others stay the code they were.
 // SHORT: the arguments came as DecodeShort, the grid is (split, KV head, batch), and there is one chunk of rows; `first`: decode_turns.
-template <int D, int TYPE, bool MASK, bool RAW, bool V8, bool PAD, bool SHORT>
+// DEEP (f16 rows, SHORT, no mask): the rows of two steps are under way while a third is worked on; q is asked for first.
+template <int D, int TYPE, bool MASK, bool RAW, bool V8, bool PAD, bool SHORT, bool DEEP = false>
 __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
     static_assert(!PAD || (TYPE == MI355X_TYPE_F16 && !RAW && !V8), "other head sizes: f16 rows, read per lane");
     static_assert(!V8 || RAW, "the int8 V stage belongs to the streamed Q8_0 path");
+    static_assert(!DEEP || (SHORT && !MASK && TYPE == MI355X_TYPE_F16), "see above");
     constexpr int KS  = D / 32;                    // reduction steps of Q.K^T (one Q8_0 block each)
     constexpr int DBK = D / 16;                    // 16-wide blocks of the output's d
     constexpr int CH  = D / 8;                     // chunks per row
@@ -521,11 +524,17 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
     uint32_t vdst[V8 ? NU : 1][V8 ? PCS / 2 : 1];
     // mask values of the lane's eight keys of the step, in the order of its scores
     u32x2_a2 mraw[2][MASK ? 2 : 1];
+    // (DEEP) Rows through a buffer that ends with the step's last valid one, or holds nothing behind the wave's last step: the request
+    // needs no branch.  With one, the compiler cannot count what is on its way behind a stage and waits for everything at each step, so
+    // that no step's rows were under way during another.  A lane's offsets of K's rows j and V's, the same for every step:
+    const uint32_t nb1  = DEEP ? (uint32_t)a.nbk1 : 0;          // (K's and V's, below 64 MiB)
+    const uint32_t koff = (uint32_t)j * nb1 + g4 * 16, voff = (uint32_t)(lane / CH) * nb1 + lane % CH * 16;
     // a partial last step: its loads are clamped to the last valid row (branch-free, in bounds) or give zeros behind it, and
     // the keys they stand for are excluded in the step
     auto issue = [&](int it, auto stage) __attribute__((always_inline)) {
         constexpr int s = decltype(stage)::value;
-        const int j0 = k_begin + it * STEP;
+        const bool on = !DEEP || it < walk_end;
+        const int  j0 = k_begin + (on ? it : 0) * STEP;
         // (One branch for the eight values where a step's registers are many; the int8 V form, with one register stage, is up to
         //  3% faster on large batches with one branch for each four.)
         if constexpr (MASK && V8) {
@@ -556,7 +565,7 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
             // One coalesced stream per tensor, through a buffer that ends with the step's last valid row: what lies behind it are
             // zeros, scales and minima among them, and the 2 * NU loads share one offset (its lane number through an asm, or
             // each of the loop's would have its own).
-            const uint32_t bytes = (uint32_t)min(STEP, k_end - j0) * RS;
+            const uint32_t bytes = (uint32_t)(MASK ? min(STEP, k_end - j0) : max(0, min(STEP, k_end - j0))) * RS;
             const auto     kb = fattn_buffer(kbase + (int64_t)j0 * RS, bytes), vb = fattn_buffer(vbase + (int64_t)j0 * RS, bytes);
             uint32_t ln = (uint32_t)lane;
             asm volatile("" : "+v"(ln));
@@ -565,6 +574,19 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
                 kun[ONE ? 0 : s][i] = buffer_stream<unit_t>(kb, (ln + i * 64) * UNIT);
                 vun[ONE ? 0 : s][i] = buffer_stream<unit_t>(vb, (ln + i * 64) * UNIT);
             }
+            return;
+        }
+        if constexpr (DEEP) {
+            const uint32_t bytes = on ? (uint32_t)(min(STEP, k_end - j0) - 1) * nb1 + (uint32_t)(PAD ? a.Dv : D) * 2 : 0;
+            const auto     kbuf = fattn_buffer(kbase + (int64_t)j0 * nb1, bytes), vbuf = fattn_buffer(vbase + (int64_t)j0 * nb1, bytes);
+#pragma unroll
+            for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+                for (int ks = 0; ks < KS; ks++)
+                    kraw[s][kb][ks].v = buffer_stream<uint4>(kbuf, !PAD || (ks * 4 + g4) * 8 < a.Dv ? koff + kb * 16 * nb1 + ks * 64 : FATTN_NO_ADDRESS);
+#pragma unroll
+            for (int i = 0; i < NV; i++)
+                vraw[s][i].v = buffer_stream<uint4>(vbuf, !PAD || lane % CH * 8 < a.Dv ? voff + i * (64 / CH) * nb1 : FATTN_NO_ADDRESS);
             return;
         }
 #pragma unroll
@@ -589,12 +611,13 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
     typedef std::integral_constant<int, 0> S0;
 
     // one step of 32 keys out of register stage s; the wave's following step `nxt` is requested into the other stage
+    // (DEEP: the one behind that into this stage, once its rows have gone on; nxt < 0: none)
     auto step = [&](const int it, const int nxt, auto stage) __attribute__((always_inline)) {
         constexpr int s = decltype(stage)::value;
         const int  j0   = k_begin + it * STEP;
         const bool tail = j0 + STEP > k_end;                  // wave-uniform
         // the following step's loads: into the other register stage, or (V8) into this one as soon as it is in LDS
-        if (!ONE && nxt < walk_end) issue(nxt, std::integral_constant<int, 1 - s>{});
+        if (!ONE && !DEEP && nxt < walk_end) issue(nxt, std::integral_constant<int, 1 - s>{});
         u32x2_a2 mcur[2];                                     // (V8's next request overwrites the stage)
         if (MASK) {
             mcur[0] = mraw[ONE ? 0 : s][0];
@@ -657,6 +680,7 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
             else     c = vraw[s][i];
             *(half8 *)&v_stage[(flat / CH) * PV + (flat % CH) * 8] = chunk_to_half8<TYPE>(c);
         }
+        if (DEEP && nxt >= 0) issue(nxt, stage);
         __builtin_amdgcn_wave_barrier();      // LDS runs a wave's instructions in order; keep the compiler from reordering
 
         // lane holds keys j0 + kb*16 + g4*4 + r of column j (V8: j0 + g4*8 + kb*4 + r)
@@ -796,7 +820,10 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
             walk = wave + first * DEC_WAVES;
         }
         convert_q();
-    } else {
+    } else if (RAW) {
+        request_q();                               // (ahead of K and V, whose request takes no branch: it is converted while they are on their way)
+        issue(wave, S0{});
+    } else if (!DEEP) {
         if (wave < n_steps) issue(wave, S0{});
     }
 
@@ -809,11 +836,45 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
 #pragma unroll
             for (int k = 0; k < PCS / 2; k++) vdst[i][k] = places[(i * 64 + lane) * (PCS / 2) + k];
     }
-    if constexpr (!MASK) {                         // (after the first K/V request: the two cold misses overlap)
-        request_q();
+    if constexpr (!MASK && !DEEP) {                // (after the first K/V request: the two cold misses overlap)
+        if (!RAW) request_q();
         convert_q();
     }
     typedef std::integral_constant<int, ONE ? 0 : 1> S1;
+    if constexpr (DEEP) {
+        // (Pairs of steps, an odd one ahead of them out of stage 1, and one way out of the loop: a way past a pair's second step would
+        //  make its rows uncountable again.)
+        const int own = n_steps > wave ? (n_steps - wave + DEC_WAVES - 1) / DEC_WAVES : 0;        // the wave's steps
+        int       it  = wave;
+        request_q();                               // (ahead of K and V: it is converted while they are on their way)
+        if (D == 128 || own <= 1) {                // (128-wide: ranges of one step a wave, see deep_rows)
+            if (own >= 1) {
+                issue(it, S0{});
+                __builtin_amdgcn_sched_barrier(0);
+                convert_q();
+                step(it, -1, S0{});
+            }
+        } else {
+            if (own & 1) {
+                issue(it, S1{});
+                issue(it + DEC_WAVES, S0{});
+                __builtin_amdgcn_sched_barrier(0);
+                convert_q();
+                step(it, it + 2 * DEC_WAVES, S1{});
+                it += DEC_WAVES;
+            } else {
+                issue(it, S0{});
+                issue(it + DEC_WAVES, S1{});
+                __builtin_amdgcn_sched_barrier(0);
+                convert_q();
+            }
+            do {
+                step(it, it + 2 * DEC_WAVES, S0{});
+                step(it + DEC_WAVES, it + 3 * DEC_WAVES, S1{});
+                it += 2 * DEC_WAVES;
+            } while (it < n_steps);
+        }
+    } else
     for (int it = walk; it < walk_end; it += 2 * DEC_WAVES) {
         step(it, it + DEC_WAVES, S0{});
         if (it + DEC_WAVES < walk_end) step(it + DEC_WAVES, it + 2 * DEC_WAVES, S1{});
@@ -929,11 +990,11 @@ fattn_decode_kernel(const FattnArgs a) {
     decode_body<D, TYPE, MASK, RAW, V8, PAD, false>(a, 0);
 }
 
-template <int D, bool MASK, int TYPE, bool RAW, bool V8, bool PAD>
+template <int D, bool MASK, int TYPE, bool RAW, bool V8, bool PAD, bool DEEP = false>
 __device__ __forceinline__ void decode_short(const DecodeShort & p) {
     FattnArgs a = decode_expand(p, D);
     if (!PAD) a.Dv = D;
-    decode_body<D, TYPE, MASK, RAW, V8, PAD, true>(a, MASK ? (int)(p.Dv >> 16) : 0);
+    decode_body<D, TYPE, MASK, RAW, V8, PAD, true, DEEP>(a, MASK ? (int)(p.Dv >> 16) : 0);
 }
 template <int D, int TYPE, bool RAW, bool V8, bool PAD>
 __global__ void __launch_bounds__(DEC_THREADS) __attribute__((amdgpu_waves_per_eu((decode_waves_min<D, TYPE, RAW>()), (decode_waves_max<D, RAW, V8>()))))
@@ -945,14 +1006,24 @@ fattn_decode_short_masked_kernel(const DecodeShort p) {
 // stream, 20 heads of 64 against 1500, one row 6.50 -> 6.27, five 6.65 -> 6.44, 8 heads of 128 against 700 6.77 -> 6.57.  A mask's look
 // and values need the tail's addresses; asked for behind K and V, or with the same head, those calls take 1 to 3% more than with a
 // structure (8 sequences of 300 to 1000 entries 14.05 and 14.35 us, 32 of Q4_0 28.9 and 29.95).
-// (64-wide f16 rows: 128 registers instead of 138, for four waves a SIMD.  That pays where workgroups share a CU and walk long
-//  ranges - 16 heads against 4000 keys, 8 sequences 28.1 -> 26.1 us, 16 of them 45.5 -> 44.5 - and costs 1 to 2% elsewhere, 5 rows x
-//  20 heads against 1500 keys 7.00 -> 7.07, 64 sequences of them 79.3 -> 80.8)
-template <int D, int TYPE, bool RAW, bool V8, bool PAD>
+// (64-wide f16 rows: 128 registers instead of 138, for four waves a SIMD, which pays where workgroups share a CU and walk long ranges; with
+//  DEEP three waves, see deep_rows.)
+template <int D, int TYPE, bool RAW, bool V8, bool PAD, bool DEEP>
 __global__ void __launch_bounds__(DEC_THREADS)
-__attribute__((amdgpu_waves_per_eu((D == 64 && TYPE == MI355X_TYPE_F16 ? 4 : decode_waves_min<D, TYPE, RAW>()), (decode_waves_max<D, RAW, V8>()))))
+__attribute__((amdgpu_waves_per_eu((D == 64 && TYPE == MI355X_TYPE_F16 ? (DEEP ? 3 : 4) : decode_waves_min<D, TYPE, RAW>()), (decode_waves_max<D, RAW, V8>()))))
 fattn_decode_short_kernel(FATTN_HEAD_PARAMS, const ArgTail<DecodeShort> tail) {
-    decode_short<D, false, TYPE, RAW, V8, PAD>(fattn_join<DecodeShort>(FATTN_HEAD_ARGS, tail));
+    decode_short<D, false, TYPE, RAW, V8, PAD, DEEP>(fattn_join<DecodeShort>(FATTN_HEAD_ARGS, tail));
+}
+
+// Unmasked f16 rows: DEEP, but for 64-wide heads where the CUs' fourth workgroups, which its registers do not leave room for, would be a
+// round of their own; on 128-wide heads, where two steps' rows take more registers than there are, ranges of one step a wave.
+// us a call inside a graph, without and with it: 5 rows x 20 heads of 64 against 1500 6.96 -> 6.85, against 375, 8 heads, 5.88 -> 5.40,
+// 64 sequences x 20 heads against 1500 77.0 -> 74.1 (1280 workgroups, two rounds either way), 8 sequences x 16 heads against 4000 27.4 ->
+// 28.8 where its three workgroups a CU cost a round (so not taken); 16 heads of 80 x 5 rows 8.2 -> 7.8; 128-wide, 8 KV heads: 663 entries
+// 7.1 -> 6.7, 2047 8.5 -> 8.0, 64 4.4 -> 4.1; with steps in pairs, spilling, 4000 10.2 -> 12.7, as taken 10.1.
+static inline bool deep_rows(int D, int64_t wgs, int n_cus, int keys_per_split) {
+    if (D == 128) return keys_per_split <= DEC_WAVES * STEP;
+    return (wgs + 3 * n_cus - 1) / (3 * n_cus) == (wgs + 4 * n_cus - 1) / (4 * n_cus);
 }
 
 template <int D, int TYPE, bool MASK, bool RAW, bool V8 = false, bool PAD = false>
@@ -973,9 +1044,16 @@ int launch_one(FattnArgs a, hipStream_t stream) {
                 if (e != hipSuccess) return (int)e;
                 fattn_launch(fattn_decode_short_masked_kernel<D, TYPE, RAW, V8, PAD>, short_grid, dim3(DEC_THREADS), lds, stream, p);
             } else {
-                const hipError_t e = fattn_allow_lds((const void *)fattn_decode_short_kernel<D, TYPE, RAW, V8, PAD>, lds, short_lds_allowed);
+                if constexpr (TYPE == MI355X_TYPE_F16) {
+                    static_assert(lds <= 64 * 1024, "no attribute to raise");
+                    if (deep_rows(D, pairs, a.n_cus, a.n_splits > 1 ? a.keys_per_split : a.Nkv)) {
+                        fattn_launch_head(fattn_decode_short_kernel<D, TYPE, RAW, V8, PAD, true>, short_grid, dim3(DEC_THREADS), lds, stream, p);
+                        return (int)hipGetLastError();
+                    }
+                }
+                const hipError_t e = fattn_allow_lds((const void *)fattn_decode_short_kernel<D, TYPE, RAW, V8, PAD, false>, lds, short_lds_allowed);
                 if (e != hipSuccess) return (int)e;
-                fattn_launch_head(fattn_decode_short_kernel<D, TYPE, RAW, V8, PAD>, short_grid, dim3(DEC_THREADS), lds, stream, p);
+                fattn_launch_head(fattn_decode_short_kernel<D, TYPE, RAW, V8, PAD, false>, short_grid, dim3(DEC_THREADS), lds, stream, p);
             }
             return (int)hipGetLastError();
         }
