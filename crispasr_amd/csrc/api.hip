@@ -857,6 +857,18 @@ void make_plan(const FattnArgs & a0, int ktype, int vtype, const mi355x_fattn_pa
         }
     }
     make_plan_core(a0, ktype, vtype, p, false, plan, steps);
+    // (calls that need no scratch without vec_takes_step, and so may overlap others on it, need none with it: whole they are no slower up to
+    //  448 keys, 8 heads of 64 x 24 x 375 7.1 us in two ranges, 5.4 whole, 8.6 the tile kernel, 20 of 128 x 16 x 440 11.0 and 23.0)
+    if (steps && plan.kernel == MI355X_FATTN_VEC && plan.workspace && vec_takes_step(a0, ktype, vtype, p)) {
+        Plan other;
+        make_plan(a0, ktype, vtype, p, other, false);
+        if (other.workspace == 0) {
+            plan.n_splits       = 1;
+            plan.keys_per_split = a0.Nkv;
+            plan.workspace      = 0;
+            plan.merge_sets     = 0;
+        }
+    }
 }
 
 // A plan that has to do with `room` bytes: a decode call that AUTO cut takes as many ranges as its partials fit there, down to those

@@ -30,11 +30,16 @@ def test_calls_next_to_the_rule(kw):
 
 
 def test_a_workspace_without_room_for_partials():
-    """as before the vector kernel took such calls: the tile kernel needs none here"""
-    case = make_case(seed=6800, D=64, Nq=24, Nkv=375, Hq=8, ktype=ora.F32)
+    """the tile kernel's, whose partials are fewer here, as before the vector kernel took such calls"""
+    case = make_case(seed=6800, D=64, Nq=5, Nkv=700, Hq=12, ktype=ora.F32)
     q, k, v = (upload(case[t]) for t in "qkv")
-    assert ggml.flash_attn_workspace_size(q, k, v, None, case["scale"]) > 4096
-    ws = torch.full((4096,), 0xA5, dtype=torch.uint8, device="cuda")
-    assert ggml.flash_attn_plan_details(q, k, v, None, case["scale"], workspace=ws[:16])["kernel"] == ggml.KERNEL_MMA
-    assert_parity(ggml.flash_attn_ext(q, k, v, None, case["scale"], workspace=ws[:16]).numpy_f32(), run_oracle(case))
-    assert (ws[16:] == 0xA5).all()
+    need = ggml.flash_attn_workspace_size(q, k, v, None, case["scale"])
+    room = ggml.flash_attn_workspace_size(q, k, v, None, case["scale"], kernel=ggml.KERNEL_MMA)
+    assert 0 < room < need
+    ws = torch.full((need,), 0xA5, dtype=torch.uint8, device="cuda")
+    assert ggml.flash_attn_plan_details(q, k, v, None, case["scale"], workspace=ws)["kernel"] == ggml.KERNEL_VEC
+    assert ggml.flash_attn_plan_details(q, k, v, None, case["scale"], workspace=ws[:room])["kernel"] == ggml.KERNEL_MMA
+    assert_parity(ggml.flash_attn_ext(q, k, v, None, case["scale"], workspace=ws[:room]).numpy_f32(), run_oracle(case))
+    assert (ws[room:] == 0xA5).all()
+    with pytest.raises(ggml.Mi355xError, match="workspace"):
+        ggml.flash_attn_ext(q, k, v, None, case["scale"], workspace=ws[:room - 16])
