@@ -772,6 +772,14 @@ void make_plan_core(const FattnArgs & a0, int ktype, int vtype, const mi355x_fat
     }
 }
 
+// the vector kernel's plan without ranges: no scratch
+void uncut(const FattnArgs & a, Plan & plan) {
+    plan.n_splits       = 1;
+    plan.keys_per_split = a.Nkv;
+    plan.workspace      = 0;
+    plan.merge_sets     = 0;
+}
+
 // Head sizes the MFMA kernels have no form for (multiples of 8 below 128 other than 64: 32 and 48, 80 and 96 of other
 // Whisper-like towers, ...) can still run on them, as the next larger of 64 and 128 with zeros behind the head's own
 // elements: the products over the padding are exact zeros, so the result is what the head size itself would give.
@@ -862,27 +870,26 @@ void make_plan(const FattnArgs & a0, int ktype, int vtype, const mi355x_fattn_pa
     if (steps && plan.kernel == MI355X_FATTN_VEC && plan.workspace && vec_takes_step(a0, ktype, vtype, p)) {
         Plan other;
         make_plan(a0, ktype, vtype, p, other, false);
-        if (other.workspace == 0) {
-            plan.n_splits       = 1;
-            plan.keys_per_split = a0.Nkv;
-            plan.workspace      = 0;
-            plan.merge_sets     = 0;
-        }
+        if (other.workspace == 0) uncut(a0, plan);
     }
 }
 
 // A plan that has to do with `room` bytes: a decode call that AUTO cut takes as many ranges as its partials fit there, down to those
 // that the price of whole steps and merges asks for (`fewest`, which was once the count itself: workspaces that programs sized by it
-// stay large enough); a call that vec_takes_step moved to the vector kernel, whose partials do not fit, is the tile kernel's, which may
-// need none (64-wide, not padded: where it needs its copies these are larger).  plan.workspace stays what the call would use at best.
-// False: the call does not fit.
+// stay large enough).  A call that vec_takes_step moved to the vector kernel, whose partials do not fit, has to do with what it had to do
+// with before: where the tile kernel's plan fits, it is that kernel's (64-wide), or, where that kernel would pad the head on copies, the
+// vector kernel's in one range.  Partials grow with the rows and copies with the keys, so that one or two heads of many rows need less
+// for the copies (96-wide, 383 rows of one head against 300 keys: 300272 bytes of partials, 153600 of copies; 10.9 us there and 9.0 in
+// one range, 32-wide 8.3 and 5.5, 72-wide 190 rows of two heads against 500 keys 12.6 and 12.5).  plan.workspace stays what a cut call
+// would use at best.  False: the call does not fit.
 bool fit_plan(FattnArgs a, int ktype, int vtype, const mi355x_fattn_params * p, size_t room, Plan & plan) {
     if (plan.workspace <= room) return true;
     if (plan.kernel == MI355X_FATTN_VEC && vec_takes_step(a, ktype, vtype, p)) {
         Plan other;
         make_plan(a, ktype, vtype, p, other, false);
-        if (other.kernel != MI355X_FATTN_MMA || other.pad || other.workspace > room) return false;
-        plan = other;
+        if (other.workspace > room) return false;
+        if (other.kernel == MI355X_FATTN_MMA && !other.pad) plan = other;
+        else uncut(a, plan);
         return true;
     }
     if (plan.kernel != MI355X_FATTN_DECODE_MMA || p->n_splits > 0 || plan.n_splits < 2 || room < plan.ws_partials) return false;

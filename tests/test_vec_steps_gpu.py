@@ -43,3 +43,17 @@ def test_a_workspace_without_room_for_partials():
     assert (ws[room:] == 0xA5).all()
     with pytest.raises(ggml.Mi355xError, match="workspace"):
         ggml.flash_attn_ext(q, k, v, None, case["scale"], workspace=ws[:room - 16])
+
+
+@pytest.mark.parametrize("D,Nq,Nkv,H,room", [(96, 383, 300, 1, 153600), (32, 383, 300, 1, 76800), (80, 360, 320, 1, 163840), (48, 380, 280, 1, 71680)])
+def test_a_workspace_of_the_padded_copies(D, Nq, Nkv, H, room):
+    """less than the vector kernel's partials take: its call in one range"""
+    case = make_case(seed=6900 + D, D=D, Nq=Nq, Nkv=Nkv, Hq=H, ktype=ora.F32)
+    print("case", D, Nq, Nkv, H, flush=True)
+    q, k, v = (upload(case[t]) for t in "qkv")
+    assert ggml.flash_attn_workspace_size(q, k, v, None, case["scale"], kernel=ggml.KERNEL_MMA) == room
+    assert ggml.flash_attn_workspace_size(q, k, v, None, case["scale"]) > room
+    ws = torch.full((room,), 0xA5, dtype=torch.uint8, device="cuda")
+    assert_parity(ggml.flash_attn_ext(q, k, v, None, case["scale"], workspace=ws).numpy_f32(), run_oracle(case))
+    with pytest.raises(ggml.Mi355xError, match="workspace"):
+        ggml.flash_attn_ext(q, k, v, None, case["scale"], workspace=ws[:room - 16])
