@@ -147,14 +147,15 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     auto dma_r = [&](int beta, char * to) __attribute__((always_inline)) { dma_rows(to, rbase, a.nbr1, p_base0 + 32 * beta, NR - 1, false); };
 
     // ---- prologue: table blocks 1 - NW .. 2, the first K tiles and V tile, Q_u and Q_v as B operands -----------------
-    // (block 1 - NW, which only the last wave reads and only here, lies in V's second half: its slot has block 2 already)
+    // (block 1 - NW, which only the last wave reads and only here, lies in V's second half: its slot has block 2 already; calls of one
+    //  tile need neither that block nor the second K tile)
     char * const first_block = vt + 32 * KP;
     dma_r(1 - NW, first_block);
 #pragma unroll 1
-    for (int beta = 2 - NW; beta <= 2; beta++) dma_r(beta, slot_of(beta));
+    for (int beta = 2 - NW; beta <= (NT > 1 ? 2 : 1); beta++) dma_r(beta, slot_of(beta));
     dma_k(0);
     dma_v(0);
-    dma_k(1);
+    if (NT > 1) dma_k(1);
     // Q_u and Q_v come along the rows, 4 of 64 values an instruction, and turn into B operands in the wave's square, as f16: fetched as
     // the operands lie an instruction takes 32 bytes of each of 32 rows
     half8 qu[KS], qv[KS];
@@ -255,7 +256,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
         };
         auto any_live = [&](float v) { return __builtin_amdgcn_ballot_w64(v > -INFINITY || v != v) != 0; };
         int live = NT;
-        if (!any_live(tile_max(NT - 1))) {
+        if (NT > 1 && !any_live(tile_max(NT - 1))) {
             live = NT - 1;
             while (live > 0) {
                 const int t0 = max(live - 4, 0);
@@ -410,23 +411,25 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
         buffer_to_lds16(rq_buf[i], off, rq_to[i], ins * 1024);
     };
 
-    // A step turns the scores of tile t, which the step before has left in registers, into probabilities beside the products of tile t + 1
-    // (the last step's are of no tile and not used), and un-skews those beside P.V: a matrix instruction is followed by its share of
-    // the vector work, its next operand and a request, and none of them moves (FR_FENCE).
+    // A step turns the scores of tile t, which the step before has left in registers, into probabilities beside the products of tile t + 1,
+    // and un-skews those beside P.V: a matrix instruction is followed by its share of the vector work, its next operand and a request,
+    // and none of them moves (FR_FENCE).  The last step stands by itself, without products and requests: as a turn of the loop like the
+    // others it took 0.6 to 0.9 us more, 8% of a call of 50 tokens (8 x 64 8.5 -> 7.7 us, 8 x 128 10.4 -> 9.6; 1000 tokens x 4 heads of 64 x 8 47.1 -> 46.0).
     uint32_t ring_at = (uint32_t)(2 - wave + NW - 1) % FR_SLOTS;              // slot of the wave's block t + 2
-#pragma unroll 1
-    for (int t = 0; t < NTL; t++) {
-        requests_of(t);
+    auto step = [&](int t, auto more) __attribute__((always_inline)) {
+        constexpr bool MORE = decltype(more)::value;
+        if (MORE) requests_of(t);
         constexpr int OPS = 2 * KS, RD = FR_RD, PER = 16 / OPS;               // products; operands read ahead; pairs of scores to each
         const uint32_t r_at = lds_ring + ring_at * 32 * KP + op0, k_at = lds_k + ((t + 1) & 1) * 32 * KP + op0;
         ring_at = ring_at + 1 == FR_SLOTS ? 0 : ring_at + 1;
         auto operand = [&](int i) __attribute__((always_inline)) { return *(lds_half8 *)(uintptr_t)((i < KS ? r_at : k_at) ^ (i % KS * 32)); };
         half8 ops[RD];
 #pragma unroll
-        for (int i = 0; i < RD; i++) ops[i] = operand(i);
+        for (int i = 0; i < (MORE ? RD : 0); i++) ops[i] = operand(i);
         FR_FENCE();
-        float16v acc;
+        float16v acc = {};
         auto product = [&](int i) __attribute__((always_inline)) {
+            if (!MORE) return;
             if (i % KS == 0) {
 #pragma unroll
                 for (int r = 0; r < 16; r++) acc[r] = 0.0f;
@@ -457,7 +460,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
             FR_FENCE();
         }
         const float16v bd_new = acc;
-        if (ADD && t + 1 < NTL) load_add(t + 1);
+        if (ADD && MORE) load_add(t + 1);
         if (__builtin_expect(32 * t + 32 > a.Nkv, 0)) {    // keys past the end of the last tile
             int key = 4 * hh;
             asm volatile("" : "+v"(key));
@@ -533,14 +536,19 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
             oacc[i / 2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vops[i % VD], p[i % 2], oacc[i / 2], 0, 0, 0);
             if (i + VD < VOPS) vops[i % VD] = v_operand(i + VD);
 #pragma unroll
-            for (int r = 16 * i / VOPS; r < 16 * (i + 1) / VOPS; r++) unskew(r, bd_prev, bd_new);
+            for (int r = 16 * i / VOPS; r < 16 * (i + 1) / VOPS; r++) if (MORE) unskew(r, bd_prev, bd_new);
             FR_FENCE();
         }
-        bd_prev = bd_new;
-        read_square();
-        meet();
-        if (ADD) have_add();
-    }
+        if constexpr (MORE) {
+            bd_prev = bd_new;
+            read_square();
+            meet();
+            if (ADD) have_add();
+        }
+    };
+#pragma unroll 1
+    for (int t = 0; t < NTL - 1; t++) step(t, std::true_type{});
+    if (NTL > 0) step(NTL - 1, std::false_type{});
 
     // ---- normalise and store: lane (il, hh) holds d = 32 db + 8 g + 4 hh + c of its query -------------------------------
     l = sum_of_halves(l);
@@ -555,8 +563,23 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
             for (int r = 0; r < 16; r++) chk = fmaf(oacc[db][r], 0.0f, chk);
         badbits = __builtin_amdgcn_ballot_w64(chk != 0.0f);
     }
-    {   // through the square, 32 values of d at a time: 8 rows of 128 bytes a store instead of 32 bytes of 32 rows
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    auto value4 = [&](int db, int g) __attribute__((always_inline)) {
+        float4v o;
+#pragma unroll
+        for (int c = 0; c < 4; c++) o[c] = oacc[db][4 * g + c] * inv;
+        return o;
+    };
+    if constexpr (D == 64) {
+        // (as they lie: the way through the square costs these short calls 0.1 to 0.2 us, 33 tokens x 8 heads 7.65 and 7.45)
+        if (i0w + il < a.Nq) {
+            float * const out = a.dst + (((int64_t)b * a.Nq + (i0w + il)) * a.H + h) * D;
+#pragma unroll
+            for (int db = 0; db < DBO; db++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) *(float4v *)(out + 32 * db + 8 * g + 4 * hh) = value4(db, g);
+        }
+    } else {   // through the square, 32 values of d at a time: 8 rows of 128 bytes a store instead of 32 bytes of 32 rows
         int         at   = lane;
         asm volatile("" : "+v"(at));                                  // (not worth registers in the loop)
         const int   orow = at >> 3, ocol = (at & 7) * 4;
@@ -564,12 +587,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
         for (int db = 0; db < DBO; db++) {
 #pragma unroll
-            for (int g = 0; g < 4; g++) {
-                float4v o;
-#pragma unroll
-                for (int c = 0; c < 4; c++) o[c] = oacc[db][4 * g + c] * inv;
-                *(float4v *)&sq[il * FR_SQP + 8 * g + 4 * hh] = o;
-            }
+            for (int g = 0; g < 4; g++) *(float4v *)&sq[il * FR_SQP + 8 * g + 4 * hh] = value4(db, g);
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const float4v o = *(const float4v *)&sq[(8 * j + orow) * FR_SQP + ocol];
