@@ -605,7 +605,10 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
         if (NQB == 1 || U == 1) cur = k_slot(cur, 1);
         PIPE_FENCE();
         // A probability that left f16's range (inf, or NaN from an infinite score) shows in the row's sum: the reference has
-        // fallen 16 binary orders behind.  Wave-uniform and rare.
+        // fallen 16 binary orders behind.  Wave-uniform and rare.  It shows in the sum of the row 16 away too, which shares columns of
+        // `ones` with it: what is still not finite under the raised reference is left out of the sums here and added to its own row's, so
+        // that a row of NaN, which comes this way with every unit, leaves the others as they are.  (v_mfma_f32_4x4x4_16b_f16, which mixes
+        // no rows, is 2 to 6% slower: 12 x 64 x 1500^2 x 4 40.5 and 43.1 us.)
         if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(lacc[QB][0] <= 1e30f)) != 0, 0)) {
             float mx = s[U][0];
 #pragma unroll
@@ -621,8 +624,6 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
                 base  = SPLAT ? delta : m[QB] + delta;
                 m[QB] += delta;
             }
-#pragma unroll
-            for (int r = 0; r < 4; r++) lacc[QB][r] = lprev * f;
             if (!MASK || __builtin_amdgcn_ballot_w64(lprev != 0.0f && f != 1.0f) != 0) {       // (not where rows see their first keys)
 #pragma unroll
                 for (int db = 0; db < DB; db++)
@@ -637,15 +638,20 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
                     for (int r = 0; r < 16; r++) s[1 - U][r] -= delta;
                 }
             }
+            float odd = 0.0f;                                      // 0, or NaN
 #pragma unroll
             for (int i = 0; i < 8; i++) {
                 e[2 * i]     = __builtin_amdgcn_exp2f(s[U][2 * i] - base);
                 e[2 * i + 1] = __builtin_amdgcn_exp2f(s[U][2 * i + 1] - base);
+                odd          = fmaf(e[2 * i] + e[2 * i + 1], 0.0f, odd);
                 pack(i);
                 PIPE_FENCE();
             }
-            add_sums(0);
-            add_sums(1);
+            odd = sum_of_halves(odd);
+#pragma unroll
+            for (int r = 0; r < 4; r++) lacc[QB][r] = fmaf(lprev, f, odd);
+#pragma unroll
+            for (int k = 0; k < 2; k++) lacc[QB] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, odd == 0.0f ? p[U][k] : zero8, lacc[QB], 0, 0, 0);
         }
     };
     typedef std::integral_constant<int, 0> I0;
