@@ -909,6 +909,7 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
             L += red_ml[w][col][1] * f[w];
         }
         bad = not_finite(L);
+        const float den = L == 0.0f ? INFINITY : L;             // (a sum of NaN makes the row NaN, as on the CPU)
         const int     ciq1 = query_of(row0 + col);
         const int     ch   = hk * a.gqa + row0 + col - ciq1 * a.gqa;
         const int64_t row  = ((int64_t)b * a.Nq + ciq1) * a.Hq + ch;
@@ -929,7 +930,7 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
             if (a.n_splits == 1) {
                 float4v o;
 #pragma unroll
-                for (int e = 0; e < 4; e++) o[e] = L > 0.0f ? acc[e] / L : 0.0f;
+                for (int e = 0; e < 4; e++) o[e] = acc[e] / den;
                 *(float4v *)(a.dst + row * dv + d) = o;
             } else {
                 float * pa = a.part_acc + (row * a.n_splits + split) * D + d;
@@ -944,7 +945,7 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
         if (a.n_splits > 1 && (tid & 15) == 0) {
             // natural-log units, as the merge expects them
             float * pm = a.part_ml + (row * a.n_splits + split) * 2;
-            const float mn = M == -INFINITY ? -INFINITY : M * 0.6931471805599453f;
+            const float mn = M == -INFINITY ? (L == L ? -INFINITY : 0.0f) : M * 0.6931471805599453f;      // (nor does the merge leave it out)
             if (a.counters) {
                 device_store2(pm, mn, L);
             } else {

@@ -43,5 +43,20 @@ def test_rows_on_their_own(kernel, variant, D, Nq, Nkv, Hq, B, mask, what):
     got = run_gpu(case, kernel=kernel, tile_variant=variant, n_splits=1)
     assert np.isfinite(ref[:, ~odd]).all()
     assert_parity(got[:, ~odd], ref[:, ~odd])
-    if np.isnan(what) and kernel != ggml.KERNEL_DECODE_MMA:
+    if np.isnan(what):
         assert np.isnan(got[:, odd]).all()
+
+
+@pytest.mark.parametrize("D,ktype", [(64, ora.F16), (128, ora.F16), (96, ora.F16), (64, ora.Q8_0), (128, ora.Q8_0), (128, ora.Q4_0)])
+@pytest.mark.parametrize("Nq,Nkv,ns", [(1, 20, 1), (1, 33, 1), (1, 300, 1), (3, 300, 2), (1, 1500, 0), (1, 1500, 7)])
+def test_decode_rows_of_nan_stay_nan(D, ktype, Nq, Nkv, ns):
+    case = make_case(seed=8100 + D + Nkv, D=D, Nq=Nq, Nkv=Nkv, Hq=4, Hkv=2, ktype=ktype)
+    q = to_f32(case["q"]).copy()
+    q[:, 1, -1, 3] = np.nan
+    case["q"] = ora.from_f32(q, ora.F32)
+    print("case", D, ktype, Nq, Nkv, ns, flush=True)
+    ref, got = run_oracle(case), run_gpu(case, kernel=ggml.KERNEL_DECODE_MMA, n_splits=ns)
+    assert np.isnan(got[:, -1, 1]).all()                     # (the exact oracle has no largest score and gives zeros; the CPU op gives NaN)
+    if ktype == ora.F16:
+        assert np.isnan(run_oracle(case, ora.MODE_GGML_LIKE)[:, -1, 1]).all()
+    assert_parity(got[:, :, [0, 2, 3]], ref[:, :, [0, 2, 3]])
