@@ -726,7 +726,7 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
                 delta = have ? fmaxf(mx, 0.0f) : mx;
                 have = true;
             }
-            const float f = __builtin_amdgcn_exp2f(-delta);
+            const float f = __builtin_amdgcn_exp2f(-fabsf(delta));      // (a first reference far below zero: nothing to scale, and 0 * inf is not 0)
             m += delta;
             l *= f;
 #pragma unroll

@@ -659,7 +659,7 @@ __global__ void __launch_bounds__(MMA_THREADS, 2) fattn_mma_kernel(const FattnAr
                         delta = st[qb].have ? fmaxf(tm, 0.0f) : tm;
                         st[qb].have = true;
                     }
-                    const float f = __builtin_amdgcn_exp2f(-delta);
+                    const float f = __builtin_amdgcn_exp2f(-fabsf(delta));      // (a first reference far below zero: nothing to scale, and 0 * inf is not 0)
                     st[qb].m += delta;
                     st[qb].l *= f;
 #pragma unroll
