@@ -1100,6 +1100,49 @@ int mi355x_fattn_plan_details(const mi355x_tensor * q, const mi355x_tensor * k, 
     return MI355X_OK;
 }
 
+int mi355x_fattn_plan_kernel_form(const mi355x_tensor * q, const mi355x_tensor * k, const mi355x_tensor * v,
+                                  const mi355x_tensor * mask, const mi355x_fattn_params * params,
+                                  int32_t * form) {
+    if (!form) return fail(MI355X_ERR_INVALID, "null argument");
+    const int rc = check(q, k, v, mask, nullptr, params);
+    if (rc) return rc;
+    FattnArgs a;
+    fill_args(a, q, k, v, mask, nullptr, params);
+    Plan plan;
+    make_plan(a, k->type, v->type, params, plan);
+    if (params->workspace) fit_plan(a, k->type, v->type, params, params->workspace_size, plan);
+    *form = MI355X_FATTN_FORM_GENERAL;
+    if ((int64_t)a.Nq * a.Hq * a.B == 0) return MI355X_OK;
+    FattnMmaVariant var;
+    int waves = 0;
+    if (plan.kernel == MI355X_FATTN_MMA) {
+        if (tile_plan(a, k->type, plan, var, waves) && waves) {
+            apply_pad(a, plan);
+            a.n_splits       = plan.n_splits;
+            a.keys_per_split = plan.keys_per_split;
+            if (fattn_pipe_alone(a, var)) *form = MI355X_FATTN_FORM_KEYS_APART;
+        }
+        return MI355X_OK;
+    }
+    // the call's arguments as its launcher is handed them, with addresses that nothing reads through
+    char * const here = (char *)(uintptr_t)4096;
+    apply_pad(a, plan);
+    int ktype = k->type;
+    if (plan.kv_to_f16) {
+        use_f16_copies(a, here);
+        ktype = MI355X_TYPE_F16;
+    }
+    if (a.masked && !a.mask) a.mask = here;
+    a.n_splits       = plan.n_splits;
+    a.keys_per_split = plan.keys_per_split;
+    if (plan.n_splits > 1) {
+        a.part_acc = (float *)here;
+        a.part_ml  = a.part_acc + (size_t)a.Nq * a.Hq * a.B * plan.n_splits * a.D;
+    }
+    *form = plan.kernel == MI355X_FATTN_VEC ? fattn_vec_form(a, ktype) : fattn_decode_supported(a, ktype) ? fattn_decode_form(a, ktype) : *form;
+    return MI355X_OK;
+}
+
 int mi355x_fattn_workspace_size(const mi355x_tensor * q, const mi355x_tensor * k, const mi355x_tensor * v,
                                 const mi355x_tensor * mask, const mi355x_fattn_params * params,
                                 size_t * bytes) {

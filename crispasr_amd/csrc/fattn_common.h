@@ -520,6 +520,7 @@ struct FattnRelposArgs {
 
 // Launchers implemented next to their kernels; all return hipError_t as int.
 int fattn_vec_launch(const FattnArgs & a, int ktype, hipStream_t stream);
+int fattn_vec_form(const FattnArgs & a, int ktype);              // mi355x_fattn_form of the call, as its launcher decides it
 int fattn_merge_launch(const FattnArgs & a, hipStream_t stream);
 int fattn_mma_launch(const FattnArgs & a, int ktype, hipStream_t stream);
 // the instantiation of the tile kernel a call takes
@@ -533,9 +534,11 @@ struct FattnMmaVariant {
 void fattn_mma_variant(const FattnArgs & a, int ktype, FattnMmaVariant & v);
 // waves of a workgroup of the pipelined kernel, which takes the variant's place, or 0: the tile kernel's (four)
 int fattn_pipe_waves(const FattnArgs & a, int ktype, const FattnMmaVariant & v);
+bool fattn_pipe_alone(const FattnArgs & a, const FattnMmaVariant & v);       // (of its calls) waves that take different keys of the same queries
 int fattn_pipe_launch(const FattnArgs & a, const FattnMmaVariant & v, int waves, hipStream_t stream);
 bool fattn_mma_supported(const FattnArgs & a, int ktype);
 int fattn_decode_launch(const FattnArgs & a, int ktype, hipStream_t stream);
+int fattn_decode_form(const FattnArgs & a, int ktype);
 bool fattn_decode_supported(const FattnArgs & a, int ktype);
 int cpy_launch(const CpyArgs & a, int stype, int dtype, hipStream_t stream);
 int set_rows_launch(const CpyArgs & a, int dtype, hipStream_t stream);

@@ -1027,6 +1027,18 @@ static inline bool deep_rows(int D, int64_t wgs, int n_cus, int keys_per_split) 
     return (wgs + 3 * n_cus - 1) / (3 * n_cus) == (wgs + 4 * n_cus - 1) / (4 * n_cus);
 }
 
+// the form of the kernel that a call takes; p: its arguments where they are short
+template <int D, int TYPE, bool RAW, bool V8>
+int form_of(const FattnArgs & a, DecodeShort & p) {
+    if constexpr (TYPE == MI355X_TYPE_F16 || V8 || (RAW && TYPE != MI355X_TYPE_Q8_0)) {      // (the rows of a cache as they usually lie)
+        if (decode_shorten(a, p))
+            return TYPE == MI355X_TYPE_F16 && !a.mask && deep_rows(D, (int64_t)a.n_splits * a.Hkv * a.B, a.n_cus, a.n_splits > 1 ? a.keys_per_split : a.Nkv)
+                       ? MI355X_FATTN_FORM_DEEP
+                       : MI355X_FATTN_FORM_SHORT;
+    }
+    return MI355X_FATTN_FORM_GENERAL;
+}
+
 template <int D, int TYPE, bool MASK, bool RAW, bool V8 = false, bool PAD = false>
 int launch_one(FattnArgs a, hipStream_t stream) {
     const int64_t pairs = (int64_t)a.n_splits * a.Hkv * a.B;
@@ -1034,9 +1046,10 @@ int launch_one(FattnArgs a, hipStream_t stream) {
     if (wgs > 0x7fffffff || a.q_chunks != (a.Nq * a.gqa + 15) / 16) return (int)hipErrorInvalidValue;
     const dim3 grid((unsigned)wgs);
     constexpr int lds = decode_lds_bytes<D, TYPE, RAW, V8>();
-    if constexpr (TYPE == MI355X_TYPE_F16 || V8 || (RAW && TYPE != MI355X_TYPE_Q8_0)) {      // (the rows of a cache as they usually lie)
+    if constexpr (TYPE == MI355X_TYPE_F16 || V8 || (RAW && TYPE != MI355X_TYPE_Q8_0)) {
         DecodeShort p;
-        if (decode_shorten(a, p)) {
+        const int   form = form_of<D, TYPE, RAW, V8>(a, p);
+        if (form != MI355X_FATTN_FORM_GENERAL) {
             if (MASK) p.Dv |= decode_turns(a, TYPE == MI355X_TYPE_F16 ? D * 2 : D / 32 * raw_block_bytes<TYPE>()) << 16;
             static std::atomic<uint64_t> short_lds_allowed{0};
             const dim3 short_grid((unsigned)a.n_splits, (unsigned)a.Hkv, (unsigned)a.B);
@@ -1047,7 +1060,7 @@ int launch_one(FattnArgs a, hipStream_t stream) {
             } else {
                 if constexpr (TYPE == MI355X_TYPE_F16) {
                     static_assert(lds <= 64 * 1024, "no attribute to raise");
-                    if (deep_rows(D, pairs, a.n_cus, a.n_splits > 1 ? a.keys_per_split : a.Nkv)) {
+                    if (form == MI355X_FATTN_FORM_DEEP) {
                         fattn_launch_head(fattn_decode_short_kernel<D, TYPE, RAW, V8, PAD, true>, short_grid, dim3(DEC_THREADS), lds, stream, p);
                         return (int)hipGetLastError();
                     }
@@ -1073,13 +1086,11 @@ int launch_one(FattnArgs a, hipStream_t stream) {
     return (int)hipGetLastError();
 }
 
-template <int D, int TYPE>
-int launch(const FattnArgs & a, hipStream_t stream) {
-    if (a.Dv != a.D) {              // another head size on f16 rows, or nothing
-        if constexpr (TYPE == MI355X_TYPE_F16)
-            return a.mask ? launch_one<D, TYPE, true, false, false, true>(a, stream) : launch_one<D, TYPE, false, false, false, true>(a, stream);
-        return (int)hipErrorInvalidValue;
-    }
+// go(RAW, V8) of a call over whole heads: quantised rows that are streamed, and whether V goes through its int8 stage
+template <int D, int TYPE, typename F>
+int by_rows(const FattnArgs & a, F go) {
+    typedef std::true_type  Yes;
+    typedef std::false_type No;
     if constexpr (FATTN_IS_BLOCK_TYPE(TYPE)) {
         // contiguous rows, and every step of every (head, batch, split) starts on a unit boundary
         constexpr int RS   = D / 32 * raw_block_bytes<TYPE>();
@@ -1091,12 +1102,29 @@ int launch(const FattnArgs & a, hipStream_t stream) {
         if (raw && !no_raw) {
             if constexpr (TYPE == MI355X_TYPE_Q8_0) {
                 static const bool f16_stage = getenv("MI355X_FATTN_DECODE_F16_STAGE") != nullptr;     // the earlier V path, for comparison runs
-                if (!f16_stage) return a.mask ? launch_one<D, TYPE, true, true, true>(a, stream) : launch_one<D, TYPE, false, true, true>(a, stream);
+                if (!f16_stage) return go(Yes{}, Yes{});
             }
-            return a.mask ? launch_one<D, TYPE, true, true>(a, stream) : launch_one<D, TYPE, false, true>(a, stream);
+            return go(Yes{}, No{});
         }
     }
-    return a.mask ? launch_one<D, TYPE, true, false>(a, stream) : launch_one<D, TYPE, false, false>(a, stream);
+    return go(No{}, No{});
+}
+
+template <int D, int TYPE>
+int launch(const FattnArgs & a, hipStream_t stream) {
+    if (a.Dv != a.D) {              // another head size on f16 rows, or nothing
+        if constexpr (TYPE == MI355X_TYPE_F16)
+            return a.mask ? launch_one<D, TYPE, true, false, false, true>(a, stream) : launch_one<D, TYPE, false, false, false, true>(a, stream);
+        return (int)hipErrorInvalidValue;
+    }
+    return by_rows<D, TYPE>(a, [&](auto raw, auto v8) {
+        return a.mask ? launch_one<D, TYPE, true, raw(), v8()>(a, stream) : launch_one<D, TYPE, false, raw(), v8()>(a, stream);
+    });
+}
+template <int D, int TYPE>
+int form(const FattnArgs & a) {
+    DecodeShort p;
+    return by_rows<D, TYPE>(a, [&](auto raw, auto v8) { return form_of<D, TYPE, raw(), v8()>(a, p); });
 }
 
 }  // namespace
@@ -1114,9 +1142,9 @@ bool fattn_decode_supported(const FattnArgs & a, int ktype) {
 }
 
 int fattn_decode_launch(const FattnArgs & a, int ktype, hipStream_t stream) {
-    if (ktype == MI355X_TYPE_F16) return a.D == 64 ? launch<64, MI355X_TYPE_F16>(a, stream) : launch<128, MI355X_TYPE_F16>(a, stream);
     switch (ktype) {
 #define DEC(T) case T: return a.D == 64 ? launch<64, T>(a, stream) : launch<128, T>(a, stream)
+        DEC(MI355X_TYPE_F16);
         DEC(MI355X_TYPE_Q8_0);
         DEC(MI355X_TYPE_Q4_0);
         DEC(MI355X_TYPE_Q4_1);
@@ -1124,5 +1152,19 @@ int fattn_decode_launch(const FattnArgs & a, int ktype, hipStream_t stream) {
         DEC(MI355X_TYPE_Q5_1);
 #undef DEC
         default: return (int)hipErrorInvalidValue;
+    }
+}
+
+int fattn_decode_form(const FattnArgs & a, int ktype) {
+    switch (ktype) {
+#define DEC(T) case T: return a.D == 64 ? form<64, T>(a) : form<128, T>(a)
+        DEC(MI355X_TYPE_F16);
+        DEC(MI355X_TYPE_Q8_0);
+        DEC(MI355X_TYPE_Q4_0);
+        DEC(MI355X_TYPE_Q4_1);
+        DEC(MI355X_TYPE_Q5_0);
+        DEC(MI355X_TYPE_Q5_1);
+#undef DEC
+        default: return MI355X_FATTN_FORM_GENERAL;
     }
 }

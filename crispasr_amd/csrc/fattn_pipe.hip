@@ -901,7 +901,8 @@ int fattn_pipe_waves(const FattnArgs & a, int ktype, const FattnMmaVariant & v) 
 // and its waves have to have keys enough for the longer hand-over.  us a call, pairs and like this, in graphs: 8 heads x 1500 13.2, 12.6,
 // x 1000 10.4, 10.1, x 768 8.9, 8.9, x 500 7.4, 7.7; 4 x 1500 12.7, 12.0, 4 x 800 9.7, 9.25.  Nearly every CU with one (all ask L2 for
 // their keys at once): 12 x 1300 14.05, 13.5, 16 x 1000 11.5, 11.8.
-static bool pipe_alone(const FattnArgs & a) {
+bool fattn_pipe_alone(const FattnArgs & a, const FattnMmaVariant & v) {
+    if (a.masked || a.D != 64 || a.Dv != a.D || v.key_split != 2) return false;
     const int64_t wgs = (int64_t)((a.Nq + 63) / 64) * a.Hq * a.B * a.n_splits;
     return a.tile_variant == 0 && wgs <= a.n_cus && (a.n_splits > 1 ? a.keys_per_split : a.Nkv) >= (wgs * 8 <= (int64_t)a.n_cus * 7 ? 768 : 1152);
 }
@@ -918,7 +919,7 @@ int fattn_pipe_launch(const FattnArgs & a, const FattnMmaVariant & v, int waves,
         return waves == 8 ? launch<64, 2, 1, 8, false>(a, stream) : launch<64, 2, 1, 4, false>(a, stream);
     }
     if (a.D == 64) {
-        if (v.key_split == 2 && !pad && pipe_alone(a)) return launch<64, 2, 4, 4, false>(a, stream);
+        if (fattn_pipe_alone(a, v)) return launch<64, 2, 4, 4, false>(a, stream);
         if (v.key_split == 2) return pad ? launch<64, 1, 2, 4, true>(a, stream) : launch<64, 1, 2, 4, false>(a, stream);
         return pad ? launch<64, 1, 1, 4, true>(a, stream) : launch<64, 1, 1, 4, false>(a, stream);
     }

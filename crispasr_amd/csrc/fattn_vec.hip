@@ -239,6 +239,11 @@ int fattn_vec_launch(const FattnArgs & a, int ktype, hipStream_t stream) {
     }
 }
 
+int fattn_vec_form(const FattnArgs & a, int ktype) {
+    VecShort p;
+    return (ktype == MI355X_TYPE_F32 || ktype == MI355X_TYPE_F16) && vec_shorten(a, ktype, p) ? MI355X_FATTN_FORM_SHORT : MI355X_FATTN_FORM_GENERAL;
+}
+
 int fattn_merge_launch(const FattnArgs & a, hipStream_t stream) {
     const int rows = a.Nq * a.Hq * a.B;
     const int rows_per_block = 4 * (64 / (a.D / 4));          // D is a multiple of 8, at most 256

@@ -32,6 +32,7 @@ TYPE_SIZE = {F32: 4, F16: 2, Q4_0: 18, Q4_1: 20, Q5_0: 22, Q5_1: 24, Q8_0: 34}
 BLOCK_SIZE = {F32: 1, F16: 1, Q4_0: 32, Q4_1: 32, Q5_0: 32, Q5_1: 32, Q8_0: QK8_0}
 
 KERNEL_AUTO, KERNEL_VEC, KERNEL_MMA, KERNEL_DECODE_MMA = 0, 1, 2, 3
+FORM_GENERAL, FORM_SHORT, FORM_DEEP, FORM_KEYS_APART = 0, 1, 2, 3
 PREC_DEFAULT, PREC_F32 = 0, 10
 # tile_variant values: 16 * key_split + query_blocks
 TILE_Q256, TILE_Q128, TILE_Q64_KEYSPLIT = 16 + 2, 16 + 1, 32 + 1
@@ -91,6 +92,7 @@ EXPORTS = [
     "mi355x_api_version", "mi355x_status_string", "mi355x_last_error",
     "mi355x_device_count", "mi355x_device_get_info", "mi355x_set_device", "mi355x_stream_synchronize",
     "mi355x_fattn_supports", "mi355x_flash_attn_ext", "mi355x_flash_attn_ext_noalloc", "mi355x_fattn_workspace_size", "mi355x_fattn_plan", "mi355x_fattn_plan_details", "mi355x_fattn_plan_form",
+    "mi355x_fattn_plan_kernel_form",
     "mi355x_relpos_bias_supports", "mi355x_relpos_bias", "mi355x_relpos_bias_workspace_size", "mi355x_flash_attn_relpos", "mi355x_fattn_relpos_workspace_size",
     "mi355x_cpy_supports", "mi355x_cpy", "mi355x_set_rows", "mi355x_set_rows_supports",
     "mi355x_buffer_alloc", "mi355x_buffer_free", "mi355x_host_buffer_alloc", "mi355x_host_buffer_free", "mi355x_host_buffer_mirror_stats", "mi355x_host_buffer_invalidate", "mi355x_buffer_memset", "mi355x_buffer_set",
@@ -124,6 +126,7 @@ def lib() -> ctypes.CDLL:
         L.mi355x_fattn_workspace_size.argtypes = [PT, PT, PT, PT, PP, ctypes.POINTER(ctypes.c_size_t)]
         L.mi355x_fattn_plan.argtypes = [PT, PT, PT, PT, PP, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)]
         L.mi355x_fattn_plan_form.argtypes = [PT, PT, PT, PT, PP, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)]
+        L.mi355x_fattn_plan_kernel_form.argtypes = [PT, PT, PT, PT, PP, ctypes.POINTER(ctypes.c_int32)]
         L.mi355x_fattn_plan_details.argtypes = [PT, PT, PT, PT, PP, ctypes.POINTER(CPlanInfo)]
         L.mi355x_relpos_bias_supports.argtypes = [PT, PT, PT, PT]
         L.mi355x_relpos_bias.argtypes = [PT, PT, PT, PT, ctypes.c_float, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
@@ -351,6 +354,16 @@ def flash_attn_plan_form(q: Tensor, k: Tensor, v: Tensor, mask: Optional[Tensor]
     _check(lib().mi355x_fattn_plan_form(q.ref(), k.ref(), v.ref(), mask.ref() if mask is not None else None,
                                         ctypes.byref(p), ctypes.byref(pipelined), ctypes.byref(waves)))
     return {"pipelined": pipelined.value, "waves": waves.value}
+
+
+def flash_attn_plan_kernel_form(q: Tensor, k: Tensor, v: Tensor, mask: Optional[Tensor] = None, scale: float = 1.0,
+                                max_bias: float = 0.0, logit_softcap: float = 0.0, kernel: int = KERNEL_AUTO,
+                                n_splits: int = 0, tile_variant: int = 0) -> int:
+    """FORM_GENERAL, FORM_SHORT, FORM_DEEP or FORM_KEYS_APART: the form of its kernel that the call takes"""
+    p = _params(scale, max_bias, logit_softcap, PREC_DEFAULT, kernel, n_splits, None, 0, tile_variant)
+    form = ctypes.c_int32()
+    _check(lib().mi355x_fattn_plan_kernel_form(q.ref(), k.ref(), v.ref(), mask.ref() if mask is not None else None, ctypes.byref(p), ctypes.byref(form)))
+    return form.value
 
 
 def flash_attn_workspace_size(q: Tensor, k: Tensor, v: Tensor, mask: Optional[Tensor] = None, scale: float = 1.0,

@@ -239,6 +239,18 @@ int mi355x_fattn_plan_form(const mi355x_tensor * q, const mi355x_tensor * k, con
                            const mi355x_tensor * mask, const mi355x_fattn_params * params,
                            int32_t * pipelined, int32_t * waves);
 
+/* The form of that kernel, where it has more than one (tests assert that a call runs the form it is meant for; it depends on the data
+ * pointers' alignment, like the plan). */
+enum mi355x_fattn_form {
+    MI355X_FATTN_FORM_GENERAL    = 0,
+    MI355X_FATTN_FORM_SHORT      = 1,  /* vector and decode kernel: arguments of 96 and 112 bytes, a grid without divisions */
+    MI355X_FATTN_FORM_DEEP       = 2,  /* decode kernel: the same, rows of two steps under way */
+    MI355X_FATTN_FORM_KEYS_APART = 3   /* pipelined kernel: waves that take different keys of the same 64 queries */
+};
+int mi355x_fattn_plan_kernel_form(const mi355x_tensor * q, const mi355x_tensor * k, const mi355x_tensor * v,
+                                  const mi355x_tensor * mask, const mi355x_fattn_params * params,
+                                  int32_t * form);
+
 /* ---- FastConformer relative-position attention (src/core/fastconformer.h:876-935) ---------- */
 
 /*

@@ -26,6 +26,12 @@ def plan_details(case: dict, **kw) -> dict:
     return ca.ggml.flash_attn_plan_details(q, k, v, m, case["scale"], case["max_bias"], case["softcap"], **kw)
 
 
+def kernel_form(case: dict, **kw) -> int:
+    q, k, v = upload(case["q"]), upload(case["k"]), upload(case["v"])
+    m = upload(case["mask"]) if case["mask"] is not None else None
+    return ca.ggml.flash_attn_plan_kernel_form(q, k, v, m, case["scale"], case["max_bias"], case["softcap"], **kw)
+
+
 def run_oracle(case: dict, mode: int = ora.MODE_EXACT) -> np.ndarray:
     return ora.flash_attn_ext(case["q"], case["k"], case["v"], case["mask"], case["scale"],
                               case["max_bias"], case["softcap"], mode)

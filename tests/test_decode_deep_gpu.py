@@ -8,10 +8,18 @@ import crispasr_amd as ca
 import oracle as ora
 from cases import errors, make_case
 from crispasr_amd import ggml
-from gpu_util import assert_parity, run_gpu, run_oracle
+from gpu_util import assert_parity, kernel_form, run_gpu, run_oracle
 from test_fattn_pipe_ends_gpu import _behind
 
 pytestmark = pytest.mark.gpu
+
+
+def _check(case, ref, ns, what=""):
+    """f16 rows: two steps under way, at (or padded to) 128 elements in ranges of one step a wave only"""
+    D, Nkv = case["k"].ne[:2]
+    keys = ((Nkv + ns - 1) // ns + 31) // 32 * 32
+    assert kernel_form(case, kernel=ggml.KERNEL_DECODE_MMA, n_splits=ns) == (ggml.FORM_DEEP if D <= 64 or keys <= 128 else ggml.FORM_SHORT)
+    assert_parity(run_gpu(case, kernel=ggml.KERNEL_DECODE_MMA, n_splits=ns), ref, what)
 
 
 @pytest.mark.parametrize("D", [64, 128, 80, 32])
@@ -21,7 +29,7 @@ def test_steps(D, Nkv):
     print("case", D, Nkv, flush=True)
     ref = run_oracle(case)
     for ns in (1, 3):
-        assert_parity(run_gpu(case, kernel=ggml.KERNEL_DECODE_MMA, n_splits=ns), ref, "%d ranges" % ns)
+        _check(case, ref, ns, "%d ranges" % ns)
 
 
 @pytest.mark.parametrize("D", [64, 128, 96])
@@ -32,13 +40,14 @@ def test_nan_bits_behind_the_last_key(D, Nkv):
     print("case", D, Nkv, flush=True)
     ref = run_oracle(case)
     for ns in (1, 2):
-        assert_parity(run_gpu(case, kernel=ggml.KERNEL_DECODE_MMA, n_splits=ns), ref, "%d ranges" % ns)
+        _check(case, ref, ns, "%d ranges" % ns)
 
 
-@pytest.mark.parametrize("Hq,B", [(12, 64), (13, 64), (16, 64), (17, 64)])          # 768, 832, 1024 and 1088 workgroups on 256 CUs
-def test_grids(Hq, B):
+@pytest.mark.parametrize("Hq,B,deep", [(12, 64, True), (13, 64, False), (16, 64, False), (17, 64, True)])          # 768, 832, 1024 and 1088 workgroups on 256 CUs
+def test_grids(Hq, B, deep):
     case = make_case(seed=7200 + Hq, D=64, Nq=1, Nkv=140, Hq=Hq, B=B)
     print("case", Hq, B, flush=True)
+    assert kernel_form(case, kernel=ggml.KERNEL_DECODE_MMA, n_splits=1) == (ggml.FORM_DEEP if deep else ggml.FORM_SHORT)
     assert_parity(run_gpu(case, kernel=ggml.KERNEL_DECODE_MMA, n_splits=1), run_oracle(case))
 
 
@@ -48,6 +57,7 @@ def test_streamed_rows(D, ktype):
     for Nkv, ns in ((1, 1), (33, 1), (97, 1), (129, 1), (300, 2), (420, 4)):
         case = make_case(seed=7300 + D + Nkv, D=D, Nq=2, Nkv=Nkv, Hq=4, Hkv=2, ktype=ktype)
         print("case", D, ktype, Nkv, ns, flush=True)
+        assert kernel_form(case, kernel=ggml.KERNEL_DECODE_MMA, n_splits=ns) == ggml.FORM_SHORT
         assert_parity(run_gpu(case, kernel=ggml.KERNEL_DECODE_MMA, n_splits=ns), run_oracle(case))
 
 
@@ -62,7 +72,9 @@ def test_rows_far_apart():
             buf[i * pitch:i * pitch + 2 * D] = x[i].view(torch.uint8)
         far.append(ca.Tensor(buf, ggml.F16, (D, n, 1, 1), (2, pitch, pitch * n, pitch * n)))
     q = torch.randn(D, device="cuda")
-    out = ca.flash_attn_ext(ca.Tensor(q.view(torch.uint8), ggml.F32, (D, 1, 1)), far[0], far[1], None, 0.125, kernel=ggml.KERNEL_DECODE_MMA).numpy_f32()
+    qt = ca.Tensor(q.view(torch.uint8), ggml.F32, (D, 1, 1))
+    assert ggml.flash_attn_plan_kernel_form(qt, far[0], far[1], None, 0.125, kernel=ggml.KERNEL_DECODE_MMA) == ggml.FORM_GENERAL
+    out = ca.flash_attn_ext(qt, far[0], far[1], None, 0.125, kernel=ggml.KERNEL_DECODE_MMA).numpy_f32()
     k, v = (x.double().cpu() for x in rows)
     ref = (torch.softmax(0.125 * (k @ q.double().cpu()), 0) @ v).numpy()
     max_abs, rel = errors(out.reshape(-1), ref)

@@ -41,3 +41,18 @@ def test_ranges_longer_than_request_addresses(mask):
         q, k = _t(ggml.F32, (128, 100, 4, 1)), ca.Tensor(None, ggml.F16, (128, 1000, 4, 1), (2, pitch, 256, pitch * 1000))
         return ggml.flash_attn_plan_form(q, k, k, _t(ggml.F16, (1000, 100, mask, 1)) if mask else None, 0.1, kernel=ggml.KERNEL_MMA, tile_variant=0x11, n_splits=ns)["pipelined"]
     assert pipelined(1 << 20) == 1 and pipelined(1 << 21) == 0 and (mask or pipelined(1 << 21, 3) == 1)
+
+
+# (256 CUs: 224 workgroups of 64 queries leave an eighth of them without one)
+@pytest.mark.parametrize("Nq,H,B,least", [(1, 1, 1, 768), (1500, 8, 1, 768), (1792, 8, 1, 768), (128, 7, 16, 768), (1856, 8, 1, 1152), (2048, 8, 1, 1152), (2049, 8, 1, None)])
+def test_waves_of_different_keys(Nq, H, B, least):
+    def form(Nkv, D=64, mask=None, kernel=ggml.KERNEL_MMA, **kw):
+        q, k = _t(ggml.F32, (D, Nq, H, B)), _t(ggml.F16, (D, Nkv, H, B))
+        return ggml.flash_attn_plan_kernel_form(q, k, k, _t(ggml.F16, (Nkv, Nq, 1, 1)) if mask else None, 0.1, kernel=kernel, **{"n_splits": 1, **kw})
+    for Nkv in (100, 767, 768, 1151, 1152, 4000):
+        assert form(Nkv) == (ggml.FORM_KEYS_APART if least and Nkv >= least else ggml.FORM_GENERAL), Nkv
+    for other in (dict(D=128), dict(D=56), dict(mask=1), dict(tile_variant=0x21), dict(logit_softcap=20.0), dict(kernel=ggml.KERNEL_VEC)):
+        assert form(1200, **other) != ggml.FORM_KEYS_APART, other
+    if least == 768:
+        assert form(1536, n_splits=2) == (ggml.FORM_KEYS_APART if H * B * ((Nq + 63) // 64) * 2 <= 224 else ggml.FORM_GENERAL)
+        assert form(1472, n_splits=2) == ggml.FORM_GENERAL                                 # (ranges of 736 keys)
