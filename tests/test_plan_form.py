@@ -55,4 +55,4 @@ def test_waves_of_different_keys(Nq, H, B, least):
         assert form(1200, **other) != ggml.FORM_KEYS_APART, other
     if least == 768:
         assert form(1536, n_splits=2) == (ggml.FORM_KEYS_APART if H * B * ((Nq + 63) // 64) * 2 <= 224 else ggml.FORM_GENERAL)
-        assert form(1472, n_splits=2) == ggml.FORM_GENERAL                                 # (ranges of 736 keys)
+        assert form(1408, n_splits=2) == ggml.FORM_GENERAL                                 # (ranges of 704 keys)
