@@ -202,8 +202,8 @@ static __device__ __forceinline__ float quad_broadcast(float x, int k) {        
 // load must not read an SGPR within five of the vector instruction that wrote it, as is the readlane of a spilled base where
 // scalar registers are short.  MOVE: the base goes through a scalar move, which may read it at once.  Without it, for kernels
 // that keep their bases in scalar registers: tests/test_kernel_resources.py fails if one of those loads has such a write close
-// before it.  (The pipelined kernel spills none, and a move in its step, wherever it stands, costs a wave that is alone on its
-// SIMD more than it looks: six layers of Whisper base 119.5 us, with a move ahead of each load 121, with one a step 124 to 130.)
+// before it.  (The pipelined kernel's forms without a mask spill none - the three masked ones 21 to 24 scalar registers - and a move in
+// their step, wherever it stands, costs a wave that is alone on its SIMD more than it looks: six layers of Whisper base 119.5 us, with a move ahead of each load 121, with one a step 124 to 130.)
 template <bool MOVE>
 static __device__ __forceinline__ void load_to_lds16(uint64_t base, uint32_t off, uint32_t to) {
     // (the readfirstlanes say that the addresses are uniform and cost nothing where the register allocator knows)
@@ -216,14 +216,6 @@ static __device__ __forceinline__ void load_to_lds16(uint64_t base, uint32_t off
     } else {
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(p), "s"(t) : "memory", "m0");
     }
-}
-
-// the same with 4 bytes a lane
-static __device__ __forceinline__ void load_to_lds4(uint64_t base, uint32_t off, uint32_t to) {
-    const uint64_t p = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(base >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)base);
-    const uint32_t t = (uint32_t)__builtin_amdgcn_readfirstlane((int)to);
-    uint64_t q;
-    asm volatile("s_mov_b64 %0, %2\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %0" : "=&s"(q) : "v"(off), "s"(p), "s"(t) : "memory", "m0");
 }
 
 // Workgroups of a masked call differ in length (causal rows, padded sequences): an XCD's are ordered from the last query tile to the

@@ -207,8 +207,13 @@ int launch_typed(const FattnArgs & a, hipStream_t stream) {
             const dim3 by((unsigned)a.n_splits, (unsigned)a.Hq, (unsigned)(a.Nq * a.B));
             auto go = [&](auto lpr) {
                 constexpr int L = decltype(lpr)::value;
-                if (pieces == 2) fattn_launch_head(fattn_vec_short_kernel<TYPE, L, 2>, by, block, 0, stream, p);
-                else             fattn_launch_head(fattn_vec_short_kernel<TYPE, L, 1>, by, block, 0, stream, p);
+                if constexpr (TYPE == MI355X_TYPE_F16) {         // (F32 rows come in the same two loads either way)
+                    if (pieces == 2) {
+                        fattn_launch_head(fattn_vec_short_kernel<TYPE, L, 2>, by, block, 0, stream, p);
+                        return;
+                    }
+                }
+                fattn_launch_head(fattn_vec_short_kernel<TYPE, L, 1>, by, block, 0, stream, p);
             };
             if (lanes <= 4)       go(std::integral_constant<int, 4>{});
             else if (lanes <= 8)  go(std::integral_constant<int, 8>{});
