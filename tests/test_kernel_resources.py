@@ -40,7 +40,7 @@ def test_matrix_instructions_are_the_compilers():
                 assert not re.search(r"v_mfma|v_smfmac|v_mov_b32|v_accvgpr", m[0]), (f, m[0])
 
 
-SOURCES = ["fattn_mma.hip", "fattn_decode.hip", "fattn_relpos.hip", "fattn_pipe.hip"]
+SOURCES = ["fattn_mma.hip", "fattn_decode.hip", "fattn_relpos.hip", "fattn_pipe.hip", "fattn_vec.hip"]
 
 
 @pytest.fixture(scope="module")
@@ -125,9 +125,37 @@ def test_tile_kernel_under_a_mask(resources):
     assert [k for k, r in forms.items() if r["ScratchSize"]] == []
 
 
+def test_short_decode_calls(resources):
+    """(D, type, RAW, V8, PAD, DEEP): 64-wide f16 rows three workgroups a CU with two steps under way and four without, streamed ones four, with
+    and without a mask; 128-wide f16 rows in ranges of one step a wave four"""
+    forms = _forms(resources, "fattn_decode_short_kernel")
+    for pad in (0, 1):
+        assert forms[(64, F16, 0, 0, pad, 1)]["VGPRs"] <= 168
+        assert forms[(64, F16, 0, 0, pad, 0)]["VGPRs"] <= 128
+        assert forms[(128, F16, 0, 0, pad, 1)]["VGPRs"] <= 128
+    masked = _forms(resources, "fattn_decode_short_masked_kernel")
+    for ktype, v8 in ((Q8_0, 1), (Q4_0, 0), (Q4_1, 0), (Q5_1, 0)):
+        assert forms[(64, ktype, 1, v8, 0, 0)]["VGPRs"] <= 128 and masked[(64, ktype, 1, v8, 0)]["VGPRs"] <= 128
+    assert [k for f in (forms, masked) for k, r in f.items() if r["ScratchSize"]] == []
+
+
+def test_short_vector_calls(resources):
+    """four workgroups a CU"""
+    forms = _forms(resources, "fattn_vec_short_kernel")
+    assert {k[1] for k in forms} == {4, 8, 16, 32}
+    assert [k for k, r in forms.items() if r["VGPRs"] > 128 or r["ScratchSize"]] == []
+
+
+def test_pipelined_kernel(resources):
+    """two waves a SIMD, three where a wave has one block of queries of a 64-wide head: nothing in scratch, whose waits would take the requests
+    on their way in with them"""
+    forms = _forms(resources, "fattn_pipe_kernel")
+    assert {(k[0], k[1]) for k in forms} == {(64, 1), (64, 2), (128, 1)}
+    assert [k for k, r in forms.items() if r["ScratchSize"] or r["VGPRs"] > (168 if k[:2] == (64, 1) else 256)] == []
+
+
 def test_relpos_scratch(resources):
-    """none inside the step loop; the forms that fill the register file hold up to three registers of the epilogue there"""
+    """none, also in the forms that fill the register file"""
     forms = _forms(resources, "fattn_relpos_kernel")
     assert {k[0] for k in forms} == {64, 128}
-    for args, r in forms.items():
-        assert r["ScratchSize"] <= (16 if args[0] == 128 else 0), (args, r)
+    assert [k for k, r in forms.items() if r["ScratchSize"]] == []
