@@ -526,6 +526,7 @@ struct FattnMmaVariant {
 void fattn_mma_variant(const FattnArgs & a, int ktype, FattnMmaVariant & v);
 // waves of a workgroup of the pipelined kernel, which takes the variant's place, or 0: the tile kernel's (four)
 int fattn_pipe_waves(const FattnArgs & a, int ktype, const FattnMmaVariant & v);
+bool fattn_pipe_reaches(const FattnArgs & a, int64_t keys, bool shared_q);   // a range of so many keys, its waves sharing their queries or not
 bool fattn_pipe_alone(const FattnArgs & a, const FattnMmaVariant & v);       // (of its calls) waves that take different keys of the same queries
 int fattn_pipe_launch(const FattnArgs & a, const FattnMmaVariant & v, int waves, hipStream_t stream);
 bool fattn_mma_supported(const FattnArgs & a, int ktype);

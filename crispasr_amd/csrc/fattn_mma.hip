@@ -988,9 +988,12 @@ int launch_mask(const FattnArgs & a, const FattnMmaVariant & v, hipStream_t stre
     if (KSP == 1 && a.softcap != 0.0f)
         return mask ? launch<D, NQB, 1, TYPE, true, true, DIRECT, false>(a, stream) : launch<D, NQB, 1, TYPE, false, true, DIRECT, false>(a, stream);
     if (!mask) {
-        // (the others are the pipelined kernel's, see fattn_mma_launch)
-        if constexpr (DIRECT && !(D == 128 && KSP == 2)) return (int)hipErrorInvalidValue;
-        else return launch<D, NQB, KSP, TYPE, false, false, DIRECT, false>(a, stream);
+        // (the others are the pipelined kernel's, see fattn_mma_launch; of those it does not reach, padded heads have no other form)
+        if constexpr (DIRECT && !(D == 128 && KSP == 2)) {
+            if constexpr (NQB == 1 && KSP == 1)
+                if (a.Dv != a.D) return launch_kernel<D, NQB, KSP, TYPE, false, false, DIRECT, false, true>(a, stream);
+            return (int)hipErrorInvalidValue;
+        } else return launch<D, NQB, KSP, TYPE, false, false, DIRECT, false>(a, stream);
     }
     if (KSP == 1 && DIRECT && v.mask_dma) return launch<D, NQB, 1, TYPE, true, false, DIRECT, DIRECT>(a, stream);
     return launch<D, NQB, KSP, TYPE, true, false, DIRECT, false>(a, stream);
@@ -1066,7 +1069,9 @@ void fattn_mma_variant(const FattnArgs & a, int ktype, FattnMmaVariant & v) {
     else                      ksp_auto = wg1 <= cus && (wg1 * 5 <= (int64_t)cus * 3 || a.Nkv >= 512);
     // (a head zero-padded to 64 keeps to one query block: the two-block form stores whole rows of D floats)
     const bool two  = a.D == 64 && a.Dv == a.D && (want_nqb ? want_nqb == 2 : two_auto);
-    const bool ksp2 = !two && ktype == MI355X_TYPE_F16 && a.softcap == 0.0f && (want_ksp ? want_ksp == 2 : ksp_auto);
+    // (64-wide without a mask the split form is the pipelined kernel's alone)
+    const bool ksp2 = !two && ktype == MI355X_TYPE_F16 && a.softcap == 0.0f && (want_ksp ? want_ksp == 2 : ksp_auto) &&
+                      (a.D == 128 || a.masked || !direct || fattn_pipe_reaches(a, a.Nkv, true));
     v.query_blocks = two ? 2 : 1;
     v.key_split    = ksp2 ? 2 : 1;
     v.queries_per_workgroup = 32 * v.query_blocks * MMA_WAVES / v.key_split;
@@ -1088,6 +1093,8 @@ int fattn_mma_launch(const FattnArgs & a, int ktype, hipStream_t stream) {
     fattn_mma_variant(a, ktype, v);
     const int waves = fattn_pipe_waves(a, ktype, v);
     if (waves) return fattn_pipe_launch(a, v, waves, stream);
+    // (unmasked ranges longer than that kernel's addresses go through registers, from 64-bit addresses)
+    if (!a.masked && a.softcap == 0.0f && a.Dv == a.D && v.key_split == 1) v.direct = false;
     switch (ktype) {
         case MI355X_TYPE_F16:  return launch_type<MI355X_TYPE_F16>(a, v, stream);
         case MI355X_TYPE_F32:  return launch_type<MI355X_TYPE_F32>(a, v, stream);

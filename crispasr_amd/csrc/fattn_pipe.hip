@@ -878,16 +878,20 @@ static bool pipe_masked(const FattnArgs & a, const FattnMmaVariant & v) {
            (v.key_split == 2 || (a.mask_al4 && !(a.Nkv & 1)));
 }
 
+// Request addresses are 32-bit numbers inside a range of a head's keys, up to 8 steps of 64 behind its end, and inside the 64 rows of Q that
+// waves share: what lies further apart is the tile kernel's.
+bool fattn_pipe_reaches(const FattnArgs & a, int64_t keys, bool shared_q) {
+    const int64_t lim = (int64_t)1 << 31;
+    return (keys + 8 * 64) * a.nbk1 < lim && (keys + 8 * 64) * a.nbv1 < lim && (!shared_q || (a.nbq1 >= 0 && a.nbq1 < 1 << 25));
+}
+
 // Plain attention over f16 rows is this kernel's.  (The pairs' form of 128-wide heads since queries come through LDS; us a layer, tile
 // kernel and this: 8 heads x 80 7.9, 6.9, x 300 11.0, 9.75, x 1500 25.6, 19.8, 10 x 1000 20.0, 15.45, 80-wide 8 x 1500 31.0, 24.9.)
 // Eight waves a workgroup where that leaves no CU with more of them than workgroups of four do: more of those than CUs, and their
 // number per CU even once rounded up.  (A caller who names the form gets four.)
-// Request addresses are 32-bit numbers inside a range of a head's keys, up to 8 steps of 64 behind its end: longer ones are the tile kernel's.
 int fattn_pipe_waves(const FattnArgs & a, int ktype, const FattnMmaVariant & v) {
     if (ktype != MI355X_TYPE_F16 || !v.direct || a.softcap != 0.0f) return 0;
-    const int64_t keys = (a.n_splits > 1 ? a.keys_per_split : a.Nkv) + 8 * 64;
-    if (keys * a.nbk1 >= ((int64_t)1 << 31) || keys * a.nbv1 >= ((int64_t)1 << 31)) return 0;
-    if (v.key_split > 1 && (a.nbq1 < 0 || a.nbq1 >= 1 << 25)) return 0;        // (64 rows of Q likewise)
+    if (!fattn_pipe_reaches(a, a.n_splits > 1 ? a.keys_per_split : a.Nkv, v.key_split > 1)) return 0;
     if (a.masked) return pipe_masked(a, v) ? 4 : 0;
     if (v.key_split == 2) return 4;
     if (a.tile_variant != 0 || (a.D == 64 && v.query_blocks != 2)) return 4;
