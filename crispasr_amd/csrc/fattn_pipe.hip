@@ -878,6 +878,15 @@ static bool pipe_masked(const FattnArgs & a, const FattnMmaVariant & v) {
            (v.key_split == 2 || (a.mask_al4 && !(a.Nkv & 1)));
 }
 
+// The pairs' form of 128-wide heads takes 128 keys a turn and starts with more requests than the tile kernel, whose waves have 64 and are done
+// sooner with few rows: those of one tile, or three, stay that kernel's.  us a call in a graph, tile kernel and pairs, 8 heads, 9 rows x
+// 32 keys 5.4, 6.35, 17 x 64 5.6, 6.25, 48 x 32 6.7, 6.9, x 64 6.7, 6.7, 64 x 64 7.15, 6.8; 3 x 129 6.7, 7.4, 17 x 160 7.0, 7.3, 24 x 129 7.25, 7.5,
+// x 192 7.25, 7.25, 32 x 160 7.55, 7.45; 9 x 100 6.2, 6.05, 9 x 193 7.55, 7.1, 40 heads, 8 x 288 8.35, 8.35; 96-wide 40 x 32 8.45, 8.8.
+static bool few_rows_of_odd_tiles(const FattnArgs & a) {
+    const int keys = a.n_splits > 1 ? a.keys_per_split : a.Nkv;
+    return a.Nq <= (keys <= 64 ? 48 : keys > 128 && keys <= 192 ? 24 : 0);
+}
+
 // Request addresses are 32-bit numbers inside a range of a head's keys, up to 8 steps of 64 behind its end, and inside the 64 rows of Q that
 // waves share: what lies further apart is the tile kernel's.
 bool fattn_pipe_reaches(const FattnArgs & a, int64_t keys, bool shared_q) {
@@ -893,7 +902,7 @@ int fattn_pipe_waves(const FattnArgs & a, int ktype, const FattnMmaVariant & v) 
     if (ktype != MI355X_TYPE_F16 || !v.direct || a.softcap != 0.0f) return 0;
     if (!fattn_pipe_reaches(a, a.n_splits > 1 ? a.keys_per_split : a.Nkv, v.key_split > 1)) return 0;
     if (a.masked) return pipe_masked(a, v) ? 4 : 0;
-    if (v.key_split == 2) return 4;
+    if (v.key_split == 2) return a.D == 128 && few_rows_of_odd_tiles(a) ? 0 : 4;
     if (a.tile_variant != 0 || (a.D == 64 && v.query_blocks != 2)) return 4;
     const int q4 = v.queries_per_workgroup;
     auto groups  = [&](int q) { return (int64_t)((a.Nq + q - 1) / q) * a.Hq * a.B * a.n_splits; };
