@@ -868,11 +868,15 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
                 __builtin_amdgcn_sched_barrier(0);
                 convert_q();
             }
-            do {
+            // (the last pair stands by itself: requests for no step are not free. 256 keys, 8 rows x 16 heads of 64 4.50 -> 4.31 us, 384, one row x 8,
+            //  4.77 -> 4.56)
+            while (it + 2 * DEC_WAVES < n_steps) {
                 step(it, it + 2 * DEC_WAVES, S0{});
                 step(it + DEC_WAVES, it + 3 * DEC_WAVES, S1{});
                 it += 2 * DEC_WAVES;
-            } while (it < n_steps);
+            }
+            step(it, -1, S0{});
+            step(it + DEC_WAVES, -1, S1{});
         }
     } else
     for (int it = walk; it < walk_end; it += 2 * DEC_WAVES) {
