@@ -157,9 +157,27 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     dma_v(0);
     if (NT > 1) dma_k(1);
     // Q_u and Q_v come along the rows, 4 of 64 values an instruction, and turn into B operands in the wave's square, as f16: fetched as
-    // the operands lie an instruction takes 32 bytes of each of 32 rows
+    // the operands lie an instruction takes 32 bytes of each of 32 rows.  (Not 128-wide calls of one tile without a mask, whose results do not
+    // take the square either: with one instruction's rows the way through LDS is what shows. 8 heads x 8 tokens 8.15 -> 7.55 us, x 17 8.45 -> 7.85,
+    // x 32 8.45 -> 8.15.)
+    constexpr bool ONE_TILE = D == 128 && !ADD;
     half8 qu[KS], qv[KS];
-    {
+    if (ONE_TILE && NT == 1) {
+        const float * pu = (const float *)(a.qu + (int64_t)iq * a.nbu1 + (int64_t)h * a.nbu2 + (int64_t)b * a.nbu3) + hh * 8;
+        const float * pv = (const float *)(a.qv + (int64_t)iq * a.nbw1 + (int64_t)h * a.nbw2 + (int64_t)b * a.nbw3) + hh * 8;
+        const float   qs = a.scale * FR_LOG2E;
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+            for (int p4 = 0; p4 < 2; p4++) {
+                const float4v u = *(const float4v *)(pu + ks * 16 + p4 * 4), w = *(const float4v *)(pv + ks * 16 + p4 * 4);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    qu[ks][4 * p4 + e] = (_Float16)(u[e] * qs);
+                    qv[ks][4 * p4 + e] = (_Float16)w[e];
+                }
+            }
+    } else {
         constexpr int QP = D / 64;                                    // pieces of 64 values a row
         const int     qr = lane >> 4, qc = lane & 15;
         float4v       raw[2 * QP][8];
@@ -570,7 +588,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
         for (int c = 0; c < 4; c++) o[c] = oacc[db][4 * g + c] * inv;
         return o;
     };
-    if constexpr (D == 64) {
+    if (D == 64 || (ONE_TILE && NT == 1)) {
         // (as they lie: the way through the square costs these short calls 0.1 to 0.2 us, 33 tokens x 8 heads 7.65 and 7.45)
         if (i0w + il < a.Nq) {
             float * const out = a.dst + (((int64_t)b * a.Nq + (i0w + il)) * a.H + h) * D;
