@@ -83,8 +83,8 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 template <bool STREAM, typename T> __device__ __forceinline__ void store16(const NarrowCopy & a, uint32_t to, T x) {
     // (buffer stores, because only their builtin takes the cache bits: 2 = non-temporal, 16 = write through)
     const auto r = __builtin_amdgcn_make_buffer_rsrc(a.dst, 0, -1, 0x00020000);
-    if (STREAM && whole_of(a) == 2) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), r, (int)to, 0, 18);
-    else if (whole_of(a))           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), r, (int)to, 0, 16);
+    if (STREAM && a.whole == 2) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), r, (int)to, 0, 18);
+    else if (a.whole)           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), r, (int)to, 0, 16);
     else                        *(T *)(a.dst + to) = x;
 }
 template <bool STREAM, typename I, typename T> __device__ __forceinline__ void store16(const WideCopy<I> & a, int64_t to, T x) {
@@ -132,8 +132,10 @@ __device__ __forceinline__ void cpy_vec_body(const A & a) {
 }
 template <typename A, typename TS, typename TD>
 __global__ void __launch_bounds__(256) cpy_vec_kernel(const A a) { cpy_vec_body<A, TS, TD>(a); }
-template <typename A, typename TS, typename TD>
-__global__ void __launch_bounds__(256) cpy_vec_kernel_head(FATTN_HEAD_PARAMS, const ArgTail<A> tail) { cpy_vec_body<A, TS, TD>(fattn_join<A>(FATTN_HEAD_ARGS, tail)); }
+template <typename TS, typename TD>
+__global__ void __launch_bounds__(256) cpy_vec_kernel_head(FATTN_HEAD_PARAMS, const ArgTail<NarrowCopyHead> tail) {
+    cpy_vec_body<NarrowCopy, TS, TD>(narrow_of(fattn_join<NarrowCopyHead>(FATTN_HEAD_ARGS, tail)));
+}
 
 // Quantise one block of 32 held by a quad of lanes, 8 consecutive elements each (lane c of the quad: elements 8c .. 8c+7),
 // and store it.  Called by all four lanes: the quad's reductions are two DPP steps, and a lane stores 8 bytes of
@@ -626,7 +628,7 @@ static void launch_plain(const CpyArgs & a, hipStream_t stream) {
         // (5 x 512 values 1.68 and 1.84 us; row writes and dequantising reads, of which steps are full, stay with the structure).
         NarrowCopy v;
         if (b.n > 65536 && b.snb[0] == (int64_t)sizeof(TS) && narrow_copy(b, E, E * sizeof(TS), E * sizeof(TD), b.n, v))
-            fattn_launch_head(cpy_vec_kernel_head<NarrowCopy, TS, TD>, dim3((unsigned)((b.n + 255) / 256)), dim3(256), 0, stream, v);
+            fattn_launch_head(cpy_vec_kernel_head<TS, TD>, dim3((unsigned)((b.n + 255) / 256)), dim3(256), 0, stream, head_first(v));
         else
             CPY_LAUNCH(b, E, sizeof(TS), E * sizeof(TS), E * sizeof(TD), b.n, true, cpy_vec_kernel, TS, TD);
     } else {
