@@ -101,12 +101,12 @@ static __device__ __forceinline__ void row_partial_merge(RowPartial & a, const R
     a.m = mn;
 }
 
-// lane ^ OFF's value, for the merge of a wave's groups: 4 through the LDS crossbar; 8, 16 and 32 in the vector unit (a rotation of
+// lane ^ OFF's value, for the merge of a wave's groups.  VECTOR: 4 through the LDS crossbar; 8, 16 and 32 in the vector unit (a rotation of
 // a row by half, and swaps of which the lower lanes' partner is the second result: only lanes that have the bit OFF clear may use it)
-template <int OFF>
+template <int OFF, bool VECTOR>
 static __device__ __forceinline__ float partner_above(float x) {
     static_assert(OFF == 4 || OFF == 8 || OFF == 16 || OFF == 32, "a power of two that a group can be wide");
-    if constexpr (OFF == 4)  return xor_shuffle(x, 4);
+    if constexpr (OFF == 4 || !VECTOR) return xor_shuffle(x, OFF);
     if constexpr (OFF == 8)  return dpp_mov<0x128>(x);               // row_ror:8
     if constexpr (OFF == 16) {
         uint32_t a = __float_as_uint(x), b = a;
@@ -115,16 +115,16 @@ static __device__ __forceinline__ float partner_above(float x) {
     }
     return both_halves(x).y;
 }
-template <int OFF>
+template <int OFF, bool VECTOR>
 static __device__ __forceinline__ void merge_groups(RowPartial & st) {
     if constexpr (OFF < 64) {
         RowPartial o;
-        o.m = partner_above<OFF>(st.m);
-        o.l = partner_above<OFF>(st.l);
+        o.m = partner_above<OFF, VECTOR>(st.m);
+        o.l = partner_above<OFF, VECTOR>(st.l);
 #pragma unroll
-        for (int e = 0; e < 8; e++) o.acc[e] = partner_above<OFF>(st.acc[e]);
+        for (int e = 0; e < 8; e++) o.acc[e] = partner_above<OFF, VECTOR>(st.acc[e]);
         row_partial_merge(st, o);
-        merge_groups<OFF * 2>(st);
+        merge_groups<OFF * 2, VECTOR>(st);
     }
 }
 
@@ -263,7 +263,7 @@ static __device__ __forceinline__ void row_scan(const RowScanArgs & a, const flo
     }
     for (; j0 < k_end; j0 += stride) step(j0, RowNothing());
     // merge the G groups of this wave (lanes with equal position in their group)
-    merge_groups<LPR>(st);
+    merge_groups<LPR, (PIECES > 0)>(st);
 }
 
 // lanes 0 .. LPR-1 hold the row's final state: write dst, or this split's partial for the merge (natural-log units).
