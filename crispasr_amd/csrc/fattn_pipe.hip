@@ -769,7 +769,7 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
     }
 
     // ---- normalise and write dst[D, Hq, Nq, B], or hand the unnormalised partial to the merge kernel -----------------------
-    const int dv = PAD ? a.Dv : D;                      // dst rows are dv floats; partial rows are D apart
+    const int dv = PAD ? a.Dv : D;                      // rows of dv floats; the partials' are D apart
     if constexpr (KSP == 1) {
         // whole rows through LDS (32 x D floats per wave, chunks XOR-swizzled by row), 16 or 32 adjacent lanes on one row
         constexpr int CPR = D / 4;                         // 16-byte chunks per output row
@@ -802,7 +802,7 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
                 const int row = k * RPI + lane / CPR, c = lane % CPR;
                 const float4 o = *(const float4 *)(stg + row * D + ((c ^ (row & (CPR - 1))) * 4));
                 typedef float f32x4 __attribute__((ext_vector_type(4)));
-                if (q_first + row < a.Nq && (!PAD || a.n_splits > 1 || c * 4 < a.Dv) && (!MASK || !(bad >> row & 1)))
+                if (q_first + row < a.Nq && (!PAD || c * 4 < a.Dv) && (!MASK || !(bad >> row & 1)))
                     __builtin_nontemporal_store(f32x4{o.x, o.y, o.z, o.w}, (f32x4 *)(out0 + row * row_stride + c * 4));
             }
             __builtin_amdgcn_wave_barrier();               // the next query block reuses the staging rows
@@ -832,7 +832,7 @@ __global__ void __launch_bounds__(W * 64, 2) fattn_pipe_kernel(const FattnArgs a
                     o.z = x[g * 4 + 2] * inv;
                     o.w = x[g * 4 + 3] * inv;
                     const int d = ((ALONE ? wave % DB : kgroup * (DB / 2)) + i) * 32 + g * 8 + hh * 4;
-                    if (!PAD || a.n_splits > 1 || d < a.Dv) *(float4 *)(out + d) = o;
+                    if (!PAD || d < a.Dv) *(float4 *)(out + d) = o;
                 }
             if (a.n_splits > 1 && hh == 0 && (ALONE ? wave % DB : kgroup) == 0) {
                 float * pm = a.part_ml + (row * a.n_splits + split) * 2;
