@@ -1061,9 +1061,13 @@ void fattn_mma_variant(const FattnArgs & a, int ktype, FattnMmaVariant & v) {
     // heads 14.9 -> 13.5 us a layer, 900 x 20 14.6 -> 13.8, 780 x 20 12.6 either way, 250 x 20 x 4 8.1 and with pairs 8.7.
     const int64_t wgp = (int64_t)((a.Nq + 63) / 64) * heads;
     const bool pipes = direct && (!a.masked || (a.Dv == 128 && a.Nkv >= 64 && a.max_bias <= 0.0f));
-    // (Of 64 keys each wave of a pair has one block: its merge shows once a quarter of the CUs run one. 64 tokens x 32 heads 4.9 us a layer
-    // either way, x 96 7.5 and with pairs 7.7, x 200 7.7, 8.85.)
-    if (a.D == 128)           ksp_auto = wg1 * 4 <= cus || (a.Nkv > 64 && (wg1 * 2 <= cus || (pipes && wgp <= cus))) || (wg1 <= cus && a.Nkv >= 2048);
+    // (Up to 64 keys each wave of a pair has one block, and its merge shows once a quarter of the CUs run one: 64 tokens x 32 heads 4.9 us a
+    // layer either way, x 96 6.9 and in pairs 7.7.  Pairs then pay where there are more workgroups of them and a mask or half a tile of keys leaves
+    // those of 128 queries to the tile kernel's order, 1185 rows x 12 heads under a mask, 33 keys, 8.8 and 11.2, 188 x 64 plain, 20 keys, 7.9 and
+    // 8.5 (without a mask up to 32 keys: 1185 x 12, 64 keys, 8.4 and 7.85), and where half of the waves of 128 queries would have none, 33 x 112
+    // plain, 20 keys, 6.35 and 6.95.)
+    const bool one_tile_pairs = a.masked ? a.Nq > 64 : a.Nq <= 48 || (a.Nq > 64 && a.Nkv <= 32);
+    if (a.D == 128)           ksp_auto = wg1 * 4 <= cus || (wg1 * 2 <= cus && (a.Nkv > 64 || one_tile_pairs)) || (a.Nkv > 64 && pipes && wgp <= cus) || (wg1 <= cus && a.Nkv >= 2048);
     else if (!a.masked)       ksp_auto = wg1 <= cus && (wg1 * 5 <= (int64_t)cus * 3 || (a.Nkv >= 768 && wg1 * 3 <= (int64_t)cus * 2) || a.Nkv >= 1024) && a.Nkv > 128;
     else if (!mdma_ok && a.Nkv >= 256) ksp_auto = wg1 * 5 <= (int64_t)cus * 8;
     else                      ksp_auto = wg1 <= cus && (wg1 * 5 <= (int64_t)cus * 3 || a.Nkv >= 512);

@@ -879,12 +879,12 @@ static bool pipe_masked(const FattnArgs & a, const FattnMmaVariant & v) {
 }
 
 // The pairs' form of 128-wide heads takes 128 keys a turn and starts with more requests than the tile kernel, whose waves have 64 and are done
-// sooner with few rows: those of one tile, or three, stay that kernel's.  us a call in a graph, tile kernel and pairs, 8 heads, 9 rows x
-// 32 keys 5.4, 6.35, 17 x 64 5.6, 6.25, 48 x 32 6.7, 6.9, x 64 6.7, 6.7, 64 x 64 7.15, 6.8; 3 x 129 6.7, 7.4, 17 x 160 7.0, 7.3, 24 x 129 7.25, 7.5,
+// sooner with few rows: those of one tile, or three, stay that kernel's, and all of half a tile.  us a call in a graph, tile kernel and pairs, 8 heads, 9 rows x
+// 32 keys 5.4, 6.35, 17 x 64 5.6, 6.25, 48 x 32 6.7, 6.9, x 64 6.7, 6.7, 64 x 32 7.1, 7.05, x 64 7.15, 6.8; 3 x 129 6.7, 7.4, 17 x 160 7.0, 7.3, 24 x 129 7.25, 7.5,
 // x 192 7.25, 7.25, 32 x 160 7.55, 7.45; 9 x 100 6.2, 6.05, 9 x 193 7.55, 7.1, 40 heads, 8 x 288 8.35, 8.35; 96-wide 40 x 32 8.45, 8.8.
 static bool few_rows_of_odd_tiles(const FattnArgs & a) {
     const int keys = a.n_splits > 1 ? a.keys_per_split : a.Nkv;
-    return a.Nq <= (keys <= 64 ? 48 : keys > 128 && keys <= 192 ? 24 : 0);
+    return keys <= 32 || a.Nq <= (keys <= 64 ? 48 : keys > 128 && keys <= 192 ? 24 : 0);
 }
 
 // Request addresses are 32-bit numbers inside a range of a head's keys, up to 8 steps of 64 behind its end, and inside the 64 rows of Q that

@@ -46,9 +46,9 @@ def test_masked_waves_of_their_own(Nq, Nkv, piped):
 
 
 @pytest.mark.parametrize("D", [128, 96, 80])
-@pytest.mark.parametrize("Nq,Nkv,piped", [(1, 1, 0), (40, 31, 0), (49, 1, 1), (70, 31, 1), (63, 33, 1), (64, 64, 1), (65, 95, 1), (100, 97, 1), (31, 128, 1), (130, 160, 1),
+@pytest.mark.parametrize("Nq,Nkv,piped", [(1, 1, 0), (40, 31, 0), (70, 32, 0), (63, 33, 1), (64, 64, 1), (65, 95, 1), (100, 97, 1), (31, 128, 1), (130, 160, 1),
                                           (70, 191, 1), (33, 300, 1), (129, 513, 1),
-                                          # few rows of one tile of keys, or three, are the tile kernel's
+                                          # half a tile of keys, and few rows of one tile or three, are the tile kernel's
                                           (48, 64, 0), (49, 64, 1), (5, 65, 1), (24, 128, 1), (24, 129, 0), (25, 129, 1), (24, 192, 0), (7, 193, 1)])
 def test_plain_pairs(D, Nq, Nkv, piped):
     case = make_case(seed=6300 + Nkv, D=D, Nq=Nq, Nkv=Nkv, Hq=4, Hkv=2, B=2, q_layout="thd", kv_layout="thd" if Nkv % 2 else "gap")

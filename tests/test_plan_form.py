@@ -56,3 +56,11 @@ def test_waves_of_different_keys(Nq, H, B, least):
     if least == 768:
         assert form(1536, n_splits=2) == (ggml.FORM_KEYS_APART if H * B * ((Nq + 63) // 64) * 2 <= 224 else ggml.FORM_GENERAL)
         assert form(1408, n_splits=2) == ggml.FORM_GENERAL                                 # (ranges of 704 keys)
+
+
+# (more than a quarter of the CUs, at most half of them, with workgroups of 128 queries)
+@pytest.mark.parametrize("Nq,H,Nkv,mask,split", [(48, 100, 64, None, 2), (49, 100, 32, None, 1), (64, 100, 33, None, 1), (65, 100, 32, None, 2), (100, 100, 33, None, 1), (100, 100, 65, None, 2),
+                                                 (64, 100, 17, 1, 1), (64, 100, 64, 1, 1), (65, 100, 17, 1, 2), (1185, 12, 33, 1, 2), (1185, 12, 64, 1, 2), (100, 64, 64, None, 2), (100, 129, 32, 1, 1)])
+def test_pairs_of_a_tile_of_keys(Nq, H, Nkv, mask, split):
+    q, k = _t(ggml.F32, (128, Nq, H, 1)), _t(ggml.F16, (128, Nkv, H, 1))
+    assert ggml.flash_attn_plan_details(q, k, k, _t(ggml.F16, (Nkv, Nq, mask, 1)) if mask else None, 0.1, kernel=ggml.KERNEL_MMA)["key_split"] == split
