@@ -565,7 +565,7 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
             // One coalesced stream per tensor, through a buffer that ends with the step's last valid row: what lies behind it are
             // zeros, scales and minima among them, and the 2 * NU loads share one offset (its lane number through an asm, or
             // each of the loop's would have its own).
-            const uint32_t bytes = (uint32_t)(MASK ? min(STEP, k_end - j0) : max(0, min(STEP, k_end - j0))) * RS;
+            const uint32_t bytes = (uint32_t)min(STEP, k_end - j0) * RS;
             const auto     kb = fattn_buffer(kbase + (int64_t)j0 * RS, bytes), vb = fattn_buffer(vbase + (int64_t)j0 * RS, bytes);
             uint32_t ln = (uint32_t)lane;
             asm volatile("" : "+v"(ln));
@@ -820,27 +820,27 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
             walk = wave + first * DEC_WAVES;
         }
         convert_q();
-    } else if (RAW) {
-        request_q();                               // (ahead of K and V, whose request takes no branch: it is converted while they are on their way)
-        issue(wave, S0{});
-    } else if (!DEEP) {
+    } else if (!RAW && !DEEP) {
         if (wave < n_steps) issue(wave, S0{});
     }
 
     // (V8) where the pieces of this lane's V units go: read behind the first K/V request, needed when that has arrived
-    if (V8) {
+    auto read_places = [&]() __attribute__((always_inline)) {
+        if (!V8) return;
         static_assert(!V8 || (V8Places<D>::RAWSZ == RAWSZ && V8Places<D>::UNITS == NU * 64 && V8Places<D>::UNIT == UNIT), "table layout");
         const uint32_t * places = (const uint32_t *)v8_places_table<D>.at;
 #pragma unroll
         for (int i = 0; i < NU; i++)
 #pragma unroll
             for (int k = 0; k < PCS / 2; k++) vdst[i][k] = places[(i * 64 + lane) * (PCS / 2) + k];
-    }
-    if constexpr (!MASK && !DEEP) {                // (after the first K/V request: the two cold misses overlap)
-        if (!RAW) request_q();
-        convert_q();
-    }
+    };
     typedef std::integral_constant<int, ONE ? 0 : 1> S1;
+    auto walk_steps = [&]() __attribute__((always_inline)) {
+        for (int it = walk; it < walk_end; it += 2 * DEC_WAVES) {
+            step(it, it + DEC_WAVES, S0{});
+            if (it + DEC_WAVES < walk_end) step(it + DEC_WAVES, it + 2 * DEC_WAVES, S1{});
+        }
+    };
     if constexpr (DEEP) {
         // (Pairs of steps, an odd one ahead of them out of stage 1, and one way out of the loop: a way past a pair's second step would
         //  make its rows uncountable again.)
@@ -878,10 +878,24 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
             step(it, -1, S0{});
             step(it + DEC_WAVES, -1, S1{});
         }
-    } else
-    for (int it = walk; it < walk_end; it += 2 * DEC_WAVES) {
-        step(it, it + DEC_WAVES, S0{});
-        if (it + DEC_WAVES < walk_end) step(it + DEC_WAVES, it + 2 * DEC_WAVES, S1{});
+    } else if constexpr (RAW && !MASK) {
+        // (Q ahead of K and V, whose request takes no branch of its own: it is converted while they are on their way.  Waves without a step ask
+        //  for nothing: from empty buffers they kept the others' requests waiting, 5 rows x 32 query and 8
+        //  KV heads of 128 against 28 Q8_0 entries 5.4 and 4.85 us, against 90 5.9 and 5.7)
+        if (wave < n_steps) {
+            request_q();
+            issue(wave, S0{});
+            read_places();
+            convert_q();
+            walk_steps();
+        }
+    } else {
+        read_places();
+        if (!MASK) {                               // (after the first K/V request: the two cold misses overlap)
+            request_q();
+            convert_q();
+        }
+        walk_steps();
     }
 
     // ---- column totals, then the four waves through LDS ----------------------------------------------
