@@ -157,10 +157,10 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     dma_v(0);
     if (NT > 1) dma_k(1);
     // Q_u and Q_v come along the rows, 4 of 64 values an instruction, and turn into B operands in the wave's square, as f16: fetched as
-    // the operands lie an instruction takes 32 bytes of each of 32 rows.  (Not 128-wide calls of one tile without a mask, whose results do not
+    // the operands lie an instruction takes 32 bytes of each of 32 rows.  (Not 128-wide calls of one tile, whose results do not
     // take the square either: with one instruction's rows the way through LDS is what shows. 8 heads x 8 tokens 8.15 -> 7.55 us, x 17 8.45 -> 7.85,
-    // x 32 8.45 -> 8.15.)
-    constexpr bool ONE_TILE = D == 128 && !ADD;
+    // x 32 8.45 -> 8.15, under an F16 mask 17 9.15 -> 8.65; under an F32 mask there are no registers for a second way.)
+    constexpr bool ONE_TILE = D == 128 && (!ADD || ADD_F16);
     half8 qu[KS], qv[KS];
     if (ONE_TILE && NT == 1) {
         const float * pu = (const float *)(a.qu + (int64_t)iq * a.nbu1 + (int64_t)h * a.nbu2 + (int64_t)b * a.nbu3) + hh * 8;
