@@ -408,6 +408,9 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr int VP8 = v8_pitch<D>();
     constexpr int PCS = UNIT / 2;                  // (V8) 2-byte pieces per unit
+    // unmasked: the request of Q ahead of the first K/V request.  (Not for 64-wide Q8_0, whose waves are bound by their steps: 3 rows x 16 heads x
+    // 16 sequences against 500 entries 6.70 us with Q behind it, 6.97 ahead, 32 query and 8 KV heads x 16 against 4000 15.4, 16.1.)
+    constexpr bool Q_FIRST = RAW && !(V8 && D == 64);
     constexpr bool ONE = V8;                       // one register stage: the next step is requested once this one is in LDS
                                                    // (two stages, as the other forms have: 102-104 against 99 us at 64 x 4096)
     constexpr int WAVE_BYTES = V8 ? RAWSZ + STEP * VP8 + KS * STEP * 2 : STEP * PV * 2 + (RAW ? 2 * RAWSZ : 0);
@@ -820,7 +823,7 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
             walk = wave + first * DEC_WAVES;
         }
         convert_q();
-    } else if (!RAW && !DEEP) {
+    } else if (!Q_FIRST && !DEEP) {
         if (wave < n_steps) issue(wave, S0{});
     }
 
@@ -878,7 +881,7 @@ __device__ __forceinline__ void decode_body(const FattnArgs & a, int first) {
             step(it, -1, S0{});
             step(it + DEC_WAVES, -1, S1{});
         }
-    } else if constexpr (RAW && !MASK) {
+    } else if constexpr (Q_FIRST && !MASK) {
         // (Q ahead of K and V, whose request takes no branch of its own: it is converted while they are on their way.  Waves without a step ask
         //  for nothing: from empty buffers they kept the others' requests waiting, 5 rows x 32 query and 8
         //  KV heads of 128 against 28 Q8_0 entries 5.4 and 4.85 us, against 90 5.9 and 5.7)
