@@ -19,8 +19,8 @@
 // range's last row, so that nothing has to hold a request back inside it, and K's and V's slots have one number.  With clamped row
 // numbers and moving bases a request took six and 6 to 12 scalar ones more a step; together with a wait for LDS reads that the
 // compiler could not count across the loop's head (a scalar load was on its way), us a pass, in turn on one box: 6 layers of 8 x 64 x
-// 1500 against 1536 with their copies 114.7 -> 111.2, 4 of 20 x 64 x 1500^2 x 4 214.7 -> 212.6, 750 x 8 heads of 128 x 8 under a bias
-// 43.5 -> 43.1, causal 407 and 2048 behind 2048 as before (90.7, 133.6: two waves a SIMD fill these gaps).  A step's requests go out one
+// 1500 against 1536 with their copies 114.7 -> 111.2, 4 of 20 x 64 x 1500^2 x 4 214.7 -> 212.6; 750 x 8 heads of 128 x 8 under a bias (43.5
+// and 43.1) and causal 407 and 2048 behind 2048 (90.7, 133.6) within the spread of the runs: two waves a SIMD fill these gaps.  A step's requests go out one
 // behind each of its first matrix instructions (a wave alone on its SIMD waits for each to be taken), the last of the prologue's behind
 // the first scores: 8 x 64 x 1500 against 1536, K and V from memory, 12.9 -> 12.5 us a launch.
 //
@@ -45,8 +45,8 @@
 // 37.2 -> 44.6).  Eight waves that share the queries of two or four (the keys in turn), for a grid that leaves CUs to one
 // workgroup of four, changed nothing at 1500 keys (8 x 64 16.0 us either way) and lost 1 us below 1000.
 // Masked calls of 128-wide heads: a wave brings the mask of its next two blocks to LDS as it does K and V, so that the waits
-// go on counting, and adds it ahead of the exponentials; the last block is the last 32 keys of the range, whole.  Against the tile
-// kernel, whole calls: 2048 causal tokens behind 2048, 32 query and 8 KV heads, with their row writes 146.8 -> 133.4 us, 1000 causal
+// go on counting, and adds it ahead of the exponentials; the last block may be partial, its keys behind the range excluded by their number.
+// Against the tile kernel, whole calls: 2048 causal tokens behind 2048, 32 query and 8 KV heads, with their row writes 146.8 -> 133.4 us, 1000 causal
 // tokens 42.5 -> 37.5, 407 (rows that start between dwords, the pairs' form) 21.4 -> 20.1 (now 17.6); under per-head masks 750 x 8 heads x 8
 // 45.7 -> 38.8, 1000 x 8 x 4 38.1 -> 32.7, 751 x 8 22.0 -> 19.2.  A step of the 407-token launch is 0.65 us, 32 KB through a CU's
 // port; the hand-over and the stores are 3 us of it.

@@ -7,8 +7,8 @@
 // The reference materialises `mask` as an F16 [T, T, H] tensor per sequence and hands it to ggml_flash_attn_ext; here
 // the position term is produced tile by tile inside the attention loop and never leaves the CU.
 //
-// A workgroup of 4 waves owns 128 consecutive queries of one (head, batch), 32 per wave (the N columns of
-// v_mfma_f32_32x32x16_f16 accumulators), and walks the keys 32 at a time.  Per step and wave:
+// A workgroup of 2 to 4 waves owns consecutive queries of one (head, batch), 32 per wave (the N columns of
+// v_mfma_f32_32x32x16_f16 accumulators), and walks the keys 32 at a time.  Per tile of keys and wave:
 //   S^T  = K tile . Q_u^T                       8 (D = 128) MFMAs, A = K rows from LDS, B = Q_u in registers
 //   BD   = R block . Q_v^T                      8 MFMAs, A = 32 rows of the table from LDS, B = Q_v in registers.
 //          Block n x the wave's 32 queries is one accumulator whose element (row, il) belongs to key
@@ -20,14 +20,15 @@
 //          32 x 32 f32 square in LDS (pitch 36: writes and the 16-byte row reads are both conflict-free) and come back
 //          in the layout of S^T.
 //   mask = f16(scale * BD + add), s = S + mask in log2 units, online softmax against a reference that is raised
-//          only when a row's maximum outgrows it by a factor 256, P -> f16
+//          only when the 16 probabilities of a lane sum to more than FR_SUM_LIMIT, P -> f16
 //   O^T += V^T . P^T                            8 MFMAs, A = V tile through ds_read_b64_tr_b16, B = P from registers
 // The waves need the same table rows one step apart, so the table is staged once per workgroup in a ring of 32-row blocks,
-// one more than there are waves.  K and V tiles and table blocks move global -> LDS without passing registers
-// (global_load_lds_dwordx4, the 16-byte chunks of a row XOR-swizzled so that the operand reads are conflict-free).  A step
-// requests the next one's into the halves and the slot that the step before it has left, and one barrier at its end waits
-// for them: K and V have two halves each.  K, V and the table are f16 with 16-byte aligned rows (the caller rounds F32 ones
-// first, as the reference's own graph does for the mask product's operands).
+// one more than there are waves.  K and V tiles and table blocks move global -> LDS without passing registers (16 bytes a lane, the
+// chunks of a row XOR-swizzled so that the operand reads are conflict-free; in the loop by buffer loads, a tensor's buffer
+// ending with its last row).  The step of tile t requests K tile t + 2, table block t + 3 and V tile t + 1, which the next step reads, into
+// the halves and the slot that the step before it has left - K and V have two halves each - and one barrier at its end waits for
+// them.  K, V and the table are f16 with 16-byte aligned rows (the caller rounds F32 ones first, as the reference's own graph does
+// for the mask product's operands).
 //
 // The vector work of a tile stands beside the matrix instructions of another: a step turns tile t's scores into probabilities beside
 // the two Q products of tile t + 1, and un-skews those beside P.V.  Q_u, Q_v and the result pass through the wave's square, so that
@@ -207,8 +208,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     constexpr int AES = ADD_F16 ? 2 : 4;
     uint32_t add_off = 0;                           // the query's row of the additive mask, from that of the wave's first query
     // (The head's and the sequence's offsets in scalar registers: the divisions leave theirs in vector ones, and the 128-wide
-    //  forms held them through the loop in scratch, for the rows that are done again.  What is left of it, one register in the
-    //  form of 3 waves and three in that of 2, belongs to the epilogue; a build without it is 1% slower at 750 tokens.)
+    //  forms held them through the loop in scratch, for the rows that are done again.)
     const char * add_head = nullptr, * add_wave = nullptr;
     if (ADD) {
         add_head = a.add + (int64_t)__builtin_amdgcn_readfirstlane(h % a.Ha) * a.nba2 + (int64_t)__builtin_amdgcn_readfirstlane(b % a.Ba) * a.nba3;
