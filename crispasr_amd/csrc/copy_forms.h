@@ -23,9 +23,11 @@ struct NarrowCopy {
 };
 static_assert(sizeof(NarrowCopy) <= 112, "arguments of a cheap launch");
 
-// The same for a large copy, whose loads' addresses come from the first 56 bytes and can be in registers when its waves start (see
-// ArgTail).  Kernels that read a structure keep the order above: in this one, whose shifts have to be taken apart and whose destination
-// is behind the first 64 bytes, a dequantising read of 663 x 8 rows of 128 took 2.51 us in a graph instead of 2.33.
+// The same with all that the loads' addresses need in the first 56 bytes: one line of the scalar cache, which for a large copy can be in
+// registers when its waves start (see ArgTail).  All kernels but the quantising ones read this order, whose second line is wanted for the
+// stores alone.  us a copy in a graph, the order above and this one, rows x 8 heads of 128: from Q8_0 663 rows of 704 2.48, 2.30, 407 2.18, 2.02,
+// 1500 of 2048 2.85, 2.68; Q8_0 as it is 663 2.37, 2.23; F32 to F16 128 2.05, 1.87, 407 2.38, 2.19; 8 x 300 rows of 37 2.17, 2.00.  Quantising
+// copies have work enough behind their loads, and the shifts to be taken apart show: F32 to Q4_0 128 rows 2.13, 2.25, 407 2.50, 2.57.
 struct NarrowCopyHead {
     const char * src;
     uint32_t     n;
@@ -33,6 +35,7 @@ struct NarrowCopyHead {
     uint32_t     snb[3], dnb[3];
     char *       dst;
     int64_t      mirror;
+    typedef uint32_t index, offset;
     template <typename F> __host__ __device__ void pointers(F f) { f(src, dst); }
 };
 static_assert(sizeof(NarrowCopyHead) <= 112 && offsetof(NarrowCopyHead, dnb) < 56, "arguments of a cheap launch");

@@ -92,8 +92,13 @@ template <bool STREAM, typename I, typename T> __device__ __forceinline__ void s
     else                        *(T *)(a.dst + to) = x;
 }
 
+// a kernel's arguments, taken apart where they come in the order of their loads
+template <typename A> __device__ __forceinline__ const A & opened(const A & a) { return a; }
+__device__ __forceinline__ NarrowCopy opened(const NarrowCopyHead & a) { return narrow_of(a); }
+
 template <typename A, typename TS, typename TD>
-__global__ void __launch_bounds__(256) cpy_scalar_kernel(const A a) {
+__global__ void __launch_bounds__(256) cpy_scalar_kernel(const A args) {
+    const auto & a = opened(args);
     typedef typename A::index I;
     const I i = thread_index<I>();
     if (i >= (I)a.n) return;
@@ -111,7 +116,7 @@ typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
 // Launched only when dimension 0 is whole such units on both sides, the elements are adjacent and rows start on the 16 bytes
 // (8 where four f16 are read) that a lane moves at once.
 template <typename TD> constexpr int vec_elements() { return 16 / (int)sizeof(TD); }
-template <typename A, typename TS, typename TD>
+template <typename TS, typename TD, typename A>
 __device__ __forceinline__ void cpy_vec_body(const A & a) {
     typedef typename A::index I;
     constexpr int E = vec_elements<TD>();
@@ -131,10 +136,10 @@ __device__ __forceinline__ void cpy_vec_body(const A & a) {
     }
 }
 template <typename A, typename TS, typename TD>
-__global__ void __launch_bounds__(256) cpy_vec_kernel(const A a) { cpy_vec_body<A, TS, TD>(a); }
+__global__ void __launch_bounds__(256) cpy_vec_kernel(const A args) { cpy_vec_body<TS, TD>(opened(args)); }
 template <typename TS, typename TD>
 __global__ void __launch_bounds__(256) cpy_vec_kernel_head(FATTN_HEAD_PARAMS, const ArgTail<NarrowCopyHead> tail) {
-    cpy_vec_body<NarrowCopy, TS, TD>(narrow_of(fattn_join<NarrowCopyHead>(FATTN_HEAD_ARGS, tail)));
+    cpy_vec_body<TS, TD>(narrow_of(fattn_join<NarrowCopyHead>(FATTN_HEAD_ARGS, tail)));
 }
 
 // Quantise one block of 32 held by a quad of lanes, 8 consecutive elements each (lane c of the quad: elements 8c .. 8c+7),
@@ -271,7 +276,8 @@ __global__ void __launch_bounds__(256) cpy_f32_block_kernel(const A a) {
 // block type -> F32; 4 elements per lane, eight lanes per block, so that with 16-byte stores (VEC) a wave writes 1 KB that lies
 // together: with 8 elements, two stores and half as many lanes 663 x 8 rows of 128 took 2.51 us instead of 2.15, 2048 x 64 20.6 instead of 11.4.
 template <typename A, int TYPE, bool VEC>
-__global__ void __launch_bounds__(256) cpy_block_f32_kernel(const A a) {
+__global__ void __launch_bounds__(256) cpy_block_f32_kernel(const A args) {
+    const auto & a = opened(args);
     typedef typename A::index I;
     const int j0  = (threadIdx.x & 7) * 4;
     for (I blk = (I)blockIdx.x * 32 + (threadIdx.x >> 3); blk < (I)a.n; blk += grid_lanes<I>() / 8) {
@@ -295,7 +301,8 @@ __global__ void __launch_bounds__(256) cpy_block_f32_kernel(const A a) {
 
 // same block type on both sides: move the blocks as halfwords
 template <typename A, int TYPE>
-__global__ void __launch_bounds__(256) cpy_block_block_kernel(const A a) {
+__global__ void __launch_bounds__(256) cpy_block_block_kernel(const A args) {
+    const auto & a = opened(args);
     typedef typename A::index I;
     constexpr int HW = BlockFormat<TYPE>::BYTES / 2;
     const I   t   = thread_index<I>();
@@ -603,12 +610,14 @@ static bool prepare_index(CpyArgs & a, int64_t unit0, int64_t threads) {
             fattn_launch((KERNEL<WideCopy<int64_t>, __VA_ARGS__>), lg_, dim3(256), 0, stream, l_);                  \
         }                                                                                                                 \
     } while (0)
-// (es: bytes of a source element, whole blocks counted as one)
-#define CPY_LAUNCH(a, unit0, es, sstep, dstep, threads, walked, KERNEL, ...)                                                   \
+// (es: bytes of a source element, whole blocks counted as one; order: head_first, or as_it_is for kernels that read a NarrowCopy)
+static inline const NarrowCopy & as_it_is(const NarrowCopy & a) { return a; }
+#define CPY_LAUNCH(a, unit0, es, sstep, dstep, threads, walked, order, KERNEL, ...)                                            \
     do {                                                                                                                  \
-        NarrowCopy v_;                                                                                                    \
+        NarrowCopy v_ = {};                                                                                               \
         const bool n_ = (a).snb[0] == (int64_t)(es) && narrow_copy(a, unit0, sstep, dstep, threads, v_);                  \
-        FORM_LAUNCH(a, unit0, threads, walked, n_, v_, whole_pieces((a).dst, walk_of((a).dne, (a).dnb, unit0, dstep), dstep), KERNEL, __VA_ARGS__); \
+        auto o_ = order(v_);                                                                                              \
+        FORM_LAUNCH(a, unit0, threads, walked, n_, o_, whole_pieces((a).dst, walk_of((a).dne, (a).dnb, unit0, dstep), dstep), KERNEL, __VA_ARGS__); \
     } while (0)
 #define ROWS_LAUNCH(a, unit0, threads, ...)                                                                               \
     do {                                                                                                                  \
@@ -630,30 +639,30 @@ static void launch_plain(const CpyArgs & a, hipStream_t stream) {
         if (b.n > 65536 && b.snb[0] == (int64_t)sizeof(TS) && narrow_copy(b, E, E * sizeof(TS), E * sizeof(TD), b.n, v))
             fattn_launch_head(cpy_vec_kernel_head<TS, TD>, dim3((unsigned)((b.n + 255) / 256)), dim3(256), 0, stream, head_first(v));
         else
-            CPY_LAUNCH(b, E, sizeof(TS), E * sizeof(TS), E * sizeof(TD), b.n, true, cpy_vec_kernel, TS, TD);
+            CPY_LAUNCH(b, E, sizeof(TS), E * sizeof(TS), E * sizeof(TD), b.n, true, head_first, cpy_vec_kernel, TS, TD);
     } else {
-        CPY_LAUNCH(a, 1, sizeof(TS), sizeof(TS), sizeof(TD), a.n, false, cpy_scalar_kernel, TS, TD);
+        CPY_LAUNCH(a, 1, sizeof(TS), sizeof(TS), sizeof(TD), a.n, false, head_first, cpy_scalar_kernel, TS, TD);
     }
 }
 
 template <int T>
 static void launch_to_blocks(const CpyArgs & a, hipStream_t stream) {
     constexpr int U = FATTN_QK8_0, BB = BlockFormat<T>::BYTES;
-    if (rows_aligned(a.src, a.sne, a.snb, 4, 16)) CPY_LAUNCH(a, U, 4, U * 4, BB, a.n * 4, false, cpy_f32_block_kernel, T, true);
-    else                                          CPY_LAUNCH(a, U, 4, U * 4, BB, a.n * 4, false, cpy_f32_block_kernel, T, false);
+    if (rows_aligned(a.src, a.sne, a.snb, 4, 16)) CPY_LAUNCH(a, U, 4, U * 4, BB, a.n * 4, false, as_it_is, cpy_f32_block_kernel, T, true);
+    else                                          CPY_LAUNCH(a, U, 4, U * 4, BB, a.n * 4, false, as_it_is, cpy_f32_block_kernel, T, false);
 }
 
 template <int T>
 static void launch_from_blocks(const CpyArgs & a, hipStream_t stream) {
     constexpr int U = FATTN_QK8_0, BB = BlockFormat<T>::BYTES;
-    if (rows_aligned(a.dst, a.dne, a.dnb, 4, 16) && a.mirror % 16 == 0) CPY_LAUNCH(a, U, BB, BB, U * 4, a.n * 8, true, cpy_block_f32_kernel, T, true);
-    else                                                                CPY_LAUNCH(a, U, BB, BB, U * 4, a.n * 8, true, cpy_block_f32_kernel, T, false);
+    if (rows_aligned(a.dst, a.dne, a.dnb, 4, 16) && a.mirror % 16 == 0) CPY_LAUNCH(a, U, BB, BB, U * 4, a.n * 8, true, head_first, cpy_block_f32_kernel, T, true);
+    else                                                                CPY_LAUNCH(a, U, BB, BB, U * 4, a.n * 8, true, head_first, cpy_block_f32_kernel, T, false);
 }
 
 template <int T>
 static void launch_blocks(const CpyArgs & a, hipStream_t stream) {
     constexpr int U = FATTN_QK8_0, BB = BlockFormat<T>::BYTES;
-    CPY_LAUNCH(a, U, BB, BB, BB, a.n * (BB / 2), false, cpy_block_block_kernel, T);
+    CPY_LAUNCH(a, U, BB, BB, BB, a.n * (BB / 2), false, head_first, cpy_block_block_kernel, T);
 }
 
 int cpy_launch(const CpyArgs & a, int stype, int dtype, hipStream_t stream) {
