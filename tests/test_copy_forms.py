@@ -67,7 +67,7 @@ int main() {
         reshaped += memcmp(a.sne, a.dne, sizeof(a.sne)) != 0;
         if ((int64_t)v.n != a.n) return printf("units %u %lld\n", v.n, (long long)a.n), 1;
         v.whole = (uint32_t)pick(0, 2);
-        const NarrowCopy w = narrow_of(head_first(v));            // the order of a large copy's arguments
+        const NarrowCopy w = narrow_of(head_first(v));            // the order of the loads
         if (w.src != v.src || w.dst != v.dst || w.mirror != v.mirror || w.n != v.n || w.whole != v.whole || memcmp(w.div, v.div, sizeof(v.div)) ||
             memcmp(w.snb, v.snb, sizeof(v.snb)) || memcmp(w.dnb, v.dnb, sizeof(v.dnb)))
             return printf("copy %d: another order\n", t), 1;
